@@ -89,6 +89,24 @@ int grid_sys(const sop_engine *e) {
   return std::max(1, std::min(e->cur_nsys, 2048));
 }
 
+// k_rebuild: a block per system of up to SORT_N_MAX beads (two are resident
+// per compute unit)
+static int grid_rebuild(const sop_engine *e) {
+  if (e->fixed_grids) return 2 * e->num_cu;
+  return std::min(e->cur_nsys - e->cur_nbig, 2048);
+}
+
+// The larger systems' kernels: blocks of 2,048 beads of the largest one, and
+// one per system.  While serving, fixed grids whenever the batch has one.
+static int grid_big_beads(const sop_engine *e) {
+  if (e->cur_nbig == 0) return 0;
+  return e->fixed_grids ? e->num_cu : std::min((e->cur_big_max + 2047) / 2048, 4 * e->num_cu);
+}
+static int grid_big_sys(const sop_engine *e) {
+  if (e->cur_nbig == 0) return 0;
+  return e->fixed_grids ? e->num_cu : std::min(e->cur_nbig, 1024);
+}
+
 // Launch grid of a persistent item kernel: `g` blocks (a multiple of 8, so
 // that item k runs on XCD k mod 8), fewer when the batch has fewer items, none
 // when it has none; fixed grids (serving) always launch g.
@@ -137,7 +155,11 @@ StepGrids filter_grids(const sop_engine *e) {
 }
 
 ListGrids list_grids(const sop_engine *e) {
-  return ListGrids{grid_tiles(e), grid_sys(e), filter_grids(e)};
+  // two streams when several systems, some built from the grid and some from
+  // their shell rows, give the filter a quarter of the device's compute units
+  // or more
+  const bool split = e->cur_nsys > 1 && 4 * (e->cur_nfitems + e->cur_nfitems_big + e->cur_nfitems_far) > e->num_cu;
+  return ListGrids{grid_tiles(e), grid_rebuild(e), grid_big_beads(e), grid_big_sys(e), split, filter_grids(e)};
 }
 
 } // namespace sopk
@@ -249,8 +271,6 @@ static sop_status ensure_capacity(sop_engine *e, int64_t beads, int64_t nat, int
     s = grow_array(e, (void **)&e->p.sysout, 8 * SYSOUT_N * (size_t)c.slots, 8 * SYSOUT_N * (size_t)nn);
     if (s) return s;
     s = grow_array(e, (void **)&e->p.syslist, 4 * (size_t)c.slots, 4 * (size_t)nn);
-    if (s) return s;
-    s = grow_array(e, (void **)&e->p.cellwork, 4 * (size_t)(c.slots + 1), 4 * (size_t)(nn + 1));
     if (s) return s;
     c.slots = nn;
     e->sys.resize((size_t)nn);
@@ -635,6 +655,7 @@ sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, in
   h.shell = engine_shell_for(e, n);
   shell_fields(P, h.shell, S);
   S.build = BUILD_NONE;
+  for (int k = 0; k < 8; ++k) S.acc[k] = k < 3 ? ACC_MIN : ACC_MAX;
   S.nl_valid = 0;
   int tmask = 0;
   for (int i = 0; i < n; ++i) tmask |= 1 << (type[i] - 1);
@@ -1050,7 +1071,13 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   e->cur_lds_big = sp.lds_big;
   e->cur_flds = fp.lds;
   e->cur_flds_big = fp.lds_big;
+  // the systems too large for one block's rebuild first
   e->h_syslist.assign(slots, slots + nslots);
+  const auto big_end = std::stable_partition(e->h_syslist.begin(), e->h_syslist.end(),
+                                             [&](int32_t s) { return e->sys[s].n > SORT_N_MAX; });
+  const int32_t nbig = (int32_t)(big_end - e->h_syslist.begin());
+  e->cur_big_max = 0;
+  for (int32_t q = 0; q < nbig; ++q) e->cur_big_max = std::max(e->cur_big_max, e->sys[e->h_syslist[q]].n);
   if ((int64_t)e->h_work.size() + 2 > e->work_cap) {
     HIPCK(hipStreamSynchronize(e->stream));
     int64_t nc = std::max<int64_t>(1024, (int64_t)e->h_work.size() * 2 + 2);
@@ -1062,9 +1089,9 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   if (!e->p.nwork) {
     HIPCK(hipMalloc((void **)&e->p.nwork, 256));
     e->p.nsys = e->p.nwork + 16;
+    e->p.nbig = e->p.nwork + 24;
     e->p.ncellwork = e->p.nwork + 32;
     e->p.nlbuild = e->p.nwork + 40;
-    e->p.gsort = e->p.nwork + 41;
     e->p.nfitems = e->p.nwork + 44;
     e->p.nfitems_big = e->p.nwork + 45;
     e->p.nfitems_far = e->p.nwork + 46;
@@ -1097,11 +1124,13 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   if (ni > 0) HIPCK(hipMemcpy(e->p.items, e->h_items.data(), sizeof(int4) * (size_t)ni, hipMemcpyHostToDevice));
   if (nfi > 0) HIPCK(hipMemcpy(e->p.fitems, e->h_fitems.data(), sizeof(int4) * (size_t)nfi, hipMemcpyHostToDevice));
   // the counters in one copy: nwork[0] = work entries, [16] batch systems,
-  // [44..46] filter items, [48] / [56] / [60] step items (LDS / far / whole-CU)
-  int32_t cnt[64];
-  HIPCK(hipMemcpy(cnt, e->p.nwork, sizeof(cnt), hipMemcpyDeviceToHost));
+  // [24] large ones, [32] home cells and [40] neighbor-list builds of a rebuild
+  // (none between rebuilds), [44..46] filter items, [48] / [56] / [60] step
+  // items (LDS / far / whole-CU)
+  int32_t cnt[64] = {0};
   cnt[0] = nw;
   cnt[16] = ns;
+  cnt[24] = nbig;
   cnt[44] = fp.n_lds;
   cnt[45] = fp.n_big;
   cnt[46] = fp.n_far;
@@ -1111,6 +1140,7 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   HIPCK(hipMemcpy(e->p.nwork, cnt, sizeof(cnt), hipMemcpyHostToDevice));
   e->cur_nwork = nw;
   e->cur_nsys = ns;
+  e->cur_nbig = nbig;
   e->cur_nitems = sp.n_lds;
   e->cur_nitems_far = sp.n_far;
   e->cur_nitems_big = sp.n_big;
@@ -1147,10 +1177,10 @@ sop_status engine_check_errors(sop_engine *e, const int32_t *slots, int32_t nslo
 static std::string graph_key(const sop_engine *e, int G, int n_nl, int n_pl) {
   std::ostringstream os;
   os << G << '|' << n_nl << '|' << n_pl << '|' << e->opts.lanes_per_bead << '|' << grid_tiles(e) << '|'
-     << grid_sys(e) << '|' << grid_items(e) << '|' << grid_items_big(e) << '|' << grid_items_far(e) << '|'
+     << grid_rebuild(e) << '|' << grid_big_beads(e) << '|' << grid_big_sys(e) << '|' << grid_items(e) << '|' << grid_items_big(e) << '|' << grid_items_far(e) << '|'
      << e->cur_lds << '|' << e->cur_lds_big;
   const StepGrids fg = filter_grids(e);
-  os << '|' << fg.grid << '|' << fg.grid_big << '|' << fg.grid_far << '|' << fg.lds << '|' << fg.lds_big;
+  os << '|' << list_grids(e).split << '|' << fg.grid << '|' << fg.grid_big << '|' << fg.grid_far << '|' << fg.lds << '|' << fg.lds_big;
   return os.str();
 }
 
@@ -1445,7 +1475,7 @@ void sop_engine_destroy(sop_engine *e) {
   for (auto &a : e->nat_arrays) if (*a.first) note(hipFree(*a.first), "hipFree(native pool)");
   for (auto &a : e->cell_arrays) if (*a.first) note(hipFree(*a.first), "hipFree(cell pool)");
   void *others[] = {e->p.nlrep_j, e->p.plrep_j, e->p.slrep_j,  e->p.tile_sys, e->p.sys,  e->p.sysout,
-                    e->p.syslist, e->p.work,    e->p.nwork,    e->p.cellwork, e->p.items};
+                    e->p.syslist, e->p.work,    e->p.nwork,    e->p.items};
   for (void *q : others) if (q) note(hipFree(q), "hipFree");
   if (e->fork.side) note(hipStreamSynchronize(e->fork.side), "hipStreamSynchronize");
   if (e->fork.fork) note(hipEventDestroy(e->fork.fork), "hipEventDestroy");

@@ -96,6 +96,7 @@ struct sop_engine {
   std::vector<int32_t> h_work, h_syslist;
   std::vector<int4> h_items, h_fitems;
   int64_t work_cap = 0, syslist_cap = 0, items_cap = 0, fitems_cap = 0;
+  int32_t cur_nbig = 0, cur_big_max = 0;  // systems of more than SORT_N_MAX beads, and the largest one's beads
   int32_t cur_nwork = 0, cur_nsys = 0, cur_nitems = 0, cur_nitems_big = 0, cur_nitems_far = 0;
   int32_t cur_nfitems = 0, cur_nfitems_big = 0, cur_nfitems_far = 0;  // shell-filter items
   size_t cur_lds = 0;     // dynamic LDS of the step kernel for the current batch

@@ -1,7 +1,7 @@
 // kernels.hip -- gfx950 kernels of the SOP overdamped hot path.
 //
-//   k_bbox / k_cell_count / k_cell_scan / k_cell_scatter / k_cell_rank /
-//   k_pl_cells / k_nl_build / k_shell_filter   list rebuilds: per-system open
+//   k_rebuild (k_big_skin / k_big_plan / k_cell_* for systems too large for
+//   one block) / k_rows / k_shell_filter   list rebuilds: per-system open
 //                cell grid, counting sort of beads into cells (histogram, DPP
 //                wave scan, scatter, deterministic in-cell ranking), 27-cell
 //                stencil with the exact FP32 predicates and ballot/mbcnt wave
@@ -179,7 +179,8 @@ __device__ __forceinline__ bool due_pl(const SysDev &S, int kstep) {
   return live(S, kstep) && ((S.step + kstep) % S.n_pl) == 0;
 }
 
-__device__ __forceinline__ int cell_index(const SysDev &S, float4 x) {
+template <typename G>
+__device__ __forceinline__ int cell_index(const G &S, float4 x) {
   int cx = (int)floorf((x.x - S.org[0]) * S.inv_edge[0]);
   int cy = (int)floorf((x.y - S.org[1]) * S.inv_edge[1]);
   int cz = (int)floorf((x.z - S.org[2]) * S.inv_edge[2]);
@@ -217,118 +218,209 @@ __device__ __forceinline__ const float4 *build_src(const DevPtrs &p, const SysDe
   return S.build == BUILD_DIRECT ? buf_in(p, S.parity + kstep) : p.pos_ref;
 }
 
-// Per system: snapshot and build decision.
-constexpr int SKIN_THREADS = 1024;
-__global__ __launch_bounds__(SKIN_THREADS) void k_skin(DevPtrs p, int kstep, int flags) {
-  constexpr int NW = SKIN_THREADS / 64;
-  __shared__ float red[2][NW];
-  __shared__ int s_build;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nsys = *p.nsys;
-  if (blockIdx.x == 0 && tid == 0) *p.gsort = 0;  // k_bbox raises it (first kernel of a rebuild)
-  for (int q = blockIdx.x; q < nsys; q += gridDim.x) {
-    const int s = p.syslist[q];
-    SysDev &S = p.sys[s];
-    const bool mat = (flags & MATERIALIZE_NL) != 0;
-    const bool nl = !mat && ((flags & FORCE_NL) || due_nl(S, kstep));
-    const bool pl = !mat && ((flags & FORCE_PL) || due_pl(S, kstep));
-    // system constants in registers (the snapshot stores below may alias S)
-    const int bo = S.bead_off, n = S.n;
-    const float4 *x = buf_in(p, S.parity + kstep);
-    const bool shell_chk = pl && S.sl_valid;
-    float d2max = 0.0f, d2sh = 0.0f;
-    if (nl || pl) {
-      // four beads per pass with no branch on the bead count, so the loads of
-      // a pass issue together (a bead past the end repeats the last one:
-      // the same snapshot store, the same displacement)
-      for (int b0 = tid; b0 < n; b0 += 4 * SKIN_THREADS) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int i = bo + min(b0 + u * SKIN_THREADS, n - 1);
-          const float4 xi = x[i];
-          if (nl) {
-            p.pos_ref[i] = xi;
-          } else {
-            const float4 r = p.pos_ref[i];
-            const float dx = xi.x - r.x, dy = xi.y - r.y, dz = xi.z - r.z;
-            d2max = fmaxf(d2max, dx * dx + dy * dy + dz * dz);
-          }
-          if (shell_chk) {
-            const float4 q = p.pos_shell[i];
-            const float ex = xi.x - q.x, ey = xi.y - q.y, ez = xi.z - q.z;
-            d2sh = fmaxf(d2sh, ex * ex + ey * ey + ez * ez);
-          }
-        }
-      }
+// A rebuild's decision for one system, from the largest displacements since
+// the two snapshots (one thread).  Returns S.build.
+__device__ __forceinline__ int decide_build(SysDev &S, int flags, bool nl, bool pl, bool shell_chk, float d2max,
+                                            float d2sh) {
+  const float dmax = sqrtf(d2max), dsh = sqrtf(d2sh);
+  int build = BUILD_NONE;
+  if (flags & MATERIALIZE_NL) {
+    build = S.nl_valid ? BUILD_NONE : BUILD_NL_ONLY;
+  } else {
+    if (nl) S.nl_valid = 0;
+    if (pl) {
+      if (S.skin > 0.0f && (nl || 2.0f * dmax < S.skin))
+        build = shell_chk && 2.0f * dsh < S.shell_ok ? BUILD_SHELL : BUILD_DIRECT;
+      else
+        build = BUILD_NL;
+    } else if (flags & FORCE_NL) {
+      build = BUILD_NL_ONLY;
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      d2max = fmaxf(d2max, __shfl_xor(d2max, o));
-      d2sh = fmaxf(d2sh, __shfl_xor(d2sh, o));
+  }
+  S.build = build;
+  if (build == BUILD_DIRECT) S.sl_valid = 1;
+  if (build == BUILD_NL) S.sl_valid = 0;  // k_rows writes its rows into the shell-row slots
+  if (build == BUILD_DIRECT || build == BUILD_SHELL || build == BUILD_NL)
+    ++S.nbuild[build == BUILD_DIRECT ? 0 : (build == BUILD_SHELL ? 1 : 2)];
+  return build;
+}
+
+// Cell grid of one axis range [a, b]: cells of the minimum edge, one more
+// than fit in the extent so the grid covers it; when that exceeds dmax, dmax
+// cells stretched over the extent (edge ext/dmax >= min_edge).  Stretching
+// every cell to ext/floor(ext/min_edge) instead would make the 27-cell
+// stencil up to 8x the volume it needs to be.
+__device__ __forceinline__ void plan_axis(float a, float b, float min_edge, int dmax, int &dims, float &inv) {
+  const float ext = b - a;
+  dims = 1;
+  inv = 0.0f;
+  if (ext > 0.0f) {
+    dims = (int)floorf(ext / min_edge) + 1;
+    if (dims <= dmax) {
+      inv = 1.0f / min_edge;
+    } else {
+      dims = dmax;
+      inv = (float)dims / ext;
     }
-    if (lane == 0) {
-      red[0][wave] = d2max;
-      red[1][wave] = d2sh;
-    }
-    __syncthreads();
-    if (tid == 0) {
-      float m0 = 0.0f, m1 = 0.0f;
-      for (int w = 0; w < NW; ++w) {
-        m0 = fmaxf(m0, red[0][w]);
-        m1 = fmaxf(m1, red[1][w]);
-      }
-      const float dmax = sqrtf(m0), dsh = sqrtf(m1);
-      int build = BUILD_NONE;
-      if (mat) {
-        build = S.nl_valid ? BUILD_NONE : BUILD_NL_ONLY;
-      } else {
-        if (nl) S.nl_valid = 0;
-        if (pl) {
-          if (S.skin > 0.0f && (nl || 2.0f * dmax < S.skin))
-            build = shell_chk && 2.0f * dsh < S.shell_ok ? BUILD_SHELL : BUILD_DIRECT;
-          else
-            build = BUILD_NL;
-        } else if (flags & FORCE_NL) {
-          build = BUILD_NL_ONLY;
-        }
-      }
-      S.build = build;
-      if (build == BUILD_DIRECT) S.sl_valid = 1;
-      if (build == BUILD_NL) S.sl_valid = 0;  // k_nl_build writes its rows into the shell-row slots
-      if (build == BUILD_DIRECT || build == BUILD_SHELL || build == BUILD_NL)
-        ++S.nbuild[build == BUILD_DIRECT ? 0 : (build == BUILD_SHELL ? 1 : 2)];
-      s_build = build;
-    }
-    __syncthreads();
-    if (s_build == BUILD_DIRECT)  // the shell rows about to be built belong to these coordinates
-      for (int b = tid; b < n; b += SKIN_THREADS) p.pos_shell[bo + b] = x[bo + b];
-    __syncthreads();
   }
 }
 
-// Per system: bounding box -> open cell grid; zero the cell histogram.
-__global__ __launch_bounds__(256) void k_bbox(DevPtrs p, int kstep) {
-  __shared__ float red[6][4];
-  __shared__ int s_ncells;
+// The cell grid of a rebuild (one thread), from the bounding box mn..mx of
+// the coordinates it sorts; a box too close to half the periodic box is
+// refused (ERR_PBC).
+struct CellGrid {
+  float org[3], inv_edge[3];
+  int dims[3];
+};
+__device__ __forceinline__ int plan_grid(SysDev &S, const float *mn, const float *mx, CellGrid &g) {
+  const float min_edge = S.build == BUILD_DIRECT ? S.cell_min_edge_sl : S.cell_min_edge;
+  const int dmax = S.dmax;
+  float ext_max = 0.0f;
+  int nc = 1;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    plan_axis(mn[d], mx[d], min_edge, dmax, g.dims[d], g.inv_edge[d]);
+    g.org[d] = mn[d];
+    nc *= g.dims[d];
+    ext_max = fmaxf(ext_max, mx[d] - mn[d]);
+    S.org[d] = g.org[d];
+    S.inv_edge[d] = g.inv_edge[d];
+    S.dims[d] = g.dims[d];
+  }
+  S.ncells = nc;
+  int ok = 1;
+  if (S.boxl > 0.0f) {
+    ok = ext_max < 0.5f * S.boxl - S.wrap_margin;
+    if (!ok) {
+      atomicOr(&S.err, ERR_PBC);
+      S.sl_valid = 0;
+    }
+  }
+  S.wrap_free = ok;
+  return nc;
+}
+
+// Rebuild of the systems whose cell sort fits one block's LDS (n <=
+// SORT_N_MAX; at most 2 n cells, so every such system), one 1024-thread block
+// per system.
+//   PH_DECIDE  neighbor-list snapshot, displacements, which build it is
+//   PH_GRID    for grid builds: bounding box, cell grid, the whole counting
+//              sort in LDS -- cell of each bead, histogram, exclusive scan,
+//              member lists, and the rank of each bead among its cell's
+//              members by index, so the in-cell order is the index order --
+//              the cell-ordered arrays, and the occupied cells appended to the
+//              batch's home-cell list (in any order: each writes its own rows)
+// What bounds it is latency: dependent round trips and block barriers of one
+// block.  Both phases in one launch (a system's beads are loaded once) when
+// the batch is small: the chain of eleven kernels it replaced, most of them
+// with nothing to do at most rebuilds, took 64 us per rebuild of one 128-bead
+// system (a rebuild and its step 107 us; now 48).  A batch that fills the device launches the phases apart, the
+// second on the side stream beside the shell builds' filter.
+constexpr int SORT_THREADS = 1024;
+constexpr int PH_DECIDE = 1, PH_GRID = 2;
+
+template <int PH>
+__global__ __launch_bounds__(SORT_THREADS) void k_rebuild(DevPtrs p, int kstep, int flags) {
+  constexpr int NW = SORT_THREADS / 64;
+  constexpr int SB = SORT_N_MAX / SORT_THREADS;  // beads per thread
+  __shared__ uint16_t s_cell[SORT_N_MAX];
+  __shared__ uint16_t s_mem[SORT_N_MAX];
+  __shared__ int s_cnt[SORT_C_MAX];  // counts, then end offsets
+  __shared__ float s_red[6][NW];
+  __shared__ int s_wsum[NW];
+  __shared__ CellGrid s_grid;
+  __shared__ int s_build, s_ncells, s_item0;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nsys = *p.nsys;
-  for (int q = blockIdx.x; q < nsys; q += gridDim.x) {
+  for (int q = *p.nbig + blockIdx.x; q < nsys; q += gridDim.x) {
     const int s = p.syslist[q];
     SysDev &S = p.sys[s];
-    if (!grid_build(S)) continue;
-    const float4 *src = build_src(p, S, kstep);
-    float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-    // four beads per pass with no branch on the count, so their loads overlap
-    // (a bead past the end repeats the last one; min and max are unchanged)
-    const int nb = S.n, bo = S.bead_off;
-    for (int b0 = tid; b0 < nb; b0 += 4 * (int)blockDim.x) {
+    // system constants in registers (the stores below may alias S)
+    const int bo = S.bead_off, n = S.n;
+    const float4 *x = buf_in(p, S.parity + kstep);
+    float4 xs[SB];
+    int build;
+    bool loaded = false;
+    if (PH & PH_DECIDE) {
+      const bool mat = (flags & MATERIALIZE_NL) != 0;
+      const bool nl = !mat && ((flags & FORCE_NL) || due_nl(S, kstep));
+      const bool pl = !mat && ((flags & FORCE_PL) || due_pl(S, kstep));
+      const bool shell_chk = pl && S.sl_valid;
+      float d2max = 0.0f, d2sh = 0.0f;
+      loaded = nl || pl;
+      if (loaded) {
+        // no branch on the bead count, so the loads issue together (a bead
+        // past the end repeats the last one: the same snapshot store, the
+        // same displacement)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float4 x = src[bo + min(b0 + u * (int)blockDim.x, nb - 1)];
-        mn[0] = fminf(mn[0], x.x); mx[0] = fmaxf(mx[0], x.x);
-        mn[1] = fminf(mn[1], x.y); mx[1] = fmaxf(mx[1], x.y);
-        mn[2] = fminf(mn[2], x.z); mx[2] = fmaxf(mx[2], x.z);
+        for (int u = 0; u < SB; ++u) xs[u] = x[bo + min(tid + u * SORT_THREADS, n - 1)];
+        if (nl) {
+#pragma unroll
+          for (int u = 0; u < SB; ++u)
+            if (u * SORT_THREADS < n) p.pos_ref[bo + min(tid + u * SORT_THREADS, n - 1)] = xs[u];
+        } else {
+#pragma unroll
+          for (int u = 0; u < SB; ++u) {
+            const float4 r = p.pos_ref[bo + min(tid + u * SORT_THREADS, n - 1)];
+            const float dx = xs[u].x - r.x, dy = xs[u].y - r.y, dz = xs[u].z - r.z;
+            d2max = fmaxf(d2max, dx * dx + dy * dy + dz * dz);
+          }
+        }
+        if (shell_chk) {
+#pragma unroll
+          for (int u = 0; u < SB; ++u) {
+            const float4 r = p.pos_shell[bo + min(tid + u * SORT_THREADS, n - 1)];
+            const float ex = xs[u].x - r.x, ey = xs[u].y - r.y, ez = xs[u].z - r.z;
+            d2sh = fmaxf(d2sh, ex * ex + ey * ey + ez * ez);
+          }
+        }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) {
+          d2max = fmaxf(d2max, __shfl_xor(d2max, o));
+          d2sh = fmaxf(d2sh, __shfl_xor(d2sh, o));
+        }
       }
+      if (lane == 0) {
+        s_red[0][wave] = d2max;
+        s_red[1][wave] = d2sh;
+      }
+      __syncthreads();
+      if (tid == 0) {
+        float m0 = 0.0f, m1 = 0.0f;
+        for (int w = 0; w < NW; ++w) {
+          m0 = fmaxf(m0, s_red[0][w]);
+          m1 = fmaxf(m1, s_red[1][w]);
+        }
+        s_build = decide_build(S, flags, nl, pl, shell_chk, m0, m1);
+        if (s_build == BUILD_NL || s_build == BUILD_NL_ONLY) atomicOr(p.nlbuild, 1);
+      }
+      __syncthreads();
+      build = s_build;
+      if (build == BUILD_DIRECT) {  // the shell rows about to be built belong to these coordinates
+#pragma unroll
+        for (int u = 0; u < SB; ++u)
+          if (u * SORT_THREADS < n) p.pos_shell[bo + min(tid + u * SORT_THREADS, n - 1)] = xs[u];
+      }
+    } else {
+      build = S.build;
+    }
+    if ((PH & PH_GRID) == 0 || build == BUILD_NONE || build == BUILD_SHELL) {
+      __syncthreads();  // the decision has been read before the next system's
+      continue;
+    }
+    // ---- cell grid and counting sort
+    const int cb = S.cell_base;
+    if (!loaded || build != BUILD_DIRECT) {
+      const float4 *src = build == BUILD_DIRECT ? x : p.pos_ref;
+#pragma unroll
+      for (int u = 0; u < SB; ++u) xs[u] = src[bo + min(tid + u * SORT_THREADS, n - 1)];
+    }
+    float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+    for (int u = 0; u < SB; ++u) {
+      mn[0] = fminf(mn[0], xs[u].x); mx[0] = fmaxf(mx[0], xs[u].x);
+      mn[1] = fminf(mn[1], xs[u].y); mx[1] = fmaxf(mx[1], xs[u].y);
+      mn[2] = fminf(mn[2], xs[u].z); mx[2] = fmaxf(mx[2], xs[u].z);
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
@@ -340,136 +432,321 @@ __global__ __launch_bounds__(256) void k_bbox(DevPtrs p, int kstep) {
     }
     if (lane == 0) {
 #pragma unroll
-      for (int d = 0; d < 3; ++d) { red[d][wave] = mn[d]; red[3 + d][wave] = mx[d]; }
+      for (int d = 0; d < 3; ++d) { s_red[d][wave] = mn[d]; s_red[3 + d][wave] = mx[d]; }
     }
     __syncthreads();
     if (tid == 0) {
-      const float min_edge = S.build == BUILD_DIRECT ? S.cell_min_edge_sl : S.cell_min_edge;
-      float ext_max = 0.0f;
-      int nc = 1;
-      for (int d = 0; d < 3; ++d) {
-        float a = red[d][0], b = red[3 + d][0];
-        for (int w = 1; w < (int)(blockDim.x >> 6); ++w) { a = fminf(a, red[d][w]); b = fmaxf(b, red[3 + d][w]); }
-        const float ext = b - a;
-        // Cells of the minimum edge, one more than fit in the extent so the
-        // grid covers it; when that exceeds dmax, dmax cells stretched over
-        // the extent (edge ext/dmax >= min_edge).  Stretching every cell to
-        // ext/floor(ext/min_edge) instead would make the 27-cell stencil up
-        // to 8x the volume it needs to be.
-        int dims = 1;
-        float inv = 0.0f;
-        if (ext > 0.0f) {
-          dims = (int)floorf(ext / min_edge) + 1;
-          if (dims <= S.dmax) {
-            inv = 1.0f / min_edge;
-          } else {
-            dims = S.dmax;
-            inv = (float)dims / ext;
-          }
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+        for (int w = 1; w < NW; ++w) {
+          mn[d] = fminf(mn[d], s_red[d][w]);
+          mx[d] = fmaxf(mx[d], s_red[3 + d][w]);
         }
-        S.org[d] = a;
-        S.inv_edge[d] = inv;
-        S.dims[d] = dims;
-        nc *= dims;
-        ext_max = fmaxf(ext_max, ext);
-      }
-      S.ncells = nc;
-      S.sort_lds = S.n <= SORT_N_MAX && nc <= SORT_C_MAX;
-      if (!S.sort_lds) atomicOr(p.gsort, 1);
-      if (S.boxl > 0.0f) {
-        const int ok = ext_max < 0.5f * S.boxl - S.wrap_margin;
-        S.wrap_free = ok;
-        if (!ok) {
-          atomicOr(&S.err, ERR_PBC);
-          S.sl_valid = 0;
-        }
-      } else {
-        S.wrap_free = 1;
-      }
-      s_ncells = nc;
+      s_ncells = plan_grid(S, mn, mx, s_grid);
     }
     __syncthreads();
     const int nc = s_ncells;
-    for (int c = tid; c < nc; c += blockDim.x) p.cell_cnt[S.cell_base + c] = 0;
+    for (int c = tid; c < nc; c += SORT_THREADS) s_cnt[c] = 0;
+    int cs[SB];
+#pragma unroll
+    for (int u = 0; u < SB; ++u) cs[u] = cell_index(s_grid, xs[u]);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < SB; ++u) {
+      const int b = tid + u * SORT_THREADS;
+      if (b < n) {
+        s_cell[b] = (uint16_t)cs[u];
+        p.cell_of[bo + b] = cs[u];
+        atomicAdd(&s_cnt[cs[u]], 1);
+      }
+    }
+    __syncthreads();
+    // exclusive scan of the counts, `per` consecutive cells per thread, with
+    // the occupied cells counted in the upper half (beads <= 5120, occupied
+    // cells <= beads: both fit 16 bits)
+    const int per = (nc + SORT_THREADS - 1) / SORT_THREADS;
+    int sum = 0;
+    for (int u = 0; u < per; ++u) {
+      const int c = tid * per + u;
+      const int v = c < nc ? s_cnt[c] : 0;
+      sum += v + (v > 0 ? 0x10000 : 0);
+    }
+    const int incl = wave_incl_scan(sum);
+    if (lane == 63) s_wsum[wave] = incl;
+    __syncthreads();
+    int off = 0, tot = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      off += w < wave ? s_wsum[w] : 0;
+      tot += s_wsum[w];
+    }
+    if (tid == 0) {
+      p.cell_start[cb + nc] = n;
+      S.ncells_used = tot >> 16;
+      s_item0 = build == BUILD_DIRECT ? atomicAdd(p.ncellwork, tot >> 16) : 0;
+    }
+    __syncthreads();
+    const int item0 = s_item0;
+    int run = off + incl - sum;
+    for (int u = 0; u < per; ++u) {
+      const int c = tid * per + u;
+      if (c >= nc) break;
+      const int v = s_cnt[c];
+      p.cell_start[cb + c] = run & 0xFFFF;
+      s_cnt[c] = run & 0xFFFF;  // cursor, ends at the cell's end offset
+      if (v > 0 && build == BUILD_DIRECT) p.cellitems[item0 + (run >> 16)] = make_int2(q, c);
+      run += v + (v > 0 ? 0x10000 : 0);
+    }
+    __syncthreads();
+    for (int b = tid; b < n; b += SORT_THREADS) s_mem[atomicAdd(&s_cnt[s_cell[b]], 1)] = (uint16_t)b;
+    // the loads of the output pass before its stores (a load issued after a
+    // store would wait for it)
+    int ns[SB], nn[SB];
+#pragma unroll
+    for (int u = 0; u < SB; ++u) {
+      const int i = bo + min(tid + u * SORT_THREADS, n - 1);
+      ns[u] = p.nat_start[i];
+      nn[u] = p.nat_cnt[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < SB; ++u) {
+      const int b = tid + u * SORT_THREADS;
+      if (b < n) {
+        const int c = s_cell[b];
+        const int st = c > 0 ? s_cnt[c - 1] : 0, en = s_cnt[c];
+        int r = 0;
+        for (int m = st; m < en; ++m) r += (int)s_mem[m] < b;
+        const int pos = st + r;
+        const int i = bo + b;
+        p.cell_pos[i] = pos;
+        p.cell_sorted[bo + pos] = i;
+        p.pos_sorted[bo + pos] = xs[u];
+        p.nat_sorted[bo + pos] = make_int2(ns[u], nn[u]);
+      }
+    }
     __syncthreads();
   }
 }
 
-// Per bead: cell id and histogram.
-__global__ __launch_bounds__(64) void k_cell_count(DevPtrs p, int kstep) {
-  if (*p.gsort == 0) return;  // every grid build of the batch sorts in LDS (k_bbox)
-  const int nwork = *p.nwork;
-  for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
-    const int t = p.work[w];
-    if (t < 0) continue;
-    const SysDev &S = p.sys[p.tile_sys[t]];
-    if (!grid_build(S) || S.sort_lds) continue;
-    const int i = t * TILE + threadIdx.x;
-    if (i < S.bead_off + S.n) {
-      const int c = cell_index(S, build_src(p, S, kstep)[i]);
-      p.cell_of[i] = c;
-      atomicAdd(&p.cell_cnt[S.cell_base + c], 1);
+// ---- systems of more than SORT_N_MAX beads (the first *nbig of the batch),
+// each spread over the whole launch: a 500,000-bead system's decision in one
+// block took longer than its step.
+
+// Order-preserving unsigned image of a float, for atomic minima and maxima.
+__device__ __forceinline__ uint32_t ord_u(float f) {
+  const uint32_t b = __float_as_uint(f);
+  return b ^ ((b >> 31) ? 0xFFFFFFFFu : 0x80000000u);
+}
+__device__ __forceinline__ float ord_f(uint32_t u) {
+  return __uint_as_float(u ^ ((u >> 31) ? 0x80000000u : 0xFFFFFFFFu));
+}
+
+// Snapshot, displacements and bounding box of the coordinates: partial maxima
+// of 2,048 beads per block into the system's accumulators (8 atomics a block).
+constexpr int BIG_THREADS = 512;
+__global__ __launch_bounds__(BIG_THREADS) void k_big_skin(DevPtrs p, int kstep, int flags) {
+  constexpr int NW = BIG_THREADS / 64, U = 4;
+  __shared__ float s_red[8][NW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nbig = *p.nbig;
+  for (int q = 0; q < nbig; ++q) {
+    SysDev &S = p.sys[p.syslist[q]];
+    const bool mat = (flags & MATERIALIZE_NL) != 0;
+    const bool nl = !mat && ((flags & FORCE_NL) || due_nl(S, kstep));
+    const bool pl = !mat && ((flags & FORCE_PL) || due_pl(S, kstep));
+    if (!nl && !pl) continue;
+    const int bo = S.bead_off, n = S.n;
+    const float4 *x = buf_in(p, S.parity + kstep);
+    const bool shell_chk = pl && S.sl_valid;
+    float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[5] = {-INFINITY, -INFINITY, -INFINITY, 0.0f, 0.0f};
+    bool any = false;
+    for (int b0 = blockIdx.x * U * BIG_THREADS; b0 < n; b0 += gridDim.x * U * BIG_THREADS) {
+      any = true;
+      float4 xi[U], r[U], sh[U];
+      int i[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        i[u] = bo + min(b0 + tid + u * BIG_THREADS, n - 1);  // past the end: the last bead again
+        xi[u] = x[i[u]];
+        r[u] = nl ? xi[u] : p.pos_ref[i[u]];
+        sh[u] = shell_chk ? p.pos_shell[i[u]] : xi[u];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (nl) p.pos_ref[i[u]] = xi[u];
+        const float dx = xi[u].x - r[u].x, dy = xi[u].y - r[u].y, dz = xi[u].z - r[u].z;
+        mx[3] = fmaxf(mx[3], dx * dx + dy * dy + dz * dz);
+        const float ex = xi[u].x - sh[u].x, ey = xi[u].y - sh[u].y, ez = xi[u].z - sh[u].z;
+        mx[4] = fmaxf(mx[4], ex * ex + ey * ey + ez * ez);
+        mn[0] = fminf(mn[0], xi[u].x); mx[0] = fmaxf(mx[0], xi[u].x);
+        mn[1] = fminf(mn[1], xi[u].y); mx[1] = fmaxf(mx[1], xi[u].y);
+        mn[2] = fminf(mn[2], xi[u].z); mx[2] = fmaxf(mx[2], xi[u].z);
+      }
+    }
+    if (!any) continue;  // the same for the whole block
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) mn[d] = fminf(mn[d], __shfl_xor(mn[d], o));
+#pragma unroll
+      for (int d = 0; d < 5; ++d) mx[d] = fmaxf(mx[d], __shfl_xor(mx[d], o));
+    }
+    __syncthreads();  // the previous system's partials have been read
+    if (lane == 0) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) s_red[d][wave] = mn[d];
+#pragma unroll
+      for (int d = 0; d < 5; ++d) s_red[3 + d][wave] = mx[d];
+    }
+    __syncthreads();
+    if (tid < 8) {
+      float v = s_red[tid][0];
+      for (int w = 1; w < NW; ++w) v = tid < 3 ? fminf(v, s_red[tid][w]) : fmaxf(v, s_red[tid][w]);
+      if (tid < 3) atomicMin(&S.acc[tid], ord_u(v));
+      else atomicMax(&S.acc[tid], ord_u(v));
     }
   }
 }
 
-// Per system: exclusive scan of the histogram (DPP wave scan + wave totals).
-__global__ __launch_bounds__(256) void k_cell_scan(DevPtrs p) {
-  if (*p.gsort == 0) return;  // every grid build of the batch sorts in LDS (k_bbox)
-  __shared__ int wsum[4], wused[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nsys = *p.nsys;
-  for (int q = blockIdx.x; q < nsys; q += gridDim.x) {
-    const int s = p.syslist[q];
-    SysDev &S = p.sys[s];
-    if (!grid_build(S) || S.sort_lds) continue;
-    const int nc = S.ncells, cb = S.cell_base;
-    int carry = 0, used = 0;
-    for (int c0 = 0; c0 < nc; c0 += 256) {
-      const int c = c0 + tid;
-      const int v = c < nc ? p.cell_cnt[cb + c] : 0;
-      const int incl = wave_incl_scan(v);
-      if (lane == 63) wsum[wave] = incl;
-      const int wu = __popcll(__ballot(v > 0));
-      if (lane == 0) wused[wave] = wu;
-      __syncthreads();
-      int off = 0, tot = 0;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        off += (w < wave) ? wsum[w] : 0;
-        tot += wsum[w];
+// Per big system: decision, cell grid, cleared histogram; the accumulators
+// go back to their empty values for the next rebuild.
+__global__ __launch_bounds__(1024) void k_big_plan(DevPtrs p, int kstep, int flags) {
+  __shared__ int s_nc;
+  const int tid = threadIdx.x;
+  const int nbig = *p.nbig;
+  for (int q = blockIdx.x; q < nbig; q += gridDim.x) {
+    SysDev &S = p.sys[p.syslist[q]];
+    if (tid == 0) {
+      const bool mat = (flags & MATERIALIZE_NL) != 0;
+      const bool nl = !mat && ((flags & FORCE_NL) || due_nl(S, kstep));
+      const bool pl = !mat && ((flags & FORCE_PL) || due_pl(S, kstep));
+      float mn[3], mx[3];
+      for (int d = 0; d < 3; ++d) {
+        mn[d] = ord_f(S.acc[d]);
+        mx[d] = ord_f(S.acc[3 + d]);
       }
-      if (c < nc) {
-        p.cell_start[cb + c] = carry + off + incl - v;
-        p.cell_cursor[cb + c] = 0;
+      const float d2max = nl || pl ? ord_f(S.acc[6]) : 0.0f, d2sh = nl || pl ? ord_f(S.acc[7]) : 0.0f;
+      for (int d = 0; d < 8; ++d) S.acc[d] = d < 3 ? ACC_MIN : ACC_MAX;
+      if (nl)  // the snapshot is these coordinates
+        for (int d = 0; d < 3; ++d) {
+          S.ref_box[d] = mn[d];
+          S.ref_box[3 + d] = mx[d];
+        }
+      const int build = decide_build(S, flags, nl, pl, pl && S.sl_valid, d2max, d2sh);
+      int nc = 0;
+      if (build != BUILD_NONE && build != BUILD_SHELL) {
+        if (build != BUILD_DIRECT)  // sorted at the snapshot
+          for (int d = 0; d < 3; ++d) {
+            mn[d] = S.ref_box[d];
+            mx[d] = S.ref_box[3 + d];
+          }
+        CellGrid g;
+        nc = plan_grid(S, mn, mx, g);
+      }
+      if (build == BUILD_NL || build == BUILD_NL_ONLY) atomicOr(p.nlbuild, 1);
+      s_nc = nc;
+    }
+    __syncthreads();
+    const int nc = s_nc, cb = S.cell_base;
+    for (int c = tid; c < nc; c += blockDim.x) p.cell_cnt[cb + c] = 0;
+    __syncthreads();
+  }
+}
+
+// Per bead: cell id and histogram; the shell snapshot of a direct build.
+__global__ __launch_bounds__(256) void k_cell_count(DevPtrs p, int kstep) {
+  const int nbig = *p.nbig;
+  for (int q = 0; q < nbig; ++q) {
+    const SysDev &S = p.sys[p.syslist[q]];
+    if (!grid_build(S)) continue;
+    const float4 *src = build_src(p, S, kstep);
+    const bool direct = S.build == BUILD_DIRECT;
+    const int bo = S.bead_off, n = S.n, cb = S.cell_base;
+    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < n; b += gridDim.x * blockDim.x) {
+      const float4 x = src[bo + b];
+      const int c = cell_index(S, x);
+      p.cell_of[bo + b] = c;
+      if (direct) p.pos_shell[bo + b] = x;
+      atomicAdd(&p.cell_cnt[cb + c], 1);
+    }
+  }
+}
+
+// Per big system: exclusive scan of the histogram (DPP wave scan + wave
+// totals), 4 consecutive cells per thread, and its occupied cells appended to
+// the batch's home-cell list.
+__global__ __launch_bounds__(1024) void k_cell_scan(DevPtrs p) {
+  constexpr int NW = 16, PER = 4;
+  __shared__ int wsum[NW], wused[NW], s_item0;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nbig = *p.nbig;
+  for (int q = blockIdx.x; q < nbig; q += gridDim.x) {
+    SysDev &S = p.sys[p.syslist[q]];
+    if (!grid_build(S)) continue;
+    const int nc = S.ncells, cb = S.cell_base, n = S.n;
+    const bool direct = S.build == BUILD_DIRECT;
+    int carry = 0, used = 0;
+    for (int c0 = 0; c0 < nc; c0 += 1024 * PER) {
+      int v[PER], sum = 0, u = 0;
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int c = c0 + tid * PER + k;
+        v[k] = c < nc ? p.cell_cnt[cb + c] : 0;
+        sum += v[k];
+        u += v[k] > 0;
+      }
+      const int incl = wave_incl_scan(sum), iused = wave_incl_scan(u);
+      if (lane == 63) {
+        wsum[wave] = incl;
+        wused[wave] = iused;
+      }
+      __syncthreads();
+      int off = 0, tot = 0, uoff = 0, utot = 0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        off += w < wave ? wsum[w] : 0;
+        tot += wsum[w];
+        uoff += w < wave ? wused[w] : 0;
+        utot += wused[w];
+      }
+      if (tid == 0) s_item0 = direct ? atomicAdd(p.ncellwork, utot) : 0;
+      __syncthreads();
+      int run = carry + off + incl - sum, it = s_item0 + uoff + iused - u;
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int c = c0 + tid * PER + k;
+        if (c < nc) {
+          p.cell_start[cb + c] = run;
+          p.cell_cursor[cb + c] = 0;
+          if (direct && v[k] > 0) p.cellitems[it++] = make_int2(q, c);
+        }
+        run += v[k];
       }
       carry += tot;
-      used += wused[0] + wused[1] + wused[2] + wused[3];
+      used += utot;
       __syncthreads();
     }
     if (tid == 0) {
       S.ncells_used = used;
       p.cell_start[cb + nc] = carry;
-      if (carry != S.n) atomicOr(&S.err, ERR_INTERNAL);
+      if (carry != n) atomicOr(&S.err, ERR_INTERNAL);
     }
   }
 }
 
 // Per bead: scatter into its cell's segment (arbitrary in-cell order).
-__global__ __launch_bounds__(64) void k_cell_scatter(DevPtrs p) {
-  if (*p.gsort == 0) return;  // every grid build of the batch sorts in LDS (k_bbox)
-  const int nwork = *p.nwork;
-  for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
-    const int t = p.work[w];
-    if (t < 0) continue;
-    const SysDev &S = p.sys[p.tile_sys[t]];
-    if (!grid_build(S) || S.sort_lds) continue;
-    const int i = t * TILE + threadIdx.x;
-    if (i < S.bead_off + S.n) {
-      const int c = p.cell_of[i];
-      const int slot = atomicAdd(&p.cell_cursor[S.cell_base + c], 1);
-      const int pos = p.cell_start[S.cell_base + c] + slot;
-      if (pos >= 0 && pos < S.n) p.cell_tmp[S.bead_off + pos] = i;
+__global__ __launch_bounds__(256) void k_cell_scatter(DevPtrs p) {
+  const int nbig = *p.nbig;
+  for (int q = 0; q < nbig; ++q) {
+    const SysDev &S = p.sys[p.syslist[q]];
+    if (!grid_build(S)) continue;
+    const int bo = S.bead_off, n = S.n, cb = S.cell_base;
+    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < n; b += gridDim.x * blockDim.x) {
+      const int c = p.cell_of[bo + b];
+      const int slot = atomicAdd(&p.cell_cursor[cb + c], 1);
+      const int pos = p.cell_start[cb + c] + slot;
+      if (pos >= 0 && pos < n) p.cell_tmp[bo + pos] = bo + b;
     }
   }
 }
@@ -477,27 +754,26 @@ __global__ __launch_bounds__(64) void k_cell_scatter(DevPtrs p) {
 // Per bead: rank among the beads of its cell by index -> sorted segment, with
 // a cell-ordered copy of the coordinates.  The in-cell order, and with it every
 // list, is independent of the order of the atomics above.
-__global__ __launch_bounds__(64) void k_cell_rank(DevPtrs p, int kstep) {
-  if (*p.gsort == 0) return;  // every grid build of the batch sorts in LDS (k_bbox)
-  const int nwork = *p.nwork;
-  for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
-    const int t = p.work[w];
-    if (t < 0) continue;
-    const SysDev &S = p.sys[p.tile_sys[t]];
-    if (!grid_build(S) || S.sort_lds) continue;
-    const int i = t * TILE + threadIdx.x;
-    if (i < S.bead_off + S.n) {
+__global__ __launch_bounds__(256) void k_cell_rank(DevPtrs p, int kstep) {
+  const int nbig = *p.nbig;
+  for (int q = 0; q < nbig; ++q) {
+    const SysDev &S = p.sys[p.syslist[q]];
+    if (!grid_build(S)) continue;
+    const float4 *src = build_src(p, S, kstep);
+    const int bo = S.bead_off, n = S.n, cb = S.cell_base;
+    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < n; b += gridDim.x * blockDim.x) {
+      const int i = bo + b;
       const int c = p.cell_of[i];
-      const int st = p.cell_start[S.cell_base + c], en = p.cell_start[S.cell_base + c + 1];
+      const int st = p.cell_start[cb + c], en = p.cell_start[cb + c + 1];
       int rank = 0;
-      if (st >= 0 && en <= S.n) {
-        for (int m = st; m < en; ++m) rank += p.cell_tmp[S.bead_off + m] < i;
+      if (st >= 0 && en <= n) {
+        for (int m = st; m < en; ++m) rank += p.cell_tmp[bo + m] < i;
         const int pos = st + rank;
-        if (pos < S.n) {
+        if (pos < n) {
           p.cell_pos[i] = pos;
-          p.nat_sorted[S.bead_off + pos] = make_int2(p.nat_start[i], p.nat_cnt[i]);
-          p.cell_sorted[S.bead_off + pos] = i;
-          p.pos_sorted[S.bead_off + pos] = build_src(p, S, kstep)[i];
+          p.nat_sorted[bo + pos] = make_int2(p.nat_start[i], p.nat_cnt[i]);
+          p.cell_sorted[bo + pos] = i;
+          p.pos_sorted[bo + pos] = src[i];
         }
       }
     }
@@ -580,174 +856,6 @@ __device__ __forceinline__ int scan_cells(const DevPtrs &p, const SysDev &S, int
     }
   natbits_mark(bits, natj, nn, S.bead_off, false);
   return cnt;
-}
-
-// Per system (one 1024-thread block) whose sort fits LDS: the whole counting
-// sort of the global kernels above in LDS -- cell of each bead, histogram,
-// exclusive scan, member lists, and the rank of each bead among its cell's
-// members by index, so the in-cell order is the index order -- then the
-// cell-ordered arrays written out in one pass.
-constexpr int SORT_THREADS = 1024;
-
-__global__ __launch_bounds__(SORT_THREADS) void k_cell_sort_lds(DevPtrs p, int kstep) {
-  __shared__ int s_cell[SORT_N_MAX];
-  __shared__ int s_mem[SORT_N_MAX];
-  __shared__ int s_cnt[SORT_C_MAX];  // counts, then end offsets
-  __shared__ int s_wsum[SORT_THREADS / 64], s_wused[SORT_THREADS / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nsys = *p.nsys;
-  for (int q = blockIdx.x; q < nsys; q += gridDim.x) {
-    const int s = p.syslist[q];
-    SysDev &S = p.sys[s];
-    if (!grid_build(S) || !S.sort_lds) continue;
-    const int n = S.n, nc = S.ncells, bo = S.bead_off, cb = S.cell_base;
-    const float4 *src = build_src(p, S, kstep);
-    for (int c = tid; c < nc; c += SORT_THREADS) s_cnt[c] = 0;
-    // this thread's beads (at most SB): every load and cell index before the
-    // first store (a load issued after a store would wait for it)
-    constexpr int SB = SORT_N_MAX / SORT_THREADS;
-    float4 xs[SB];
-    int cs[SB];
-#pragma unroll
-    for (int u = 0; u < SB; ++u) {
-      xs[u] = src[bo + min(tid + u * SORT_THREADS, n - 1)];
-      cs[u] = cell_index(S, xs[u]);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < SB; ++u) {
-      const int b = tid + u * SORT_THREADS;
-      if (b < n) {
-        s_cell[b] = cs[u];
-        p.cell_of[bo + b] = cs[u];
-        atomicAdd(&s_cnt[cs[u]], 1);
-      }
-    }
-    __syncthreads();
-    // exclusive scan of the counts: 4 consecutive cells per thread
-    constexpr int PER = SORT_C_MAX / SORT_THREADS;
-    int v[PER], sum = 0, used = 0;
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int c = tid * PER + u;
-      v[u] = c < nc ? s_cnt[c] : 0;
-      sum += v[u];
-      used += v[u] > 0;
-    }
-    const int incl = wave_incl_scan(sum);
-    const int wu = wave_sum_i(used);
-    if (lane == 63) s_wsum[wave] = incl;
-    if (lane == 0) s_wused[wave] = wu;
-    __syncthreads();
-    int off = 0, tot_used = 0;
-    for (int w = 0; w < SORT_THREADS / 64; ++w) {
-      off += w < wave ? s_wsum[w] : 0;
-      tot_used += s_wused[w];
-    }
-    int run = off + incl - sum;
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int c = tid * PER + u;
-      if (c < nc) {
-        p.cell_start[cb + c] = run;
-        s_cnt[c] = run;  // cursor, ends at the cell's end offset
-      }
-      run += v[u];
-    }
-    if (tid == 0) {
-      p.cell_start[cb + nc] = n;
-      S.ncells_used = tot_used;
-    }
-    __syncthreads();
-    for (int b = tid; b < n; b += SORT_THREADS) s_mem[atomicAdd(&s_cnt[s_cell[b]], 1)] = b;
-    __syncthreads();
-    int ns[SB], nn[SB];
-#pragma unroll
-    for (int u = 0; u < SB; ++u) {
-      const int i = bo + min(tid + u * SORT_THREADS, n - 1);
-      ns[u] = p.nat_start[i];
-      nn[u] = p.nat_cnt[i];
-    }
-#pragma unroll
-    for (int u = 0; u < SB; ++u) {
-      const int b = tid + u * SORT_THREADS;
-      if (b < n) {
-        const int c = s_cell[b];
-        const int st = c > 0 ? s_cnt[c - 1] : 0, en = s_cnt[c];
-        int r = 0;
-        for (int m = st; m < en; ++m) r += s_mem[m] < b;
-        const int pos = st + r;
-        const int i = bo + b;
-        p.cell_pos[i] = pos;
-        p.cell_sorted[bo + pos] = i;
-        p.pos_sorted[bo + pos] = xs[u];
-        p.nat_sorted[bo + pos] = make_int2(ns[u], nn[u]);
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// Per batch: exclusive scan of the home-cell counts of the systems that build
-// their pair list directly (one block).
-__global__ __launch_bounds__(256) void k_cellwork(DevPtrs p) {
-  __shared__ int wsum[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nsys = *p.nsys;
-  int carry = 0;
-  bool nl = false;  // some system materializes its neighbor list at this rebuild
-  for (int q0 = 0; q0 < nsys; q0 += 256) {
-    const int q = q0 + tid;
-    int v = 0;
-    if (q < nsys) {
-      const SysDev &S = p.sys[p.syslist[q]];
-      v = S.build == BUILD_DIRECT ? S.ncells_used : 0;
-      nl |= S.build == BUILD_NL || S.build == BUILD_NL_ONLY;
-    }
-    const int incl = wave_incl_scan(v);
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    int off = 0, tot = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      off += (w < wave) ? wsum[w] : 0;
-      tot += wsum[w];
-    }
-    if (q < nsys) p.cellwork[q] = carry + off + incl - v;
-    carry += tot;
-    __syncthreads();
-  }
-  const int any_nl = __syncthreads_or(nl);
-  if (tid == 0) {
-    p.cellwork[nsys] = carry;
-    *p.ncellwork = carry;
-    *p.nlbuild = any_nl;
-  }
-}
-
-// Per system of the batch: list its home cells for the direct build.
-__global__ __launch_bounds__(256) void k_cellexpand(DevPtrs p) {
-  __shared__ int wsum[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nsys = *p.nsys;
-  for (int q = blockIdx.x; q < nsys; q += gridDim.x) {
-    const SysDev &S = p.sys[p.syslist[q]];
-    if (S.build != BUILD_DIRECT) continue;
-    const int off = p.cellwork[q], nc = S.ncells, cb = S.cell_base;
-    int base = 0;
-    for (int c0 = 0; c0 < nc; c0 += 256) {
-      const int c = c0 + tid;
-      const bool used = c < nc && p.cell_start[cb + c + 1] > p.cell_start[cb + c];
-      const uint64_t m = __ballot(used);
-      if (lane == 0) wsum[wave] = __popcll(m);
-      __syncthreads();
-      int o = base;
-      for (int w = 0; w < wave; ++w) o += wsum[w];
-      if (used) p.cellitems[off + o + lanes_below(m)] = make_int2(q, c);
-      base += wsum[0] + wsum[1] + wsum[2] + wsum[3];
-      __syncthreads();
-    }
-  }
 }
 
 // Block per home cell: the shell rows of the cell's beads straight from the
@@ -850,13 +958,14 @@ __device__ __forceinline__ int pl_scan_fast(const float4 *s_cand, const int *s_c
   return cnt;
 }
 
-__global__ __launch_bounds__(256) void k_pl_cells(DevPtrs p, int kstep) {
-  __shared__ float4 s_home[HOME_MAX];
-  __shared__ int s_hj[HOME_MAX], s_hcnt[HOME_MAX], s_hnn[HOME_MAX], s_hns[HOME_MAX];
-  __shared__ uint32_t s_excl[HOME_MAX][EXCL_WORDS];  // per home bead: candidate slots it must skip
-  __shared__ float4 s_cand[CAND_MAX];
-  __shared__ int s_cj[CAND_MAX];
-  __shared__ int s_rst[9], s_roff[10], s_hrange[2];
+constexpr int PLC_BYTES = 16 * (CAND_MAX + HOME_MAX) + 4 * (CAND_MAX + HOME_MAX * (4 + EXCL_WORDS)) + 96;
+__device__ __forceinline__ void pl_cells(const DevPtrs &p, int kstep, char *s_raw) {
+  float4 *s_cand = reinterpret_cast<float4 *>(s_raw), *s_home = s_cand + CAND_MAX;
+  int *s_cj = reinterpret_cast<int *>(s_home + HOME_MAX);
+  int *s_hj = s_cj + CAND_MAX, *s_hcnt = s_hj + HOME_MAX, *s_hnn = s_hcnt + HOME_MAX, *s_hns = s_hnn + HOME_MAX;
+  uint32_t(*s_excl)[EXCL_WORDS] = reinterpret_cast<uint32_t(*)[EXCL_WORDS]>(s_hns + HOME_MAX);  // per home bead:
+                                                                                     // slots it must skip
+  int *s_rst = reinterpret_cast<int *>(s_excl + HOME_MAX), *s_roff = s_rst + 9, *s_hrange = s_roff + 10;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int total = *p.ncellwork;
@@ -1048,10 +1157,9 @@ __global__ __launch_bounds__(256) void k_pl_cells(DevPtrs p, int kstep) {
 // pass without materializing the neighbor list: the native pair list in each
 // bead's native slots, the non-native rows in the shell-row slots (the shell
 // filter packs them into the pair list), which therefore stop holding shell
-// rows (k_skin clears sl_valid).
-__global__ __launch_bounds__(256) void k_nl_build(DevPtrs p, int kstep) {
-  if (*p.nlbuild == 0) return;  // no system of the batch needs it (k_cellwork)
-  __shared__ uint32_t s_bits[4][NATBITS_WORDS];
+// rows (decide_build clears sl_valid).
+__device__ __forceinline__ void nl_build(const DevPtrs &p, int kstep, char *s_raw) {
+  uint32_t(*s_bits)[NATBITS_WORDS] = reinterpret_cast<uint32_t(*)[NATBITS_WORDS]>(s_raw);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int k = lane; k < NATBITS_WORDS; k += 64) s_bits[wave][k] = 0u;
   __builtin_amdgcn_wave_barrier();
@@ -1146,33 +1254,16 @@ __global__ __launch_bounds__(256) void k_nl_build(DevPtrs p, int kstep) {
   }
 }
 
-// Per tile of a system whose pair list is rebuilt from its neighbor list: the
-// order in which the step kernel's lane groups take the tile's beads, by
-// decreasing row length (non-native + native), ties by index, so the beads
-// that one round of lane groups computes together run loops of similar
-// length (grid and shell builds: the shell filter computes the same order).
-// Results do not depend on the order: each bead is computed by one group the
-// same way.
-__global__ __launch_bounds__(256) void k_tile_order(DevPtrs p) {
-  if (*p.nlbuild == 0) return;  // shell and grid builds: the shell filter orders their tiles
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nwork = *p.nwork;
-  for (int w = blockIdx.x * 4 + wave; w < nwork; w += gridDim.x * 4) {
-    const int t = p.work[w];
-    if (t < 0) continue;
-    const SysDev &S = p.sys[p.tile_sys[t]];
-    if (S.build != BUILD_NL) continue;
-    const int b0 = t * TILE, i = b0 + lane;
-    // grid and shell builds: shell-row counts (the pair lists are filtered
-    // after this); neighbor-list builds: the previous pair-list counts
-    const int nrep = S.build == BUILD_NL ? p.plrep_cnt[i] : p.slrep_cnt[i];
-    const int key = i < S.bead_off + S.n ? nrep + p.platt_cnt[i] : -1;
-    int rank = 0;
-    for (int j = 0; j < TILE; ++j) {
-      const int kj = __shfl(key, j);
-      rank += (kj > key) | ((kj == key) & (j < lane));
-    }
-    p.tile_ord[b0 + rank] = (uint8_t)lane;
+// Rows of one rebuild: the home cells of the batch's grid builds, then the
+// neighbor-list builds, which are rare (one launch: a kernel of their own cost
+// 5 us a rebuild with nothing to do).
+__global__ __launch_bounds__(256) void k_rows(DevPtrs p, int kstep) {
+  constexpr int NLB_BYTES = 4 * 4 * NATBITS_WORDS;
+  __shared__ __align__(16) char s_raw[PLC_BYTES > NLB_BYTES ? PLC_BYTES : NLB_BYTES];
+  pl_cells(p, kstep, s_raw);
+  if (*p.nlbuild != 0) {
+    __syncthreads();
+    nl_build(p, kstep, s_raw);
   }
 }
 
@@ -1205,7 +1296,7 @@ __device__ __forceinline__ void wave_tile(const DevPtrs &p, const SysDev &S, int
   // at each rebuild (ERR_PBC), so every separation here is below boxl/2.
   const int64_t step = S.step + kstep;
   const int q1 = S.type_mask == 2 ? 3 : 0;  // type-pair index of a one-type system
-  // slot q of the tile's order (k_tile_order) is computed in round q / GPW by
+  // slot q of the tile's order (tile_ord) is computed in round q / GPW by
   // group q % GPW; lane m's own bead b0 + m sits in slot qm
   const int ordm = p.tile_ord[b0 + lane];
   const int qm = __builtin_amdgcn_ds_permute(ordm << 2, lane);
@@ -1553,7 +1644,7 @@ __device__ __forceinline__ void step_items(const DevPtrs &p, int kstep, float4 *
 // Pair list of one tile's beads = their shell rows filtered at x with the
 // reference's exact predicate (d2 < rc_pl^2, squares summed in order without
 // contraction), for grid and shell builds, and the native pair list from the
-// native CSR.  Neighbor-list builds: k_nl_build has left the filtered rows in
+// native CSR.  Neighbor-list builds: k_rows has left the filtered rows in
 // the shell-row slots and written the native pair list; the rows are packed
 // here as they are.  4 lanes per bead, 16 beads per round: lane l
 // takes 4-entry chunks l, l + 4, ... of the row, kept entries are compacted
@@ -1577,24 +1668,24 @@ __device__ __forceinline__ void filter_tile(const DevPtrs &p, const SysDev &S, i
   const int bo = S.bead_off, pl_cap = S.pl_cap;
   const int64_t pl_base = S.pl_base;
   const int bend = min(t * TILE + TILE, bo + S.n);
-  const bool nlb = S.build == BUILD_NL;  // neighbor-list build: rows already filtered (k_nl_build)
+  const bool nlb = S.build == BUILD_NL;  // neighbor-list build: rows already filtered (k_rows)
   // cutoffs as wave-uniform values (a per-lane indexed load would be a vector
   // load, and waiting for it would also wait for the earlier stores)
   const float rc11 = S.rc2_pl_rep[0], rc12 = S.rc2_pl_rep[1], rc21 = S.rc2_pl_rep[2], rc22 = S.rc2_pl_rep[3];
   // row lengths of the whole tile in one load, picked up by shuffles; beads
-  // in the tile's order (k_tile_order), slot q = 16 r + g
+  // in the tile's order (tile_ord), slot q = 16 r + g
   const bool tin = t * TILE + lane < bend;
   const int t_nr = tin ? p.slrep_cnt[t * TILE + lane] : 0;
   const int t_ns = tin ? p.nat_start[t * TILE + lane] : 0, t_nn = tin ? p.nat_cnt[t * TILE + lane] : 0;
-  // the tile's bead order for this filter and the step kernel (k_tile_order's
-  // key: shell-row length + the native pair-list length of the last rebuild,
-  // decreasing, ties by index), read before this pass rewrites platt_cnt.
-  // Computed at grid builds only: shell builds keep the order of the grid
-  // build that made their shell rows (row lengths change little between
-  // them), and neighbor-list builds the order k_tile_order gave them.  The
-  // order only groups beads into rounds; no result depends on it.
+  // the tile's bead order for this filter and the step kernel: decreasing row
+  // length (shell-row length + the native pair-list length), ties by index, so
+  // that the beads one round of lane groups takes together run loops of
+  // similar length.  Computed at grid and neighbor-list builds: shell builds
+  // keep the order of the grid build that made their shell rows (row lengths
+  // change little between them).  The order only groups beads into rounds; no
+  // result depends on it.
   int ordm;
-  if (nlb || S.build == BUILD_SHELL) {
+  if (S.build == BUILD_SHELL) {
     ordm = p.tile_ord[t * TILE + lane];
   } else {
     const int key = tin ? t_nr + p.platt_cnt[t * TILE + lane] : -1;
@@ -1832,6 +1923,12 @@ __global__ __launch_bounds__(STEP_THREADS) void k_shell_filter(DevPtrs p, int ks
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   char *s_stage = reinterpret_cast<char *>(s_pos) + stage_off;
+  // the filter of the grid builds runs after their rows: the rebuild's work
+  // counters go back to empty for the next one
+  if (blockIdx.x == 0 && tid == 0 && ((builds >> BUILD_DIRECT) & 1)) {
+    *p.ncellwork = 0;
+    *p.nlbuild = 0;
+  }
   int w0, w1;
   item_range<KLDS, true>(p, tier, w0, w1);
   for (int w = w0 + blockIdx.x; w < w1; w += gridDim.x) {
@@ -2202,38 +2299,44 @@ static void launch_filter(const DevPtrs &p, const StepGrids &sg, int kstep, int 
                        p, kstep, 0, 0, 2 * FILTER_STAGE_BYTES, builds);
 }
 
-// One list-rebuild point for the current batch: snapshot / decision, cell
-// grid and counting sort, then whichever of the direct pair-list build or the
-// neighbor-list materialization + filter each system needs.
+// One list-rebuild point for the current batch: decision, cell grid and
+// counting sort, the rows of grid and neighbor-list builds, then the filter.
+// lg.split (and fk): the systems whose pair list comes from their shell rows
+// need nothing from the cell grid, so their filter runs beside the grid chain,
+// and the filter of the grid-built systems follows the chain on the second
+// stream (the two filters take disjoint systems).  A batch whose filter does
+// not fill the device gains nothing from that and pays for the fork and for
+// the launches with nothing to do: it runs the whole rebuild in three launches
+// on one stream.
 hipError_t launch_lists(const DevPtrs &p, const ListGrids &lg, int kstep, int flags, hipStream_t st,
                         const StepFork *fk) {
-  const int grid_tiles = lg.grid_tiles, grid_sys = lg.grid_sys;
-  hipLaunchKernelGGL(k_skin, dim3(grid_sys), dim3(SKIN_THREADS), 0, st, p, kstep, flags);
-  hipLaunchKernelGGL(k_bbox, dim3(grid_sys), dim3(256), 0, st, p, kstep);
-  // Systems whose pair list comes from their shell rows need nothing from
-  // the cell grid: with a second stream (fk) their filter runs beside the
-  // grid chain, and the filter of the grid-built systems follows the chain on
-  // the second stream.  The two filters take disjoint systems.
   constexpr int ALL = (1 << BUILD_DIRECT) | (1 << BUILD_SHELL) | (1 << BUILD_NL);
   constexpr int SHELL_ONLY = 1 << BUILD_SHELL;
+  const bool split = fk && lg.split;
+  if (lg.grid_big > 0) {
+    hipLaunchKernelGGL(k_big_skin, dim3(lg.grid_big), dim3(BIG_THREADS), 0, st, p, kstep, flags);
+    hipLaunchKernelGGL(k_big_plan, dim3(lg.grid_nbig), dim3(1024), 0, st, p, kstep, flags);
+  }
   hipStream_t cs = st;  // the grid chain's stream
-  if (fk) {
+  if (split) {
+    if (lg.grid_sys > 0)
+      hipLaunchKernelGGL(k_rebuild<PH_DECIDE>, dim3(lg.grid_sys), dim3(SORT_THREADS), 0, st, p, kstep, flags);
     const hipError_t h = fork_begin(fk, st);
     if (h != hipSuccess) return h;
     cs = fk->side;
+    if (lg.grid_sys > 0)
+      hipLaunchKernelGGL(k_rebuild<PH_GRID>, dim3(lg.grid_sys), dim3(SORT_THREADS), 0, cs, p, kstep, flags);
+  } else if (lg.grid_sys > 0) {
+    hipLaunchKernelGGL(k_rebuild<PH_DECIDE | PH_GRID>, dim3(lg.grid_sys), dim3(SORT_THREADS), 0, cs, p, kstep, flags);
   }
-  hipLaunchKernelGGL(k_cell_sort_lds, dim3(grid_sys), dim3(SORT_THREADS), 0, cs, p, kstep);
-  hipLaunchKernelGGL(k_cell_count, dim3(grid_tiles), dim3(64), 0, cs, p, kstep);
-  hipLaunchKernelGGL(k_cell_scan, dim3(grid_sys), dim3(256), 0, cs, p);
-  hipLaunchKernelGGL(k_cell_scatter, dim3(grid_tiles), dim3(64), 0, cs, p);
-  hipLaunchKernelGGL(k_cell_rank, dim3(grid_tiles), dim3(64), 0, cs, p, kstep);
-  hipLaunchKernelGGL(k_cellwork, dim3(1), dim3(256), 0, cs, p);
-  hipLaunchKernelGGL(k_cellexpand, dim3(grid_sys), dim3(256), 0, cs, p);
-  hipLaunchKernelGGL(k_pl_cells, dim3(grid_tiles), dim3(256), 0, cs, p, kstep);
-  hipLaunchKernelGGL(k_tile_order, dim3(grid_tiles), dim3(256), 0, cs, p);
-  // neighbor-list builds: their rows before the shell filter packs them
-  hipLaunchKernelGGL(k_nl_build, dim3(grid_tiles), dim3(256), 0, cs, p, kstep);
-  if (fk) {
+  if (lg.grid_big > 0) {
+    hipLaunchKernelGGL(k_cell_count, dim3(4 * lg.grid_big), dim3(256), 0, cs, p, kstep);
+    hipLaunchKernelGGL(k_cell_scan, dim3(lg.grid_nbig), dim3(1024), 0, cs, p);
+    hipLaunchKernelGGL(k_cell_scatter, dim3(4 * lg.grid_big), dim3(256), 0, cs, p);
+    hipLaunchKernelGGL(k_cell_rank, dim3(4 * lg.grid_big), dim3(256), 0, cs, p, kstep);
+  }
+  hipLaunchKernelGGL(k_rows, dim3(lg.grid_tiles), dim3(256), 0, cs, p, kstep);
+  if (split) {
     launch_filter(p, lg.fg, kstep, ALL & ~SHELL_ONLY, cs);
     launch_filter(p, lg.fg, kstep, SHELL_ONLY, st);
     const hipError_t h = fork_end(fk, st);

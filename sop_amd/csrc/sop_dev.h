@@ -71,13 +71,12 @@ struct SysDev {
   int32_t sl_valid;       // 1: the shell rows match pos_shell
   int32_t nbuild[3];      // pair-list rebuilds: grid (BUILD_DIRECT), shell, neighbor list
   float wrap_margin;
-  // cell grid, written by k_bbox at each neighbor-list rebuild
+  // cell grid, written at each grid build
   float org[3];
   float inv_edge[3];
   int32_t dims[3];
   int32_t ncells;
   int32_t ncells_used; // cells holding at least one bead
-  int32_t sort_lds;    // this rebuild's cell sort runs in one block's LDS
   int32_t wrap_free; // 1: every pair separation is below boxl/2 (minimum image is the identity)
   // list state, device-written.  The neighbor list is defined by the snapshot
   // pos_ref taken at its last rebuild; it is materialized only when needed.
@@ -87,7 +86,15 @@ struct SysDev {
   // status, device-written
   int32_t err;
   int32_t row_max;   // longest shell row (or neighbor-list build row) since the host last read it
+  // systems of more than SORT_N_MAX beads: this rebuild's bounding box (minima,
+  // maxima) and largest squared displacements, as order-preserving unsigned
+  // images (ACC_MIN / ACC_MAX when empty), and the box of the pos_ref snapshot
+  uint32_t acc[8];
+  float ref_box[6];
 };
+
+// SysDev::acc when empty: the images of +infinity and -infinity
+constexpr uint32_t ACC_MIN = 0xFF800000u, ACC_MAX = 0x007FFFFFu;
 
 // SysDev::build
 constexpr int BUILD_NONE = 0;    // no list work at this step
@@ -96,7 +103,7 @@ constexpr int BUILD_NL = 2;      // pair list = neighbor list of pos_ref filtere
 constexpr int BUILD_NL_ONLY = 3; // materialize the neighbor list only
 constexpr int BUILD_SHELL = 4;   // pair list = shell rows filtered at x (no cell grid)
 
-// k_skin flags
+// rebuild flags
 constexpr int FORCE_NL = 1;      // rebuild the neighbor list now (snapshot)
 constexpr int FORCE_PL = 2;      // rebuild the pair list now
 constexpr int MATERIALIZE_NL = 4;// materialize the neighbor list of the current snapshot
@@ -145,12 +152,11 @@ struct DevPtrs {
   uint8_t *tile_ord;    // per tile: TILE bead offsets in the order the step kernel's lane groups take them
   int32_t *work;        // tile ids to process (-1 = padding), XCD-interleaved
   int32_t *nwork;
-  int32_t *syslist;     // system slots of the current batch
+  int32_t *syslist;     // system slots of the current batch, those of more than SORT_N_MAX beads first
   int32_t *nsys;
-  int32_t *cellwork;    // per batch position: first home cell of the direct pair-list build
-  int32_t *ncellwork;   // total home cells of the direct pair-list build
-  int32_t *nlbuild;     // 1 if a system of the batch materializes its neighbor list at this rebuild
-  int32_t *gsort;       // nonzero if a grid build of this rebuild sorts in global memory (too big for LDS)
+  int32_t *nbig;        // systems of more than SORT_N_MAX beads
+  int32_t *ncellwork;   // home cells of this rebuild's grid builds (0 between rebuilds)
+  int32_t *nlbuild;     // 1 if a system of the batch builds from its neighbor list at this rebuild
   int2 *cellitems;      // home cells of the direct build: {batch position, cell}
   int4 *items;          // step-kernel work: {first tile, tiles | waves per tile << 8, first staged
                         // bead or -1, staged beads}; the waves of a tile split its rounds
@@ -186,10 +192,13 @@ struct StepFork {
   hipEvent_t fork, join;
 };
 
-// Grids of the list kernels: per tile, per system, and the shell filter's
-// work items (staged in LDS like the step kernel's).
+// Grids of the list kernels: home cells, systems of up to SORT_N_MAX beads
+// (one block each), beads (blocks of 2,048) and number of the larger ones, and
+// the shell filter's work items (staged in LDS like the step kernel's).
+// split: the shell builds' filter on one stream beside the grid chain.
 struct ListGrids {
-  int grid_tiles, grid_sys;
+  int grid_tiles, grid_sys, grid_big, grid_nbig;
+  bool split;
   StepGrids fg;
 };
 
@@ -197,9 +206,10 @@ struct ListGrids {
 __host__ __device__ inline int item_tiles(int y) { return y & 0xFF; }
 __host__ __device__ inline int item_split(int y) { return y >> 8; }
 
-// systems whose cell sort fits one block's LDS
+// systems whose cell sort fits one block's LDS: a system of n beads has at
+// most max(64, 2 n) cells
 constexpr int SORT_N_MAX = 5120;
-constexpr int SORT_C_MAX = 4096;
+constexpr int SORT_C_MAX = 2 * SORT_N_MAX;
 
 constexpr int EPART_N = 6;   // bond, angle, native, rep, virial, contacts
 constexpr int SYSOUT_N = 16; // e[0..5], contacts, rgsq, sum x,y,z, n
