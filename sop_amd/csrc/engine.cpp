@@ -100,11 +100,11 @@ static int grid_rebuild(const sop_engine *e) {
 // one per system.  While serving, fixed grids whenever the batch has one.
 static int grid_big_beads(const sop_engine *e) {
   if (e->cur_nbig == 0) return 0;
-  return e->fixed_grids ? e->num_cu : std::min((e->cur_big_max + 2047) / 2048, 4 * e->num_cu);
+  return e->fixed_grids ? 8 : std::min((e->cur_big_max + 2047) / 2048, 4 * e->num_cu);
 }
 static int grid_big_sys(const sop_engine *e) {
   if (e->cur_nbig == 0) return 0;
-  return e->fixed_grids ? e->num_cu : std::min(e->cur_nbig, 1024);
+  return e->fixed_grids ? 64 : std::min(e->cur_nbig, 1024);
 }
 
 // Launch grid of a persistent item kernel: `g` blocks (a multiple of 8, so

@@ -530,8 +530,10 @@ __global__ __launch_bounds__(SORT_THREADS) void k_rebuild(DevPtrs p, int kstep, 
 }
 
 // ---- systems of more than SORT_N_MAX beads (the first *nbig of the batch),
-// each spread over the whole launch: a 500,000-bead system's decision in one
-// block took longer than its step.
+// each spread over many blocks: a 200,000-bead system's decision in one block
+// took 174 us.  Grid: x blocks over a system's beads, y over the systems (64
+// 8,000-bead systems one after another, each over the whole launch, took
+// twice as long as side by side).
 
 // Order-preserving unsigned image of a float, for atomic minima and maxima.
 __device__ __forceinline__ uint32_t ord_u(float f) {
@@ -550,7 +552,7 @@ __global__ __launch_bounds__(BIG_THREADS) void k_big_skin(DevPtrs p, int kstep, 
   __shared__ float s_red[8][NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nbig = *p.nbig;
-  for (int q = 0; q < nbig; ++q) {
+  for (int q = blockIdx.y; q < nbig; q += gridDim.y) {
     SysDev &S = p.sys[p.syslist[q]];
     const bool mat = (flags & MATERIALIZE_NL) != 0;
     const bool nl = !mat && ((flags & FORCE_NL) || due_nl(S, kstep));
@@ -657,7 +659,7 @@ __global__ __launch_bounds__(1024) void k_big_plan(DevPtrs p, int kstep, int fla
 // Per bead: cell id and histogram; the shell snapshot of a direct build.
 __global__ __launch_bounds__(256) void k_cell_count(DevPtrs p, int kstep) {
   const int nbig = *p.nbig;
-  for (int q = 0; q < nbig; ++q) {
+  for (int q = blockIdx.y; q < nbig; q += gridDim.y) {
     const SysDev &S = p.sys[p.syslist[q]];
     if (!grid_build(S)) continue;
     const float4 *src = build_src(p, S, kstep);
@@ -738,7 +740,7 @@ __global__ __launch_bounds__(1024) void k_cell_scan(DevPtrs p) {
 // Per bead: scatter into its cell's segment (arbitrary in-cell order).
 __global__ __launch_bounds__(256) void k_cell_scatter(DevPtrs p) {
   const int nbig = *p.nbig;
-  for (int q = 0; q < nbig; ++q) {
+  for (int q = blockIdx.y; q < nbig; q += gridDim.y) {
     const SysDev &S = p.sys[p.syslist[q]];
     if (!grid_build(S)) continue;
     const int bo = S.bead_off, n = S.n, cb = S.cell_base;
@@ -756,7 +758,7 @@ __global__ __launch_bounds__(256) void k_cell_scatter(DevPtrs p) {
 // list, is independent of the order of the atomics above.
 __global__ __launch_bounds__(256) void k_cell_rank(DevPtrs p, int kstep) {
   const int nbig = *p.nbig;
-  for (int q = 0; q < nbig; ++q) {
+  for (int q = blockIdx.y; q < nbig; q += gridDim.y) {
     const SysDev &S = p.sys[p.syslist[q]];
     if (!grid_build(S)) continue;
     const float4 *src = build_src(p, S, kstep);
@@ -2314,7 +2316,7 @@ hipError_t launch_lists(const DevPtrs &p, const ListGrids &lg, int kstep, int fl
   constexpr int SHELL_ONLY = 1 << BUILD_SHELL;
   const bool split = fk && lg.split;
   if (lg.grid_big > 0) {
-    hipLaunchKernelGGL(k_big_skin, dim3(lg.grid_big), dim3(BIG_THREADS), 0, st, p, kstep, flags);
+    hipLaunchKernelGGL(k_big_skin, dim3(lg.grid_big, lg.grid_nbig), dim3(BIG_THREADS), 0, st, p, kstep, flags);
     hipLaunchKernelGGL(k_big_plan, dim3(lg.grid_nbig), dim3(1024), 0, st, p, kstep, flags);
   }
   hipStream_t cs = st;  // the grid chain's stream
@@ -2330,10 +2332,10 @@ hipError_t launch_lists(const DevPtrs &p, const ListGrids &lg, int kstep, int fl
     hipLaunchKernelGGL(k_rebuild<PH_DECIDE | PH_GRID>, dim3(lg.grid_sys), dim3(SORT_THREADS), 0, cs, p, kstep, flags);
   }
   if (lg.grid_big > 0) {
-    hipLaunchKernelGGL(k_cell_count, dim3(4 * lg.grid_big), dim3(256), 0, cs, p, kstep);
+    hipLaunchKernelGGL(k_cell_count, dim3(4 * lg.grid_big, lg.grid_nbig), dim3(256), 0, cs, p, kstep);
     hipLaunchKernelGGL(k_cell_scan, dim3(lg.grid_nbig), dim3(1024), 0, cs, p);
-    hipLaunchKernelGGL(k_cell_scatter, dim3(4 * lg.grid_big), dim3(256), 0, cs, p);
-    hipLaunchKernelGGL(k_cell_rank, dim3(4 * lg.grid_big), dim3(256), 0, cs, p, kstep);
+    hipLaunchKernelGGL(k_cell_scatter, dim3(4 * lg.grid_big, lg.grid_nbig), dim3(256), 0, cs, p);
+    hipLaunchKernelGGL(k_cell_rank, dim3(4 * lg.grid_big, lg.grid_nbig), dim3(256), 0, cs, p, kstep);
   }
   hipLaunchKernelGGL(k_rows, dim3(lg.grid_tiles), dim3(256), 0, cs, p, kstep);
   if (split) {
