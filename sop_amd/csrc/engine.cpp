@@ -128,7 +128,13 @@ int grid_items(const sop_engine *e) {
   return items_grid(e->step_blocks > 0 ? e->step_blocks : default_step_blocks(e), e->fixed_grids, e->cur_nitems);
 }
 
+// A block per tile; while serving a fixed grid whenever the batch has such
+// tiles (three blocks are resident per compute unit).
 int grid_items_far(const sop_engine *e) { return items_grid(2 * e->num_cu, e->fixed_grids, e->cur_nitems_far); }
+int grid_step_tiles(const sop_engine *e) {
+  if (e->cur_ntiles == 0) return 0;
+  return e->fixed_grids ? 4 * e->num_cu : e->cur_ntiles;
+}
 
 // Whole-CU LDS items: one block per compute unit (the block takes all of
 // the unit's LDS).  While serving, a fixed grid whenever the batch has such
@@ -141,7 +147,7 @@ static int items_grid_big(const sop_engine *e, int count) {
 int grid_items_big(const sop_engine *e) { return items_grid_big(e, e->cur_nitems_big); }
 
 StepGrids step_grids(const sop_engine *e) {
-  return StepGrids{grid_items(e), grid_items_big(e), grid_items_far(e), e->cur_lds, e->cur_lds_big};
+  return StepGrids{grid_items(e), grid_items_big(e), grid_items_far(e), e->cur_lds, e->cur_lds_big, grid_step_tiles(e)};
 }
 
 // The shell filter's LDS launch: one block per item (a block leaves its
@@ -151,7 +157,7 @@ StepGrids filter_grids(const sop_engine *e) {
   const int g = e->step_blocks > 0 ? e->step_blocks : default_step_blocks(e);
   return StepGrids{items_grid(e->fixed_grids ? g : std::max(g, 8 * e->num_cu), e->fixed_grids, e->cur_nfitems),
                    items_grid_big(e, e->cur_nfitems_big),
-                   items_grid(2 * e->num_cu, e->fixed_grids, e->cur_nfitems_far), e->cur_flds, e->cur_flds_big};
+                   items_grid(2 * e->num_cu, e->fixed_grids, e->cur_nfitems_far), e->cur_flds, e->cur_flds_big, 0};
 }
 
 ListGrids list_grids(const sop_engine *e) {
@@ -903,6 +909,42 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   int32_t per_step = e->opts.step_tiles;
   if (per_step <= 0) per_step = total_tiles > slots_w ? STEP_WAVES : (2 * total_tiles > slots_w ? 8 : 4);
   e->cur_step_tiles = per_step;
+  // the step's tiles with a block each (k_step_tile): all of a batch of up to
+  // TILE_STEP_PER_CU tiles per compute unit; else the systems too large for
+  // two LDS blocks per unit while theirs are that few, and the ones too large
+  // for any LDS tier up to TILE_STEP_FAR_PER_CU.  Step times by tile against
+  // the other kernel (us): 2 x 8,000 beads 8.2 / 13.8 whole-CU, 6 x 8,000
+  // 17.9 / 14.4; 32 x 4,000 and 4 x 8,000 together 34.8 / 40.8; 12 x 4,000
+  // 14.0 / 12.9 LDS; 20,000 beads 12.7 / 33.7 global-gather items, 60,000
+  // 24.6 / 36.3, 100,000 56.5 / 42.0.
+  const int64_t tile_cap = (int64_t)TILE_STEP_PER_CU * e->num_cu;
+  int64_t mid_tiles = 0, far_tiles = 0;
+  for (int32_t q = 0; q < nslots; ++q) {
+    const int64_t len = e->sys[slots[q]].bead_len;
+    if (len > lds_cap) (len > big_cap ? far_tiles : mid_tiles) += len / TILE;
+  }
+  const bool own_items = e->opts.step_tiles > 0;  // item size asked for
+  const bool by_tile = total_tiles <= tile_cap && !own_items;
+  const bool mid_by_tile = mid_tiles + far_tiles <= tile_cap && !own_items;
+  const bool far_by_tile = far_tiles <= (int64_t)TILE_STEP_FAR_PER_CU * e->num_cu && !own_items;
+  auto tile_step = [&](const SysHost &h) {
+    return by_tile || (h.bead_len > lds_cap && (mid_by_tile || (far_by_tile && h.bead_len > big_cap)));
+  };
+  std::vector<int2> tiles;
+  {
+    // each XCD (tile k of the table runs on XCD k mod 8) a run of consecutive
+    // tiles, whose gathers share much of their range of the coordinates
+    std::vector<int2> all;
+    for (int32_t sl : by_arena) {
+      const SysHost &h = e->sys[sl];
+      if (!tile_step(h)) continue;
+      for (int64_t t = h.bead_off / TILE; t < (h.bead_off + h.bead_len) / TILE; ++t)
+        all.push_back(make_int2((int32_t)t, sl));
+    }
+    const size_t run = (all.size() + NX - 1) / NX;
+    tiles.assign(run * NX, make_int2(-1, 0));
+    for (size_t k = 0; k < all.size(); ++k) tiles[(k % run) * NX + k / run] = all[k];
+  }
   struct Plan {
     std::vector<int4> items;
     int32_t n_lds = 0, n_big = 0, n_far = 0;
@@ -934,6 +976,7 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     };
     for (int32_t sl : by_arena) {
       const SysHost &h = e->sys[sl];
+      if (split && tile_step(h)) continue;
       const int32_t t0 = (int32_t)(h.bead_off / TILE), nt = (int32_t)(h.bead_len / TILE);
       const int32_t per = per_fixed > 0 ? per_fixed : per_of(h);
       if (h.bead_len <= lds_cap) {
@@ -1086,6 +1129,14 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     e->work_cap = nc;
     invalidate_graphs(e);
   }
+  if ((int64_t)tiles.size() > e->tiles_cap) {
+    HIPCK(hipStreamSynchronize(e->stream));
+    const int64_t nc = std::max<int64_t>(1024, (int64_t)tiles.size() * 2);
+    if (e->p.tiles) HIPCK(hipFree(e->p.tiles));
+    HIPCK(hipMalloc((void **)&e->p.tiles, sizeof(int2) * (size_t)nc));
+    e->tiles_cap = nc;
+    invalidate_graphs(e);
+  }
   if (!e->p.nwork) {
     HIPCK(hipMalloc((void **)&e->p.nwork, 256));
     e->p.nsys = e->p.nwork + 16;
@@ -1097,6 +1148,7 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     e->p.nfitems_far = e->p.nwork + 46;
     e->p.nitems = e->p.nwork + 48;
     e->p.nitems_far = e->p.nwork + 56;
+    e->p.ntiles = e->p.nwork + 57;
     e->p.nitems_big = e->p.nwork + 60;
     invalidate_graphs(e);
   }
@@ -1120,13 +1172,16 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   const int32_t nw = (int32_t)e->h_work.size(), ns = nslots;
   if (nw > 0) HIPCK(hipMemcpy(e->p.work, e->h_work.data(), 4 * (size_t)nw, hipMemcpyHostToDevice));
   if (ns > 0) HIPCK(hipMemcpy(e->p.syslist, e->h_syslist.data(), 4 * (size_t)ns, hipMemcpyHostToDevice));
+  e->cur_ntiles = (int32_t)tiles.size();
+  if (!tiles.empty())
+    HIPCK(hipMemcpy(e->p.tiles, tiles.data(), sizeof(int2) * tiles.size(), hipMemcpyHostToDevice));
   const int32_t ni = (int32_t)e->h_items.size(), nfi = (int32_t)e->h_fitems.size();
   if (ni > 0) HIPCK(hipMemcpy(e->p.items, e->h_items.data(), sizeof(int4) * (size_t)ni, hipMemcpyHostToDevice));
   if (nfi > 0) HIPCK(hipMemcpy(e->p.fitems, e->h_fitems.data(), sizeof(int4) * (size_t)nfi, hipMemcpyHostToDevice));
   // the counters in one copy: nwork[0] = work entries, [16] batch systems,
   // [24] large ones, [32] home cells and [40] neighbor-list builds of a rebuild
   // (none between rebuilds), [44..46] filter items, [48] / [56] / [60] step
-  // items (LDS / far / whole-CU)
+  // items (LDS / far / whole-CU), [57] step tiles
   int32_t cnt[64] = {0};
   cnt[0] = nw;
   cnt[16] = ns;
@@ -1136,14 +1191,15 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   cnt[46] = fp.n_far;
   cnt[48] = sp.n_lds;
   cnt[56] = sp.n_far;
+  cnt[57] = (int32_t)tiles.size();
   cnt[60] = sp.n_big;
   HIPCK(hipMemcpy(e->p.nwork, cnt, sizeof(cnt), hipMemcpyHostToDevice));
   e->cur_nwork = nw;
   e->cur_nsys = ns;
   e->cur_nbig = nbig;
   e->cur_nitems = sp.n_lds;
-  e->cur_nitems_far = sp.n_far;
   e->cur_nitems_big = sp.n_big;
+  e->cur_nitems_far = sp.n_far;
   e->cur_nfitems = fp.n_lds;
   e->cur_nfitems_far = fp.n_far;
   e->cur_nfitems_big = fp.n_big;
@@ -1177,10 +1233,10 @@ sop_status engine_check_errors(sop_engine *e, const int32_t *slots, int32_t nslo
 static std::string graph_key(const sop_engine *e, int G, int n_nl, int n_pl) {
   std::ostringstream os;
   os << G << '|' << n_nl << '|' << n_pl << '|' << e->opts.lanes_per_bead << '|' << grid_tiles(e) << '|'
-     << grid_rebuild(e) << '|' << grid_big_beads(e) << '|' << grid_big_sys(e) << '|' << grid_items(e) << '|' << grid_items_big(e) << '|' << grid_items_far(e) << '|'
+     << grid_rebuild(e) << '|' << grid_big_beads(e) << '|' << grid_big_sys(e) << '|' << grid_items(e) << '|' << grid_items_big(e) << '|'
      << e->cur_lds << '|' << e->cur_lds_big;
   const StepGrids fg = filter_grids(e);
-  os << '|' << list_grids(e).split << '|' << fg.grid << '|' << fg.grid_big << '|' << fg.grid_far << '|' << fg.lds << '|' << fg.lds_big;
+  os << '|' << step_grids(e).tiles << '|' << grid_items_far(e) << '|' << list_grids(e).split << '|' << fg.grid << '|' << fg.grid_big << '|' << fg.grid_far << '|' << fg.lds << '|' << fg.lds_big;
   return os.str();
 }
 
@@ -1475,7 +1531,8 @@ void sop_engine_destroy(sop_engine *e) {
   for (auto &a : e->nat_arrays) if (*a.first) note(hipFree(*a.first), "hipFree(native pool)");
   for (auto &a : e->cell_arrays) if (*a.first) note(hipFree(*a.first), "hipFree(cell pool)");
   void *others[] = {e->p.nlrep_j, e->p.plrep_j, e->p.slrep_j,  e->p.tile_sys, e->p.sys,  e->p.sysout,
-                    e->p.syslist, e->p.work,    e->p.nwork,    e->p.items};
+                    e->p.syslist, e->p.work,    e->p.nwork,    e->p.items,
+                    e->p.tiles};
   for (void *q : others) if (q) note(hipFree(q), "hipFree");
   if (e->fork.side) note(hipStreamSynchronize(e->fork.side), "hipStreamSynchronize");
   if (e->fork.fork) note(hipEventDestroy(e->fork.fork), "hipEventDestroy");

@@ -1278,6 +1278,115 @@ __device__ __forceinline__ float4 partner(const float4 *__restrict__ pin, const 
   return LDS ? s_pos[j - base] : pin[j];
 }
 
+// Force of the chain terms on bead b0 + lane of a tile, one bead per lane.
+template <bool LDS>
+__device__ __forceinline__ float3 chain_force(const DevPtrs &p, const SysDev &S, int s, int b0,
+                                              const float4 *__restrict__ pin, const float4 *s_pos, int lds0, float t_br,
+                                              float br_before) {
+  const int lane = threadIdx.x & 63;
+  const int bead_off = S.bead_off, n = S.n;
+  const int bend = min(b0 + TILE, bead_off + n);
+  // Chain terms, each pair once, over the tile's lanes: lane m computes the
+  // FENE bond (i, i+1) and the i,i+2 soft sphere of its bead i = b0 + m (the
+  // force on i; the partner takes the opposite), and takes the partner halves
+  // of the bond (i-1, i) and the pair (i-2, i) from lanes m-1 and m-2.  The
+  // pairs that start before the tile come from lanes 0 and 1 themselves.
+  const int i = b0 + lane;
+  const int send = bead_off + n;
+  float4 xc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (i < bend) xc = partner<LDS>(pin, s_pos, lds0, i);
+  // force on a from the pair (a, b) of chain offset off (1: FENE bond of
+  // length r0, 2: soft sphere); zero across chains
+  auto chain_pair = [&](float4 xa, int ja, int off, float r0, float &ox, float &oy, float &oz) {
+    ox = oy = oz = 0.0f;
+    const int jb = ja + off;
+    if (ja < bead_off || jb >= send) return;
+    const float4 xb = partner<LDS>(pin, s_pos, lds0, jb);
+    if ((__float_as_int(xb.w) >> 2) != (__float_as_int(xa.w) >> 2)) return;
+    const float dx = xb.x - xa.x, dy = xb.y - xa.y, dz = xb.z - xa.z;
+    const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+    float c;
+    if (off == 1) {
+      const float d = sqrtf(d2);
+      const float dev = d - r0;
+      const float gg = 1.0f - dev * dev * S.inv_R0sq;
+      c = S.k_bnd * dev * rcpf(d * gg);
+      if (gg <= 0.0f) atomicOr(&p.sys[s].err, ERR_BOND);
+    } else {
+      const float ir2 = rcpf(d2);
+      const float ir4 = ir2 * ir2;
+      c = -S.ss_f6 * (ir4 * ir4);
+    }
+    ox = c * dx;
+    oy = c * dy;
+    oz = c * dz;
+  };
+  float bx, by, bz, sx, sy, sz;
+  chain_pair(xc, i < bend ? i : send, 1, t_br, bx, by, bz);
+  chain_pair(xc, i < bend ? i : send, 2, 0.0f, sx, sy, sz);
+  // the partner halves from lanes m-1 (bond) and m-2 (soft sphere)
+  const int m1 = lane >= 1 ? lane - 1 : 0, m2 = lane >= 2 ? lane - 2 : 0;
+  float pbx = __shfl(bx, m1), pby = __shfl(by, m1), pbz = __shfl(bz, m1);
+  float psx = __shfl(sx, m2), psy = __shfl(sy, m2), psz = __shfl(sz, m2);
+  if (lane < 2 && i < bend) {  // pairs that start before the tile
+    float ex, ey, ez;
+    const float4 xp2 = i - 2 >= bead_off ? partner<LDS>(pin, s_pos, lds0, i - 2) : xc;
+    chain_pair(xp2, i - 2 >= bead_off ? i - 2 : send, 2, 0.0f, ex, ey, ez);
+    psx = ex; psy = ey; psz = ez;
+    if (lane == 0) {
+      const float4 xp1 = i - 1 >= bead_off ? partner<LDS>(pin, s_pos, lds0, i - 1) : xc;
+      chain_pair(xp1, i - 1 >= bead_off ? i - 1 : send, 1, br_before, ex, ey, ez);
+      pbx = ex; pby = ey; pbz = ez;
+    }
+  }
+  return make_float3((bx + sx) - (pbx + psx), (by + sy) - (pby + psy), (bz + sz) - (pbz + psz));
+}
+
+// The move of bead b0 + lane (or the force output) from its force mf without
+// noise and its three normals n0, n1, n2 of this step.
+template <bool LDS>
+__device__ __forceinline__ void integrate(const DevPtrs &p, const SysDev &S, int s, int i, int mode,
+                                          const float4 *__restrict__ pin, float4 *__restrict__ pout,
+                                          const float4 *s_pos, int lds0, float mfx, float mfy, float mfz, float n0,
+                                          float n1, float n2) {
+  if (mode == MODE_FORCE) {
+    p.fout[i] = make_float4(mfx, mfy, mfz, 0.0f);
+    return;
+  }
+  const float var = S.var;
+  const float ftx = mfx + n0 * var, fty = mfy + n1 * var, ftz = mfz + n2 * var;
+  if (mode == MODE_FORCE_NOISE) {
+    p.fout[i] = make_float4(ftx, fty, ftz, 0.0f);
+    return;
+  }
+  float4 x = partner<LDS>(pin, s_pos, lds0, i);
+  if (S.dyn == 0) {
+    // overdamped (sop.cu:487-520): x += (h/zeta) F
+    const float a5 = S.a5;
+    x.x = x.x + a5 * ftx;
+    x.y = x.y + a5 * fty;
+    x.z = x.z + a5 * ftz;
+  } else {
+    // underdamped (sop.cu:421-484): the reference's velocity update after its
+    // force evaluation, v = a3 incr + a4 F, happens here at the start of the
+    // next step, then incr = a1 v + a2 F, x += incr
+    const float4 st = p.vel[i];
+    float vx2 = st.x, vy2 = st.y, vz2 = st.z;
+    if (__float_as_int(st.w) == 1) {
+      vx2 = S.a3 * st.x + S.a4 * ftx;
+      vy2 = S.a3 * st.y + S.a4 * fty;
+      vz2 = S.a3 * st.z + S.a4 * ftz;
+    }
+    const float ix = S.a1 * vx2 + S.a2 * ftx, iy = S.a1 * vy2 + S.a2 * fty, iz = S.a1 * vz2 + S.a2 * ftz;
+    x.x = x.x + ix;
+    x.y = x.y + iy;
+    x.z = x.z + iz;
+    p.vel[i] = S.vupd ? make_float4(ix, iy, iz, __int_as_float(1)) : make_float4(vx2, vy2, vz2, 0.0f);
+  }
+  pout[i] = x;
+  if (!(isfinite(x.x) && isfinite(x.y) && isfinite(x.z))) atomicOr(&p.sys[s].err, ERR_NAN);
+}
+
 // One wave, one tile of 64 beads.  LPB lanes per bead gather its partners and
 // reduce with DPP; GPW = 64 / LPB beads per round, LPB rounds.  After each
 // round, lane m picks up the force of bead m of the tile from the group that
@@ -1296,7 +1405,6 @@ __device__ __forceinline__ void wave_tile(const DevPtrs &p, const SysDev &S, int
   const int bend = min(b0 + TILE, bead_off + n);
   // No minimum image: a state whose extent reaches boxl/2 - margin is refused
   // at each rebuild (ERR_PBC), so every separation here is below boxl/2.
-  const int64_t step = S.step + kstep;
   const int q1 = S.type_mask == 2 ? 3 : 0;  // type-pair index of a one-type system
   // slot q of the tile's order (tile_ord) is computed in round q / GPW by
   // group q % GPW; lane m's own bead b0 + m sits in slot qm
@@ -1441,105 +1549,12 @@ __device__ __forceinline__ void wave_tile(const DevPtrs &p, const SysDev &S, int
       mfz = vz;
     }
   }
-  // Chain terms, each pair once, over the tile's lanes: lane m computes the
-  // FENE bond (i, i+1) and the i,i+2 soft sphere of its bead i = b0 + m (the
-  // force on i; the partner takes the opposite), and takes the partner halves
-  // of the bond (i-1, i) and the pair (i-2, i) from lanes m-1 and m-2.  The
-  // pairs that start before the tile come from lanes 0 and 1 themselves.
-  {
-    const int i = b0 + lane;
-    const int send = bead_off + n;
-    float4 xc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (i < bend) xc = partner<LDS>(pin, s_pos, lds0, i);
-    // force on a from the pair (a, b) of chain offset off (1: FENE bond of
-    // length r0, 2: soft sphere); zero across chains
-    auto chain_pair = [&](float4 xa, int ja, int off, float r0, float &ox, float &oy, float &oz) {
-      ox = oy = oz = 0.0f;
-      const int jb = ja + off;
-      if (ja < bead_off || jb >= send) return;
-      const float4 xb = partner<LDS>(pin, s_pos, lds0, jb);
-      if ((__float_as_int(xb.w) >> 2) != (__float_as_int(xa.w) >> 2)) return;
-      const float dx = xb.x - xa.x, dy = xb.y - xa.y, dz = xb.z - xa.z;
-      const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-      float c;
-      if (off == 1) {
-        const float d = sqrtf(d2);
-        const float dev = d - r0;
-        const float gg = 1.0f - dev * dev * S.inv_R0sq;
-        c = S.k_bnd * dev * rcpf(d * gg);
-        if (gg <= 0.0f) atomicOr(&p.sys[s].err, ERR_BOND);
-      } else {
-        const float ir2 = rcpf(d2);
-        const float ir4 = ir2 * ir2;
-        c = -S.ss_f6 * (ir4 * ir4);
-      }
-      ox = c * dx;
-      oy = c * dy;
-      oz = c * dz;
-    };
-    float bx, by, bz, sx, sy, sz;
-    chain_pair(xc, i < bend ? i : send, 1, t_br, bx, by, bz);
-    chain_pair(xc, i < bend ? i : send, 2, 0.0f, sx, sy, sz);
-    // the partner halves from lanes m-1 (bond) and m-2 (soft sphere)
-    const int m1 = lane >= 1 ? lane - 1 : 0, m2 = lane >= 2 ? lane - 2 : 0;
-    float pbx = __shfl(bx, m1), pby = __shfl(by, m1), pbz = __shfl(bz, m1);
-    float psx = __shfl(sx, m2), psy = __shfl(sy, m2), psz = __shfl(sz, m2);
-    if (lane < 2 && i < bend) {  // pairs that start before the tile
-      float ex, ey, ez;
-      const float4 xp2 = i - 2 >= bead_off ? partner<LDS>(pin, s_pos, lds0, i - 2) : xc;
-      chain_pair(xp2, i - 2 >= bead_off ? i - 2 : send, 2, 0.0f, ex, ey, ez);
-      psx = ex; psy = ey; psz = ez;
-      if (lane == 0) {
-        const float4 xp1 = i - 1 >= bead_off ? partner<LDS>(pin, s_pos, lds0, i - 1) : xc;
-        chain_pair(xp1, i - 1 >= bead_off ? i - 1 : send, 1, br_before, ex, ey, ez);
-        pbx = ex; pby = ey; pbz = ez;
-      }
-    }
-    mfx += (bx + sx) - (pbx + psx);
-    mfy += (by + sy) - (pby + psy);
-    mfz += (bz + sz) - (pbz + psz);
-  }
-  const int i = b0 + lane;
-  if (i >= bend) return;
-  if (rm < r0 || rm >= r1) return;  // the other wave of a split tile computed this bead
-  if (MODE == MODE_FORCE) {
-    p.fout[i] = make_float4(mfx, mfy, mfz, 0.0f);
-    return;
-  }
-  float n0, n1, n2;
-  normals3(S.seed_lo, S.seed_hi, (uint32_t)(i - bead_off), step, n0, n1, n2);
-  const float var = S.var;
-  const float ftx = mfx + n0 * var, fty = mfy + n1 * var, ftz = mfz + n2 * var;
-  if (MODE == MODE_FORCE_NOISE) {
-    p.fout[i] = make_float4(ftx, fty, ftz, 0.0f);
-    return;
-  }
-  float4 x = partner<LDS>(pin, s_pos, lds0, i);
-  if (S.dyn == 0) {
-    // overdamped (sop.cu:487-520): x += (h/zeta) F
-    const float a5 = S.a5;
-    x.x = x.x + a5 * ftx;
-    x.y = x.y + a5 * fty;
-    x.z = x.z + a5 * ftz;
-  } else {
-    // underdamped (sop.cu:421-484): the reference's velocity update after its
-    // force evaluation, v = a3 incr + a4 F, happens here at the start of the
-    // next step, then incr = a1 v + a2 F, x += incr
-    const float4 st = p.vel[i];
-    float vx2 = st.x, vy2 = st.y, vz2 = st.z;
-    if (__float_as_int(st.w) == 1) {
-      vx2 = S.a3 * st.x + S.a4 * ftx;
-      vy2 = S.a3 * st.y + S.a4 * fty;
-      vz2 = S.a3 * st.z + S.a4 * ftz;
-    }
-    const float ix = S.a1 * vx2 + S.a2 * ftx, iy = S.a1 * vy2 + S.a2 * fty, iz = S.a1 * vz2 + S.a2 * ftz;
-    x.x = x.x + ix;
-    x.y = x.y + iy;
-    x.z = x.z + iz;
-    p.vel[i] = S.vupd ? make_float4(ix, iy, iz, __int_as_float(1)) : make_float4(vx2, vy2, vz2, 0.0f);
-  }
-  pout[i] = x;
-  if (!(isfinite(x.x) && isfinite(x.y) && isfinite(x.z))) atomicOr(&p.sys[s].err, ERR_NAN);
+  const float3 ch = chain_force<LDS>(p, S, s, b0, pin, s_pos, lds0, t_br, br_before);
+  if (b0 + lane >= bend || rm < r0 || rm >= r1) return;  // (a split tile's other beads are its other waves')
+  float n0 = 0.0f, n1 = 0.0f, n2 = 0.0f;
+  if (MODE != MODE_FORCE)
+    normals3(S.seed_lo, S.seed_hi, (uint32_t)(b0 + lane - bead_off), S.step + kstep, n0, n1, n2);
+  integrate<LDS>(p, S, s, b0 + lane, MODE, pin, pout, s_pos, lds0, mfx + ch.x, mfy + ch.y, mfz + ch.z, n0, n1, n2);
 }
 
 // Stage an item's arena beads [z, z + w) (whole tiles) into LDS.  Wave v
@@ -1593,13 +1608,12 @@ __device__ __forceinline__ void item_range(const DevPtrs &p, int tier, int &w0, 
 // Fused step over work items {first tile, tiles | waves per tile << 8, first
 // staged bead or -1, staged beads}: with s waves per tile, waves s k .. s k +
 // s - 1 of the block share tile first + k, each taking LPB / s consecutive
-// rounds (tiles * s <= STEP_WAVES).  The
-// LDS kernel (KLDS) takes the items whose systems fit in LDS and first copies
-// the staged arena beads (whole systems, each from its own coordinate buffer)
-// into dynamic LDS, so every partner gather is an LDS read; the other kernel
-// takes the items that gather from global memory (items[nitems .. nitems +
-// nitems_far)).  The result is identical either way.  Both are launched each
-// step, so each has its own register budget.
+// rounds (tiles * s <= STEP_WAVES).  The LDS kernel (KLDS) takes the items
+// whose systems fit in LDS and first copies the staged arena beads (whole
+// systems, each from its own coordinate buffer) into dynamic LDS, so every
+// partner gather is an LDS read; the other kernel takes the items that gather
+// from global memory (items[nitems .. nitems + nitems_far)).  The result is
+// identical either way, and k_step_tile's.
 template <int LPB, int MODE, bool KLDS>
 __device__ __forceinline__ void step_items(const DevPtrs &p, int kstep, float4 *s_pos, int tier) {
   const int tid = threadIdx.x;
@@ -1633,12 +1647,13 @@ __device__ __forceinline__ void step_items(const DevPtrs &p, int kstep, float4 *
       continue;
     }
     const int lds0 = KLDS ? it.z : 0;
+    // (staged systems are small enough for 16-bit rows)
     if (S.type_mask != 3) {
-      if (S.idx16) wave_tile<LPB, MODE, KLDS, true, true>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
-      else wave_tile<LPB, MODE, KLDS, false, true>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
+      if (KLDS || S.idx16) wave_tile<LPB, MODE, KLDS, true, true>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
+      else wave_tile<LPB, MODE, false, false, true>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
     } else {
-      if (S.idx16) wave_tile<LPB, MODE, KLDS, true, false>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
-      else wave_tile<LPB, MODE, KLDS, false, false>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
+      if (KLDS || S.idx16) wave_tile<LPB, MODE, KLDS, true, false>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
+      else wave_tile<LPB, MODE, false, false, false>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
     }
   }
 }
@@ -1992,6 +2007,240 @@ __global__ __launch_bounds__(STEP_THREADS) void k_step_far(DevPtrs p, int kstep)
   step_items<LPB, MODE, false>(p, kstep, nullptr, 0);
 }
 
+// ---- a block per tile
+//
+// The step of a small batch (at most TILE_STEP_PER_CU tiles per compute unit)
+// and of the systems too large to stage in LDS.  A small batch is bound by
+// latency, not by the vector ALUs: each compute unit has a handful of waves,
+// and with whole systems staged in LDS a 4,999-bead step spent 18,000 of its
+// 26,000 cycles waiting for the 80 KB copies of 79 blocks.  So nothing is
+// staged -- the positions are in the L2s, and a wave's gathers are issued in
+// batches of sixteen -- and a tile's work is spread over as many waves as it
+// has parts:
+//   - up to 8 waves take the rounds (64 / LPB beads each): heads, the row's
+//     chunks and native entries, gathers, forces, left in LDS;
+//   - one more wave draws the tile's noise and computes its chain terms beside
+//     them, then adds the forces up and moves the beads.
+// The arithmetic of a bead and its order are those of the item kernels:
+// results are identical.
+
+// The lane's bead of round r and its list ranges, from the tile's heads.
+struct RoundAt {
+  int li, i, ns, nc, nr;
+  uint32_t row;  // first entry of the row in the system's segment
+};
+template <int LPB>
+__device__ __forceinline__ RoundAt round_at(int r, int b0, int bend, int ordm, uint2 hd, int nat0, int reg0) {
+  constexpr int GPW = 64 / LPB;
+  RoundAt a;
+  a.li = __shfl(ordm, r * GPW + (int)(threadIdx.x & 63) / LPB);
+  const uint32_t cn = (uint32_t)__shfl((int)hd.x, a.li), po = (uint32_t)__shfl((int)hd.y, a.li);
+  a.i = b0 + a.li;
+  const bool in = a.i < bend;
+  a.nc = in ? (int)(cn & 0xFFFFu) : 0;
+  a.nr = in ? (int)(cn >> 16) : 0;
+  a.ns = nat0 + (int)(po >> 16);
+  a.row = (uint32_t)reg0 + (uint32_t)ROW_PAD * (po & 0xFFFFu);
+  return a;
+}
+
+// Gathered native and non-native force on the lane group's bead.
+template <int LPB, bool IDX16, bool ONE>
+__device__ __forceinline__ float3 tile_round(const DevPtrs &p, const SysDev &S, const float4 *__restrict__ pin, int self,
+                                             const RoundAt &a) {
+  const int l = (int)(threadIdx.x & 63) % LPB;
+  constexpr uint32_t ESZ = IDX16 ? 2u : 4u;
+  // buffer resources in scalar registers: the system's pair-list segment and
+  // the natives
+  const __amdgpu_buffer_rsrc_t rrow = buf_rsrc(p.plrep_j + S.pl_base, (uint32_t)S.n * (uint32_t)S.pl_cap * ESZ);
+  const __amdgpu_buffer_rsrc_t rnat = buf_rsrc(p.platt, 0xFFFFFFFFu);
+  constexpr int D = IDX16 ? 8 : 4;  // chunks of four entries held per lane
+  constexpr int NB = 4;             // natives held per lane
+  uint32_t q[16];
+  auto load_chunks = [&](int c0) {  // without a condition: past the segment a buffer load returns zeros
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      const uint32_t off = ESZ * a.row + 4u * ESZ * (uint32_t)(l + LPB * (c0 + k));
+      if constexpr (IDX16) {
+        const int2 v = load_i2(rrow, off);
+        q[2 * k] = (uint32_t)v.x;
+        q[2 * k + 1] = (uint32_t)v.y;
+      } else {
+        const uint4 v = load_b128(rrow, off);
+        q[4 * k] = v.x; q[4 * k + 1] = v.y; q[4 * k + 2] = v.z; q[4 * k + 3] = v.w;
+      }
+    }
+  };
+  int2 en[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    en[b] = make_int2(self, 0);  // past the list: the bead itself, which contributes nothing
+    if (l + LPB * b < a.nc) en[b] = load_i2(rnat, 8u * (uint32_t)(a.ns + l + LPB * b));
+  }
+  load_chunks(0);
+  const float4 xi = pin[self];
+  const int bead_off = S.bead_off;
+  const int row = ONE ? (S.type_mask == 2 ? 3 : 0) : (w_type(xi.w) - 1) * 2;  // type-pair index
+  const int nch = (a.nr + 3) >> 2;
+  const uint32_t sv = (uint32_t)(self - bead_off) * 0x10001u;
+  const float4 *__restrict__ base = pin + bead_off;
+  // the four partners of chunk position k (a lane past its row: the bead
+  // itself, whose d2 = 0 fails the guard)
+  auto gather = [&](int k, bool on, float4 *x) {
+    if constexpr (IDX16) {
+      const uint32_t w0 = on ? q[2 * k] : sv, w1 = on ? q[2 * k + 1] : sv;
+      x[0] = base[w0 & 0xFFFFu];
+      x[1] = base[w0 >> 16];
+      x[2] = base[w1 & 0xFFFFu];
+      x[3] = base[w1 >> 16];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = pin[on ? q[4 * k + e] : (uint32_t)self];
+    }
+  };
+  constexpr int R = 4;  // chunks in flight
+  float4 xn[NB], xr[R][4];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) xn[b] = pin[en[b].x];
+#pragma unroll
+  for (int k = 0; k < R; ++k)
+    if (__ballot(l + LPB * k < nch) != 0) gather(k, l + LPB * k < nch, xr[k]);
+  float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+  // native LJ: c = -12 eps u q6 (q6 - 1) with u = 1/d2, q6 = (r0^2 u)^3, as
+  // fma(t, q6, -t) with t = -12 eps u q6
+  {
+    const float eA = -12.0f * S.eps_att[row], eB = ONE ? eA : -12.0f * S.eps_att[row + 1];
+    auto nat = [&](float4 xj, float r0) {
+      const float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
+      const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+      const float eps = ONE ? eA : (w_type(xj.w) == 2 ? eB : eA);
+      const float r02 = r0 * r0;
+      const float ir2 = rcpf(d2);
+      const float q2 = r02 * ir2;
+      const float q6 = q2 * q2 * q2;
+      const float t = eps * ir2 * q6;
+      float c = fmaf(t, q6, -t);
+      c = d2 > 1.0e-7f * r02 ? c : 0.0f;
+      fx = fmaf(c, dx, fx);
+      fy = fmaf(c, dy, fy);
+      fz = fmaf(c, dz, fz);
+    };
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      if (__ballot(l + LPB * b < a.nc) != 0) nat(xn[b], __int_as_float(en[b].y));
+    for (int k = l + NB * LPB; k < a.nc; k += LPB) {
+      const int2 e = load_i2(rnat, 8u * (uint32_t)(a.ns + k));
+      nat(pin[e.x], __int_as_float(e.y));
+    }
+  }
+  // non-native repulsion: c = u q6 (m12 q6 + m6) with u = 1/d2, q6 =
+  // (sigma^2 u)^3, as u^4 (a u^3 + b) with a = m12 sigma^12, b = m6 sigma^6
+  {
+    const float aA = S.rep_a[row], aB = ONE ? aA : S.rep_a[row + 1];
+    const float bA = S.rep_b[row], bB = ONE ? bA : S.rep_b[row + 1];
+    const float gA = S.rep_guard[row], gB = ONE ? gA : S.rep_guard[row + 1];
+    auto rep = [&](const float4 *x) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float4 xj = x[e];
+        const float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
+        const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+        const bool tb = !ONE && w_type(xj.w) == 2;
+        const float u = rcpf(d2);
+        const float u2 = u * u;
+        float c = (u2 * u2) * fmaf(tb ? aB : aA, u2 * u, tb ? bB : bA);
+        c = d2 > (tb ? gB : gA) ? c : 0.0f;
+        fx = fmaf(c, dx, fx);
+        fy = fmaf(c, dy, fy);
+        fz = fmaf(c, dz, fz);
+      }
+    };
+    for (int c0 = 0;;) {
+#pragma unroll
+      for (int k = 0; k < D; ++k) {
+        if (__ballot(l + LPB * (c0 + k) < nch) == 0) break;
+        rep(xr[k % R]);
+        if (k + R < D && __ballot(l + LPB * (c0 + k + R) < nch) != 0)
+          gather((k + R) % D, l + LPB * (c0 + k + R) < nch, xr[k % R]);
+      }
+      c0 += D;
+      if (__ballot(l + LPB * c0 < nch) == 0) break;
+      load_chunks(c0);  // rows of more than D chunks a lane
+#pragma unroll
+      for (int k = 0; k < R; ++k) gather(k, l + LPB * (c0 + k) < nch, xr[k]);
+    }
+  }
+  return make_float3(group_sum<LPB>(fx), group_sum<LPB>(fy), group_sum<LPB>(fz));
+}
+
+// waves of a tile's rounds: one round each for up to 8 lanes per bead
+constexpr int tile_waves(int lpb) { return lpb < 8 ? lpb : 8; }
+
+template <int LPB>
+__global__ __launch_bounds__(64 * (tile_waves(LPB) + 1)) void k_step_tile(DevPtrs p, int kstep, int mode) {
+  constexpr int W = tile_waves(LPB);
+  __shared__ float s_f[3][TILE];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: system data in scalar registers
+  const int ntiles = *p.ntiles;
+  for (int w = blockIdx.x; w < ntiles; w += gridDim.x) {
+    if (w != (int)blockIdx.x) __syncthreads();  // the previous tile's forces have been read
+    const int2 it = p.tiles[w];
+    if (it.x < 0) continue;
+    const int t = it.x, s = it.y;
+    const int b0 = t * TILE;
+    const SysDev &S = p.sys[s];
+    if (wave < W) {
+      const int ordm = p.tile_ord[b0 + lane];
+      const uint2 hd = p.plhead[b0 + lane];
+      const int nat0 = p.nat_start[b0];
+      const int bead_off = S.bead_off;
+      const int bend = min(b0 + TILE, bead_off + S.n);
+      const float4 *__restrict__ pin = buf_in(p, S.parity + kstep);
+      if (mode != MODE_STEP || S.step + kstep < S.step_end) {
+        for (int r = wave; r < LPB; r += W) {
+          const RoundAt a = round_at<LPB>(r, b0, bend, ordm, hd, nat0, (b0 - bead_off) * S.pl_cap);
+          const int self = a.i < bend ? a.i : b0;  // a bead of this system: safe to gather
+          float3 f;
+          if (S.type_mask != 3)
+            f = S.idx16 ? tile_round<LPB, true, true>(p, S, pin, self, a) : tile_round<LPB, false, true>(p, S, pin, self, a);
+          else
+            f = S.idx16 ? tile_round<LPB, true, false>(p, S, pin, self, a) : tile_round<LPB, false, false>(p, S, pin, self, a);
+          if (lane % LPB == 0) {
+            s_f[0][a.li] = f.x;
+            s_f[1][a.li] = f.y;
+            s_f[2][a.li] = f.z;
+          }
+        }
+      }
+      __syncthreads();
+    } else {
+      const float br = p.bond_r0[b0 + lane], brb = p.bond_r0[max(b0 - 1, 0)];
+      const int bead_off = S.bead_off;
+      const int bend = min(b0 + TILE, bead_off + S.n);
+      const int par = S.parity + kstep;
+      const int64_t step = S.step + kstep;
+      const float4 *__restrict__ pin = buf_in(p, par);
+      float4 *__restrict__ pout = buf_out(p, par);
+      const int i = b0 + lane;
+      const bool over = mode == MODE_STEP && step >= S.step_end;
+      float n0 = 0.0f, n1 = 0.0f, n2 = 0.0f;
+      float3 ch = make_float3(0.0f, 0.0f, 0.0f);
+      if (over) {
+        // finished inside this block of steps: carry the coordinates over
+        if (i < bend) pout[i] = pin[i];
+      } else {
+        ch = chain_force<false>(p, S, s, b0, pin, nullptr, 0, i < bend ? br : 0.0f, b0 > bead_off ? brb : 0.0f);
+        if (mode != MODE_FORCE) normals3(S.seed_lo, S.seed_hi, (uint32_t)(i - bead_off), step, n0, n1, n2);
+      }
+      __syncthreads();
+      if (!over && i < bend)
+        integrate<false>(p, S, s, i, mode, pin, pout, nullptr, 0, s_f[0][lane] + ch.x, s_f[1][lane] + ch.y,
+                         s_f[2][lane] + ch.z, n0, n1, n2);
+    }
+  }
+}
+
 // ------------------------------------------------ energies / observables
 
 // 16 lanes per bead; FP32 pair energies, FP64 accumulation; pairs are seen
@@ -2263,14 +2512,8 @@ __global__ void k_selftest(int *out, float *fout) {
 
 #define SOPK_LAUNCH_CHECK() hipGetLastError()
 
-// The whole-CU and global-gather launches of the step kernel and of the shell
-// filter go on a side stream beside the two-blocks-per-unit LDS launch when
-// both sides have work: fork (side waits for st) and join (st waits for
-// side).  Under graph capture these become two graph branches.
-static bool fork_wanted(const StepFork *fk, const StepGrids &sg) {
-  return fk && sg.grid > 0 && (sg.grid_big > 0 || sg.grid_far > 0);
-}
-
+// Fork (the side stream waits for st) and join (st waits for the side
+// stream).  Under graph capture these become two graph branches.
 static hipError_t fork_begin(const StepFork *fk, hipStream_t st) {
   hipError_t h = hipEventRecord(fk->fork, st);
   if (h == hipSuccess) h = hipStreamWaitEvent(fk->side, fk->fork, 0);
@@ -2350,9 +2593,21 @@ hipError_t launch_lists(const DevPtrs &p, const ListGrids &lg, int kstep, int fl
 }
 
 template <int MODE>
+static void launch_step_lds(const DevPtrs &p, int lpb, int grid, size_t lds, int kstep, int tier, hipStream_t st) {
+  const dim3 g(grid), b(STEP_THREADS);
+  switch (lpb) {
+    case 4: hipLaunchKernelGGL((k_step<4, MODE>), g, b, lds, st, p, kstep, tier); break;
+    case 8: hipLaunchKernelGGL((k_step<8, MODE>), g, b, lds, st, p, kstep, tier); break;
+    case 32: hipLaunchKernelGGL((k_step<32, MODE>), g, b, lds, st, p, kstep, tier); break;
+    default: hipLaunchKernelGGL((k_step<16, MODE>), g, b, lds, st, p, kstep, tier); break;
+  }
+}
+
+template <int MODE>
 static hipError_t launch_step_mode(const DevPtrs &p, int lpb, const StepGrids &sg, int kstep, hipStream_t st,
                                    const StepFork *fk) {
-  const bool fork = fork_wanted(fk, sg);
+  // the whole-CU and per-tile launches beside the two-blocks-per-unit one
+  const bool fork = fk && sg.grid > 0 && (sg.grid_big > 0 || sg.grid_far > 0 || sg.tiles > 0);
   if (fork) {
     const hipError_t h = fork_begin(fk, st);
     if (h != hipSuccess) return h;
@@ -2360,21 +2615,25 @@ static hipError_t launch_step_mode(const DevPtrs &p, int lpb, const StepGrids &s
   const hipStream_t far_st = fork ? fk->side : st;
   for (int tier = 0; tier < 2; ++tier) {
     const int grid = tier ? sg.grid_big : sg.grid;
-    const size_t lds = tier ? sg.lds_big : sg.lds;
-    hipStream_t ts = tier ? far_st : st;
-    if (grid > 0) switch (lpb) {
-      case 4: hipLaunchKernelGGL((k_step<4, MODE>), dim3(grid), dim3(STEP_THREADS), lds, ts, p, kstep, tier); break;
-      case 8: hipLaunchKernelGGL((k_step<8, MODE>), dim3(grid), dim3(STEP_THREADS), lds, ts, p, kstep, tier); break;
-      case 32: hipLaunchKernelGGL((k_step<32, MODE>), dim3(grid), dim3(STEP_THREADS), lds, ts, p, kstep, tier); break;
-      default: hipLaunchKernelGGL((k_step<16, MODE>), dim3(grid), dim3(STEP_THREADS), lds, ts, p, kstep, tier); break;
+    if (grid > 0) launch_step_lds<MODE>(p, lpb, grid, tier ? sg.lds_big : sg.lds, kstep, tier, tier ? far_st : st);
+  }
+  if (sg.grid_far > 0) {
+    const dim3 g(sg.grid_far), b(STEP_THREADS);
+    switch (lpb) {
+      case 4: hipLaunchKernelGGL((k_step_far<4, MODE>), g, b, 0, far_st, p, kstep); break;
+      case 8: hipLaunchKernelGGL((k_step_far<8, MODE>), g, b, 0, far_st, p, kstep); break;
+      case 32: hipLaunchKernelGGL((k_step_far<32, MODE>), g, b, 0, far_st, p, kstep); break;
+      default: hipLaunchKernelGGL((k_step_far<16, MODE>), g, b, 0, far_st, p, kstep); break;
     }
   }
-  const int grid_far = sg.grid_far;
-  if (grid_far > 0) switch (lpb) {
-    case 4: hipLaunchKernelGGL((k_step_far<4, MODE>), dim3(grid_far), dim3(STEP_THREADS), 0, far_st, p, kstep); break;
-    case 8: hipLaunchKernelGGL((k_step_far<8, MODE>), dim3(grid_far), dim3(STEP_THREADS), 0, far_st, p, kstep); break;
-    case 32: hipLaunchKernelGGL((k_step_far<32, MODE>), dim3(grid_far), dim3(STEP_THREADS), 0, far_st, p, kstep); break;
-    default: hipLaunchKernelGGL((k_step_far<16, MODE>), dim3(grid_far), dim3(STEP_THREADS), 0, far_st, p, kstep); break;
+  if (sg.tiles > 0) {
+    const dim3 g(sg.tiles), b(64 * (tile_waves(lpb) + 1));
+    switch (lpb) {
+      case 4: hipLaunchKernelGGL(k_step_tile<4>, g, b, 0, far_st, p, kstep, MODE); break;
+      case 8: hipLaunchKernelGGL(k_step_tile<8>, g, b, 0, far_st, p, kstep, MODE); break;
+      case 32: hipLaunchKernelGGL(k_step_tile<32>, g, b, 0, far_st, p, kstep, MODE); break;
+      default: hipLaunchKernelGGL(k_step_tile<16>, g, b, 0, far_st, p, kstep, MODE); break;
+    }
   }
   hipError_t h = SOPK_LAUNCH_CHECK();
   if (fork && h == hipSuccess) h = fork_end(fk, st);
@@ -2391,13 +2650,13 @@ hipError_t launch_step(const DevPtrs &p, int mode, int lpb, const StepGrids &sg,
 // Allow the step kernels dynamic LDS up to `bytes`.
 hipError_t step_lds_limit(size_t bytes) {
   hipError_t h = hipSuccess;
-#define SOPK_LDS_ATTR(L, M)                                                                                      \
-  if (h == hipSuccess)                                                                                           \
-    h = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_step<L, M>), hipFuncAttributeMaxDynamicSharedMemorySize, \
-                            (int)bytes);
-  SOPK_LDS_ATTR(4, 0) SOPK_LDS_ATTR(8, 0) SOPK_LDS_ATTR(16, 0) SOPK_LDS_ATTR(32, 0)
-  SOPK_LDS_ATTR(4, 1) SOPK_LDS_ATTR(8, 1) SOPK_LDS_ATTR(16, 1) SOPK_LDS_ATTR(32, 1)
-  SOPK_LDS_ATTR(4, 2) SOPK_LDS_ATTR(8, 2) SOPK_LDS_ATTR(16, 2) SOPK_LDS_ATTR(32, 2)
+  auto allow = [&](auto *k) {
+    if (h == hipSuccess)
+      h = hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  };
+#define SOPK_LDS_ATTR(L)                                                                            \
+  allow(&k_step<L, MODE_STEP>), allow(&k_step<L, MODE_FORCE>), allow(&k_step<L, MODE_FORCE_NOISE>);
+  SOPK_LDS_ATTR(4) SOPK_LDS_ATTR(8) SOPK_LDS_ATTR(16) SOPK_LDS_ATTR(32)
 #undef SOPK_LDS_ATTR
   return h;
 }

@@ -151,6 +151,8 @@ struct DevPtrs {
   int32_t *tile_sys;    // system slot of each tile
   uint8_t *tile_ord;    // per tile: TILE bead offsets in the order the step kernel's lane groups take them
   int32_t *work;        // tile ids to process (-1 = padding), XCD-interleaved
+  int2 *tiles;          // tiles that step with a block each: {tile, system slot}, tile -1 = padding
+  int32_t *ntiles;
   int32_t *nwork;
   int32_t *syslist;     // system slots of the current batch, those of more than SORT_N_MAX beads first
   int32_t *nsys;
@@ -176,12 +178,19 @@ struct DevPtrs {
 constexpr int STEP_WAVES = 16;
 constexpr int STEP_THREADS = 64 * STEP_WAVES;
 
-// Grids of the step kernel's three launches: items staged in LDS at two
-// blocks per compute unit, items staged in a whole compute unit's LDS, items
-// that gather from global memory.
+// Batches of up to this many tiles per compute unit step with a block per
+// tile (k_step_tile), whatever their systems' sizes.
+constexpr int TILE_STEP_PER_CU = 2;
+// The tiles of systems that gather from global memory do so up to this many.
+constexpr int TILE_STEP_FAR_PER_CU = 4;
+
+// Grids of the step's launches: items staged in LDS at two blocks per compute
+// unit, items staged in a whole compute unit's LDS, items that gather from
+// global memory, and tiles with a block each (the step kernel only).
 struct StepGrids {
   int grid, grid_big, grid_far;
   size_t lds, lds_big;
+  int tiles;
 };
 
 // A second stream and two events: the step launches of the whole-CU and

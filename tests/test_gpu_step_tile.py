@@ -1,0 +1,103 @@
+"""The step with a block per tile against the item kernels, on device 0.
+
+Small batches, and the few systems too large to stage, take a block per tile;
+step_tiles asks for the item kernels instead.  Both run the same arithmetic in
+the same order, so coordinates, forces and velocities are bitwise equal: at
+tile remainders, with rows longer than one block of held chunks, native lists
+longer than the held ones, no natives, two bead types, several chains, jobs
+that end inside a block of steps, underdamped dynamics, every lane count, and
+either side of the tile counts where the launch changes.
+"""
+import numpy as np
+import pytest
+
+import sop_amd as S
+from sop_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def chain(seed, n, types=1, under=False, natives=True, chains=1):
+    s = S.make_chain_system(seed, n)
+    rng = np.random.default_rng(seed)
+    s.params.seed = W.philox_key(41, seed)
+    if types == 2:
+        s.type = rng.integers(1, 3, n).astype(np.int32)
+        for i in (1, 2):
+            for j in (1, 2):
+                s.params.sigma_rep[i][j] = 3.8 + 0.1 * (i + j - 2)
+                s.params.eps_att[i][j] = 1.0 - 0.1 * (i + j - 2)
+    if under:
+        s.params.dynamics, s.params.h, s.params.zeta = S._abi.DYN_UNDERDAMPED, 2.5e-3, 0.05
+        s.vel = rng.normal(0, 0.7, (n, 3)).astype(np.float32)
+    if not natives:
+        s.nat_i, s.nat_j, s.nat_r0 = (np.zeros(0, d) for d in (np.int32, np.int32, np.float32))
+    if chains > 1:
+        s.chain = np.sort(rng.integers(0, chains, n)).astype(np.int32)
+        keep = ~((s.chain[s.nat_i] == s.chain[s.nat_j]) & (s.nat_j - s.nat_i <= 2))
+        s.nat_i, s.nat_j, s.nat_r0 = s.nat_i[keep], s.nat_j[keep], s.nat_r0[keep]
+    return s
+
+
+def outputs(systems, steps, **opts):
+    with S.Engine(0, **opts) as e:
+        ids = [e.add(s) for s in systems]
+        f0 = [e.force_eval(i, with_noise=k % 2 == 1) for k, i in enumerate(ids)]
+        e.run(ids, steps)
+        return f0 + [e.coords(i) for i in ids] + [e.velocities(i) for i in ids]
+
+
+@pytest.mark.parametrize("systems,steps,lanes", [
+    ([(1, 1), (2, 2), (3, 63), (4, 64), (5, 65)], 60, 4),
+    ([(6, 700, 2)], 60, 4),
+    ([(7, 700, 2, True), (8, 129)], 60, 4),
+    ([(9, 900, 1, False, False)], 30, 4),
+    ([(10, 900, 1, False, True, 5)], 55, 4),
+    ([(11, 1500)], 30, 8),
+    ([(12, 600, 2)], 30, 16),
+    ([(13, 600)], 30, 32),
+    ([(14, 11000)], 20, 4),
+    ([(15, 66000, 1, False, False)], 12, 4),  # 32-bit rows
+    ([(16, 8000), (17, 3000), (18, 8000)], 12, 4),
+])
+def test_tile_step_equals_item_step(systems, steps, lanes):
+    made = [chain(*a) for a in systems]
+    got = outputs(made, steps, lanes_per_bead=lanes)
+    want = outputs(made, steps, lanes_per_bead=lanes, step_tiles=16)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+
+
+def test_dense_rows_and_many_natives():
+    """Rows of several hundred partners and up to 40 natives a bead."""
+    n = 1400
+    s = chain(21, n)
+    s.xyz = (s.xyz * np.float32(0.55)).astype(np.float32)
+    s.bond_r0 = (s.bond_r0 * np.float32(0.55)).astype(np.float32)
+    rng = np.random.default_rng(3)
+    i, j = np.triu_indices(n, 3)
+    pick = rng.random(len(i)) < 40.0 / n
+    s.nat_i, s.nat_j = i[pick].astype(np.int32), j[pick].astype(np.int32)
+    s.nat_r0 = np.linalg.norm(s.xyz[s.nat_i] - s.xyz[s.nat_j], axis=1).astype(np.float32)
+    f = []
+    for tiles in (0, 16):
+        with S.Engine(0, step_tiles=tiles) as e:
+            k = e.add(s)
+            assert e.rows(k)[1] > 256
+            f.append(e.force_eval(k))
+    assert np.array_equal(*f)
+
+
+@pytest.mark.parametrize("replicas,n", [(8, 4032), (8, 4096), (9, 4096)])
+def test_either_side_of_the_tile_count(replicas, n):
+    base = chain(31, n)
+    made = []
+    for r in range(replicas):
+        t = S.System(xyz=base.xyz, params=S.copy_params(base.params), bond_r0=base.bond_r0, nat_i=base.nat_i,
+                     nat_j=base.nat_j, nat_r0=base.nat_r0)
+        t.params.seed = W.philox_key(43, r)
+        made.append(t)
+    got = outputs(made, 20)
+    want = outputs(made, 20, step_tiles=16)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
