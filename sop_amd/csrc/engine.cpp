@@ -157,7 +157,7 @@ StepGrids filter_grids(const sop_engine *e) {
   const int g = e->step_blocks > 0 ? e->step_blocks : default_step_blocks(e);
   return StepGrids{items_grid(e->fixed_grids ? g : std::max(g, 8 * e->num_cu), e->fixed_grids, e->cur_nfitems),
                    items_grid_big(e, e->cur_nfitems_big),
-                   items_grid(2 * e->num_cu, e->fixed_grids, e->cur_nfitems_far), e->cur_flds, e->cur_flds_big, 0};
+                   items_grid(2 * e->num_cu, e->fixed_grids, e->cur_nfitems_far), e->cur_flds, e->cur_flds_big, grid_step_tiles(e)};
 }
 
 ListGrids list_grids(const sop_engine *e) {
@@ -909,7 +909,8 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   int32_t per_step = e->opts.step_tiles;
   if (per_step <= 0) per_step = total_tiles > slots_w ? STEP_WAVES : (2 * total_tiles > slots_w ? 8 : 4);
   e->cur_step_tiles = per_step;
-  // the step's tiles with a block each (k_step_tile): all of a batch of up to
+  // the tiles with a block each in the step and the shell filter (k_step_tile,
+  // k_filter_tile): all of a batch of up to
   // TILE_STEP_PER_CU tiles per compute unit; else the systems too large for
   // two LDS blocks per unit while theirs are that few, and the ones too large
   // for any LDS tier up to TILE_STEP_FAR_PER_CU.  Step times by tile against
@@ -928,6 +929,7 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   const bool mid_by_tile = mid_tiles + far_tiles <= tile_cap && !own_items;
   const bool far_by_tile = far_tiles <= (int64_t)TILE_STEP_FAR_PER_CU * e->num_cu && !own_items;
   auto tile_step = [&](const SysHost &h) {
+    if (h.n > 65536) return false;  // 16-bit rows only
     return by_tile || (h.bead_len > lds_cap && (mid_by_tile || (far_by_tile && h.bead_len > big_cap)));
   };
   std::vector<int2> tiles;
@@ -976,7 +978,7 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     };
     for (int32_t sl : by_arena) {
       const SysHost &h = e->sys[sl];
-      if (split && tile_step(h)) continue;
+      if (tile_step(h)) continue;
       const int32_t t0 = (int32_t)(h.bead_off / TILE), nt = (int32_t)(h.bead_len / TILE);
       const int32_t per = per_fixed > 0 ? per_fixed : per_of(h);
       if (h.bead_len <= lds_cap) {

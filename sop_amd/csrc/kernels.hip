@@ -1658,6 +1658,27 @@ __device__ __forceinline__ void step_items(const DevPtrs &p, int kstep, float4 *
   }
 }
 
+// The tile's bead order for the filter and the step kernel: decreasing row
+// length (shell-row length + the last native pair-list length), ties by
+// index, so that the beads one round of lane groups takes together run loops
+// of similar length.  Computed at grid and neighbor-list builds (before this
+// pass rewrites platt_cnt): shell builds keep the order of the grid build that
+// made their shell rows (row lengths change little between them).  The order
+// only groups beads into rounds; no result depends on it.  Returns the bead of
+// slot `lane`; beads past the system's end come last.
+__device__ __forceinline__ int tile_order(const DevPtrs &p, int t, int build, bool tin, int nr, bool write) {
+  const int lane = threadIdx.x & 63;
+  if (build == BUILD_SHELL) return p.tile_ord[t * TILE + lane];
+  const int key = tin ? nr + p.platt_cnt[t * TILE + lane] : -1;
+  int rank = 0;
+  for (int j = 0; j < TILE; ++j) {
+    const int kj = __builtin_amdgcn_readlane(key, j);
+    rank += (kj > key) | ((kj == key) & (j < lane));
+  }
+  if (write) p.tile_ord[t * TILE + rank] = (uint8_t)lane;
+  return __builtin_amdgcn_ds_permute(rank << 2, lane);  // slot lane holds the bead of that rank
+}
+
 // Pair list of one tile's beads = their shell rows filtered at x with the
 // reference's exact predicate (d2 < rc_pl^2, squares summed in order without
 // contraction), for grid and shell builds, and the native pair list from the
@@ -1694,26 +1715,7 @@ __device__ __forceinline__ void filter_tile(const DevPtrs &p, const SysDev &S, i
   const bool tin = t * TILE + lane < bend;
   const int t_nr = tin ? p.slrep_cnt[t * TILE + lane] : 0;
   const int t_ns = tin ? p.nat_start[t * TILE + lane] : 0, t_nn = tin ? p.nat_cnt[t * TILE + lane] : 0;
-  // the tile's bead order for this filter and the step kernel: decreasing row
-  // length (shell-row length + the native pair-list length), ties by index, so
-  // that the beads one round of lane groups takes together run loops of
-  // similar length.  Computed at grid and neighbor-list builds: shell builds
-  // keep the order of the grid build that made their shell rows (row lengths
-  // change little between them).  The order only groups beads into rounds; no
-  // result depends on it.
-  int ordm;
-  if (S.build == BUILD_SHELL) {
-    ordm = p.tile_ord[t * TILE + lane];
-  } else {
-    const int key = tin ? t_nr + p.platt_cnt[t * TILE + lane] : -1;
-    int rank = 0;
-    for (int j = 0; j < TILE; ++j) {
-      const int kj = __shfl(key, j);
-      rank += (kj > key) | ((kj == key) & (j < lane));
-    }
-    p.tile_ord[t * TILE + rank] = (uint8_t)lane;
-    ordm = __builtin_amdgcn_ds_permute(rank << 2, lane);  // slot lane holds bead ordm
-  }
+  const int ordm = tile_order(p, t, S.build, tin, t_nr, true);
   const double plf = S.pl_factor;
   const float pla = S.pl_abs;
   ent_t *const seg = reinterpret_cast<ent_t *>(p.plrep_j + pl_base);
@@ -1995,6 +1997,249 @@ __global__ __launch_bounds__(STEP_THREADS) void k_shell_filter(DevPtrs p, int ks
   }
 }
 
+// ---- the same by a block per tile
+//
+// The filter of the systems that step with a block per tile.  One wave per
+// tile is a chain of some 40 dependent round trips (the rounds' row batches,
+// gathers, natives and write passes): 25 us for a 4,999-bead system, 46 for
+// 10,000, in which most compute units stood empty.  Here eight waves take eight
+// rows each, a row 64 entries per pass -- all their entries loaded, then all
+// their partners gathered, at once -- and four waves the natives of sixteen
+// beads each; one exchange of the waves' totals gives every list its place,
+// and the kept entries are written from registers.  Lane 16 q + 4 e + l takes
+// entry 16 q + 4 l + e of its pass: a row's kept entries come out in the order
+// of the item kernel.  The native lists are packed in bead order.
+constexpr int FILTER_ROW_WAVES = 8, FILTER_NAT_WAVES = 4;
+constexpr int FILTER_TILE_THREADS = 64 * (FILTER_ROW_WAVES + FILTER_NAT_WAVES);
+
+template <bool ONE>
+__device__ __forceinline__ void filter_rows(const DevPtrs &p, const SysDev &S, int b0, int nb, int wave,
+                                            const float4 *__restrict__ pin, int *s_len, const int *s_nlen,
+                                            const int2 *s_nat) {
+  constexpr int R = TILE / FILTER_ROW_WAVES, NP = 2;  // rows of the wave, passes held in registers
+  constexpr uint32_t PAST = 0xFFFFFF00u;  // beyond any segment: a load returns 0, a store is dropped
+  const int lane = threadIdx.x & 63;
+  const int bo = S.bead_off, pl_cap = S.pl_cap;
+  const bool nlb = S.build == BUILD_NL;
+  const uint32_t bytes = (uint32_t)S.n * (uint32_t)pl_cap * 2u;  // 16-bit entries
+  const __amdgpu_buffer_rsrc_t rin = buf_rsrc(p.slrep_j + S.pl_base, bytes), rout = buf_rsrc(p.plrep_j + S.pl_base, bytes);
+  const uint32_t region = (uint32_t)(b0 - bo) * (uint32_t)pl_cap;  // this tile's first entry
+  auto load = [&](uint32_t entry, bool on) -> int {
+    return (int)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rin, (int)(on ? 2u * entry : PAST), 0, 0);
+  };
+  auto store = [&](uint32_t entry, bool on, int v) {
+    __builtin_amdgcn_raw_buffer_store_b16((unsigned short)v, rout, (int)(on ? 2u * entry : PAST), 0, 0);
+  };
+  const bool tin = lane < nb;
+  const int t_nr = tin ? p.slrep_cnt[b0 + lane] : 0;
+  const int ordm = tile_order(p, b0 / TILE, S.build, tin, t_nr, wave == 0);
+  const int o_nr = __shfl(t_nr, ordm);  // by slot
+  const int eo = (lane & 48) + 4 * (lane & 3) + ((lane >> 2) & 3);
+  const float4 *__restrict__ base = pin + bo;
+  const int vself = b0 - bo;  // a lane without an entry gathers a bead of the system
+  int nr[R], li[R], e[R][NP];
+#pragma unroll
+  for (int g = 0; g < R; ++g) {
+    nr[g] = __builtin_amdgcn_readlane(o_nr, R * wave + g);
+    li[g] = __builtin_amdgcn_readlane(ordm, R * wave + g);
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+      e[g][u] = load(region + (uint32_t)(li[g] * pl_cap + 64 * u + eo), 64 * u + eo < nr[g]);
+  }
+  const float rc11 = S.rc2_pl_rep[0], rc12 = S.rc2_pl_rep[1], rc21 = S.rc2_pl_rep[2], rc22 = S.rc2_pl_rep[3];
+  float4 xi[R];
+#pragma unroll
+  for (int g = 0; g < R; ++g) xi[g] = pin[b0 + min(li[g], nb - 1)];
+  // the reference's predicate without the minimum image, which is the identity
+  // here (a grid build whose extent reaches boxl/2 - margin raises ERR_PBC, and
+  // beads move less than the margin before the next)
+  auto kept = [&](int g, bool valid, float4 xj) {
+    const bool t2 = w_type(xi[g].w) == 2;
+    const float rcA = ONE ? (t2 ? rc22 : rc11) : (t2 ? rc21 : rc11), rcB = t2 ? rc22 : rc12;
+    const float dx = xj.x - xi[g].x, dy = xj.y - xi[g].y, dz = xj.z - xi[g].z;
+    const float rc = ONE ? rcA : (w_type(xj.w) == 2 ? rcB : rcA);
+    return valid & (nlb | (((dx * dx + dy * dy) + dz * dz) < rc));
+  };
+  uint64_t m[R][NP];
+#pragma unroll
+  for (int h = 0; h < R; h += R / 2) {  // half the wave's rows gathered at a time
+    float4 xj[R / 2][NP];
+#pragma unroll
+    for (int g = 0; g < R / 2; ++g)
+#pragma unroll
+      for (int u = 0; u < NP; ++u) xj[g][u] = base[64 * u + eo < nr[h + g] ? e[h + g][u] : vself];
+#pragma unroll
+    for (int g = 0; g < R / 2; ++g)
+#pragma unroll
+      for (int u = 0; u < NP; ++u)
+        m[h + g][u] = __builtin_amdgcn_ballot_w64(kept(h + g, 64 * u + eo < nr[h + g], xj[g][u]));
+  }
+  // passes past the held ones: counted now, filtered again when written
+  auto tail = [&](int g, bool write, int at) {
+    int c = 0;
+    for (int m0 = 64 * NP; m0 < nr[g]; m0 += 64) {
+      const bool valid = m0 + eo < nr[g];
+      const int v = load(region + (uint32_t)(li[g] * pl_cap + m0 + eo), valid);
+      const bool k = kept(g, valid, base[valid ? v : vself]);
+      const uint64_t mk = __builtin_amdgcn_ballot_w64(k);
+      if (write) store(region + (uint32_t)(at + c + lanes_below(mk)), k, v);
+      c += __popcll(mk);
+    }
+    return c;
+  };
+  int cnt[R], sum = 0;
+#pragma unroll
+  for (int g = 0; g < R; ++g) {
+    cnt[g] = tail(g, false, 0);
+#pragma unroll
+    for (int u = 0; u < NP; ++u) cnt[g] += __popcll(m[g][u]);
+    sum += (cnt[g] + ROW_PAD - 1) & ~(ROW_PAD - 1);
+  }
+  if (lane == 0) s_len[wave] = sum;
+  __syncthreads();
+  int packed = 0;
+  for (int v = 0; v < wave; ++v) packed += s_len[v];
+  int c_q = 0, s_q = 0;
+#pragma unroll
+  for (int g = 0; g < R; ++g) {
+    int at = packed;
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      store(region + (uint32_t)(at + lanes_below(m[g][u])), (m[g][u] >> lane) & 1, e[g][u]);
+      at += __popcll(m[g][u]);
+    }
+    if (nr[g] > 64 * NP) at += tail(g, true, at);
+    // padded to a multiple of ROW_PAD with the bead itself (its d2 = 0 fails the
+    // step kernel's repulsion guard)
+    const int len = (cnt[g] + ROW_PAD - 1) & ~(ROW_PAD - 1);
+    store(region + (uint32_t)(at + lane), lane < len - cnt[g], b0 - bo + li[g]);
+    c_q = lane == g ? cnt[g] : c_q;
+    s_q = lane == g ? packed : s_q;
+    packed += len;
+  }
+  const int lb = __shfl(ordm, R * wave + (lane & (R - 1)));
+  if (lane < R && lb < nb) {
+    int2 nat = s_nat[lb];  // {length, offset within its wave's sixteen beads}
+    if (!nlb)
+      for (int v = 0; v < lb / 16; ++v) nat.y += s_nlen[v];
+    const int i = b0 + lb;
+    p.plrep_cnt[i] = c_q;
+    p.plrep_off[i] = (int)region + s_q;
+    p.plhead[i] = make_uint2((uint32_t)nat.x | ((uint32_t)c_q << 16), (uint32_t)(s_q / ROW_PAD) | ((uint32_t)nat.y << 16));
+  }
+}
+
+// Natives within their pair cutoff of sixteen beads, four lanes each: keep
+// decisions and counts, then the entries at the lists' places.  Keep bits hold
+// 32 batches of four (128 natives of a bead); past them the decision is made
+// again for the writes, and batches past the first NB are loaded again.
+__device__ __forceinline__ void filter_nats(const DevPtrs &p, const SysDev &S, int b0, int nb, int wave,
+                                            const float4 *__restrict__ pin, int *s_nlen, int2 *s_nat) {
+  constexpr int NB = 4;
+  const int lane = threadIdx.x & 63, g = lane >> 2, l = lane & 3;
+  const uint32_t below = (1u << l) - 1u;
+  const int lb = 16 * wave + g;
+  const bool act = lb < nb, nlb = S.build == BUILD_NL;
+  const int i = b0 + min(lb, nb - 1);
+  const int nat0 = p.nat_start[b0];
+  const int ns = p.nat_start[i], nn = act && !nlb ? p.nat_cnt[i] : 0;
+  if (nlb) {  // k_rows has left the lists in the beads' own slots
+    if (act && l == 0) s_nat[lb] = make_int2(p.platt_cnt[i], p.platt_off[i] - nat0);
+    __syncthreads();
+    return;
+  }
+  const double plf = S.pl_factor;
+  const float pla = S.pl_abs;
+  int j[NB];
+  float r0[NB];
+  auto load = [&](int m0) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int k = l + 4 * (m0 + b);
+      j[b] = i;
+      r0[b] = 0.0f;
+      if (k < nn) {
+        j[b] = p.nat_j[ns + k];
+        r0[b] = p.nat_r0[ns + k];
+      }
+    }
+  };
+  load(0);
+  const float4 xi = pin[i];
+  const bool multi = __ballot(nn > 4 * NB) != 0;
+  uint32_t km = 0;  // keep bits: bit m0 + b for the lane's entry l + 4 (m0 + b)
+  auto pass = [&](bool wr, int o0) {
+    int c = 0;
+    for (int m0 = 0; __ballot(l + 4 * m0 < nn) != 0; m0 += NB) {
+      if (m0 > 0 || (wr && multi)) load(m0);
+      float4 xj[NB];
+      const bool test = !wr || m0 >= 32;
+      if (test) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) xj[b] = pin[j[b]];
+      }
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const int bit = m0 + b;
+        bool keep;
+        if (test) {
+          const float rc = cutoff_of(plf, pla, r0[b]);
+          const float dx = xj[b].x - xi.x, dy = xj[b].y - xi.y, dz = xj[b].z - xi.z;
+          keep = (l + 4 * bit < nn) & (((dx * dx + dy * dy) + dz * dz) < rc * rc);
+          if (!wr && bit < 32 && keep) km |= 1u << bit;
+        } else {
+          keep = (km >> bit) & 1u;
+        }
+        const uint32_t bits = (uint32_t)(__ballot(keep) >> (4 * g)) & 0xFu;
+        if (wr && keep) p.platt[o0 + c + __popc(bits & below)] = make_int2(j[b], __float_as_int(r0[b]));
+        c += __popc(bits);
+      }
+    }
+    return c;
+  };
+  const int c = pass(false, 0);
+  const int incl = wave_incl_scan(l == 0 ? c : 0);
+  if (lane == 63) s_nlen[wave] = incl;
+  if (act && l == 0) s_nat[lb] = make_int2(c, incl - c);
+  __syncthreads();
+  int off = incl - c;
+  for (int v = 0; v < wave; ++v) off += s_nlen[v];
+  pass(true, nat0 + off);
+  if (act && l == 0) {
+    p.platt_cnt[i] = c;
+    p.platt_off[i] = nat0 + off;
+  }
+}
+
+__global__ __launch_bounds__(FILTER_TILE_THREADS) void k_filter_tile(DevPtrs p, int kstep, int builds) {
+  __shared__ int s_len[FILTER_ROW_WAVES], s_nlen[FILTER_NAT_WAVES];
+  __shared__ int2 s_nat[TILE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // the filter of the grid builds runs after their rows: the rebuild's work
+  // counters go back to empty for the next one
+  if (blockIdx.x == 0 && threadIdx.x == 0 && ((builds >> BUILD_DIRECT) & 1)) {
+    *p.ncellwork = 0;
+    *p.nlbuild = 0;
+  }
+  const int ntiles = *p.ntiles;
+  for (int w = blockIdx.x; w < ntiles; w += gridDim.x) {
+    if (w != (int)blockIdx.x) __syncthreads();  // the previous tile's totals have been read
+    const int2 it = p.tiles[w];
+    if (it.x < 0) continue;
+    const SysDev &S = p.sys[it.y];
+    if (((builds >> S.build) & 1) == 0) continue;
+    const int b0 = it.x * TILE, nb = min(TILE, S.bead_off + S.n - b0);
+    const float4 *__restrict__ pin = buf_in(p, S.parity + kstep);
+    if (wave >= FILTER_ROW_WAVES) {
+      filter_nats(p, S, b0, nb, wave - FILTER_ROW_WAVES, pin, s_nlen, s_nat);
+    } else if (S.type_mask != 3) {
+      filter_rows<true>(p, S, b0, nb, wave, pin, s_len, s_nlen, s_nat);
+    } else {
+      filter_rows<false>(p, S, b0, nb, wave, pin, s_len, s_nlen, s_nat);
+    }
+  }
+}
+
 // 8 waves per SIMD: two blocks per compute unit
 template <int LPB, int MODE>
 __global__ __launch_bounds__(STEP_THREADS, 8) void k_step(DevPtrs p, int kstep, int tier) {
@@ -2045,30 +2290,23 @@ __device__ __forceinline__ RoundAt round_at(int r, int b0, int bend, int ordm, u
 }
 
 // Gathered native and non-native force on the lane group's bead.
-template <int LPB, bool IDX16, bool ONE>
+template <int LPB, bool ONE>
 __device__ __forceinline__ float3 tile_round(const DevPtrs &p, const SysDev &S, const float4 *__restrict__ pin, int self,
                                              const RoundAt &a) {
   const int l = (int)(threadIdx.x & 63) % LPB;
-  constexpr uint32_t ESZ = IDX16 ? 2u : 4u;
-  // buffer resources in scalar registers: the system's pair-list segment and
-  // the natives
-  const __amdgpu_buffer_rsrc_t rrow = buf_rsrc(p.plrep_j + S.pl_base, (uint32_t)S.n * (uint32_t)S.pl_cap * ESZ);
+  // buffer resources in scalar registers: the system's pair-list segment
+  // (16-bit entries) and the natives
+  const __amdgpu_buffer_rsrc_t rrow = buf_rsrc(p.plrep_j + S.pl_base, (uint32_t)S.n * (uint32_t)S.pl_cap * 2u);
   const __amdgpu_buffer_rsrc_t rnat = buf_rsrc(p.platt, 0xFFFFFFFFu);
-  constexpr int D = IDX16 ? 8 : 4;  // chunks of four entries held per lane
-  constexpr int NB = 4;             // natives held per lane
-  uint32_t q[16];
+  constexpr int D = 8;   // chunks of four entries held per lane
+  constexpr int NB = 4;  // natives held per lane
+  uint32_t q[2 * D];
   auto load_chunks = [&](int c0) {  // without a condition: past the segment a buffer load returns zeros
 #pragma unroll
     for (int k = 0; k < D; ++k) {
-      const uint32_t off = ESZ * a.row + 4u * ESZ * (uint32_t)(l + LPB * (c0 + k));
-      if constexpr (IDX16) {
-        const int2 v = load_i2(rrow, off);
-        q[2 * k] = (uint32_t)v.x;
-        q[2 * k + 1] = (uint32_t)v.y;
-      } else {
-        const uint4 v = load_b128(rrow, off);
-        q[4 * k] = v.x; q[4 * k + 1] = v.y; q[4 * k + 2] = v.z; q[4 * k + 3] = v.w;
-      }
+      const int2 v = load_i2(rrow, 2u * a.row + 8u * (uint32_t)(l + LPB * (c0 + k)));
+      q[2 * k] = (uint32_t)v.x;
+      q[2 * k + 1] = (uint32_t)v.y;
     }
   };
   int2 en[NB];
@@ -2087,16 +2325,11 @@ __device__ __forceinline__ float3 tile_round(const DevPtrs &p, const SysDev &S, 
   // the four partners of chunk position k (a lane past its row: the bead
   // itself, whose d2 = 0 fails the guard)
   auto gather = [&](int k, bool on, float4 *x) {
-    if constexpr (IDX16) {
-      const uint32_t w0 = on ? q[2 * k] : sv, w1 = on ? q[2 * k + 1] : sv;
-      x[0] = base[w0 & 0xFFFFu];
-      x[1] = base[w0 >> 16];
-      x[2] = base[w1 & 0xFFFFu];
-      x[3] = base[w1 >> 16];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = pin[on ? q[4 * k + e] : (uint32_t)self];
-    }
+    const uint32_t w0 = on ? q[2 * k] : sv, w1 = on ? q[2 * k + 1] : sv;
+    x[0] = base[w0 & 0xFFFFu];
+    x[1] = base[w0 >> 16];
+    x[2] = base[w1 & 0xFFFFu];
+    x[3] = base[w1 >> 16];
   };
   constexpr int R = 4;  // chunks in flight
   float4 xn[NB], xr[R][4];
@@ -2161,7 +2394,7 @@ __device__ __forceinline__ float3 tile_round(const DevPtrs &p, const SysDev &S, 
         if (__ballot(l + LPB * (c0 + k) < nch) == 0) break;
         rep(xr[k % R]);
         if (k + R < D && __ballot(l + LPB * (c0 + k + R) < nch) != 0)
-          gather((k + R) % D, l + LPB * (c0 + k + R) < nch, xr[k % R]);
+          gather(k + R, l + LPB * (c0 + k + R) < nch, xr[k % R]);
       }
       c0 += D;
       if (__ballot(l + LPB * c0 < nch) == 0) break;
@@ -2201,11 +2434,7 @@ __global__ __launch_bounds__(64 * (tile_waves(LPB) + 1)) void k_step_tile(DevPtr
         for (int r = wave; r < LPB; r += W) {
           const RoundAt a = round_at<LPB>(r, b0, bend, ordm, hd, nat0, (b0 - bead_off) * S.pl_cap);
           const int self = a.i < bend ? a.i : b0;  // a bead of this system: safe to gather
-          float3 f;
-          if (S.type_mask != 3)
-            f = S.idx16 ? tile_round<LPB, true, true>(p, S, pin, self, a) : tile_round<LPB, false, true>(p, S, pin, self, a);
-          else
-            f = S.idx16 ? tile_round<LPB, true, false>(p, S, pin, self, a) : tile_round<LPB, false, false>(p, S, pin, self, a);
+          const float3 f = S.type_mask != 3 ? tile_round<LPB, true>(p, S, pin, self, a) : tile_round<LPB, false>(p, S, pin, self, a);
           if (lane % LPB == 0) {
             s_f[0][a.li] = f.x;
             s_f[1][a.li] = f.y;
@@ -2531,6 +2760,8 @@ static hipError_t fork_end(const StepFork *fk, hipStream_t st) {
 static void launch_filter(const DevPtrs &p, const StepGrids &sg, int kstep, int builds, hipStream_t st) {
   // row staging after the staged positions where LDS has room for it
   const bool stage0 = sg.lds + FILTER_STAGE_BYTES <= LDS_BYTES_MAX;
+  if (sg.tiles > 0)
+    hipLaunchKernelGGL(k_filter_tile, dim3(sg.tiles), dim3(FILTER_TILE_THREADS), 0, st, p, kstep, builds);
   if (sg.grid > 0)
     hipLaunchKernelGGL(k_shell_filter<true>, dim3(sg.grid), dim3(STEP_THREADS),
                        sg.lds + (stage0 ? FILTER_STAGE_BYTES : 0), st, p, kstep, 0, stage0 ? (int)sg.lds : -1,

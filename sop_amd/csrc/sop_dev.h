@@ -151,7 +151,7 @@ struct DevPtrs {
   int32_t *tile_sys;    // system slot of each tile
   uint8_t *tile_ord;    // per tile: TILE bead offsets in the order the step kernel's lane groups take them
   int32_t *work;        // tile ids to process (-1 = padding), XCD-interleaved
-  int2 *tiles;          // tiles that step with a block each: {tile, system slot}, tile -1 = padding
+  int2 *tiles;          // tiles that step and filter with a block each: {tile, system slot}, tile -1 = padding
   int32_t *ntiles;
   int32_t *nwork;
   int32_t *syslist;     // system slots of the current batch, those of more than SORT_N_MAX beads first
@@ -186,7 +186,7 @@ constexpr int TILE_STEP_FAR_PER_CU = 4;
 
 // Grids of the step's launches: items staged in LDS at two blocks per compute
 // unit, items staged in a whole compute unit's LDS, items that gather from
-// global memory, and tiles with a block each (the step kernel only).
+// global memory, and tiles with a block each.
 struct StepGrids {
   int grid, grid_big, grid_far;
   size_t lds, lds_big;

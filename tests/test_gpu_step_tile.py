@@ -1,4 +1,4 @@
-"""The step with a block per tile against the item kernels, on device 0.
+"""Step and shell filter with a block per tile against the item kernels, on device 0.
 
 Small batches, and the few systems too large to stage, take a block per tile;
 step_tiles asks for the item kernels instead.  Both run the same arithmetic in
@@ -6,7 +6,8 @@ the same order, so coordinates, forces and velocities are bitwise equal: at
 tile remainders, with rows longer than one block of held chunks, native lists
 longer than the held ones, no natives, two bead types, several chains, jobs
 that end inside a block of steps, underdamped dynamics, every lane count, and
-either side of the tile counts where the launch changes.
+either side of the tile counts where the launch changes.  The filter's lists
+come out in the same order, for shell, grid and neighbor-list builds.
 """
 import numpy as np
 import pytest
@@ -57,7 +58,7 @@ def outputs(systems, steps, **opts):
     ([(12, 600, 2)], 30, 16),
     ([(13, 600)], 30, 32),
     ([(14, 11000)], 20, 4),
-    ([(15, 66000, 1, False, False)], 12, 4),  # 32-bit rows
+    ([(15, 65536, 1, False, False)], 12, 4),  # the largest system with 16-bit rows
     ([(16, 8000), (17, 3000), (18, 8000)], 12, 4),
 ])
 def test_tile_step_equals_item_step(systems, steps, lanes):
@@ -99,5 +100,53 @@ def test_either_side_of_the_tile_count(replicas, n):
         made.append(t)
     got = outputs(made, 20)
     want = outputs(made, 20, step_tiles=16)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+
+
+def lists_after_moves(s, tiles, moves):
+    out = []
+    rng = np.random.default_rng(5)
+    with S.Engine(0, step_tiles=tiles) as e:
+        i = e.add(s)
+        x = s.xyz
+        for d in moves:
+            # (a larger move shifts the whole system: the bonds hold)
+            x = x + rng.normal(0, 0.05, x.shape).astype(np.float32) + np.float32(d if d > 1 else 0.0)
+            e.set_coords(i, x)
+            e.update_pair_list(i)
+            out += [e.get_list(i, w) for w in (S.LIST_PL_REP, S.LIST_PL_NATIVE)]
+            st = e.list_stats(i)
+            out.append(np.array([st.grid_builds, st.shell_builds, st.nl_builds, st.pl_rep, st.pl_native]))
+            out.append(e.force_eval(i))
+    return out
+
+
+@pytest.mark.parametrize("n,types,scale,natives,skin,model", [
+    (1, 1, 1.0, 8, 16.0, "config"), (63, 1, 1.0, 8, 16.0, "config"), (130, 2, 1.0, 8, 16.0, "config"),
+    (1400, 1, 0.6, 8, 16.0, "config"),      # rows past two passes of 64
+    (400, 1, 0.6, 300, 16.0, "config"),     # more than 128 natives a bead
+    (700, 2, 1.0, 40, 16.0, "reference"),   # factor cutoffs
+    (700, 1, 1.0, 8, 0.05, "config"),       # neighbor-list builds
+    (12000, 1, 1.0, 8, 16.0, "config")])
+def test_tile_filter_gives_the_item_filters_lists(n, types, scale, natives, skin, model):
+    s = chain(100 + n, n, types)
+    if model == "reference":
+        p = S.params_reference()
+        p.zeta, p.boxl, p.seed = 50.0, 0.0, 9
+        s.params = p
+    else:
+        s.params.nl_abs = s.params.pl_abs + skin
+    s.xyz = (s.xyz * np.float32(scale)).astype(np.float32)
+    s.bond_r0 = (s.bond_r0 * np.float32(scale)).astype(np.float32)
+    if natives != 8:
+        rng = np.random.default_rng(n)
+        i, j = np.triu_indices(n, 3)
+        pick = rng.random(len(i)) < natives / n
+        s.nat_i, s.nat_j = i[pick].astype(np.int32), j[pick].astype(np.int32)
+        s.nat_r0 = np.linalg.norm(s.xyz[s.nat_i] - s.xyz[s.nat_j], axis=1).astype(np.float32)
+    moves = (0.05, 0.05, 2.0, 0.05)  # shell builds, a grid build (or one from the snapshot), a shell build
+    got, want = lists_after_moves(s, 0, moves), lists_after_moves(s, 16, moves)
+    assert len(got) == len(want)
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
