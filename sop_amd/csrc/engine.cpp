@@ -165,7 +165,7 @@ ListGrids list_grids(const sop_engine *e) {
   // their shell rows, give the filter a quarter of the device's compute units
   // or more
   const bool split = e->cur_nsys > 1 && 4 * (e->cur_nfitems + e->cur_nfitems_big + e->cur_nfitems_far) > e->num_cu;
-  return ListGrids{grid_tiles(e), grid_rebuild(e), grid_big_beads(e), grid_big_sys(e), split, filter_grids(e)};
+  return ListGrids{grid_tiles(e), std::min(16 * e->cur_nwork, 8 * e->num_cu), grid_rebuild(e), grid_big_beads(e), grid_big_sys(e), split, filter_grids(e)};
 }
 
 } // namespace sopk

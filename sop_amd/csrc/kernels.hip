@@ -796,6 +796,7 @@ __device__ __forceinline__ bool native_pair(const int32_t *nj, int nn, int j) {
 // (local index mod 65536); a set bit is confirmed by the exact search unless
 // the system is small enough for the key to be the index itself.
 constexpr int NATBITS_WORDS = 2048;
+constexpr int NLB_BEADS = 1;  // beads of a wave's unit in neighbor-list builds
 
 __device__ __forceinline__ void natbits_mark(uint32_t *bits, const int32_t *natj, int nn, int bead_off, bool set) {
   const int lane = threadIdx.x & 63;
@@ -819,7 +820,9 @@ __device__ __forceinline__ int scan_cells(const DevPtrs &p, const SysDev &S, int
                                           Emit emit) {
   const int lane = threadIdx.x & 63;
   const int wi = __float_as_int(xi.w), ci = wi >> 2;
+  // (in registers: the emitted entries may alias S)
   const float boxl = S.boxl;
+  const int bo = S.bead_off, n = S.n;
   const int cx = min(max((int)floorf((xi.x - S.org[0]) * S.inv_edge[0]), 0), S.dims[0] - 1);
   const int cy = min(max((int)floorf((xi.y - S.org[1]) * S.inv_edge[1]), 0), S.dims[1] - 1);
   const int cz = min(max((int)floorf((xi.z - S.org[2]) * S.inv_edge[2]), 0), S.dims[2] - 1);
@@ -833,27 +836,37 @@ __device__ __forceinline__ int scan_cells(const DevPtrs &p, const SysDev &S, int
       const int row = (zz * S.dims[1] + yy) * S.dims[0];
       const int st = max(p.cell_start[S.cell_base + row + x0], 0);
       const int en = min(p.cell_start[S.cell_base + row + x1 + 1], S.n);
-      for (int m0 = st; m0 < en; m0 += 64) {
-        const int m = m0 + lane;
-        bool pred = false;
-        int j = 0;
-        if (m < en) {
-          j = p.cell_sorted[S.bead_off + m];
-          const float4 xj = p.pos_sorted[S.bead_off + m];
+      // U x 64 candidates' loads in flight together
+      constexpr int U = 4;
+      for (int m0 = st; m0 < en; m0 += 64 * U) {
+        int jj[U];
+        float4 xx[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int m = min(m0 + 64 * u + lane, en - 1);
+          jj[u] = p.cell_sorted[bo + m];
+          xx[u] = p.pos_sorted[bo + m];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (m0 + 64 * u >= en) break;
+          const int j = jj[u];
+          const float4 xj = xx[u];
           const int wj = __float_as_int(xj.w);
           const int dj = j - i;
-          const bool excl = (j == i) || (((wj >> 2) == ci) && dj >= -2 && dj <= 2) ||
-                            j < S.bead_off || j >= S.bead_off + S.n;
+          const bool excl = m0 + 64 * u + lane >= en || (j == i) || (((wj >> 2) == ci) && dj >= -2 && dj <= 2) ||
+                            j < bo || j >= bo + n;
+          bool pred = false;
           if (!excl && dist2_exact(xi, xj, boxl) < ((wj & 3) == 2 ? rcB : rcA)) {
-            const int jl = (j - S.bead_off) & 0xFFFF;
+            const int jl = (j - bo) & 0xFFFF;
             bool nat = (bits[jl >> 5] >> (jl & 31)) & 1u;
             if (nat && !exact_key) nat = native_pair(natj, nn, j);
             pred = !nat && extra(j, wj);
           }
+          const uint64_t mk = __ballot(pred);
+          if (pred) emit(cnt + lanes_below(mk), j);
+          cnt += __popcll(mk);
         }
-        const uint64_t mk = __ballot(pred);
-        if (pred) emit(cnt + lanes_below(mk), j);
-        cnt += __popcll(mk);
       }
     }
   natbits_mark(bits, natj, nn, S.bead_off, false);
@@ -1165,9 +1178,13 @@ __device__ __forceinline__ void nl_build(const DevPtrs &p, int kstep, char *s_ra
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int k = lane; k < NATBITS_WORDS; k += 64) s_bits[wave][k] = 0u;
   __builtin_amdgcn_wave_barrier();
-  const int nwork = *p.nwork;
-  for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
-    const int t = p.work[w];
+  // units of NLB_BEADS beads: a wave scans a bead's 27 cells one load batch
+  // after another, so the beads go out over as many waves as the launch has
+  // (a wave took sixteen: 860 us for the neighbor list of 5,000 beads)
+  constexpr int UNITS = TILE / NLB_BEADS;
+  const int nunit = *p.nwork * UNITS;
+  for (int w = blockIdx.x * 4 + wave; w < nunit; w += gridDim.x * 4) {
+    const int t = p.work[w / UNITS];
     if (t < 0) continue;
     const int s = p.tile_sys[t];
     const SysDev &S = p.sys[s];
@@ -1177,8 +1194,8 @@ __device__ __forceinline__ void nl_build(const DevPtrs &p, int kstep, char *s_ra
     const float4 *pin = buf_in(p, S.parity + kstep);
     const float boxl = S.boxl;
     const int bend = min(t * TILE + TILE, S.bead_off + S.n);
-    for (int q = 0; q < TILE / 4; ++q) {
-      const int i = t * TILE + wave * (TILE / 4) + q;
+    for (int q = 0; q < NLB_BEADS; ++q) {
+      const int i = t * TILE + (w % UNITS) * NLB_BEADS + q;
       if (i >= bend) break;
       const float4 xi = ref[i];
       const float4 xn = pin[i];
@@ -2811,7 +2828,9 @@ hipError_t launch_lists(const DevPtrs &p, const ListGrids &lg, int kstep, int fl
     hipLaunchKernelGGL(k_cell_scatter, dim3(4 * lg.grid_big, lg.grid_nbig), dim3(256), 0, cs, p);
     hipLaunchKernelGGL(k_cell_rank, dim3(4 * lg.grid_big, lg.grid_nbig), dim3(256), 0, cs, p, kstep);
   }
-  hipLaunchKernelGGL(k_rows, dim3(lg.grid_tiles), dim3(256), 0, cs, p, kstep);
+  // the neighbor list asked for: a wave per bead
+  const int grid_rows = flags == FORCE_NL || (flags & MATERIALIZE_NL) ? lg.grid_nl : lg.grid_tiles;
+  hipLaunchKernelGGL(k_rows, dim3(grid_rows), dim3(256), 0, cs, p, kstep);
   if (split) {
     launch_filter(p, lg.fg, kstep, ALL & ~SHELL_ONLY, cs);
     launch_filter(p, lg.fg, kstep, SHELL_ONLY, st);

@@ -201,12 +201,13 @@ struct StepFork {
   hipEvent_t fork, join;
 };
 
-// Grids of the list kernels: home cells, systems of up to SORT_N_MAX beads
+// Grids of the list kernels: home cells, beads of neighbor-list builds (a wave
+// each), systems of up to SORT_N_MAX beads
 // (one block each), beads (blocks of 2,048) and number of the larger ones, and
 // the shell filter's work items (staged in LDS like the step kernel's).
 // split: the shell builds' filter on one stream beside the grid chain.
 struct ListGrids {
-  int grid_tiles, grid_sys, grid_big, grid_nbig;
+  int grid_tiles, grid_nl, grid_sys, grid_big, grid_nbig;
   bool split;
   StepGrids fg;
 };
