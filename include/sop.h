@@ -194,8 +194,8 @@ sop_status sop_energy_eval(sop_engine *e, int32_t sys, double *energies);
 /* sop_energy_eval without any device allocation: no hipMalloc, hipFree or
  * allocating library call.  No counterpart in the reference; for callers that
  * cannot allocate (code under HIP graph capture, serving loops, harnesses
- * that forbid it).  The work table and the energy partials live in a
- * file-scope device array of the library, ~3 MiB per device, held until the
+ * that forbid it).  The energy partials live in a file-scope device array of
+ * the library, ~80 KiB per device, held until the
  * process ends; systems of up to 65,536 beads (SOP_ERR_CAPACITY above).
  * Same kernels and summation order as sop_energy_eval: identical results.
  * Every call on one device shares that device's array: calls that overlap on

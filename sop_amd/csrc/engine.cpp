@@ -1767,9 +1767,9 @@ sop_status sop_get_forces(sop_engine *e, int32_t sys, float *f3n) {
 }
 
 static sop_status eval_energy(sop_engine *e, int32_t sys, double *out) {
-  sop_status st = engine_set_batch(e, &sys, 1);
-  if (st) return st;
-  HIPCK(launch_energy(e->p, grid_tiles(e), grid_sys(e), e->stream));
+  const SysHost &h = e->sys[sys];
+  const int nt = (int)(h.bead_len / TILE);
+  HIPCK(launch_energy_one(e->p, (int)(h.bead_off / TILE), nt, sys, std::min(nt, 2 * e->num_cu), nullptr, e->stream));
   HIPCK(hipMemcpyAsync(out, e->p.sysout + (int64_t)sys * SYSOUT_N, 8 * SYSOUT_N, hipMemcpyDeviceToHost, e->stream));
   HIPCK(hipStreamSynchronize(e->stream));
   return SOP_OK;
@@ -1794,20 +1794,15 @@ sop_status sop_energy_eval_noalloc(sop_engine *e, int32_t sys, double *energies)
        << NOALLOC_BEADS;
     return set_error(e, SOP_ERR_CAPACITY, os.str());
   }
-  // the engine's arrays, with the work table, counters and partials in scratch
+  // the engine's arrays, with the partials and values in scratch
   DevPtrs q = e->p;
   char *b = static_cast<char *>(e->scratch);
-  q.work = reinterpret_cast<int32_t *>(b + NOALLOC_OFF_WORK);
-  q.nwork = reinterpret_cast<int32_t *>(b + NOALLOC_OFF_CNT);
-  q.nsys = q.nwork + 16;
-  q.syslist = reinterpret_cast<int32_t *>(b + NOALLOC_OFF_SYSLIST);
-  q.epart = reinterpret_cast<double *>(b + NOALLOC_OFF_EPART);
+  q.epart = reinterpret_cast<double *>(b);
   q.epart_base = (int32_t)h.bead_off;
   q.sysout = reinterpret_cast<double *>(b + NOALLOC_OFF_SYSOUT);
   q.sysout_base = sys;
-  const int t0 = (int)(h.bead_off / TILE), nt = (int)(h.bead_len / TILE);
-  const int grid = std::max(8, std::min(8 * e->num_cu, (nt + 7) / 8 * 8));
-  HIPCK(launch_noalloc_energy(q, t0, nt, sys, grid, e->stream));
+  const int nt = (int)(h.bead_len / TILE);
+  HIPCK(launch_energy_one(q, (int)(h.bead_off / TILE), nt, sys, std::min(nt, 2 * e->num_cu), nullptr, e->stream));
   double o[SYSOUT_N];
   HIPCK(hipMemcpyAsync(o, q.sysout, sizeof(o), hipMemcpyDeviceToHost, e->stream));
   HIPCK(hipStreamSynchronize(e->stream));

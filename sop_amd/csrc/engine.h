@@ -25,13 +25,13 @@ hipError_t launch_step(const DevPtrs &p, int mode, int lpb, const StepGrids &sg,
 hipError_t step_lds_limit(size_t bytes);
 hipError_t filter_lds_init();
 hipError_t launch_energy(const DevPtrs &p, int grid_tiles, int grid_sys, hipStream_t st);
+hipError_t launch_energy_one(const DevPtrs &p, int t0, int nt, int slot, int grid_tiles, double *out, hipStream_t st);
 hipError_t launch_advance(const DevPtrs &p, int nsteps, hipStream_t st);
 hipError_t launch_relayout(const DevPtrs &p, int bo, int n, int idx16, int64_t old_base, int old_cap,
                            int64_t new_base, int new_cap, hipStream_t st);
 hipError_t launch_begin(const DevPtrs &p, int64_t nsteps, hipStream_t st);
 hipError_t launch_selftest(int *out, float *fout, hipStream_t st);
 hipError_t noalloc_scratch(int device, void **ptr);
-hipError_t launch_noalloc_energy(const DevPtrs &p, int t0, int nt, int slot, int grid_tiles, hipStream_t st);
 
 // First-fit range allocator over [0, cap).
 class RangeAlloc {

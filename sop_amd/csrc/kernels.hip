@@ -2491,14 +2491,20 @@ __global__ __launch_bounds__(64 * (tile_waves(LPB) + 1)) void k_step_tile(DevPtr
 
 // 16 lanes per bead; FP32 pair energies, FP64 accumulation; pairs are seen
 // from both beads and weighted 1/2.  Native contacts (d/r0 < 1.25 over all
-// natives) are counted from the lower index.
-__global__ __launch_bounds__(256) void k_energy(DevPtrs p) {
-  constexpr int LPB = 16, GPW = 4, ROUNDS = TILE / 16;
+// natives) are counted from the lower index.  A block of 16 waves takes a tile,
+// every bead at once (four waves took sixteen rounds of load chains: 17 us for
+// 701 beads, 6 now), and leaves the tile's sums: its 6 energy partials, then
+// sum x, y, z, |r|^2.  nt > 0: tiles t0 .. t0 + nt - 1 (one system, no work
+// table); else the work table's tiles.
+constexpr int ENERGY_THREADS = 1024;
+__global__ __launch_bounds__(ENERGY_THREADS) void k_energy(DevPtrs p, int t0, int nt) {
+  constexpr int LPB = 16;
+  __shared__ double sh[ENERGY_THREADS / 64][TPART_N];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane / LPB, l = lane % LPB;
-  const int nwork = *p.nwork;
+  const int nwork = nt > 0 ? nt : *p.nwork;
   for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
-    const int t = p.work[w];
+    const int t = nt > 0 ? t0 + w : p.work[w];
     if (t < 0) continue;
     const int s = p.tile_sys[t];
     const SysDev &S = p.sys[s];
@@ -2508,11 +2514,12 @@ __global__ __launch_bounds__(256) void k_energy(DevPtrs p) {
     const float4 *pin = buf_in(p, S.parity);
     const float boxl = S.boxl, inv_boxl = S.inv_boxl;
     const bool wrapf = S.wrap_free != 0 || boxl <= 0.0f;
-    for (int r = 0; r < ROUNDS; ++r) {
-      const int i = b0 + r * (4 * GPW) + wave * GPW + g;
+    {
+      const int i = b0 + wave * (64 / LPB) + g;
+      float4 xi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       double eb = 0.0, ea = 0.0, en = 0.0, er = 0.0, vir = 0.0, con = 0.0;
       if (i < bend) {
-        const float4 xi = pin[i];
+        xi = pin[i];
         const int wi = __float_as_int(xi.w);
         const int row = ((wi & 3) - 1) * 2;
         if (l < 4) {
@@ -2607,48 +2614,63 @@ __global__ __launch_bounds__(256) void k_energy(DevPtrs p) {
         vir += __shfl_xor(vir, o);
         con += __shfl_xor(con, o);
       }
-      if (l == 0 && i < bend) {
-        double *o = p.epart + (int64_t)(i - p.epart_base) * EPART_N;
-        o[0] = eb; o[1] = ea; o[2] = en; o[3] = er; o[4] = vir; o[5] = con;
+      // the wave's four beads, then the block's sixteen waves in order
+      double v[TPART_N] = {eb, ea, en, er, vir, con, 0.0, 0.0, 0.0, 0.0};
+      if (i < bend) {
+        v[6] = xi.x;
+        v[7] = xi.y;
+        v[8] = xi.z;
+        v[9] = (double)xi.x * xi.x + (double)xi.y * xi.y + (double)xi.z * xi.z;
+      }
+#pragma unroll
+      for (int k = 0; k < TPART_N; ++k) {
+        v[k] += __shfl_xor(v[k], 16);
+        v[k] += __shfl_xor(v[k], 32);
+      }
+      __syncthreads();  // the previous tile's sums have been read
+      if (lane == 0) {
+#pragma unroll
+        for (int k = 0; k < TPART_N; ++k) sh[wave][k] = v[k];
+      }
+      __syncthreads();
+      if (tid < TPART_N) {
+        double a = 0.0;
+        for (int q = 0; q < ENERGY_THREADS / 64; ++q) a += sh[q][tid];
+        p.epart[(int64_t)(t - p.epart_base / TILE) * TPART_N + tid] = a;
       }
     }
   }
 }
 
-// Per system, fixed-order reduction of the bead partials plus Rg^2 from the
-// centroid form (1/N) sum |r|^2 - |r_cm|^2, identical to the reference's
-// pair sum / N^2 (sop.cu:564-580).
-__global__ __launch_bounds__(256) void k_sys_reduce(DevPtrs p) {
-  __shared__ double sh[4][10];
+// Per system, fixed-order sum of the tile partials plus Rg^2 from the centroid
+// form (1/N) sum |r|^2 - |r_cm|^2, identical to the reference's pair sum / N^2
+// (sop.cu:564-580).  slot >= 0: that system alone, its values also to out (when
+// not null); else the batch's systems.
+__global__ __launch_bounds__(256) void k_sys_reduce(DevPtrs p, int slot, double *out) {
+  __shared__ double sh[4][TPART_N];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nsys = *p.nsys;
+  const int nsys = slot >= 0 ? 1 : *p.nsys;
   for (int q = blockIdx.x; q < nsys; q += gridDim.x) {
-    const int s = p.syslist[q];
+    const int s = slot >= 0 ? slot : p.syslist[q];
     const SysDev &S = p.sys[s];
-    const float4 *pin = buf_in(p, S.parity);
-    double acc[10];
+    const int nt = (S.n + TILE - 1) / TILE;
+    const double *e = p.epart + (int64_t)(S.bead_off - p.epart_base) / TILE * TPART_N;
+    double acc[TPART_N];
 #pragma unroll
-    for (int k = 0; k < 10; ++k) acc[k] = 0.0;
-    for (int b = tid; b < S.n; b += blockDim.x) {
-      const int i = S.bead_off + b;
-      const double *e = p.epart + (int64_t)(i - p.epart_base) * EPART_N;
+    for (int k = 0; k < TPART_N; ++k) acc[k] = 0.0;
+    for (int b = tid; b < nt; b += 256) {
 #pragma unroll
-      for (int k = 0; k < 6; ++k) acc[k] += e[k];
-      const float4 x = pin[i];
-      acc[6] += x.x;
-      acc[7] += x.y;
-      acc[8] += x.z;
-      acc[9] += (double)x.x * x.x + (double)x.y * x.y + (double)x.z * x.z;
+      for (int k = 0; k < TPART_N; ++k) acc[k] += e[b * TPART_N + k];
     }
 #pragma unroll
-    for (int k = 0; k < 10; ++k) acc[k] = wave_sum_d(acc[k]);
+    for (int k = 0; k < TPART_N; ++k) acc[k] = wave_sum_d(acc[k]);
     if (lane == 0)
-      for (int k = 0; k < 10; ++k) sh[wave][k] = acc[k];
+      for (int k = 0; k < TPART_N; ++k) sh[wave][k] = acc[k];
     __syncthreads();
     if (tid == 0) {
-      double tot[10];
-      for (int k = 0; k < 10; ++k) tot[k] = sh[0][k] + sh[1][k] + sh[2][k] + sh[3][k];
-      double *o = p.sysout + (int64_t)(s - p.sysout_base) * SYSOUT_N;
+      double tot[TPART_N];
+      for (int k = 0; k < TPART_N; ++k) tot[k] = sh[0][k] + sh[1][k] + sh[2][k] + sh[3][k];
+      double o[SYSOUT_N] = {0.0};
       o[0] = tot[0]; o[1] = tot[1]; o[2] = tot[2]; o[3] = tot[3];
       o[4] = tot[0] + tot[1] + tot[2] + tot[3];
       o[5] = tot[4];
@@ -2658,6 +2680,11 @@ __global__ __launch_bounds__(256) void k_sys_reduce(DevPtrs p) {
       o[7] = tot[9] * inv - (cx * cx + cy * cy + cz * cz);
       o[8] = tot[6]; o[9] = tot[7]; o[10] = tot[8];
       o[11] = (double)S.n;
+      double *d = p.sysout + (int64_t)(s - p.sysout_base) * SYSOUT_N;
+      for (int k = 0; k < 12; ++k) {
+        d[k] = o[k];
+        if (out) out[k] = o[k];
+      }
     }
     __syncthreads();
   }
@@ -2930,8 +2957,15 @@ hipError_t launch_relayout(const DevPtrs &p, int bo, int n, int idx16, int64_t o
 }
 
 hipError_t launch_energy(const DevPtrs &p, int grid_tiles, int grid_sys, hipStream_t st) {
-  hipLaunchKernelGGL(k_energy, dim3(grid_tiles), dim3(256), 0, st, p);
-  hipLaunchKernelGGL(k_sys_reduce, dim3(grid_sys), dim3(256), 0, st, p);
+  hipLaunchKernelGGL(k_energy, dim3(std::min(grid_tiles, 512)), dim3(ENERGY_THREADS), 0, st, p, 0, 0);
+  hipLaunchKernelGGL(k_sys_reduce, dim3(grid_sys), dim3(256), 0, st, p, -1, nullptr);
+  return SOPK_LAUNCH_CHECK();
+}
+
+// One system (tiles t0 .. t0 + nt - 1, slot), without a work table.
+hipError_t launch_energy_one(const DevPtrs &p, int t0, int nt, int slot, int grid_tiles, double *out, hipStream_t st) {
+  hipLaunchKernelGGL(k_energy, dim3(grid_tiles), dim3(ENERGY_THREADS), 0, st, p, t0, nt);
+  hipLaunchKernelGGL(k_sys_reduce, dim3(1), dim3(256), 0, st, p, slot, out);
   return SOPK_LAUNCH_CHECK();
 }
 
@@ -2947,8 +2981,8 @@ hipError_t launch_begin(const DevPtrs &p, int64_t nsteps, hipStream_t st) {
 
 // ------------------------------------------ allocation-free energy entry point
 //
-// The work table, counters and energy partials of sop_energy_eval_noalloc
-// live in this file-scope array instead of memory the library allocates.
+// The energy partials and values of sop_energy_eval_noalloc live in this
+// file-scope array instead of memory the library allocates.
 // Host code never passes the array's name to a kernel or a copy (in host
 // code it stands for no device address): the address of each device's copy
 // comes from hipGetSymbolAddress, once per device, and only that address is
@@ -2975,25 +3009,6 @@ hipError_t noalloc_scratch(int device, void **ptr) {
   g_scratch_ptr[device] = p;
   *ptr = p;
   return hipSuccess;
-}
-
-// Work table of one system (tiles t0 .. t0 + nt - 1) and its counters, in
-// the scratch that p.work / p.nwork / p.nsys / p.syslist point into.
-__global__ void k_noalloc_setup(DevPtrs p, int t0, int nt, int slot) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nt; k += gridDim.x * blockDim.x) p.work[k] = t0 + k;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *p.nwork = nt;
-    *p.nsys = 1;
-    p.syslist[0] = slot;
-  }
-}
-
-hipError_t launch_noalloc_energy(const DevPtrs &p, int t0, int nt, int slot, int grid_tiles, hipStream_t st) {
-  hipLaunchKernelGGL(k_noalloc_setup, dim3(std::max(1, std::min(64, (nt + 255) / 256))), dim3(256), 0, st, p, t0,
-                     nt, slot);
-  hipLaunchKernelGGL(k_energy, dim3(grid_tiles), dim3(256), 0, st, p);
-  hipLaunchKernelGGL(k_sys_reduce, dim3(1), dim3(256), 0, st, p);
-  return SOPK_LAUNCH_CHECK();
 }
 
 hipError_t launch_selftest(int *out, float *fout, hipStream_t st) {

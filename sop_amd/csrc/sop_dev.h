@@ -146,7 +146,7 @@ struct DevPtrs {
   float4 *vel;          // underdamped state per bead: w = 1: xyz = last increment;
                         // w = 0: xyz = velocity entering the next step
   float4 *fout;         // forces (force-eval modes)
-  double *epart;        // per bead: 6 energy partials
+  double *epart;        // per tile: TPART_N partial sums
   double *sysout;       // per system slot: SYSOUT_N reduced values
   int32_t *tile_sys;    // system slot of each tile
   uint8_t *tile_ord;    // per tile: TILE bead offsets in the order the step kernel's lane groups take them
@@ -222,18 +222,14 @@ constexpr int SORT_N_MAX = 5120;
 constexpr int SORT_C_MAX = 2 * SORT_N_MAX;
 
 constexpr int EPART_N = 6;   // bond, angle, native, rep, virial, contacts
+constexpr int TPART_N = 10;  // per tile: the EPART_N sums, then sum x, y, z, |r|^2 of its beads
 constexpr int SYSOUT_N = 16; // e[0..5], contacts, rgsq, sum x,y,z, n
 
 // Scratch of the allocation-free energy entry point: one system of up to
-// NOALLOC_BEADS beads.  Layout in bytes: work table (one entry per tile),
-// counters (the engine's nwork layout: [0] work entries, [16] systems),
-// system list, per-bead energy partials, the system's reduced values.
+// NOALLOC_BEADS beads.  Layout in bytes: per-tile energy partials, the
+// system's reduced values.
 constexpr int NOALLOC_BEADS = 65536;
-constexpr size_t NOALLOC_OFF_WORK = 0;
-constexpr size_t NOALLOC_OFF_CNT = NOALLOC_OFF_WORK + 4 * (NOALLOC_BEADS / TILE) + 256;
-constexpr size_t NOALLOC_OFF_SYSLIST = NOALLOC_OFF_CNT + 256;
-constexpr size_t NOALLOC_OFF_EPART = NOALLOC_OFF_SYSLIST + 256;
-constexpr size_t NOALLOC_OFF_SYSOUT = NOALLOC_OFF_EPART + 8 * EPART_N * (size_t)NOALLOC_BEADS;
+constexpr size_t NOALLOC_OFF_SYSOUT = 8 * TPART_N * (size_t)(NOALLOC_BEADS / TILE);
 constexpr size_t NOALLOC_BYTES = NOALLOC_OFF_SYSOUT + 8 * SYSOUT_N;
 
 } // namespace sopk
