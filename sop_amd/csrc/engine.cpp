@@ -205,6 +205,21 @@ static sop_status grow_array(sop_engine *e, void **ptr, size_t old_bytes, size_t
   return SOP_OK;
 }
 
+namespace sopk {
+// Pinned host memory of at least `bytes` (the stream is idle when it moves).
+sop_status engine_io(sop_engine *e, HostBuf &b, size_t bytes) {
+  if (b.bytes >= bytes) return SOP_OK;
+  HIPCK(hipStreamSynchronize(e->stream));
+  const size_t nb = std::max<size_t>(bytes + bytes / 2, (size_t)64 << 10);
+  void *q = nullptr;
+  HIPCK(hipHostMalloc(&q, nb, hipHostMallocDefault));
+  if (b.ptr) (void)hipHostFree(b.ptr);
+  b.ptr = q;
+  b.bytes = nb;
+  return SOP_OK;
+}
+} // namespace sopk
+
 static void invalidate_graphs(sop_engine *e) {
   for (auto &kv : e->graphs) (void)hipGraphExecDestroy(kv.second);
   e->graphs.clear();
@@ -278,6 +293,11 @@ static sop_status ensure_capacity(sop_engine *e, int64_t beads, int64_t nat, int
     if (s) return s;
     s = grow_array(e, (void **)&e->p.syslist, 4 * (size_t)c.slots, 4 * (size_t)nn);
     if (s) return s;
+    int2 *rep = nullptr;
+    HIPCK(hipHostMalloc((void **)&rep, sizeof(int2) * (size_t)nn, hipHostMallocDefault));
+    for (int64_t q = 0; q < nn; ++q) rep[q] = q < c.slots ? e->p.rep[q] : make_int2(0, 0);
+    if (e->p.rep) (void)hipHostFree(e->p.rep);
+    e->p.rep = rep;
     c.slots = nn;
     e->sys.resize((size_t)nn);
     changed = true;
@@ -541,11 +561,9 @@ sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, in
     std::memcpy(q, src, bytes);
     return hipMemcpyAsync(dst, q, bytes, hipMemcpyHostToDevice, up);
   };
-  h.wbits.resize((size_t)n);
   int32_t cur = 0;
   for (int i = 0; i < n; ++i) {
     const int32_t wb = (chain[i] << 2) | type[i];
-    h.wbits[i] = wb;
     float wf;
     std::memcpy(&wf, &wb, 4);
     pos[i] = make_float4(d->xyz[3 * i], d->xyz[3 * i + 1], d->xyz[3 * i + 2], wf);
@@ -723,16 +741,16 @@ sop_status engine_resize_rows(sop_engine *e, int32_t slot, int32_t cap, bool kee
 // Systems whose longest row came within an eighth of their row capacity get
 // a larger one; their rows move and no result changes.  With fixed pools a
 // capacity that finds no room stays as it is (a row that outgrows it is
-// reported as an overflow).  The engine stream must be idle; sd is the
-// systems' current state.  *grown receives each system's added bytes.
-sop_status engine_grow_rows(sop_engine *e, const int32_t *slots, int32_t n, const std::vector<SysDev> &sd,
+// reported as an overflow).  The engine stream must be idle; row_max[q] is the
+// longest row of slots[q] so far.  *grown receives each system's added bytes.
+sop_status engine_grow_rows(sop_engine *e, const int32_t *slots, int32_t n, const int32_t *row_max,
                             std::vector<int64_t> *grown) {
   if (grown) grown->assign((size_t)n, 0);
   if (!e->grow_rows) return SOP_OK;
   for (int32_t q = 0; q < n; ++q) {
     const int32_t s = slots[q];
     const SysHost &h = e->sys[s];
-    const int32_t m = sd[s].row_max;
+    const int32_t m = row_max[q];
     if (!pl_cap_short(e, h, m)) continue;
     const int64_t before = engine_system_bytes(e, s);
     const sop_status st = engine_resize_rows(e, s, pl_cap_target(e, h.n, m), true);
@@ -813,8 +831,12 @@ sop_status engine_init_lists(sop_engine *e, const int32_t *slots, int32_t n, sop
   HIPCK(hipStreamSynchronize(e->stream));
   st = engine_fit_new(e, slots, n);
   if (st) return st;
+  st = engine_set_batch(e, slots, n);  // (engine_fit_new may have left a part of it)
+  if (st) return st;
+  HIPCK(launch_report(e->p, e->stream));
+  HIPCK(hipStreamSynchronize(e->stream));
   for (int32_t q = 0; q < n; ++q) {
-    status[q] = engine_check_errors(e, &slots[q], 1);
+    status[q] = engine_error_status(e, slots[q], e->p.rep[slots[q]].x);
     if (status[q]) engine_remove_system(e, slots[q]);
   }
   return SOP_OK;
@@ -851,6 +873,25 @@ sop_status engine_remove_system(sop_engine *e, int32_t slot) {
 // tiles of a system share one XCD's L2.
 sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots) {
   constexpr int NX = 8;
+  // everything the tables are made from: while it is what it was, so are they
+  std::vector<int64_t> key;
+  key.reserve(20 + 3 * (size_t)nslots);
+  for (int64_t v : {(int64_t)nslots, (int64_t)e->fixed_grids, (int64_t)e->opts.lanes_per_bead, (int64_t)e->opts.step_tiles,
+                    (int64_t)e->opts.lds_beads_max, (int64_t)e->lds_limit, e->lds_big_cap, (int64_t)e->num_cu,
+                    (int64_t)e->tune.nb, (int64_t)e->tune.tail})
+    key.push_back(v);
+  for (int b = 0; b < 3; ++b) {
+    key.push_back(e->tune.max_beads[b]);
+    key.push_back(e->tune.tiles[b]);
+  }
+  for (int32_t q = 0; q < nslots; ++q) {
+    const SysHost &h = e->sys[slots[q]];
+    key.push_back(slots[q]);
+    key.push_back(h.bead_off);
+    key.push_back(h.n);
+  }
+  if (key == e->batch_key) return SOP_OK;
+  e->batch_key.clear();
   std::vector<int32_t> order(slots, slots + nslots);
   std::sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
     if (e->sys[a].bead_len != e->sys[b].bead_len) return e->sys[a].bead_len > e->sys[b].bead_len;
@@ -1172,18 +1213,11 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   }
   if (nslots > e->cap.slots) return set_error(e, SOP_ERR_INVALID, "batch larger than slot capacity");
   const int32_t nw = (int32_t)e->h_work.size(), ns = nslots;
-  if (nw > 0) HIPCK(hipMemcpy(e->p.work, e->h_work.data(), 4 * (size_t)nw, hipMemcpyHostToDevice));
-  if (ns > 0) HIPCK(hipMemcpy(e->p.syslist, e->h_syslist.data(), 4 * (size_t)ns, hipMemcpyHostToDevice));
-  e->cur_ntiles = (int32_t)tiles.size();
-  if (!tiles.empty())
-    HIPCK(hipMemcpy(e->p.tiles, tiles.data(), sizeof(int2) * tiles.size(), hipMemcpyHostToDevice));
   const int32_t ni = (int32_t)e->h_items.size(), nfi = (int32_t)e->h_fitems.size();
-  if (ni > 0) HIPCK(hipMemcpy(e->p.items, e->h_items.data(), sizeof(int4) * (size_t)ni, hipMemcpyHostToDevice));
-  if (nfi > 0) HIPCK(hipMemcpy(e->p.fitems, e->h_fitems.data(), sizeof(int4) * (size_t)nfi, hipMemcpyHostToDevice));
-  // the counters in one copy: nwork[0] = work entries, [16] batch systems,
-  // [24] large ones, [32] home cells and [40] neighbor-list builds of a rebuild
-  // (none between rebuilds), [44..46] filter items, [48] / [56] / [60] step
-  // items (LDS / far / whole-CU), [57] step tiles
+  // the counters: nwork[0] = work entries, [16] batch systems, [24] large
+  // ones, [32] home cells and [40] neighbor-list builds of a rebuild (none
+  // between rebuilds), [44..46] filter items, [48] / [56] / [60] step items
+  // (LDS / far / whole-CU), [57] step tiles
   int32_t cnt[64] = {0};
   cnt[0] = nw;
   cnt[16] = ns;
@@ -1195,7 +1229,30 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   cnt[56] = sp.n_far;
   cnt[57] = (int32_t)tiles.size();
   cnt[60] = sp.n_big;
-  HIPCK(hipMemcpy(e->p.nwork, cnt, sizeof(cnt), hipMemcpyHostToDevice));
+  // all of it through the staging buffer, in one launch
+  const std::pair<void *, std::pair<const void *, size_t>> parts[TABLE_PARTS] = {
+      {e->p.nwork, {cnt, 64}},
+      {e->p.work, {e->h_work.data(), (size_t)nw}},
+      {e->p.syslist, {e->h_syslist.data(), (size_t)ns}},
+      {e->p.items, {e->h_items.data(), 4 * (size_t)ni}},
+      {e->p.fitems, {e->h_fitems.data(), 4 * (size_t)nfi}},
+      {e->p.tiles, {tiles.data(), 2 * tiles.size()}}};
+  size_t words = 0;
+  for (const auto &q : parts) words += q.second.second;
+  HIPCK(hipStreamSynchronize(e->stream));  // the launch that read the last tables has passed
+  sop_status st = engine_io(e, e->stage, 4 * words);
+  if (st) return st;
+  TableParts tp;
+  tp.stage = static_cast<const uint32_t *>(e->stage.ptr);
+  size_t at = 0;
+  for (int k = 0; k < TABLE_PARTS; ++k) {
+    const auto &q = parts[k];
+    if (q.second.second) std::memcpy(static_cast<uint32_t *>(e->stage.ptr) + at, q.second.first, 4 * q.second.second);
+    tp.part[k] = TablePart{static_cast<uint32_t *>(q.first), (uint32_t)at, (uint32_t)q.second.second};
+    at += q.second.second;
+  }
+  HIPCK(launch_tables(tp, e->stream));
+  e->cur_ntiles = (int32_t)tiles.size();
   e->cur_nwork = nw;
   e->cur_nsys = ns;
   e->cur_nbig = nbig;
@@ -1205,6 +1262,7 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   e->cur_nfitems = fp.n_lds;
   e->cur_nfitems_far = fp.n_far;
   e->cur_nfitems_big = fp.n_big;
+  e->batch_key.swap(key);
   return SOP_OK;
 }
 
@@ -1222,11 +1280,13 @@ sop_status engine_error_status(sop_engine *e, int32_t s, int32_t err) {
   return set_error(e, st, os.str());
 }
 
+// Status of the listed systems, which are the current batch's: reported by the
+// device and read once the stream is done.
 sop_status engine_check_errors(sop_engine *e, const int32_t *slots, int32_t nslots) {
-  std::vector<SysDev> sd((size_t)e->cap.slots);
-  HIPCK(hipMemcpy(sd.data(), e->p.sys, sizeof(SysDev) * sd.size(), hipMemcpyDeviceToHost));
+  HIPCK(launch_report(e->p, e->stream));
+  HIPCK(hipStreamSynchronize(e->stream));
   for (int q = 0; q < nslots; ++q) {
-    const sop_status st = engine_error_status(e, slots[q], sd[slots[q]].err);
+    const sop_status st = engine_error_status(e, slots[q], e->p.rep[slots[q]].x);
     if (st) return st;
   }
   return SOP_OK;
@@ -1305,6 +1365,13 @@ static void mirror_advance(sop_engine *e, const int32_t *sys, int32_t nsys, int6
   }
 }
 
+// Row capacities after steps, from what the last k_advance reported.
+static sop_status grow_reported(sop_engine *e, const int32_t *sys, int32_t nsys) {
+  std::vector<int32_t> longest((size_t)nsys);
+  for (int32_t q = 0; q < nsys; ++q) longest[q] = e->p.rep[sys[q]].y;
+  return engine_grow_rows(e, sys, nsys, longest.data(), nullptr);
+}
+
 // nsteps of the listed systems in one batch: hipGraph blocks of n_nl steps
 // while the schedule is uniform and aligned, host-driven launches for the
 // rest.  With events, ev0 is recorded after the batch's tables are set and
@@ -1342,11 +1409,8 @@ sop_status engine_run(sop_engine *e, const int32_t *sys, int32_t nsys, int64_t n
       left -= G;
       // row capacities checked every GROW_BLOCKS blocks of a long run
       if (++blocks % GROW_BLOCKS == 0 && left >= G && !ev1) {
-        std::vector<SysDev> sd;
         HIPCK(hipStreamSynchronize(e->stream));
-        st = read_sys_all(e, sd);
-        if (st) return st;
-        st = engine_grow_rows(e, sys, nsys, sd, nullptr);
+        st = grow_reported(e, sys, nsys);
         if (st) return st;
       }
     }
@@ -1358,13 +1422,10 @@ sop_status engine_run(sop_engine *e, const int32_t *sys, int32_t nsys, int64_t n
   }
   if (ev1) HIPCK(hipEventRecord(ev1, e->stream));
   HIPCK(hipStreamSynchronize(e->stream));
-  std::vector<SysDev> sd;
-  st = read_sys_all(e, sd);
-  if (st) return st;
-  st = engine_grow_rows(e, sys, nsys, sd, nullptr);
+  st = grow_reported(e, sys, nsys);
   if (st) return st;
   for (int32_t q = 0; q < nsys; ++q) {
-    st = engine_error_status(e, sys[q], sd[sys[q]].err);
+    st = engine_error_status(e, sys[q], e->p.rep[sys[q]].x);
     if (st) return st;
   }
   return SOP_OK;
@@ -1536,6 +1597,8 @@ void sop_engine_destroy(sop_engine *e) {
                     e->p.syslist, e->p.work,    e->p.nwork,    e->p.items,
                     e->p.tiles};
   for (void *q : others) if (q) note(hipFree(q), "hipFree");
+  for (void *q : {e->io.ptr, e->stage.ptr, (void *)e->p.rep}) if (q) note(hipHostFree(q), "hipHostFree");
+  if (e->p.fitems) note(hipFree(e->p.fitems), "hipFree");
   if (e->fork.side) note(hipStreamSynchronize(e->fork.side), "hipStreamSynchronize");
   if (e->fork.fork) note(hipEventDestroy(e->fork.fork), "hipEventDestroy");
   if (e->fork.join) note(hipEventDestroy(e->fork.join), "hipEventDestroy");
@@ -1596,7 +1659,6 @@ sop_status sop_update_neighbor_list(sop_engine *e, int32_t sys) {
   st = engine_set_batch(e, &sys, 1);
   if (st) return st;
   HIPCK(launch_lists(e->p, list_grids(e), 0, FORCE_NL, e->stream));
-  HIPCK(hipStreamSynchronize(e->stream));
   return engine_check_errors(e, &sys, 1);
 }
 
@@ -1605,7 +1667,6 @@ sop_status sop_update_pair_list(sop_engine *e, int32_t sys) {
   sop_status st = engine_set_batch(e, &sys, 1);
   if (st) return st;
   HIPCK(launch_lists(e->p, list_grids(e), 0, FORCE_PL, e->stream));
-  HIPCK(hipStreamSynchronize(e->stream));
   return engine_check_errors(e, &sys, 1);
 }
 
@@ -1616,7 +1677,6 @@ static sop_status materialize_nl(sop_engine *e, int32_t sys) {
   st = engine_set_batch(e, &sys, 1);
   if (st) return st;
   HIPCK(launch_lists(e->p, list_grids(e), 0, MATERIALIZE_NL, e->stream));
-  HIPCK(hipStreamSynchronize(e->stream));
   return engine_check_errors(e, &sys, 1);
 }
 
@@ -1748,30 +1808,41 @@ sop_status sop_force_eval(sop_engine *e, int32_t sys, int32_t with_noise) {
   if (st) return st;
   HIPCK(launch_step(e->p, with_noise ? MODE_FORCE_NOISE : MODE_FORCE, e->opts.lanes_per_bead, step_grids(e), 0,
                     e->stream));
-  HIPCK(hipStreamSynchronize(e->stream));
   return engine_check_errors(e, &sys, 1);
+}
+
+// Per-bead values of a system in the host buffer (after a 64-byte header),
+// with the stream done.
+static sop_status read_beads(sop_engine *e, int32_t sys, int what, const float **out, int64_t *step) {
+  const SysHost &h = e->sys[sys];
+  sop_status st = engine_io(e, e->io, 64 + 16 * (size_t)h.n);
+  if (st) return st;
+  float *f = reinterpret_cast<float *>(static_cast<char *>(e->io.ptr) + 64);
+  HIPCK(launch_read(e->p, sys, h.n, what, f, static_cast<int64_t *>(e->io.ptr), e->stream));
+  HIPCK(hipStreamSynchronize(e->stream));
+  *out = f;
+  if (step) *step = *static_cast<const int64_t *>(e->io.ptr);
+  return SOP_OK;
 }
 
 sop_status sop_get_forces(sop_engine *e, int32_t sys, float *f3n) {
   if (!valid_sys(e, sys) || !f3n) return set_error(e, SOP_ERR_INVALID, "bad arguments");
-  HIPCK(hipStreamSynchronize(e->stream));
-  const SysHost &h = e->sys[sys];
-  std::vector<float4> f((size_t)h.n);
-  HIPCK(hipMemcpy(f.data(), e->p.fout + h.bead_off, 16 * (size_t)h.n, hipMemcpyDeviceToHost));
-  for (int i = 0; i < h.n; ++i) {
-    f3n[3 * i] = f[i].x;
-    f3n[3 * i + 1] = f[i].y;
-    f3n[3 * i + 2] = f[i].z;
-  }
+  const float *f = nullptr;
+  const sop_status st = read_beads(e, sys, READ_FORCES, &f, nullptr);
+  if (st) return st;
+  std::memcpy(f3n, f, 12 * (size_t)e->sys[sys].n);
   return SOP_OK;
 }
 
 static sop_status eval_energy(sop_engine *e, int32_t sys, double *out) {
   const SysHost &h = e->sys[sys];
+  const sop_status st = engine_io(e, e->io, 8 * SYSOUT_N);
+  if (st) return st;
   const int nt = (int)(h.bead_len / TILE);
-  HIPCK(launch_energy_one(e->p, (int)(h.bead_off / TILE), nt, sys, std::min(nt, 2 * e->num_cu), nullptr, e->stream));
-  HIPCK(hipMemcpyAsync(out, e->p.sysout + (int64_t)sys * SYSOUT_N, 8 * SYSOUT_N, hipMemcpyDeviceToHost, e->stream));
+  HIPCK(launch_energy_one(e->p, (int)(h.bead_off / TILE), nt, sys, std::min(nt, 2 * e->num_cu),
+                          static_cast<double *>(e->io.ptr), e->stream));
   HIPCK(hipStreamSynchronize(e->stream));
+  std::memcpy(out, e->io.ptr, 8 * 12);
   return SOP_OK;
 }
 
@@ -1851,76 +1922,54 @@ sop_status sop_run_plain(sop_engine *e, const int32_t *sys, int32_t nsys, int64_
     mirror_advance(e, &sys[q], 1, nsteps);
   }
   HIPCK(hipStreamSynchronize(e->stream));
-  return engine_check_errors(e, sys, nsys);
-}
-
-static sop_status read_coords(sop_engine *e, int32_t sys, std::vector<float4> &x) {
-  SysDev S;
-  sop_status st = engine_read_sys(e, sys, &S);
-  if (st) return st;
-  const SysHost &h = e->sys[sys];
-  x.resize((size_t)h.n);
-  HIPCK(hipMemcpy(x.data(), (S.parity & 1 ? e->p.pos1 : e->p.pos0) + h.bead_off, 16 * (size_t)h.n,
-                  hipMemcpyDeviceToHost));
+  for (int q = 0; q < nsys; ++q) {  // as k_advance reported them
+    st = engine_error_status(e, sys[q], e->p.rep[sys[q]].x);
+    if (st) return st;
+  }
   return SOP_OK;
 }
 
 sop_status sop_get_coords(sop_engine *e, int32_t sys, float *xyz, int64_t *step) {
   if (!valid_sys(e, sys)) return set_error(e, SOP_ERR_INVALID, "no such system");
-  std::vector<float4> x;
-  sop_status st = read_coords(e, sys, x);
+  const float *x = nullptr;
+  const sop_status st = read_beads(e, sys, READ_COORDS, &x, step);
   if (st) return st;
-  if (xyz)
-    for (size_t i = 0; i < x.size(); ++i) {
-      xyz[3 * i] = x[i].x;
-      xyz[3 * i + 1] = x[i].y;
-      xyz[3 * i + 2] = x[i].z;
-    }
-  if (step) {
-    SysDev S;
-    st = engine_read_sys(e, sys, &S);
-    if (st) return st;
-    *step = S.step;
-  }
+  if (xyz) std::memcpy(xyz, x, 12 * (size_t)e->sys[sys].n);
   return SOP_OK;
 }
 
 sop_status sop_get_wrapped_coords(sop_engine *e, int32_t sys, float *xyz) {
   if (!valid_sys(e, sys) || !xyz) return set_error(e, SOP_ERR_INVALID, "bad arguments");
-  std::vector<float4> x;
-  sop_status st = read_coords(e, sys, x);
+  const float *x = nullptr;
+  const sop_status st = read_beads(e, sys, READ_COORDS, &x, nullptr);
   if (st) return st;
   const float boxl = e->sys[sys].params.boxl;
-  for (size_t i = 0; i < x.size(); ++i) {
-    float v[3] = {x[i].x, x[i].y, x[i].z};
-    for (int d = 0; d < 3; ++d) {
-      if (boxl > 0.0f) v[d] = v[d] - boxl * rintf(v[d] / boxl);
-      xyz[3 * i + d] = v[d];
-    }
-  }
+  const size_t m = 3 * (size_t)e->sys[sys].n;
+  for (size_t k = 0; k < m; ++k) xyz[k] = boxl > 0.0f ? x[k] - boxl * rintf(x[k] / boxl) : x[k];
   return SOP_OK;
 }
 
 // Forces with noise of the current step (kstep 0) or of the last step taken
-// (kstep -1: the other coordinate buffer and step - 1) into fout, copied out.
-static sop_status noisy_forces(sop_engine *e, int32_t sys, int kstep, std::vector<float4> &f) {
+// (kstep -1: the other coordinate buffer and step - 1), three floats a bead.
+static sop_status noisy_forces(sop_engine *e, int32_t sys, int kstep, std::vector<float> &f) {
   sop_status st = engine_set_batch(e, &sys, 1);
   if (st) return st;
   HIPCK(launch_step(e->p, MODE_FORCE_NOISE, e->opts.lanes_per_bead, step_grids(e), kstep, e->stream));
-  HIPCK(hipStreamSynchronize(e->stream));
   st = engine_check_errors(e, &sys, 1);
   if (st) return st;
-  const SysHost &h = e->sys[sys];
-  f.resize((size_t)h.n);
-  HIPCK(hipMemcpy(f.data(), e->p.fout + h.bead_off, 16 * (size_t)h.n, hipMemcpyDeviceToHost));
+  const float *x = nullptr;
+  st = read_beads(e, sys, READ_FORCES, &x, nullptr);
+  if (st) return st;
+  f.assign(x, x + 3 * (size_t)e->sys[sys].n);
   return SOP_OK;
 }
 
 static sop_status read_vel_state(sop_engine *e, int32_t sys, std::vector<float4> &v) {
-  HIPCK(hipStreamSynchronize(e->stream));
-  const SysHost &h = e->sys[sys];
-  v.resize((size_t)h.n);
-  HIPCK(hipMemcpy(v.data(), e->p.vel + h.bead_off, 16 * (size_t)h.n, hipMemcpyDeviceToHost));
+  const float *x = nullptr;
+  const sop_status st = read_beads(e, sys, READ_VEL, &x, nullptr);
+  if (st) return st;
+  v.resize((size_t)e->sys[sys].n);
+  std::memcpy(v.data(), x, 16 * v.size());
   return SOP_OK;
 }
 
@@ -1937,7 +1986,8 @@ sop_status sop_get_velocities(sop_engine *e, int32_t sys, float *v3n) {
     std::fill(v3n, v3n + 3 * (size_t)h.n, 0.0f);
     return SOP_OK;
   }
-  std::vector<float4> v, f;
+  std::vector<float4> v;
+  std::vector<float> f;
   sop_status st = read_vel_state(e, sys, v);
   if (st) return st;
   bool any = false;
@@ -1948,9 +1998,9 @@ sop_status sop_get_velocities(sop_engine *e, int32_t sys, float *v3n) {
   for (int i = 0; i < h.n; ++i) {
     const float4 s = v[i];
     if (incr_flag(s)) {
-      v3n[3 * i] = a[2] * s.x + a[3] * f[i].x;
-      v3n[3 * i + 1] = a[2] * s.y + a[3] * f[i].y;
-      v3n[3 * i + 2] = a[2] * s.z + a[3] * f[i].z;
+      v3n[3 * i] = a[2] * s.x + a[3] * f[3 * i];
+      v3n[3 * i + 1] = a[2] * s.y + a[3] * f[3 * i + 1];
+      v3n[3 * i + 2] = a[2] * s.z + a[3] * f[3 * i + 2];
     } else {
       v3n[3 * i] = s.x;
       v3n[3 * i + 1] = s.y;
@@ -1963,7 +2013,8 @@ sop_status sop_get_velocities(sop_engine *e, int32_t sys, float *v3n) {
 sop_status sop_get_increments(sop_engine *e, int32_t sys, float *d3n) {
   if (!valid_sys(e, sys) || !d3n) return set_error(e, SOP_ERR_INVALID, "bad arguments");
   const SysHost &h = e->sys[sys];
-  std::vector<float4> v, f;
+  std::vector<float4> v;
+  std::vector<float> f;
   sop_status st;
   if (h.params.dynamics == SOP_DYN_UNDERDAMPED) {
     if ((st = read_vel_state(e, sys, v))) return st;
@@ -1979,9 +2030,9 @@ sop_status sop_get_increments(sop_engine *e, int32_t sys, float *d3n) {
         d3n[3 * i + 1] = s.y;
         d3n[3 * i + 2] = s.z;
       } else {
-        d3n[3 * i] = a[0] * s.x + a[1] * f[i].x;
-        d3n[3 * i + 1] = a[0] * s.y + a[1] * f[i].y;
-        d3n[3 * i + 2] = a[0] * s.z + a[1] * f[i].z;
+        d3n[3 * i] = a[0] * s.x + a[1] * f[3 * i];
+        d3n[3 * i + 1] = a[0] * s.y + a[1] * f[3 * i + 1];
+        d3n[3 * i + 2] = a[0] * s.z + a[1] * f[3 * i + 2];
       }
     }
     return SOP_OK;
@@ -1989,11 +2040,7 @@ sop_status sop_get_increments(sop_engine *e, int32_t sys, float *d3n) {
   if ((st = noisy_forces(e, sys, -1, f))) return st;
   float a5, var;
   sop_params_derived(&h.params, &a5, &var);
-  for (int i = 0; i < h.n; ++i) {
-    d3n[3 * i] = a5 * f[i].x;
-    d3n[3 * i + 1] = a5 * f[i].y;
-    d3n[3 * i + 2] = a5 * f[i].z;
-  }
+  for (size_t k = 0; k < f.size(); ++k) d3n[k] = a5 * f[k];
   return SOP_OK;
 }
 
@@ -2016,21 +2063,13 @@ sop_status sop_set_rng(sop_engine *e, int32_t sys, uint64_t seed, int64_t step) 
 
 sop_status sop_set_coords(sop_engine *e, int32_t sys, const float *xyz) {
   if (!valid_sys(e, sys) || !xyz) return set_error(e, SOP_ERR_INVALID, "bad arguments");
-  SysDev S;
-  sop_status st = engine_read_sys(e, sys, &S);
+  const size_t bytes = 12 * (size_t)e->sys[sys].n;
+  sop_status st = engine_io(e, e->io, bytes);
   if (st) return st;
-  const SysHost &h = e->sys[sys];
-  std::vector<float4> x((size_t)h.n);
-  for (int i = 0; i < h.n; ++i) {
-    float wf;
-    std::memcpy(&wf, &h.wbits[i], 4);
-    x[i] = make_float4(xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], wf);
-  }
-  HIPCK(hipMemcpy((S.parity & 1 ? e->p.pos1 : e->p.pos0) + h.bead_off, x.data(), 16 * (size_t)h.n,
-                  hipMemcpyHostToDevice));
+  std::memcpy(e->io.ptr, xyz, bytes);
   // new coordinates clear the system's sticky error bits
-  const int32_t zero = 0;
-  HIPCK(hipMemcpy((char *)(e->p.sys + sys) + offsetof(SysDev, err), &zero, 4, hipMemcpyHostToDevice));
+  HIPCK(launch_write_coords(e->p, sys, e->sys[sys].n, static_cast<const float *>(e->io.ptr), e->stream));
+  HIPCK(hipStreamSynchronize(e->stream));  // the buffer is the next call's
   return SOP_OK;
 }
 

@@ -26,6 +26,10 @@ hipError_t step_lds_limit(size_t bytes);
 hipError_t filter_lds_init();
 hipError_t launch_energy(const DevPtrs &p, int grid_tiles, int grid_sys, hipStream_t st);
 hipError_t launch_energy_one(const DevPtrs &p, int t0, int nt, int slot, int grid_tiles, double *out, hipStream_t st);
+hipError_t launch_tables(const TableParts &tp, hipStream_t st);
+hipError_t launch_report(const DevPtrs &p, hipStream_t st);
+hipError_t launch_read(const DevPtrs &p, int slot, int n, int what, float *out, int64_t *step, hipStream_t st);
+hipError_t launch_write_coords(const DevPtrs &p, int slot, int n, const float *in, hipStream_t st);
 hipError_t launch_advance(const DevPtrs &p, int nsteps, hipStream_t st);
 hipError_t launch_relayout(const DevPtrs &p, int bo, int n, int idx16, int64_t old_base, int old_cap,
                            int64_t new_base, int new_cap, hipStream_t st);
@@ -48,8 +52,8 @@ class RangeAlloc {
   std::map<int64_t, int64_t> free_;
 };
 
-// Device array that can grow, keeping its contents.
-struct DevBuf {
+// Pinned host memory that kernels read and write, grown as needed.
+struct HostBuf {
   void *ptr = nullptr;
   size_t bytes = 0;
 };
@@ -64,7 +68,6 @@ struct SysHost {
   int64_t step = 0;  // host mirror (exact outside serving)
   int32_t parity = 0;
   sop_params params{};
-  std::vector<int32_t> wbits;  // w component of each bead (chain<<2|type)
 };
 
 struct Pools {
@@ -91,6 +94,12 @@ struct sop_engine {
   sopk::DevPtrs p{};
   // raw buffers in allocation order (for growth/free)
   std::vector<std::pair<void **, size_t>> bead_arrays, nat_arrays, cell_arrays;
+
+  // the host's end of a call: results, and the tables staged for a batch
+  // (reusable once the engine stream has passed the launch that reads them)
+  sopk::HostBuf io, stage;
+  // what the tables on the device were made from (empty: nothing yet)
+  std::vector<int64_t> batch_key;
 
   // work tables (host staging)
   std::vector<int32_t> h_work, h_syslist;
@@ -178,6 +187,7 @@ int64_t job_bytes_estimate(const sop_engine *e, const sop_system_desc *d);
 int64_t engine_system_bytes(const sop_engine *e, int32_t slot);
 sop_status engine_fit_new(sop_engine *e, const int32_t *slots, int32_t n);
 sop_status engine_fit_shell(sop_engine *e, int32_t slot, float shell);
-sop_status engine_grow_rows(sop_engine *e, const int32_t *slots, int32_t n, const std::vector<SysDev> &sd,
+sop_status engine_grow_rows(sop_engine *e, const int32_t *slots, int32_t n, const int32_t *row_max,
                             std::vector<int64_t> *grown);
+sop_status engine_io(sop_engine *e, HostBuf &b, size_t bytes);
 } // namespace sopk

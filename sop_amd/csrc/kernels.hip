@@ -2690,6 +2690,56 @@ __global__ __launch_bounds__(256) void k_sys_reduce(DevPtrs p, int slot, double 
   }
 }
 
+// ---- the host's end of a call
+//
+// A call's tables come from one pinned host buffer and its results go to
+// another, both read and written by kernels in stream order: a call is its
+// launches and one wait for the stream (7 synchronous copies of tables and 2
+// of results, 15 us each, were 120 us of every call).
+
+// Tables of a batch from the pinned staging buffer to their device arrays.
+__global__ __launch_bounds__(256) void k_tables(TableParts tp) {
+  const int k = blockIdx.y;
+  const uint32_t *src = tp.stage + tp.part[k].src;
+  uint32_t *dst = tp.part[k].dst;
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < tp.part[k].words; i += gridDim.x * 256) dst[i] = src[i];
+}
+
+// {error bits, longest row} of the batch's systems, for the host.
+__device__ __forceinline__ void report(const DevPtrs &p, int s, const SysDev &S) {
+  p.rep[s] = make_int2(S.err, S.row_max);
+}
+__global__ void k_report(DevPtrs p) {
+  const int nsys = *p.nsys;
+  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < nsys; q += gridDim.x * blockDim.x)
+    report(p, p.syslist[q], p.sys[p.syslist[q]]);
+}
+
+// Per-bead values of one system to the host buffer: the current coordinates or
+// the forces, three floats a bead, or the underdamped state, four; step: the
+// system's completed steps (when not null).
+__global__ __launch_bounds__(256) void k_read(DevPtrs p, int slot, int what, float *out, int64_t *step) {
+  const SysDev &S = p.sys[slot];
+  const float4 *src = what == READ_COORDS ? buf_in(p, S.parity) : (what == READ_FORCES ? p.fout : p.vel);
+  const float *f = reinterpret_cast<const float *>(src + S.bead_off);
+  const int w = what == READ_VEL ? 4 : 3, m = S.n * w;
+  for (int k = blockIdx.x * 256 + threadIdx.x; k < m; k += gridDim.x * 256) out[k] = f[4 * (k / w) + k % w];
+  if (step && blockIdx.x == 0 && threadIdx.x == 0) *step = S.step;
+}
+
+// New coordinates of one system from the host buffer (type and chain stay),
+// and its error bits cleared.
+__global__ __launch_bounds__(256) void k_write_coords(DevPtrs p, int slot, const float *in) {
+  SysDev &S = p.sys[slot];
+  float4 *x = const_cast<float4 *>(buf_in(p, S.parity)) + S.bead_off;
+  const int n = S.n;
+  for (int b = blockIdx.x * 256 + threadIdx.x; b < n; b += gridDim.x * 256) {
+    const float4 o = x[b];
+    x[b] = make_float4(in[3 * b], in[3 * b + 1], in[3 * b + 2], o.w);
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) S.err = 0;
+}
+
 // Per system: open a run of nsteps (the step kernel moves a system while
 // step < step_end).
 __global__ void k_begin(DevPtrs p, int64_t nsteps) {
@@ -2733,7 +2783,8 @@ __global__ __launch_bounds__(64) void k_relayout(DevPtrs p, int bo, int n, int i
   else relayout_tile<uint32_t>(p, bo, n, t, ob, oc, nb, nc);
 }
 
-// Per system: advance the step counter after a block of kernel steps.
+// Per system: advance the step counter after a block of kernel steps, and
+// report to the host.
 __global__ void k_advance(DevPtrs p, int nsteps) {
   const int nsys = *p.nsys;
   for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < nsys; q += gridDim.x * blockDim.x) {
@@ -2741,6 +2792,7 @@ __global__ void k_advance(DevPtrs p, int nsteps) {
     const int64_t st = S.step + nsteps;
     S.step = st < S.step_end ? st : (S.step_end > S.step ? S.step_end : S.step);
     S.parity = (S.parity + nsteps) & 1;
+    report(p, p.syslist[q], S);
   }
 }
 
@@ -2966,6 +3018,29 @@ hipError_t launch_energy(const DevPtrs &p, int grid_tiles, int grid_sys, hipStre
 hipError_t launch_energy_one(const DevPtrs &p, int t0, int nt, int slot, int grid_tiles, double *out, hipStream_t st) {
   hipLaunchKernelGGL(k_energy, dim3(grid_tiles), dim3(ENERGY_THREADS), 0, st, p, t0, nt);
   hipLaunchKernelGGL(k_sys_reduce, dim3(1), dim3(256), 0, st, p, slot, out);
+  return SOPK_LAUNCH_CHECK();
+}
+
+hipError_t launch_tables(const TableParts &tp, hipStream_t st) {
+  uint32_t most = 1;
+  for (const TablePart &q : tp.part) most = std::max(most, q.words);
+  hipLaunchKernelGGL(k_tables, dim3(std::min(64u, (most + 255) / 256), TABLE_PARTS), dim3(256), 0, st, tp);
+  return SOPK_LAUNCH_CHECK();
+}
+
+hipError_t launch_report(const DevPtrs &p, hipStream_t st) {
+  hipLaunchKernelGGL(k_report, dim3(4), dim3(256), 0, st, p);
+  return SOPK_LAUNCH_CHECK();
+}
+
+hipError_t launch_read(const DevPtrs &p, int slot, int n, int what, float *out, int64_t *step, hipStream_t st) {
+  hipLaunchKernelGGL(k_read, dim3(std::max(1, std::min(512, (4 * n + 255) / 256))), dim3(256), 0, st, p, slot, what,
+                     out, step);
+  return SOPK_LAUNCH_CHECK();
+}
+
+hipError_t launch_write_coords(const DevPtrs &p, int slot, int n, const float *in, hipStream_t st) {
+  hipLaunchKernelGGL(k_write_coords, dim3(std::max(1, std::min(512, (n + 255) / 256))), dim3(256), 0, st, p, slot, in);
   return SOPK_LAUNCH_CHECK();
 }
 

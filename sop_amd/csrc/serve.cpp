@@ -122,7 +122,9 @@ sop_status retire_and_start(sop_engine *e, sop_engine::Serve *sv, const std::vec
     std::vector<int32_t> ks;
     for (sop_engine::Job *j : keep) ks.push_back(j->slot);
     std::vector<int64_t> grown;
-    st = engine_grow_rows(e, ks.data(), (int32_t)ks.size(), sd, &grown);
+    std::vector<int32_t> longest;
+    for (int32_t s : ks) longest.push_back(sd[s].row_max);
+    st = engine_grow_rows(e, ks.data(), (int32_t)ks.size(), longest.data(), &grown);
     if (st) return st;
     std::lock_guard<std::mutex> lk(sv->mu);
     for (size_t q = 0; q < keep.size(); ++q) {

@@ -150,6 +150,7 @@ struct DevPtrs {
   double *sysout;       // per system slot: SYSOUT_N reduced values
   int32_t *tile_sys;    // system slot of each tile
   uint8_t *tile_ord;    // per tile: TILE bead offsets in the order the step kernel's lane groups take them
+  int2 *rep;            // per system slot, in pinned host memory: {err, row_max} as of the last report
   int32_t *work;        // tile ids to process (-1 = padding), XCD-interleaved
   int2 *tiles;          // tiles that step and filter with a block each: {tile, system slot}, tile -1 = padding
   int32_t *ntiles;
@@ -211,6 +212,20 @@ struct ListGrids {
   bool split;
   StepGrids fg;
 };
+
+// A batch's tables in the pinned staging buffer (32-bit words).
+constexpr int TABLE_PARTS = 6;
+struct TablePart {
+  uint32_t *dst;
+  uint32_t src, words;
+};
+struct TableParts {
+  TablePart part[TABLE_PARTS];
+  const uint32_t *stage;
+};
+
+// what launch_read copies out
+constexpr int READ_COORDS = 0, READ_FORCES = 1, READ_VEL = 2;
 
 // step-kernel item: tiles in the low byte of .y, waves per tile above it
 __host__ __device__ inline int item_tiles(int y) { return y & 0xFF; }
