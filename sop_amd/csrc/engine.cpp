@@ -109,11 +109,12 @@ static int grid_big_sys(const sop_engine *e) {
 
 // Launch grid of a persistent item kernel: `g` blocks (a multiple of 8, so
 // that item k runs on XCD k mod 8), fewer when the batch has fewer items, none
-// when it has none; fixed grids (serving) always launch g.
+// when it has none; with fixed grids (serving) g or none, so that a few
+// captured graphs serve every batch.
 static int items_grid(int g, bool fixed, int count) {
   g = std::max(8, g / 8 * 8);
-  if (fixed) return g;
   if (count == 0) return 0;  // no launch
+  if (fixed) return g;
   return std::max(8, std::min(g, (count + 7) / 8 * 8));
 }
 
@@ -137,13 +138,8 @@ int grid_step_tiles(const sop_engine *e) {
 }
 
 // Whole-CU LDS items: one block per compute unit (the block takes all of
-// the unit's LDS).  While serving, a fixed grid whenever the batch has such
-// items and no launch when it has none (two graph variants; a light load of
-// small jobs then pays for no empty launch).
-static int items_grid_big(const sop_engine *e, int count) {
-  if (e->fixed_grids) return count > 0 ? items_grid(e->num_cu, true, count) : 0;
-  return items_grid(e->num_cu, false, count);
-}
+// the unit's LDS).
+static int items_grid_big(const sop_engine *e, int count) { return items_grid(e->num_cu, e->fixed_grids, count); }
 int grid_items_big(const sop_engine *e) { return items_grid_big(e, e->cur_nitems_big); }
 
 StepGrids step_grids(const sop_engine *e) {
@@ -293,9 +289,9 @@ static sop_status ensure_capacity(sop_engine *e, int64_t beads, int64_t nat, int
     if (s) return s;
     s = grow_array(e, (void **)&e->p.syslist, 4 * (size_t)c.slots, 4 * (size_t)nn);
     if (s) return s;
-    int2 *rep = nullptr;
-    HIPCK(hipHostMalloc((void **)&rep, sizeof(int2) * (size_t)nn, hipHostMallocDefault));
-    for (int64_t q = 0; q < nn; ++q) rep[q] = q < c.slots ? e->p.rep[q] : make_int2(0, 0);
+    int4 *rep = nullptr;
+    HIPCK(hipHostMalloc((void **)&rep, sizeof(int4) * (size_t)nn, hipHostMallocDefault));
+    for (int64_t q = 0; q < nn; ++q) rep[q] = q < c.slots ? e->p.rep[q] : make_int4(0, 0, 0, 0);
     if (e->p.rep) (void)hipHostFree(e->p.rep);
     e->p.rep = rep;
     c.slots = nn;
@@ -406,9 +402,15 @@ int64_t job_bytes_estimate(const sop_engine *e, const sop_system_desc *d) {
   return beads * per_bead + 24 * 2 * (int64_t)d->n_native + 2 * esz * n * pl_cap + per_cell * cell_cap;
 }
 
+sop_status upload_drain(sop_engine *e, Upload *upl) {
+  HIPCK(hipStreamSynchronize(upl->stream));
+  upl->used = 0;
+  return SOP_OK;
+}
+
 // Validate and upload one system, without its first lists (engine_init_lists).
 sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, int64_t step_end, int32_t *slot_out,
-                                     const Upload *upl) {
+                                     Upload *upl) {
   hipStream_t up = upl ? upl->stream : nullptr;
   if (!d || d->n_beads < 1 || !d->xyz) return set_error(e, SOP_ERR_INVALID, "system: need n_beads >= 1 and xyz");
   const int32_t n = d->n_beads;
@@ -434,7 +436,7 @@ sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, in
   const int32_t nn = d->n_native;
   if (nn < 0 || (nn > 0 && (!d->nat_i || !d->nat_j || !d->nat_r0)))
     return set_error(e, SOP_ERR_INVALID, "native arrays");
-  std::vector<std::vector<std::pair<int32_t, float>>> nat(n);
+  std::vector<int32_t> nstart((size_t)n + 1, 0);
   for (int k = 0; k < nn; ++k) {
     const int i = d->nat_i[k], j = d->nat_j[k];
     if (i < 0 || j < 0 || i >= n || j >= n || i >= j)
@@ -442,22 +444,32 @@ sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, in
     if (chain[i] == chain[j] && j - i <= 2)
       return set_error(e, SOP_ERR_INVALID, "native pair inside the |i-j| <= 2 exclusion");
     if (!(d->nat_r0[k] > 0.0f)) return set_error(e, SOP_ERR_INVALID, "native r0 must be > 0");
-    nat[i].push_back({j, d->nat_r0[k]});
-    nat[j].push_back({i, d->nat_r0[k]});
+    ++nstart[(size_t)i + 1];
+    ++nstart[(size_t)j + 1];
+  }
+  for (int i = 0; i < n; ++i) nstart[(size_t)i + 1] += nstart[i];
+  std::vector<std::pair<int32_t, float>> nat((size_t)2 * nn);
+  {
+    // pairs sorted by (i, j) come out sorted by partner
+    std::vector<int32_t> at(nstart.begin(), nstart.end() - 1);
+    for (int k = 0; k < nn; ++k) {
+      const int i = d->nat_i[k], j = d->nat_j[k];
+      nat[(size_t)at[i]++] = {j, d->nat_r0[k]};
+      nat[(size_t)at[j]++] = {i, d->nat_r0[k]};
+    }
   }
   for (int i = 0; i < n; ++i) {
-    std::sort(nat[i].begin(), nat[i].end());
-    for (size_t q = 1; q < nat[i].size(); ++q)
-      if (nat[i][q].first == nat[i][q - 1].first) return set_error(e, SOP_ERR_INVALID, "duplicate native pair");
-    if (nat[i].size() > 65535) return set_error(e, SOP_ERR_CAPACITY, "more than 65535 native partners of one bead");
+    const auto lo = nat.begin() + nstart[i], hi = nat.begin() + nstart[(size_t)i + 1];
+    if (!std::is_sorted(lo, hi)) std::sort(lo, hi);
+    for (auto q = lo; q < hi; ++q)
+      if (q > lo && q->first == (q - 1)->first) return set_error(e, SOP_ERR_INVALID, "duplicate native pair");
+    if (hi - lo > 65535) return set_error(e, SOP_ERR_CAPACITY, "more than 65535 native partners of one bead");
   }
   // the step kernel holds a native list's offset within its tile's native
   // slots in 16 bits
-  for (int t0 = 0; t0 < n; t0 += TILE) {
-    size_t tn = 0;
-    for (int i = t0; i < std::min(n, t0 + TILE); ++i) tn += nat[i].size();
-    if (tn > 65535) return set_error(e, SOP_ERR_CAPACITY, "more than 65535 native partners in one 64-bead tile");
-  }
+  for (int t0 = 0; t0 < n; t0 += TILE)
+    if (nstart[std::min(n, t0 + TILE)] - nstart[t0] > 65535)
+      return set_error(e, SOP_ERR_CAPACITY, "more than 65535 native partners in one 64-bead tile");
   // capacities
   const int32_t nl_cap = round_up(std::max(1, std::min(n - 1, e->opts.nl_cap_max)), 16);
   const int32_t pl_cap = pl_cap_start(e, n);
@@ -483,10 +495,23 @@ sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, in
   h.step = d->step0;
   h.parity = 0;
   h.params = P;
-  // with an upload stream, every upload goes through the pinned staging
-  // buffer (a copy from pageable memory would wait for the engine stream)
-  const size_t bl = (size_t)h.bead_len, nl_b = (size_t)h.nat_len;
-  const size_t stage_need = 32 * 256 + 16 * bl * 3 + 4 * bl * 9 + 8 * nl_b + bl + 4 * (bl / TILE) + sizeof(SysDev);
+  // the upload: one pinned blob that a kernel unpacks (a copy from pageable
+  // memory would wait for the engine stream)
+  AddSystem up_a{};
+  uint32_t words = 0;
+  auto part = [&](uint32_t &off, size_t w) {
+    off = words;
+    words += (uint32_t)((w + 15) / 16 * 16);
+  };
+  part(up_a.xyz, 3 * (size_t)n);
+  part(up_a.wbits, (size_t)n);
+  part(up_a.bond, (size_t)n);
+  part(up_a.nstart, (size_t)n + 1);
+  part(up_a.natj, 2 * (size_t)nn);
+  part(up_a.natr, 2 * (size_t)nn);
+  part(up_a.vel, d->vel ? 3 * (size_t)n : 0);
+  part(up_a.sys, sizeof(SysDev) / 4);
+  const size_t stage_need = 4 * (size_t)words;
   if (up && stage_need > upl->stage_bytes) return SOP_ERR_BUSY;
   sop_status st;
   // with an upload stream, free ranges only: growing a pool reallocates
@@ -536,64 +561,28 @@ sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, in
     }
     if (slot < 0) return set_error(e, SOP_ERR_CAPACITY, "no free system slot");
   }
-  // host staging
   const int64_t b0 = h.bead_off;
-  std::vector<float4> pos((size_t)h.bead_len, make_float4(0, 0, 0, 0));
-  std::vector<float> bond((size_t)h.bead_len, 0.0f);
-  std::vector<int32_t> nstart((size_t)h.bead_len, (int32_t)h.nat_off), ncnt((size_t)h.bead_len, 0);
-  std::vector<int32_t> zeros((size_t)h.bead_len, 0);
-  std::vector<int32_t> natj((size_t)h.nat_len, 0);
-  std::vector<float> natr((size_t)h.nat_len, 0.0f);
-  std::vector<float4> v((size_t)h.bead_len, make_float4(0, 0, 0, 0));
-  std::vector<uint8_t> ord((size_t)h.bead_len);
-  std::vector<int32_t> ts((size_t)(h.bead_len / TILE), slot);
-  SysDev S;
-  // host buffers above stay alive until the uploads that read them are done
-  struct UploadDrain {
-    hipStream_t s;
-    ~UploadDrain() { if (s) (void)hipStreamSynchronize(s); }
-  } drain{up};
-  size_t staged = 0;
-  auto put = [&](void *dst, const void *src, size_t bytes) {
-    if (!up) return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
-    char *q = static_cast<char *>(upl->stage) + staged;
-    staged += (bytes + 255) / 256 * 256;
-    std::memcpy(q, src, bytes);
-    return hipMemcpyAsync(dst, q, bytes, hipMemcpyHostToDevice, up);
-  };
-  int32_t cur = 0;
-  for (int i = 0; i < n; ++i) {
-    const int32_t wb = (chain[i] << 2) | type[i];
-    float wf;
-    std::memcpy(&wf, &wb, 4);
-    pos[i] = make_float4(d->xyz[3 * i], d->xyz[3 * i + 1], d->xyz[3 * i + 2], wf);
-    bond[i] = d->bond_r0 ? d->bond_r0[i] : 3.8f;
-    nstart[i] = (int32_t)h.nat_off + cur;
-    ncnt[i] = (int32_t)nat[i].size();
-    for (auto &pr : nat[i]) {
-      natj[cur] = (int32_t)b0 + pr.first;
-      natr[cur] = pr.second;
-      ++cur;
-    }
+  if (up) {
+    if (upl->used + stage_need > upl->stage_bytes && (st = upload_drain(e, upl))) return st;
+  } else {
+    HIPCK(hipStreamSynchronize(e->stream));  // the launch that read the staging buffer last has passed
+    if ((st = engine_io(e, e->stage, stage_need))) return st;
   }
-  const DevPtrs &p = e->p;
-  HIPCK(put(p.pos0 + b0, pos.data(), 16 * h.bead_len));
-  HIPCK(put(p.pos1 + b0, pos.data(), 16 * h.bead_len));
-  HIPCK(put(p.bond_r0 + b0, bond.data(), 4 * h.bead_len));
-  HIPCK(put(p.nat_start + b0, nstart.data(), 4 * h.bead_len));
-  HIPCK(put(p.nat_cnt + b0, ncnt.data(), 4 * h.bead_len));
-  for (int32_t *arr : {p.nlatt_cnt, p.platt_cnt, p.nlrep_cnt, p.plrep_cnt, p.plrep_off, p.platt_off})
-    HIPCK(put(arr + b0, zeros.data(), 4 * h.bead_len));
-  // underdamped state: the velocities entering the first step (w = 0)
-  if (d->vel)
-    for (int i = 0; i < n; ++i) v[i] = make_float4(d->vel[3 * i], d->vel[3 * i + 1], d->vel[3 * i + 2], 0.0f);
-  HIPCK(put(p.vel + b0, v.data(), 16 * h.bead_len));
-  HIPCK(put(p.nat_j + h.nat_off, natj.data(), 4 * h.nat_len));
-  HIPCK(put(p.nat_r0 + h.nat_off, natr.data(), 4 * h.nat_len));
-  // identity bead order per tile until the first pair list orders it
-  for (size_t k = 0; k < ord.size(); ++k) ord[k] = (uint8_t)(k % TILE);
-  HIPCK(put(p.tile_ord + b0, ord.data(), ord.size()));
-  HIPCK(put(p.tile_sys + b0 / TILE, ts.data(), 4 * ts.size()));
+  uint32_t *blob = reinterpret_cast<uint32_t *>(up ? static_cast<char *>(upl->stage) + upl->used
+                                                   : static_cast<char *>(e->stage.ptr));
+  std::memcpy(blob + up_a.xyz, d->xyz, 12 * (size_t)n);
+  std::memcpy(blob + up_a.nstart, nstart.data(), 4 * nstart.size());
+  if (d->vel) std::memcpy(blob + up_a.vel, d->vel, 12 * (size_t)n);
+  for (int i = 0; i < n; ++i) {
+    const float r0 = d->bond_r0 ? d->bond_r0[i] : 3.8f;
+    blob[up_a.wbits + i] = (uint32_t)((chain[i] << 2) | type[i]);
+    std::memcpy(blob + up_a.bond + i, &r0, 4);
+  }
+  for (size_t k = 0; k < nat.size(); ++k) {
+    blob[up_a.natj + k] = (uint32_t)nat[k].first;
+    std::memcpy(blob + up_a.natr + k, &nat[k].second, 4);
+  }
+  SysDev S;
   // device descriptor
   std::memset(&S, 0, sizeof(S));
   S.bead_off = (int32_t)b0;
@@ -688,8 +677,17 @@ sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, in
   S.dims[0] = S.dims[1] = S.dims[2] = 1;
   S.ncells = 1;
   S.wrap_free = 0;
-  HIPCK(put(p.sys + slot, &S, sizeof(SysDev)));
-  if (up) HIPCK(hipStreamSynchronize(up));
+  std::memcpy(blob + up_a.sys, &S, sizeof(SysDev));
+  up_a.blob = blob;
+  up_a.bead_off = (int32_t)b0;
+  up_a.bead_len = (int32_t)h.bead_len;
+  up_a.n = n;
+  up_a.nat_off = (int32_t)h.nat_off;
+  up_a.n_nat = 2 * nn;
+  up_a.slot = slot;
+  up_a.has_vel = d->vel ? 1 : 0;
+  HIPCK(launch_add_system(e->p, up_a, up ? up : e->stream));
+  if (up) upl->used += (stage_need + 255) / 256 * 256;
   e->sys[slot] = std::move(h);
   *slot_out = slot;
   return SOP_OK;
@@ -786,18 +784,17 @@ sop_status engine_fit_shell(sop_engine *e, int32_t slot, float shell) {
 // coordinates (the lists a fitted first build gives); its build counts are
 // set back to one build.  Capacities only grow, so a system never holds less
 // than job_bytes_estimate charged for it.
+// (From what the device reported after those lists.)
 sop_status engine_fit_new(sop_engine *e, const int32_t *slots, int32_t n) {
-  std::vector<SysDev> sd;
-  sop_status st = read_sys_all(e, sd);
-  if (st) return st;
+  sop_status st = SOP_OK;
   std::vector<int32_t> redo;
   for (int32_t q = 0; q < n; ++q) {
     const int32_t s = slots[q];
     const SysHost &h = e->sys[s];
-    const SysDev &S = sd[s];
-    if (S.err & ~ERR_PL_OVF) continue;  // failed for another reason: reported as it is
-    const int32_t m = S.row_max, want = pl_cap_target(e, h.n, m);
-    const bool over = (S.err & ERR_PL_OVF) != 0;
+    const int32_t err = e->p.rep[s].x;
+    if (err & ~ERR_PL_OVF) continue;  // failed for another reason: reported as it is
+    const int32_t m = e->p.rep[s].y, want = pl_cap_target(e, h.n, m);
+    const bool over = (err & ERR_PL_OVF) != 0;
     if (!over && !pl_cap_short(e, h, m)) continue;
     if (want == h.pl_cap || want < m) continue;  // at the limit: an overflow stands
     st = engine_resize_rows(e, s, want, false);
@@ -805,6 +802,8 @@ sop_status engine_fit_new(sop_engine *e, const int32_t *slots, int32_t n) {
     redo.push_back(s);
   }
   if (redo.empty()) return SOP_OK;
+  std::vector<SysDev> sd;
+  if ((st = read_sys_all(e, sd))) return st;
   const int32_t zero = 0;
   for (int32_t s : redo) {
     HIPCK(hipMemcpy(&e->p.sys[s].err, &zero, sizeof(zero), hipMemcpyHostToDevice));
@@ -813,6 +812,7 @@ sop_status engine_fit_new(sop_engine *e, const int32_t *slots, int32_t n) {
   st = engine_set_batch(e, redo.data(), (int32_t)redo.size());
   if (st) return st;
   HIPCK(launch_lists(e->p, list_grids(e), 0, FORCE_NL | FORCE_PL, e->stream));
+  HIPCK(launch_report(e->p, e->stream));
   HIPCK(hipStreamSynchronize(e->stream));
   for (int32_t s : redo)
     HIPCK(hipMemcpy(e->p.sys[s].nbuild, sd[s].nbuild, sizeof(sd[s].nbuild), hipMemcpyHostToDevice));
@@ -828,13 +828,10 @@ sop_status engine_init_lists(sop_engine *e, const int32_t *slots, int32_t n, sop
   sop_status st = engine_set_batch(e, slots, n);
   if (st) return st;
   HIPCK(launch_lists(e->p, list_grids(e), 0, FORCE_NL | FORCE_PL, e->stream));
+  HIPCK(launch_report(e->p, e->stream));
   HIPCK(hipStreamSynchronize(e->stream));
   st = engine_fit_new(e, slots, n);
   if (st) return st;
-  st = engine_set_batch(e, slots, n);  // (engine_fit_new may have left a part of it)
-  if (st) return st;
-  HIPCK(launch_report(e->p, e->stream));
-  HIPCK(hipStreamSynchronize(e->stream));
   for (int32_t q = 0; q < n; ++q) {
     status[q] = engine_error_status(e, slots[q], e->p.rep[slots[q]].x);
     if (status[q]) engine_remove_system(e, slots[q]);

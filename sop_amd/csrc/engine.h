@@ -24,7 +24,8 @@ hipError_t launch_step(const DevPtrs &p, int mode, int lpb, const StepGrids &sg,
                        const StepFork *fk = nullptr);
 hipError_t step_lds_limit(size_t bytes);
 hipError_t filter_lds_init();
-hipError_t launch_energy(const DevPtrs &p, int grid_tiles, int grid_sys, hipStream_t st);
+hipError_t launch_energy(const DevPtrs &p, int grid_tiles, int grid_sys, double *out, hipStream_t st);
+hipError_t launch_add_system(const DevPtrs &p, const AddSystem &a, hipStream_t st);
 hipError_t launch_energy_one(const DevPtrs &p, int t0, int nt, int slot, int grid_tiles, double *out, hipStream_t st);
 hipError_t launch_tables(const TableParts &tp, hipStream_t st);
 hipError_t launch_report(const DevPtrs &p, hipStream_t st);
@@ -146,19 +147,22 @@ sop_status set_error(sop_engine *e, sop_status st, const std::string &msg);
 sop_status hip_check(sop_engine *e, hipError_t h, const char *what);
 sop_status engine_add_system(sop_engine *e, const sop_system_desc *d, int32_t *slot);
 // A stream for uploads beside the engine stream's work, and a pinned host
-// buffer every upload is staged through.
+// buffer every upload is staged through; used: bytes of it that uploads in
+// flight may still read.
 struct Upload {
   hipStream_t stream;
   void *stage;
   size_t stage_bytes;
+  size_t used;
 };
 // With `upl`, the system goes into free pool ranges and a free slot only
 // (SOP_ERR_BUSY, nothing changed, when it does not fit without growing a
-// pool, or its uploads do not fit the staging buffer) and is uploaded on
-// upl->stream, which the call drains before returning; work in flight on the
-// engine stream is not waited for and not touched.
+// pool, or its upload does not fit the staging buffer) and is uploaded on
+// upl->stream, which the caller drains (upload_drain) before the system is
+// used; work in flight on the engine stream is not waited for and not touched.
 sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, int64_t step_end, int32_t *slot,
-                                     const Upload *upl = nullptr);
+                                     Upload *upl = nullptr);
+sop_status upload_drain(sop_engine *e, Upload *upl);
 sop_status engine_init_lists(sop_engine *e, const int32_t *slots, int32_t n, sop_status *status);
 sop_status engine_remove_system(sop_engine *e, int32_t slot);
 sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots);

@@ -2644,8 +2644,8 @@ __global__ __launch_bounds__(ENERGY_THREADS) void k_energy(DevPtrs p, int t0, in
 
 // Per system, fixed-order sum of the tile partials plus Rg^2 from the centroid
 // form (1/N) sum |r|^2 - |r_cm|^2, identical to the reference's pair sum / N^2
-// (sop.cu:564-580).  slot >= 0: that system alone, its values also to out (when
-// not null); else the batch's systems.
+// (sop.cu:564-580).  slot >= 0: that system alone; else the batch's systems.
+// The values also to out (when not null), in batch order.
 __global__ __launch_bounds__(256) void k_sys_reduce(DevPtrs p, int slot, double *out) {
   __shared__ double sh[4][TPART_N];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -2683,7 +2683,7 @@ __global__ __launch_bounds__(256) void k_sys_reduce(DevPtrs p, int slot, double 
       double *d = p.sysout + (int64_t)(s - p.sysout_base) * SYSOUT_N;
       for (int k = 0; k < 12; ++k) {
         d[k] = o[k];
-        if (out) out[k] = o[k];
+        if (out) out[(slot >= 0 ? 0 : q) * SYSOUT_N + k] = o[k];
       }
     }
     __syncthreads();
@@ -2705,14 +2705,49 @@ __global__ __launch_bounds__(256) void k_tables(TableParts tp) {
   for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < tp.part[k].words; i += gridDim.x * 256) dst[i] = src[i];
 }
 
-// {error bits, longest row} of the batch's systems, for the host.
+// A system's state, for the host.
 __device__ __forceinline__ void report(const DevPtrs &p, int s, const SysDev &S) {
-  p.rep[s] = make_int2(S.err, S.row_max);
+  p.rep[s] = make_int4(S.err, S.row_max, S.step >= S.step_end ? 1 : 0, 0);
 }
 __global__ void k_report(DevPtrs p) {
   const int nsys = *p.nsys;
   for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < nsys; q += gridDim.x * blockDim.x)
     report(p, p.syslist[q], p.sys[p.syslist[q]]);
+}
+
+// A new system unpacked from its upload: every array of its ranges in one
+// launch (21 copies of host-made arrays, half of them zeros, took 300 us a
+// system, half a served job's admission).
+__global__ __launch_bounds__(256) void k_add_system(DevPtrs p, AddSystem a) {
+  const int id = blockIdx.x * 256 + threadIdx.x, stride = gridDim.x * 256;
+  const float *xyz = reinterpret_cast<const float *>(a.blob + a.xyz), *bond = reinterpret_cast<const float *>(a.blob + a.bond);
+  const float *vel = reinterpret_cast<const float *>(a.blob + a.vel);
+  const int *wb = reinterpret_cast<const int *>(a.blob + a.wbits), *ns = reinterpret_cast<const int *>(a.blob + a.nstart);
+  for (int k = id; k < a.bead_len; k += stride) {
+    const int i = a.bead_off + k;
+    const bool in = k < a.n;
+    const float4 x = in ? make_float4(xyz[3 * k], xyz[3 * k + 1], xyz[3 * k + 2], __int_as_float(wb[k]))
+                        : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    p.pos0[i] = x;
+    p.pos1[i] = x;
+    p.bond_r0[i] = in ? bond[k] : 0.0f;
+    p.nat_start[i] = a.nat_off + (in ? ns[k] : 0);
+    p.nat_cnt[i] = in ? ns[k + 1] - ns[k] : 0;
+    p.nlatt_cnt[i] = p.platt_cnt[i] = p.nlrep_cnt[i] = p.plrep_cnt[i] = p.plrep_off[i] = p.platt_off[i] = 0;
+    // underdamped state: the velocities entering the first step (w = 0)
+    p.vel[i] = in && a.has_vel ? make_float4(vel[3 * k], vel[3 * k + 1], vel[3 * k + 2], 0.0f)
+                               : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    p.tile_ord[i] = (uint8_t)(k % TILE);  // identity bead order until the first pair list orders it
+    if (k % TILE == 0) p.tile_sys[i / TILE] = a.slot;
+  }
+  const int *nj = reinterpret_cast<const int *>(a.blob + a.natj);
+  const float *nr = reinterpret_cast<const float *>(a.blob + a.natr);
+  for (int k = id; k < a.n_nat; k += stride) {
+    p.nat_j[a.nat_off + k] = a.bead_off + nj[k];
+    p.nat_r0[a.nat_off + k] = nr[k];
+  }
+  uint32_t *d = reinterpret_cast<uint32_t *>(p.sys + a.slot);
+  for (int k = id; k < (int)(sizeof(SysDev) / 4); k += stride) d[k] = a.blob[a.sys + k];
 }
 
 // Per-bead values of one system to the host buffer: the current coordinates or
@@ -3008,9 +3043,9 @@ hipError_t launch_relayout(const DevPtrs &p, int bo, int n, int idx16, int64_t o
   return SOPK_LAUNCH_CHECK();
 }
 
-hipError_t launch_energy(const DevPtrs &p, int grid_tiles, int grid_sys, hipStream_t st) {
+hipError_t launch_energy(const DevPtrs &p, int grid_tiles, int grid_sys, double *out, hipStream_t st) {
   hipLaunchKernelGGL(k_energy, dim3(std::min(grid_tiles, 512)), dim3(ENERGY_THREADS), 0, st, p, 0, 0);
-  hipLaunchKernelGGL(k_sys_reduce, dim3(grid_sys), dim3(256), 0, st, p, -1, nullptr);
+  hipLaunchKernelGGL(k_sys_reduce, dim3(grid_sys), dim3(256), 0, st, p, -1, out);
   return SOPK_LAUNCH_CHECK();
 }
 
@@ -3025,6 +3060,12 @@ hipError_t launch_tables(const TableParts &tp, hipStream_t st) {
   uint32_t most = 1;
   for (const TablePart &q : tp.part) most = std::max(most, q.words);
   hipLaunchKernelGGL(k_tables, dim3(std::min(64u, (most + 255) / 256), TABLE_PARTS), dim3(256), 0, st, tp);
+  return SOPK_LAUNCH_CHECK();
+}
+
+hipError_t launch_add_system(const DevPtrs &p, const AddSystem &a, hipStream_t st) {
+  const int m = std::max(a.bead_len, a.n_nat);
+  hipLaunchKernelGGL(k_add_system, dim3(std::max(1, std::min(1024, (m + 255) / 256))), dim3(256), 0, st, p, a);
   return SOPK_LAUNCH_CHECK();
 }
 

@@ -50,7 +50,7 @@ struct sop_engine::Serve {
   std::string fatal;
   sop_serve_stats stats{};
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  Upload up{nullptr, nullptr, 0};  // uploads of admitted jobs beside the block in flight
+  Upload up{nullptr, nullptr, 0, 0};  // uploads of admitted jobs beside the block in flight
 };
 
 namespace {
@@ -63,15 +63,13 @@ namespace {
 // error bits before the list launch, the admitted jobs' from theirs after it.
 sop_status retire_and_start(sop_engine *e, sop_engine::Serve *sv, const std::vector<sop_engine::Job *> &added,
                             const std::vector<int32_t> &added_slots) {
-  std::vector<SysDev> sd((size_t)e->cap.slots);
-  sop_status st = hip_check(e, hipMemcpy(sd.data(), e->p.sys, sizeof(SysDev) * sd.size(), hipMemcpyDeviceToHost),
-                            "retire");
+  // wait for the block: its last kernel reported every running job's state
+  sop_status st = hip_check(e, hipStreamSynchronize(e->stream), "retire");
   if (st) return st;
   std::vector<sop_engine::Job *> keep, fin;
   std::vector<int32_t> slots;
   for (sop_engine::Job *j : sv->running) {
-    const SysDev &S = sd[j->slot];
-    if (S.step >= S.step_end || S.err) {
+    if (e->p.rep[j->slot].z || e->p.rep[j->slot].x) {
       fin.push_back(j);
       slots.push_back(j->slot);
     } else {
@@ -82,24 +80,38 @@ sop_status retire_and_start(sop_engine *e, sop_engine::Serve *sv, const std::vec
   slots.insert(slots.end(), added_slots.begin(), added_slots.end());
   st = engine_set_batch(e, slots.data(), (int32_t)slots.size());
   if (st) return st;
-  std::vector<double> out(fin.size() * SYSOUT_N);
-  std::vector<std::vector<float4>> xs(fin.size());
+  // the finished jobs' error bits and the running ones' longest rows, before
+  // the lists below report again
+  std::vector<int32_t> fin_err, keep_rows;
+  for (sop_engine::Job *j : fin) fin_err.push_back(e->p.rep[j->slot].x);
+  for (sop_engine::Job *j : keep) keep_rows.push_back(e->p.rep[j->slot].y);
+  // energies (in batch order) and coordinates go to the pinned result buffer
+  std::unordered_map<int32_t, size_t> order;
+  for (size_t q = 0; q < e->h_syslist.size(); ++q) order[e->h_syslist[q]] = q;
+  std::vector<size_t> at(fin.size());
+  size_t bytes = (8 * SYSOUT_N * slots.size() + 255) / 256 * 256;
+  for (size_t q = 0; q < fin.size(); ++q) {
+    at[q] = bytes;
+    bytes += (12 * (size_t)e->sys[fin[q]->slot].n + 255) / 256 * 256;
+  }
   if (!fin.empty()) {
-    st = hip_check(e, launch_energy(e->p, grid_tiles(e), grid_sys(e), e->stream), "energy");
+    st = engine_io(e, e->io, bytes);
+    if (st) return st;
+    st = hip_check(e, launch_energy(e->p, grid_tiles(e), grid_sys(e), static_cast<double *>(e->io.ptr), e->stream),
+                   "energy");
     if (st) return st;
   }
+  const char *io = static_cast<const char *>(e->io.ptr);
   for (size_t q = 0; q < fin.size(); ++q) {
-    const SysDev &S = sd[fin[q]->slot];
-    st = hip_check(e, hipMemcpyAsync(&out[q * SYSOUT_N], e->p.sysout + (int64_t)fin[q]->slot * SYSOUT_N,
-                                     8 * SYSOUT_N, hipMemcpyDeviceToHost, e->stream), "energy copy");
-    if (st) return st;
-    xs[q].resize((size_t)S.n);
-    st = hip_check(e, hipMemcpyAsync(xs[q].data(), (S.parity & 1 ? e->p.pos1 : e->p.pos0) + S.bead_off,
-                                     16 * (size_t)S.n, hipMemcpyDeviceToHost, e->stream), "coords copy");
+    float *xyz = reinterpret_cast<float *>(static_cast<char *>(e->io.ptr) + at[q]);
+    const int32_t s = fin[q]->slot;
+    st = hip_check(e, launch_read(e->p, s, e->sys[s].n, READ_COORDS, xyz, nullptr, e->stream), "coords");
     if (st) return st;
   }
   if (!added.empty()) {
     st = hip_check(e, launch_lists(e->p, list_grids(e), 0, FORCE_NL | FORCE_PL, e->stream), "first lists");
+    if (st) return st;
+    st = hip_check(e, launch_report(e->p, e->stream), "report");
     if (st) return st;
   }
   st = hip_check(e, hipStreamSynchronize(e->stream), "retire sync");
@@ -122,9 +134,7 @@ sop_status retire_and_start(sop_engine *e, sop_engine::Serve *sv, const std::vec
     std::vector<int32_t> ks;
     for (sop_engine::Job *j : keep) ks.push_back(j->slot);
     std::vector<int64_t> grown;
-    std::vector<int32_t> longest;
-    for (int32_t s : ks) longest.push_back(sd[s].row_max);
-    st = engine_grow_rows(e, ks.data(), (int32_t)ks.size(), longest.data(), &grown);
+    st = engine_grow_rows(e, ks.data(), (int32_t)ks.size(), keep_rows.data(), &grown);
     if (st) return st;
     std::lock_guard<std::mutex> lk(sv->mu);
     for (size_t q = 0; q < keep.size(); ++q) {
@@ -132,25 +142,15 @@ sop_status retire_and_start(sop_engine *e, sop_engine::Serve *sv, const std::vec
       sv->used += grown[q];
     }
   }
-  std::vector<SysDev> sa;
-  if (!added.empty()) {
-    sa.resize((size_t)e->cap.slots);
-    st = hip_check(e, hipMemcpy(sa.data(), e->p.sys, sizeof(SysDev) * sa.size(), hipMemcpyDeviceToHost),
-                   "admitted status");
-    if (st) return st;
-  }
   const double now = sop_clock_seconds();
   for (size_t q = 0; q < fin.size(); ++q) {
     sop_engine::Job *j = fin[q];
-    const int32_t status = engine_error_status(e, j->slot, sd[j->slot].err);
+    const int32_t status = engine_error_status(e, j->slot, fin_err[q]);
+    const size_t row = order[j->slot];
     engine_remove_system(e, j->slot);
     std::lock_guard<std::mutex> lk(sv->mu);
-    for (size_t i = 0; i < xs[q].size(); ++i) {
-      j->xyz[3 * i] = xs[q][i].x;
-      j->xyz[3 * i + 1] = xs[q][i].y;
-      j->xyz[3 * i + 2] = xs[q][i].z;
-    }
-    for (int k = 0; k < SOP_E_COUNT; ++k) j->energies[k] = out[q * SYSOUT_N + k];
+    std::memcpy(j->xyz.data(), io + at[q], 4 * j->xyz.size());
+    std::memcpy(j->energies, io + 8 * SYSOUT_N * row, sizeof(j->energies));
     j->status = status;
     j->t_done = now;
     j->done = 1;
@@ -158,7 +158,7 @@ sop_status retire_and_start(sop_engine *e, sop_engine::Serve *sv, const std::vec
     sv->used -= j->bytes;
   }
   for (sop_engine::Job *j : added) {
-    const sop_status status = engine_error_status(e, j->slot, sa[j->slot].err);
+    const sop_status status = engine_error_status(e, j->slot, e->p.rep[j->slot].x);
     if (status != SOP_OK) engine_remove_system(e, j->slot);
     std::lock_guard<std::mutex> lk(sv->mu);
     j->t_admit = now;
@@ -182,7 +182,7 @@ sop_status retire_and_start(sop_engine *e, sop_engine::Serve *sv, const std::vec
 // the engine stream; a job that would need a pool to grow goes back to the
 // queue front with the ones behind it, *deferred counts them, and the caller
 // admits them once the engine is idle.
-void admit(sop_engine *e, sop_engine::Serve *sv, const Upload *up, std::vector<sop_engine::Job *> &added,
+void admit(sop_engine *e, sop_engine::Serve *sv, Upload *up, std::vector<sop_engine::Job *> &added,
            std::vector<int32_t> &added_slots, size_t *deferred) {
   std::vector<sop_engine::Job *> take;
   {
@@ -289,7 +289,11 @@ void serve_loop(sop_engine *e) {
     std::vector<sop_engine::Job *> added;
     std::vector<int32_t> added_slots;
     size_t deferred = 0;
-    if (st == SOP_OK) admit(e, sv, run && sv->up.stream ? &sv->up : nullptr, added, added_slots, &deferred);
+    if (st == SOP_OK) {
+      Upload *up = run && sv->up.stream ? &sv->up : nullptr;
+      admit(e, sv, up, added, added_slots, &deferred);
+      if (up && !added.empty()) st = upload_drain(e, up);  // before their first lists
+    }
     const size_t beside = run && sv->up.stream ? added.size() : 0;
     const double ta = sop_clock_seconds();
     // 3. retire finished jobs and start the admitted ones (waits for the block)

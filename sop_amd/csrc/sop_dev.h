@@ -150,7 +150,7 @@ struct DevPtrs {
   double *sysout;       // per system slot: SYSOUT_N reduced values
   int32_t *tile_sys;    // system slot of each tile
   uint8_t *tile_ord;    // per tile: TILE bead offsets in the order the step kernel's lane groups take them
-  int2 *rep;            // per system slot, in pinned host memory: {err, row_max} as of the last report
+  int4 *rep;            // per system slot, in pinned host memory: {err, row_max, steps done} as of the last report
   int32_t *work;        // tile ids to process (-1 = padding), XCD-interleaved
   int2 *tiles;          // tiles that step and filter with a block each: {tile, system slot}, tile -1 = padding
   int32_t *ntiles;
@@ -222,6 +222,14 @@ struct TablePart {
 struct TableParts {
   TablePart part[TABLE_PARTS];
   const uint32_t *stage;
+};
+
+// A new system's upload: its place, and the word offsets of its parts in the
+// pinned blob (nstart: n + 1 offsets into the natives; natj: local indices).
+struct AddSystem {
+  const uint32_t *blob;
+  uint32_t xyz, wbits, bond, nstart, natj, natr, vel, sys;
+  int32_t bead_off, bead_len, n, nat_off, n_nat, slot, has_vel;
 };
 
 // what launch_read copies out
