@@ -50,6 +50,7 @@ struct sop_engine::Serve {
   std::string fatal;
   sop_serve_stats stats{};
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  HostBuf io;                         // results of finished jobs (the loop's own: e->io is the driving thread's)
   Upload up{nullptr, nullptr, 0, 0};  // uploads of admitted jobs beside the block in flight
 };
 
@@ -95,15 +96,15 @@ sop_status retire_and_start(sop_engine *e, sop_engine::Serve *sv, const std::vec
     bytes += (12 * (size_t)e->sys[fin[q]->slot].n + 255) / 256 * 256;
   }
   if (!fin.empty()) {
-    st = engine_io(e, e->io, bytes);
+    st = engine_io(e, sv->io, bytes);
     if (st) return st;
-    st = hip_check(e, launch_energy(e->p, grid_tiles(e), grid_sys(e), static_cast<double *>(e->io.ptr), e->stream),
+    st = hip_check(e, launch_energy(e->p, grid_tiles(e), grid_sys(e), static_cast<double *>(sv->io.ptr), e->stream),
                    "energy");
     if (st) return st;
   }
-  const char *io = static_cast<const char *>(e->io.ptr);
+  const char *io = static_cast<const char *>(sv->io.ptr);
   for (size_t q = 0; q < fin.size(); ++q) {
-    float *xyz = reinterpret_cast<float *>(static_cast<char *>(e->io.ptr) + at[q]);
+    float *xyz = reinterpret_cast<float *>(static_cast<char *>(sv->io.ptr) + at[q]);
     const int32_t s = fin[q]->slot;
     st = hip_check(e, launch_read(e->p, s, e->sys[s].n, READ_COORDS, xyz, nullptr, e->stream), "coords");
     if (st) return st;
@@ -481,6 +482,7 @@ sop_status sop_serve_stop(sop_engine *e) {
   if (sv->ev1) (void)hipEventDestroy(sv->ev1);
   if (sv->up.stream) (void)hipStreamDestroy(sv->up.stream);
   if (sv->up.stage) (void)hipHostFree(sv->up.stage);
+  if (sv->io.ptr) (void)hipHostFree(sv->io.ptr);
   delete sv;
   e->serve = nullptr;
   e->fixed_grids = false;
