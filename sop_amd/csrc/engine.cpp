@@ -1678,70 +1678,32 @@ static sop_status materialize_nl(sop_engine *e, int32_t sys) {
 }
 
 sop_status sop_get_list(sop_engine *e, int32_t sys, int32_t which, int32_t *ij, int64_t cap, int64_t *n) {
+  static_assert(LIST_NL_ATT == SOP_LIST_NL_NATIVE && LIST_NL_REP == SOP_LIST_NL_REP &&
+                    LIST_PL_ATT == SOP_LIST_PL_NATIVE && LIST_PL_REP == SOP_LIST_PL_REP, "list ids");
   if (!valid_sys(e, sys) || !n) return set_error(e, SOP_ERR_INVALID, "bad arguments");
-  HIPCK(hipStreamSynchronize(e->stream));
+  if (which < LIST_NL_ATT || which > LIST_PL_REP) return set_error(e, SOP_ERR_INVALID, "unknown list");
+  sop_status st = SOP_OK;
   if (which == SOP_LIST_NL_NATIVE || which == SOP_LIST_NL_REP) {
-    sop_status st = materialize_nl(e, sys);
+    st = materialize_nl(e, sys);
     if (st) return st;
   }
-  const SysHost &h = e->sys[sys];
-  const int32_t nb = h.n;
-  std::vector<int32_t> cnt((size_t)nb);
-  std::vector<int32_t> ent;
-  std::vector<int32_t> start((size_t)nb);
-  int32_t *cnt_d = nullptr;
-  int64_t seg_len = 0;
-  if (which == SOP_LIST_NL_NATIVE || which == SOP_LIST_PL_NATIVE) {
-    cnt_d = which == SOP_LIST_NL_NATIVE ? e->p.nlatt_cnt : e->p.platt_cnt;
-    // the neighbor list's natives sit in each bead's native slots; the native
-    // pair list is packed per tile (platt_off)
-    HIPCK(hipMemcpy(start.data(), (which == SOP_LIST_NL_NATIVE ? e->p.nat_start : e->p.platt_off) + h.bead_off,
-                    4 * (size_t)nb, hipMemcpyDeviceToHost));
-    ent.resize((size_t)h.nat_len);
-    if (which == SOP_LIST_NL_NATIVE) {
-      HIPCK(hipMemcpy(ent.data(), e->p.nlatt_j + h.nat_off, 4 * (size_t)h.nat_len, hipMemcpyDeviceToHost));
-    } else {
-      std::vector<int2> pe((size_t)h.nat_len);
-      HIPCK(hipMemcpy(pe.data(), e->p.platt + h.nat_off, 8 * (size_t)h.nat_len, hipMemcpyDeviceToHost));
-      for (size_t k = 0; k < pe.size(); ++k) ent[k] = pe[k].x;
-    }
-    for (int i = 0; i < nb; ++i) start[i] -= (int32_t)h.nat_off;
-  } else if (which == SOP_LIST_NL_REP || which == SOP_LIST_PL_REP) {
-    const bool nl = which == SOP_LIST_NL_REP;
-    cnt_d = nl ? e->p.nlrep_cnt : e->p.plrep_cnt;
-    seg_len = nl ? h.nl_len : (int64_t)h.n * h.pl_cap;  // entries
-    ent.resize((size_t)seg_len);
-    if (!nl && h.n <= 65536) {
-      // 16-bit local indices from the segment start
-      std::vector<uint16_t> e16((size_t)seg_len);
-      HIPCK(hipMemcpy(e16.data(), e->p.plrep_j + h.pl_off, 2 * (size_t)seg_len, hipMemcpyDeviceToHost));
-      for (int64_t q = 0; q < seg_len; ++q) ent[(size_t)q] = (int32_t)h.bead_off + e16[(size_t)q];
-    } else {
-      HIPCK(hipMemcpy(ent.data(), (nl ? e->p.nlrep_j + h.nl_off : e->p.plrep_j + h.pl_off), 4 * (size_t)seg_len,
-                      hipMemcpyDeviceToHost));
-    }
-    if (nl) {
-      for (int i = 0; i < nb; ++i) start[i] = i * h.nl_cap;
-    } else {  // pair-list rows are packed per tile: each bead's row start is stored
-      HIPCK(hipMemcpy(start.data(), e->p.plrep_off + h.bead_off, 4 * (size_t)nb, hipMemcpyDeviceToHost));
-    }
-  } else {
-    return set_error(e, SOP_ERR_INVALID, "unknown list");
+  const int32_t nb = e->sys[sys].n;
+  if ((st = engine_io(e, e->io, 64))) return st;
+  HIPCK(launch_list_places(e->p, sys, nb, which, 0, static_cast<int64_t *>(e->io.ptr), e->stream));
+  HIPCK(hipStreamSynchronize(e->stream));
+  const int64_t total = *static_cast<const int64_t *>(e->io.ptr);
+  *n = total;
+  const int64_t want = ij ? std::min(total, cap) : 0;
+  constexpr int64_t WINDOW = (int64_t)4 << 20;  // pairs through the host buffer at a time
+  if (want > 0 && (st = engine_io(e, e->io, 8 * (size_t)(std::min(want, WINDOW) + 1)))) return st;
+  for (int64_t lo = 0; lo < want; lo += WINDOW) {
+    const int64_t m = std::min(WINDOW, want - lo);
+    if (lo)  // (the total again, behind the window)
+      HIPCK(launch_list_places(e->p, sys, nb, which, lo, static_cast<int64_t *>(e->io.ptr) + WINDOW, e->stream));
+    HIPCK(launch_list_write(e->p, sys, nb, which, static_cast<int2 *>(e->io.ptr), (int)m, e->stream));
+    HIPCK(hipStreamSynchronize(e->stream));
+    std::memcpy(ij + 2 * lo, e->io.ptr, 8 * (size_t)m);
   }
-  HIPCK(hipMemcpy(cnt.data(), cnt_d + h.bead_off, 4 * (size_t)nb, hipMemcpyDeviceToHost));
-  int64_t m = 0;
-  for (int i = 0; i < nb; ++i)
-    for (int k = 0; k < cnt[i]; ++k) {
-      const int32_t j = ent[(size_t)start[i] + k] - (int32_t)h.bead_off;
-      if (j > i) {
-        if (ij && m < cap) {
-          ij[2 * m] = i;
-          ij[2 * m + 1] = j;
-        }
-        ++m;
-      }
-    }
-  *n = m;
   return SOP_OK;
 }
 

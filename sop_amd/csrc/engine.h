@@ -30,6 +30,8 @@ hipError_t launch_energy_one(const DevPtrs &p, int t0, int nt, int slot, int gri
 hipError_t launch_tables(const TableParts &tp, hipStream_t st);
 hipError_t launch_report(const DevPtrs &p, hipStream_t st);
 hipError_t launch_read(const DevPtrs &p, int slot, int n, int what, float *out, int64_t *step, hipStream_t st);
+hipError_t launch_list_places(const DevPtrs &p, int slot, int n, int which, int64_t lo, int64_t *total, hipStream_t st);
+hipError_t launch_list_write(const DevPtrs &p, int slot, int n, int which, int2 *out, int m, hipStream_t st);
 hipError_t launch_write_coords(const DevPtrs &p, int slot, int n, const float *in, hipStream_t st);
 hipError_t launch_advance(const DevPtrs &p, int nsteps, hipStream_t st);
 hipError_t launch_relayout(const DevPtrs &p, int bo, int n, int idx16, int64_t old_base, int old_cap,

@@ -232,6 +232,9 @@ struct AddSystem {
   int32_t bead_off, bead_len, n, nat_off, n_nat, slot, has_vel;
 };
 
+// the lists of launch_list_places / launch_list_write (the SOP_LIST_* values)
+constexpr int LIST_NL_ATT = 0, LIST_NL_REP = 1, LIST_PL_ATT = 2, LIST_PL_REP = 3;
+
 // what launch_read copies out
 constexpr int READ_COORDS = 0, READ_FORCES = 1, READ_VEL = 2;
 
