@@ -954,8 +954,9 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   // for any LDS tier up to TILE_STEP_FAR_PER_CU.  Step times by tile against
   // the other kernel (us): 2 x 8,000 beads 8.2 / 13.8 whole-CU, 6 x 8,000
   // 17.9 / 14.4; 32 x 4,000 and 4 x 8,000 together 34.8 / 40.8; 12 x 4,000
-  // 14.0 / 12.9 LDS; 20,000 beads 12.7 / 33.7 global-gather items, 60,000
-  // 24.6 / 36.3, 100,000 56.5 / 42.0.
+  // 14.0 / 12.9 LDS; against global-gather items, step and run per step:
+  // 20,000 beads 12.7 and 18.6 / 17.8 and 29.2, 45,000 19.2 and 29.1 / 18.8 and
+  // 31.8, 65,000 27.0 and 39.8 / 20.0 and 34.5.
   const int64_t tile_cap = (int64_t)TILE_STEP_PER_CU * e->num_cu;
   int64_t mid_tiles = 0, far_tiles = 0;
   for (int32_t q = 0; q < nslots; ++q) {
@@ -990,10 +991,17 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     int32_t n_lds = 0, n_big = 0, n_far = 0;
     size_t lds = 0, lds_big = 0;
   };
-  // tiles per item of a system: its size bucket's tuned value, else per_step
-  auto per_of = [&](const SysHost &h) {
+  // tiles per item of the global-gather systems: one item per compute unit, of
+  // 4 to 16 tiles (a wave's share of a tile repeats the tile's chain terms and
+  // noise, and a second item on some of the units lasts as long as on all).
+  // Step times for chains of 500 beads by items of 4 / 8 / 16 tiles (us):
+  // 200,000 beads 53.6 / 42.8 / 36.2, by this rule (13) 34.2; 100,000 beads
+  // 26.9 / 21.8 / 34.0, by this rule (7) 21.2
+  const int32_t per_far = (int32_t)std::clamp<int64_t>((far_tiles + e->num_cu - 1) / e->num_cu, 4, STEP_WAVES);
+  // tiles per item of a system: its size bucket's tuned value, else the rule's
+  auto per_of = [&](const SysHost &h, int32_t otherwise) {
     const int b = engine_bucket(e, h.n);
-    return b >= 0 && e->tune.tiles[b] > 0 ? e->tune.tiles[b] : per_step;
+    return b >= 0 && e->tune.tiles[b] > 0 ? e->tune.tiles[b] : otherwise;
   };
   auto plan = [&](int32_t per_fixed, bool split, Plan &out) {
     // waves per tile of an item of nt tiles
@@ -1018,7 +1026,7 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
       const SysHost &h = e->sys[sl];
       if (tile_step(h)) continue;
       const int32_t t0 = (int32_t)(h.bead_off / TILE), nt = (int32_t)(h.bead_len / TILE);
-      const int32_t per = per_fixed > 0 ? per_fixed : per_of(h);
+      const int32_t per = per_fixed > 0 ? per_fixed : per_of(h, per_step);
       if (h.bead_len <= lds_cap) {
         out.lds = std::max(out.lds, (size_t)h.bead_len * 16);
         if (nt > per) {
@@ -1045,7 +1053,8 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
       } else {
         flush();
         std::vector<int4> v;
-        for (int32_t k = 0; k < nt; k += per) v.push_back(mk(t0 + k, std::min(per, nt - k), -1, 0));
+        const int32_t pf = own_items ? per : (split ? per_of(h, per_far) : per_far);
+        for (int32_t k = 0; k < nt; k += pf) v.push_back(mk(t0 + k, std::min(pf, nt - k), -1, 0));
         far_items.push_back(v);
       }
     }
@@ -1113,11 +1122,15 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     std::sort(far_items.begin(), far_items.end(), [](const std::vector<int4> &u, const std::vector<int4> &v) {
       return u.size() != v.size() ? u.size() > v.size() : u[0].x < v[0].x;
     });
-    // a system with more items than one XCD's share of the global-gather
-    // launch (2 blocks per compute unit) goes out in contiguous runs of that
-    // share, each run to the least-loaded XCD: one XCD would leave the rest of
-    // the device idle, and so large a system outgrows one L2 anyway
-    const size_t share = (size_t)std::max(1, 2 * e->num_cu / NX);
+    // a system with more items than an XCD's share of them all (at most its
+    // share of the launch's two blocks per compute unit) goes out in contiguous
+    // runs of that share, each run to the least-loaded XCD: so large a system
+    // outgrows one L2 anyway.  (Runs of the launch's share alone: 391 items
+    // filled six XCDs and left one nearly idle and one idle; the shell filter's
+    // 196 filled three and took 124 us instead of 67.)
+    size_t n_far = 0;
+    for (const auto &v : far_items) n_far += v.size();
+    const size_t share = std::max<size_t>(1, std::min<size_t>(2 * e->num_cu / NX, (n_far + NX - 1) / NX));
     for (const auto &v : far_items) {
       for (size_t k0 = 0; k0 < v.size(); k0 += share) {
         const int x = (int)(std::min_element(fload.begin(), fload.end()) - fload.begin());

@@ -183,7 +183,7 @@ constexpr int STEP_THREADS = 64 * STEP_WAVES;
 // tile (k_step_tile), whatever their systems' sizes.
 constexpr int TILE_STEP_PER_CU = 2;
 // The tiles of systems that gather from global memory do so up to this many.
-constexpr int TILE_STEP_FAR_PER_CU = 4;
+constexpr int TILE_STEP_FAR_PER_CU = 3;
 
 // Grids of the step's launches: items staged in LDS at two blocks per compute
 // unit, items staged in a whole compute unit's LDS, items that gather from

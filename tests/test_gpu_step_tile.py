@@ -69,6 +69,16 @@ def test_tile_step_equals_item_step(systems, steps, lanes):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("sizes", [(49152,), (49153,), (66000,), (30000, 12000, 11000), (1000, 60000, 3000)])
+def test_global_gather_items_by_count(sizes):
+    """Items of the systems too large to stage, on either side of the last batch
+    with a block per tile, against items of 16 tiles: 16- and 32-bit rows,
+    several systems, and beside systems that are staged."""
+    made = [chain(60 + k, n, 1, False, False) for k, n in enumerate(sizes)]
+    for a, b in zip(outputs(made, 12), outputs(made, 12, step_tiles=16)):
+        assert np.array_equal(a, b)
+
+
 def test_dense_rows_and_many_natives():
     """Rows of several hundred partners and up to 40 natives a bead."""
     n = 1400
