@@ -79,6 +79,23 @@ def test_global_gather_items_by_count(sizes):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("n,types,lanes", [(300, 1, 4), (1500, 2, 4), (700, 1, 8), (6000, 1, 4), (12000, 2, 4)])
+def test_beads_on_one_another(n, types, lanes):
+    """Pairs below the repulsion's guard, in the middle of rows and at their ends:
+    the item kernels' loops meet them without the guard first."""
+    s = chain(200 + n, n, types)
+    rng = np.random.default_rng(n)
+    on = rng.choice(np.arange(0, n - 4, 4), 40, replace=False)
+    for a, b in zip(on[:20], on[20:]):
+        s.xyz[a] = s.xyz[b]
+    s.bond_r0[:-1] = np.linalg.norm(s.xyz[1:].astype(np.float64) - s.xyz[:-1], axis=1)  # bonds at rest
+    f = []
+    for tiles in (0, 16):
+        with S.Engine(0, step_tiles=tiles, lanes_per_bead=lanes) as e:
+            f.append(e.force_eval(e.add(s)))
+    assert np.array_equal(*f) and np.all(np.isfinite(f[0]))
+
+
 def test_dense_rows_and_many_natives():
     """Rows of several hundred partners and up to 40 natives a bead."""
     n = 1400
