@@ -1800,6 +1800,12 @@ __device__ __forceinline__ int tile_order(const DevPtrs &p, int t, int build, bo
 // known; the entries past FILTER_SROW, and every entry without staging, come
 // from a second pass over the round's rows, which repeats the first's
 // compaction order.  Rows are padded to ROW_PAD entries for the step kernel.
+// Bound by latency and memory together: a staging block has a compute unit to
+// itself (three waves per SIMD at work on average), reads 0.3 GB of shell rows
+// and natives and writes 0.2 GB of lists for 512 replicas, with the vector ALUs
+// at half and LDS at 43 %.  Addresses by one multiply-add an entry, the row's
+// end tested only in chunks that reach it, and one word of keep bits per chunk
+// took it from 229 to 209 us.
 template <bool LDS, bool IDX16, bool STAGE, bool ONE>
 __device__ __forceinline__ void filter_tile(const DevPtrs &p, const SysDev &S, int s, int t,
                                             const float4 *__restrict__ pin, const float4 *s_pos, int lds0,
@@ -1807,7 +1813,7 @@ __device__ __forceinline__ void filter_tile(const DevPtrs &p, const SysDev &S, i
   using ent_t = typename std::conditional<IDX16, uint16_t, uint32_t>::type;
   using chunk_t = typename std::conditional<IDX16, uint2, uint4>::type;
   const int lane = threadIdx.x & 63, g = lane >> 2, l = lane & 3;
-  const uint32_t below = (1u << l) - 1u;
+  const uint32_t lb = 1u << l, below = lb - 1u;
   // system constants in registers: the stores below may alias SysDev as far
   // as the compiler knows, and a reload would wait for every earlier store
   const int bo = S.bead_off, pl_cap = S.pl_cap;
@@ -1826,6 +1832,8 @@ __device__ __forceinline__ void filter_tile(const DevPtrs &p, const SysDev &S, i
   const double plf = S.pl_factor;
   const float pla = S.pl_abs;
   ent_t *const seg = reinterpret_cast<ent_t *>(p.plrep_j + pl_base);
+  const PosAt<LDS> pos(pin, s_pos, lds0);
+  const uint32_t row0 = pos.at0 + 16u * (uint32_t)bo;  // of row index 0
   // this tile's region of the segment, and the rows packed so far; the same
   // for the native pair list, whose region is the tile's native CSR range
   const int region = (t * TILE - bo) * pl_cap;
@@ -1860,10 +1868,7 @@ __device__ __forceinline__ void filter_tile(const DevPtrs &p, const SysDev &S, i
     const bool t2 = (__float_as_int(xi.w) & 3) == 2;
     // the cutoffs by the partner's type (one-type systems: the one of their type)
     const float rcA = ONE ? (t2 ? rc22 : rc11) : (t2 ? rc21 : rc11), rcB = t2 ? rc22 : rc12;
-    // entry value of the bead itself, and entry value -> staged position (LDS)
-    // or arena index
-    const int vself = IDX16 ? self - bo : self;
-    const int vpos = LDS ? (IDX16 ? bo - lds0 : -lds0) : (IDX16 ? bo : 0);
+    const uint32_t self_off = pos.at0 + 16u * (uint32_t)self;
     const chunk_t *src = reinterpret_cast<const chunk_t *>(
         reinterpret_cast<const ent_t *>(p.slrep_j + pl_base) + (int64_t)(self - bo) * pl_cap);
     ent_t *s_row = STAGE ? reinterpret_cast<ent_t *>(s_stage) + g * FILTER_SROW : nullptr;  // this group's staged row
@@ -1877,6 +1882,58 @@ __device__ __forceinline__ void filter_tile(const DevPtrs &p, const SysDev &S, i
       const int nch = (m + 3) >> 2;
       const int clast = max(nch - 1, 0);
       int cnt = 0;
+      // one chunk of each lane; full: no lane's is past its row's end.  Staged
+      // positions: the keep bits of a group's four lanes, position-major as
+      // the row's order, meet in one word, and entry (e, l) goes behind the
+      // bits below 4 e + l; gathered ones are decided as each arrives (waiting
+      // for all four cost 2 us of 67 for 200,000 beads).
+      auto chunk = [&](const chunk_t &ch, int c, auto full) {
+        ent_t v[4];
+        uint32_t off[4];
+        if constexpr (IDX16) {
+          v[0] = (ent_t)ch.x; v[1] = (ent_t)(ch.x >> 16); v[2] = (ent_t)ch.y; v[3] = (ent_t)(ch.y >> 16);
+          off[0] = mad16<false>(ch.x, row0); off[1] = mad16<true>(ch.x, row0);
+          off[2] = mad16<false>(ch.y, row0); off[3] = mad16<true>(ch.y, row0);
+        } else {
+          v[0] = ch.x; v[1] = ch.y; v[2] = ch.z; v[3] = ch.w;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) off[e] = pos.at0 + 16u * v[e];
+        }
+        float4 xj[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          // (an entry past the row's end reads the bead itself)
+          if constexpr (!full) off[e] = 4 * c + e < m ? off[e] : self_off;
+          xj[e] = pos.template get<ONE>(off[e]);
+        }
+        bool keep[4];
+        uint32_t bits = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          // the reference's predicate without the minimum image, which is the
+          // identity here (a grid build whose extent reaches boxl/2 - margin
+          // raises ERR_PBC, and beads move less than the margin before the next)
+          const float dx = xj[e].x - xi.x, dy = xj[e].y - xi.y, dz = xj[e].z - xi.z;
+          const float rc = ONE ? rcA : (w_type(xj[e].w) == 2 ? rcB : rcA);
+          keep[e] = ((dx * dx + dy * dy) + dz * dz) < rc;
+          if (nlb) keep[e] = true;
+          if constexpr (!full) keep[e] = keep[e] & (4 * c + e < m);
+          if constexpr (LDS) {
+            bits |= keep[e] ? lb << (4 * e) : 0u;
+          } else {
+            const uint32_t eb = (uint32_t)(__builtin_amdgcn_ballot_w64(keep[e]) >> (4 * g)) & 0xFu;
+            if (keep[e]) put(cnt + __popc(eb & below), v[e]);
+            cnt += __popc(eb);
+          }
+        }
+        if constexpr (!LDS) return;
+        bits |= (uint32_t)__builtin_amdgcn_mov_dpp((int)bits, 0xB1, 0xF, 0xF, true);
+        bits |= (uint32_t)__builtin_amdgcn_mov_dpp((int)bits, 0x4E, 0xF, 0xF, true);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (keep[e]) put(cnt + __popc(bits & ((lb << (4 * e)) - 1u)), v[e]);
+        cnt += __popc(bits);
+      };
       for (int m0 = 0; __ballot(l + 4 * m0 < nch) != 0; m0 += CB) {
         chunk_t ch[CB];
 #pragma unroll
@@ -1885,35 +1942,8 @@ __device__ __forceinline__ void filter_tile(const DevPtrs &p, const SysDev &S, i
         for (int b = 0; b < CB; ++b) {
           const int c = l + 4 * (m0 + b);
           if (__ballot(c < nch) == 0) break;
-          // entry values as stored (16-bit local or 32-bit arena indices);
-          // an entry past the row's end reads the bead itself
-          int v[4];
-          if constexpr (IDX16) {
-            v[0] = (int)(ch[b].x & 0xFFFFu); v[1] = (int)(ch[b].x >> 16);
-            v[2] = (int)(ch[b].y & 0xFFFFu); v[3] = (int)(ch[b].y >> 16);
-          } else {
-            v[0] = (int)ch[b].x; v[1] = (int)ch[b].y; v[2] = (int)ch[b].z; v[3] = (int)ch[b].w;
-          }
-          bool ok[4];
-          float4 xj[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            ok[e] = 4 * c + e < m;
-            const int q = (ok[e] ? v[e] : vself) + vpos;
-            xj[e] = LDS ? s_pos[q] : pin[q];
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            // the reference's predicate without the minimum image, which is the
-            // identity here (a grid build whose extent reaches boxl/2 - margin
-            // raises ERR_PBC, and beads move less than the margin before the next)
-            const float dx = xj[e].x - xi.x, dy = xj[e].y - xi.y, dz = xj[e].z - xi.z;
-            const float rc = ONE ? rcA : (w_type(xj[e].w) == 2 ? rcB : rcA);
-            const bool keep = ok[e] & (nlb | (((dx * dx + dy * dy) + dz * dz) < rc));
-            const uint32_t bits = (uint32_t)(__builtin_amdgcn_ballot_w64(keep) >> (4 * g)) & 0xFu;
-            if (keep) put(cnt + __popc(bits & below), v[e]);
-            cnt += __popc(bits);
-          }
+          if (LDS && __ballot(4 * c + 4 > m) == 0) chunk(ch[b], c, std::true_type());
+          else chunk(ch[b], c, std::false_type());
         }
       }
       return cnt;
@@ -1921,11 +1951,11 @@ __device__ __forceinline__ void filter_tile(const DevPtrs &p, const SysDev &S, i
     const int mrow = act ? nr : 0;
     int cnt;
     if constexpr (STAGE) {
-      cnt = pass(mrow, [&](int o, int v) {
-        if (o < FILTER_SROW) s_row[o] = (ent_t)v;
+      cnt = pass(mrow, [&](int o, ent_t v) {
+        if (o < FILTER_SROW) s_row[o] = v;
       });
     } else {
-      cnt = pass(mrow, [](int, int) {});
+      cnt = pass(mrow, [](int, ent_t) {});
     }
     // native pair list: natives within their pair cutoff, in native order,
     // packed per tile like the rows (platt_off): the keep decisions first,
@@ -2030,8 +2060,8 @@ __device__ __forceinline__ void filter_tile(const DevPtrs &p, const SysDev &S, i
     // the entries not staged: a second pass over the rows that have them
     const int lo = STAGE ? FILTER_SROW : 0;
     if (__ballot(c > lo) != 0) {
-      pass(c > lo ? mrow : 0, [&](int o, int v) {
-        if (o >= lo && o < c) dst[o] = (ent_t)v;
+      pass(c > lo ? mrow : 0, [&](int o, ent_t v) {
+        if (o >= lo && o < c) dst[o] = v;
       });
     }
   }
@@ -2090,16 +2120,17 @@ __global__ __launch_bounds__(STEP_THREADS) void k_shell_filter(DevPtrs p, int ks
     const bool st32 = stage_off >= 0 && stage_bytes >= 2 * FILTER_STAGE_BYTES;
     // one-type systems: every partner has the bead's type (one cutoff)
     const bool one = S.type_mask != 3;
-    if (S.idx16) {
+    if (KLDS || S.idx16) {  // (staged systems have 16-bit rows)
       if (st16) {
         if (one) filter_tile<KLDS, true, true, true>(p, S, s, t, pin, s_pos, lds0, wst);
         else filter_tile<KLDS, true, true, false>(p, S, s, t, pin, s_pos, lds0, wst);
       } else {
         filter_tile<KLDS, true, false, false>(p, S, s, t, pin, s_pos, lds0, nullptr);
       }
-    } else {
-      if (st32) filter_tile<KLDS, false, true, false>(p, S, s, t, pin, s_pos, lds0, wst);
-      else filter_tile<KLDS, false, false, false>(p, S, s, t, pin, s_pos, lds0, nullptr);
+    } else if constexpr (!KLDS) {
+      if (!st32) filter_tile<false, false, false, false>(p, S, s, t, pin, s_pos, lds0, nullptr);
+      else if (one) filter_tile<false, false, true, true>(p, S, s, t, pin, s_pos, lds0, wst);
+      else filter_tile<false, false, true, false>(p, S, s, t, pin, s_pos, lds0, wst);
     }
   }
 }
