@@ -123,10 +123,13 @@ static int items_grid(int g, bool fixed, int count) {
 // are resident per unit and the dispatcher starts each on whichever unit
 // frees first; A/B on one box, 512 replicas: 6.61e9 -> 6.90e9 bead-steps/s
 // against two per unit) and two while serving (fixed grids).
-int default_step_blocks(const sop_engine *e) { return (e->fixed_grids ? 2 : 4) * e->num_cu; }
+// (A mixed launch four in either: its items may be more than are resident, and
+// a block that took two would double the step.)
+int default_step_blocks(const sop_engine *e) { return (e->fixed_grids && !e->cur_mixed ? 2 : 4) * e->num_cu; }
 
 int grid_items(const sop_engine *e) {
-  return items_grid(e->step_blocks > 0 ? e->step_blocks : default_step_blocks(e), e->fixed_grids, e->cur_nitems);
+  return items_grid(e->step_blocks > 0 ? e->step_blocks : default_step_blocks(e), e->fixed_grids,
+                    e->cur_nitems + (e->cur_mixed ? e->cur_nitems_far : 0));
 }
 
 // A block per tile; while serving a fixed grid whenever the batch has such
@@ -143,7 +146,8 @@ static int items_grid_big(const sop_engine *e, int count) { return items_grid(e-
 int grid_items_big(const sop_engine *e) { return items_grid_big(e, e->cur_nitems_big); }
 
 StepGrids step_grids(const sop_engine *e) {
-  return StepGrids{grid_items(e), grid_items_big(e), grid_items_far(e), e->cur_lds, e->cur_lds_big, grid_step_tiles(e)};
+  if (e->cur_mixed) return StepGrids{grid_items(e), 0, 0, e->cur_lds, 0, 0, true};
+  return StepGrids{grid_items(e), grid_items_big(e), grid_items_far(e), e->cur_lds, e->cur_lds_big, grid_step_tiles(e), false};
 }
 
 // The shell filter's LDS launch: one block per item (a block leaves its
@@ -153,7 +157,7 @@ StepGrids filter_grids(const sop_engine *e) {
   const int g = e->step_blocks > 0 ? e->step_blocks : default_step_blocks(e);
   return StepGrids{items_grid(e->fixed_grids ? g : std::max(g, 8 * e->num_cu), e->fixed_grids, e->cur_nfitems),
                    items_grid_big(e, e->cur_nfitems_big),
-                   items_grid(2 * e->num_cu, e->fixed_grids, e->cur_nfitems_far), e->cur_flds, e->cur_flds_big, grid_step_tiles(e)};
+                   items_grid(2 * e->num_cu, e->fixed_grids, e->cur_nfitems_far), e->cur_flds, e->cur_flds_big, grid_step_tiles(e), false};
 }
 
 ListGrids list_grids(const sop_engine *e) {
@@ -967,10 +971,14 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   const bool by_tile = total_tiles <= tile_cap && !own_items;
   const bool mid_by_tile = mid_tiles + far_tiles <= tile_cap && !own_items;
   const bool far_by_tile = far_tiles <= (int64_t)TILE_STEP_FAR_PER_CU * e->num_cu && !own_items;
-  auto tile_step = [&](const SysHost &h) {
+  auto tile_filter = [&](const SysHost &h) {
     if (h.n > 65536) return false;  // 16-bit rows only
     return by_tile || (h.bead_len > lds_cap && (mid_by_tile || (far_by_tile && h.bead_len > big_cap)));
   };
+  // a batch of LDS and global-gather systems alone steps in one launch of
+  // items of both (k_step_mixed)
+  e->cur_mixed = !by_tile && mid_tiles == 0 && far_tiles > 0 && far_tiles < total_tiles;
+  auto tile_step = [&](const SysHost &h) { return !e->cur_mixed && tile_filter(h); };
   std::vector<int2> tiles;
   {
     // each XCD (tile k of the table runs on XCD k mod 8) a run of consecutive
@@ -978,7 +986,7 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     std::vector<int2> all;
     for (int32_t sl : by_arena) {
       const SysHost &h = e->sys[sl];
-      if (!tile_step(h)) continue;
+      if (!tile_filter(h)) continue;
       for (int64_t t = h.bead_off / TILE; t < (h.bead_off + h.bead_len) / TILE; ++t)
         all.push_back(make_int2((int32_t)t, sl));
     }
@@ -998,6 +1006,14 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   // 200,000 beads 53.6 / 42.8 / 36.2, by this rule (13) 34.2; 100,000 beads
   // 26.9 / 21.8 / 34.0, by this rule (7) 21.2
   const int32_t per_far = (int32_t)std::clamp<int64_t>((far_tiles + e->num_cu - 1) / e->num_cu, 4, STEP_WAVES);
+  // in a mixed launch the fewest of 4, 8 or 16 tiles with which all items are
+  // resident at once, two per unit (the batch's item size instead: 60 systems
+  // of 1,500 beads and 3 of 18,000 60.8 us per step against 49.4, 120 and 8
+  // 105 against 96)
+  int32_t per_mixed = 4;
+  while (per_mixed < STEP_WAVES &&
+         (total_tiles - far_tiles) / per_step + far_tiles / per_mixed > 2 * (int64_t)e->num_cu)
+    per_mixed *= 2;
   // tiles per item of a system: its size bucket's tuned value, else the rule's
   auto per_of = [&](const SysHost &h, int32_t otherwise) {
     const int b = engine_bucket(e, h.n);
@@ -1024,7 +1040,7 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     };
     for (int32_t sl : by_arena) {
       const SysHost &h = e->sys[sl];
-      if (tile_step(h)) continue;
+      if (split ? tile_step(h) : tile_filter(h)) continue;
       const int32_t t0 = (int32_t)(h.bead_off / TILE), nt = (int32_t)(h.bead_len / TILE);
       const int32_t per = per_fixed > 0 ? per_fixed : per_of(h, per_step);
       if (h.bead_len <= lds_cap) {
@@ -1053,7 +1069,7 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
       } else {
         flush();
         std::vector<int4> v;
-        const int32_t pf = own_items ? per : (split ? per_of(h, per_far) : per_far);
+        const int32_t pf = own_items ? per : !split ? per_far : per_of(h, e->cur_mixed ? per_mixed : per_far);
         for (int32_t k = 0; k < nt; k += pf) v.push_back(mk(t0 + k, std::min(pf, nt - k), -1, 0));
         far_items.push_back(v);
       }
@@ -1308,7 +1324,7 @@ static std::string graph_key(const sop_engine *e, int G, int n_nl, int n_pl) {
      << grid_rebuild(e) << '|' << grid_big_beads(e) << '|' << grid_big_sys(e) << '|' << grid_items(e) << '|' << grid_items_big(e) << '|'
      << e->cur_lds << '|' << e->cur_lds_big;
   const StepGrids fg = filter_grids(e);
-  os << '|' << step_grids(e).tiles << '|' << grid_items_far(e) << '|' << list_grids(e).split << '|' << fg.grid << '|' << fg.grid_big << '|' << fg.grid_far << '|' << fg.lds << '|' << fg.lds_big;
+  os << '|' << e->cur_mixed << '|' << grid_step_tiles(e) << '|' << grid_items_far(e) << '|' << list_grids(e).split << '|' << fg.grid << '|' << fg.grid_big << '|' << fg.grid_far << '|' << fg.lds << '|' << fg.lds_big;
   return os.str();
 }
 

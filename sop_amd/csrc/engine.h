@@ -111,7 +111,8 @@ struct sop_engine {
   int32_t cur_nbig = 0, cur_big_max = 0;  // systems of more than SORT_N_MAX beads, and the largest one's beads
   int32_t cur_nwork = 0, cur_nsys = 0, cur_nitems = 0, cur_nitems_big = 0, cur_nitems_far = 0;
   int32_t cur_nfitems = 0, cur_nfitems_big = 0, cur_nfitems_far = 0;  // shell-filter items
-  int32_t cur_ntiles = 0; // tiles that step with a block each
+  int32_t cur_ntiles = 0; // tiles with a block each in the shell filter, and in the step unless cur_mixed
+  bool cur_mixed = false; // the step takes LDS and global-gather items in one launch
   int64_t tiles_cap = 0;
   size_t cur_lds = 0;     // dynamic LDS of the step kernel for the current batch
   size_t cur_lds_big = 0; // dynamic LDS of the whole-CU tier

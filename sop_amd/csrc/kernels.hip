@@ -1455,7 +1455,8 @@ __device__ __forceinline__ void integrate(const DevPtrs &p, const SysDev &S, int
 // computed it, so the random force and the move run on all 64 lanes, one bead
 // per lane, with no block barrier.  ONE: every bead of the system has the
 // same type, so the force-field constants are wave-uniform (scalar registers).
-template <int LPB, int MODE, bool LDS, bool IDX16, bool ONE>
+// GB partners are asked for together.
+template <int LPB, int MODE, bool LDS, bool IDX16, bool ONE, int GB>
 __device__ __forceinline__ void wave_tile(const DevPtrs &p, const SysDev &S, int s, int t, int kstep,
                                           const float4 *__restrict__ pin, float4 *__restrict__ pout,
                                           const float4 *s_pos, int lds0, int r0, int r1) {
@@ -1589,7 +1590,6 @@ __device__ __forceinline__ void wave_tile(const DevPtrs &p, const SysDev &S, int
         // the E partners of one chunk; the next chunk's load goes out first,
         // without a condition: past the row it reads the rows after it, or
         // zeros past the segment (buffer range check)
-        constexpr int GB = LDS ? 2 : 4;  // partners asked for together
         auto chunk = [&](int c, auto guarded) {
           const chunk_t cur = q;
           q = load_chunk(rrow, rowoff + CB * (uint32_t)(c + LPB));
@@ -1696,13 +1696,18 @@ __device__ __forceinline__ void stage_item(const DevPtrs &p, int z, int w, int k
 }
 
 // Work items of one launch: LDS items (tier 0), whole-CU LDS items (tier 1),
-// or the items that gather from global memory (KLDS = false).
+// the items that gather from global memory (KLDS = false), or the LDS items and
+// then those (TIER_MIXED: a batch with no whole-CU items).
+constexpr int TIER_MIXED = 2;
 template <bool KLDS, bool FILTER>
 __device__ __forceinline__ void item_range(const DevPtrs &p, int tier, int &w0, int &w1) {
   const int n0 = FILTER ? *p.nfitems : *p.nitems, n1 = FILTER ? *p.nfitems_big : *p.nitems_big;
   if (!KLDS) {
     w0 = n0 + n1;
     w1 = w0 + (FILTER ? *p.nfitems_far : *p.nitems_far);
+  } else if (tier == TIER_MIXED) {
+    w0 = 0;
+    w1 = n0 + n1 + *p.nitems_far;
   } else if (tier == 0) {
     w0 = 0;
     w1 = n0;
@@ -1721,7 +1726,7 @@ __device__ __forceinline__ void item_range(const DevPtrs &p, int tier, int &w0, 
 // partner gather is an LDS read; the other kernel takes the items that gather
 // from global memory (items[nitems .. nitems + nitems_far)).  The result is
 // identical either way, and k_step_tile's.
-template <int LPB, int MODE, bool KLDS>
+template <int LPB, int MODE, bool KLDS, bool MIXED = false>
 __device__ __forceinline__ void step_items(const DevPtrs &p, int kstep, float4 *s_pos, int tier) {
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: system data in scalar registers
@@ -1730,7 +1735,8 @@ __device__ __forceinline__ void step_items(const DevPtrs &p, int kstep, float4 *
   for (int w = w0 + blockIdx.x; w < w1; w += gridDim.x) {
     const int4 it = p.items[w];
     if (it.x < 0) continue;
-    if (KLDS) {
+    const bool staged = KLDS && (!MIXED || it.z >= 0);
+    if (staged) {
       __syncthreads();  // the previous item's reads are done
       stage_item(p, it.z, it.w, kstep, s_pos, wave, tid & 63);
       __syncthreads();
@@ -1753,14 +1759,19 @@ __device__ __forceinline__ void step_items(const DevPtrs &p, int kstep, float4 *
       if (r0 == 0 && i < S.bead_off + S.n) pout[i] = pin[i];
       continue;
     }
-    const int lds0 = KLDS ? it.z : 0;
-    // (staged systems are small enough for 16-bit rows)
-    if (S.type_mask != 3) {
-      if (KLDS || S.idx16) wave_tile<LPB, MODE, KLDS, true, true>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
-      else wave_tile<LPB, MODE, false, false, true>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
-    } else {
-      if (KLDS || S.idx16) wave_tile<LPB, MODE, KLDS, true, false>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
-      else wave_tile<LPB, MODE, false, false, false>(p, S, s, t, kstep, pin, pout, s_pos, lds0, r0, r1);
+    const bool one = S.type_mask != 3;
+    if (staged) {  // (small enough for 16-bit rows)
+      if (one) wave_tile<LPB, MODE, KLDS, true, true, 2>(p, S, s, t, kstep, pin, pout, s_pos, it.z, r0, r1);
+      else wave_tile<LPB, MODE, KLDS, true, false, 2>(p, S, s, t, kstep, pin, pout, s_pos, it.z, r0, r1);
+    } else if constexpr (!KLDS || MIXED) {
+      constexpr int GB = MIXED ? 2 : 4;  // (the mixed launch has half the registers)
+      if (S.idx16) {
+        if (one) wave_tile<LPB, MODE, false, true, true, GB>(p, S, s, t, kstep, pin, pout, s_pos, 0, r0, r1);
+        else wave_tile<LPB, MODE, false, true, false, GB>(p, S, s, t, kstep, pin, pout, s_pos, 0, r0, r1);
+      } else {
+        if (one) wave_tile<LPB, MODE, false, false, true, GB>(p, S, s, t, kstep, pin, pout, s_pos, 0, r0, r1);
+        else wave_tile<LPB, MODE, false, false, false, GB>(p, S, s, t, kstep, pin, pout, s_pos, 0, r0, r1);
+      }
     }
   }
 }
@@ -2383,6 +2394,18 @@ template <int LPB, int MODE>
 __global__ __launch_bounds__(STEP_THREADS, 8) void k_step(DevPtrs p, int kstep, int tier) {
   extern __shared__ float4 s_pos[];
   step_items<LPB, MODE, true>(p, kstep, s_pos, tier);
+}
+
+// The LDS items and the global-gather ones in one launch, at two blocks per
+// compute unit.  Two launches on two streams cost the graph a fork and a join,
+// 9 us a step, and the gathering blocks got the registers of one per unit.
+// Run per step, two launches / one: 12 systems of 1,500 beads and one of
+// 18,000 40.1 / 33.5 us, 60 and 3 59.2 / 49.4, 120 and 1 62.6 / 48.7, 120 and 8
+// 102.5 / 96.0.
+template <int LPB, int MODE>
+__global__ __launch_bounds__(STEP_THREADS, 8) void k_step_mixed(DevPtrs p, int kstep) {
+  extern __shared__ float4 s_pos[];
+  step_items<LPB, MODE, true, true>(p, kstep, s_pos, TIER_MIXED);
 }
 
 template <int LPB, int MODE>
@@ -3166,8 +3189,23 @@ static void launch_step_lds(const DevPtrs &p, int lpb, int grid, size_t lds, int
 }
 
 template <int MODE>
+static void launch_step_mixed(const DevPtrs &p, int lpb, int grid, size_t lds, int kstep, hipStream_t st) {
+  const dim3 g(grid), b(STEP_THREADS);
+  switch (lpb) {
+    case 4: hipLaunchKernelGGL((k_step_mixed<4, MODE>), g, b, lds, st, p, kstep); break;
+    case 8: hipLaunchKernelGGL((k_step_mixed<8, MODE>), g, b, lds, st, p, kstep); break;
+    case 32: hipLaunchKernelGGL((k_step_mixed<32, MODE>), g, b, lds, st, p, kstep); break;
+    default: hipLaunchKernelGGL((k_step_mixed<16, MODE>), g, b, lds, st, p, kstep); break;
+  }
+}
+
+template <int MODE>
 static hipError_t launch_step_mode(const DevPtrs &p, int lpb, const StepGrids &sg, int kstep, hipStream_t st,
                                    const StepFork *fk) {
+  if (sg.mixed) {
+    launch_step_mixed<MODE>(p, lpb, sg.grid, sg.lds, kstep, st);
+    return SOPK_LAUNCH_CHECK();
+  }
   // the whole-CU and per-tile launches beside the two-blocks-per-unit one
   const bool fork = fk && sg.grid > 0 && (sg.grid_big > 0 || sg.grid_far > 0 || sg.tiles > 0);
   if (fork) {
@@ -3217,7 +3255,9 @@ hipError_t step_lds_limit(size_t bytes) {
       h = hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
   };
 #define SOPK_LDS_ATTR(L)                                                                            \
-  allow(&k_step<L, MODE_STEP>), allow(&k_step<L, MODE_FORCE>), allow(&k_step<L, MODE_FORCE_NOISE>);
+  allow(&k_step<L, MODE_STEP>), allow(&k_step<L, MODE_FORCE>), allow(&k_step<L, MODE_FORCE_NOISE>),   \
+      allow(&k_step_mixed<L, MODE_STEP>), allow(&k_step_mixed<L, MODE_FORCE>),                        \
+      allow(&k_step_mixed<L, MODE_FORCE_NOISE>);
   SOPK_LDS_ATTR(4) SOPK_LDS_ATTR(8) SOPK_LDS_ATTR(16) SOPK_LDS_ATTR(32)
 #undef SOPK_LDS_ATTR
   return h;

@@ -192,6 +192,7 @@ struct StepGrids {
   int grid, grid_big, grid_far;
   size_t lds, lds_big;
   int tiles;
+  bool mixed;  // step only: one launch of `grid` blocks takes the LDS and the global-gather items
 };
 
 // A second stream and two events: the step launches of the whole-CU and

@@ -79,6 +79,28 @@ def test_global_gather_items_by_count(sizes):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("systems,lanes", [
+    ([(70, 2000)] * 14 + [(71, 12000)], 4),
+    ([(72, 4500, 2)] * 8 + [(73, 11000, 2), (74, 64)], 4),
+    ([(75, 130)] * 3 + [(76, 70000, 1, False, False)], 4),  # 32-bit rows
+    ([(77, 700, 1, True)] * 30 + [(78, 20000, 1, True)], 8),
+])
+def test_staged_and_gathered_systems_in_one_launch(systems, lanes):
+    """LDS and global-gather items of one launch, against each system alone."""
+    made = [chain(*a) for a in systems]
+    for k, s in enumerate(made):
+        s.params.seed = W.philox_key(47, k)
+    got = outputs(made, 20, lanes_per_bead=lanes)
+    n = len(made)
+    for k in (0, n - 2, n - 1):
+        with S.Engine(0, lanes_per_bead=lanes) as e:
+            i = e.add(made[k])
+            assert np.array_equal(got[k], e.force_eval(i, with_noise=k % 2 == 1))
+            e.run([i], 20)
+            assert np.array_equal(got[n + k], e.coords(i))
+            assert np.array_equal(got[2 * n + k], e.velocities(i))
+
+
 @pytest.mark.parametrize("n,types,lanes", [(300, 1, 4), (1500, 2, 4), (700, 1, 8), (6000, 1, 4), (12000, 2, 4)])
 def test_beads_on_one_another(n, types, lanes):
     """Pairs below the repulsion's guard, in the middle of rows and at their ends:
