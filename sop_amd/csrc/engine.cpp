@@ -1200,7 +1200,8 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   }
   if ((int64_t)tiles.size() > e->tiles_cap) {
     HIPCK(hipStreamSynchronize(e->stream));
-    const int64_t nc = std::max<int64_t>(1024, (int64_t)tiles.size() * 2);
+    // (room for every block of the launch: a block reads its first entry at once)
+    const int64_t nc = std::max<int64_t>(std::max(1024, 4 * e->num_cu), (int64_t)tiles.size() * 2);
     if (e->p.tiles) HIPCK(hipFree(e->p.tiles));
     HIPCK(hipMalloc((void **)&e->p.tiles, sizeof(int2) * (size_t)nc));
     e->tiles_cap = nc;

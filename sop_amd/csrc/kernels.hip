@@ -113,6 +113,18 @@ __device__ __forceinline__ double wave_sum_d(double v) {
   return v;
 }
 
+// Maximum over the wave of values >= 0, in lane 63.
+__device__ __forceinline__ float wave_max63(float v) {
+  auto step = [&](int shifted) { v = fmaxf(v, __int_as_float(shifted)); };
+  step(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x111, 0xF, 0xF, false));
+  step(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x112, 0xF, 0xF, false));
+  step(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x114, 0xF, 0xF, false));
+  step(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x118, 0xF, 0xF, false));
+  step(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xA, 0xF, false));
+  step(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xC, 0xF, false));
+  return v;
+}
+
 // Inclusive prefix sum across the 64 lanes of a wave with DPP: Hillis-Steele
 // inside each 16-lane row (row_shr 1,2,4,8), then row_bcast15 / row_bcast31
 // carry row totals into the rows above.
@@ -171,12 +183,47 @@ __device__ __forceinline__ void normals3(uint32_t k0, uint32_t k1, uint32_t bead
   n2 = rb * cb;
 }
 
-__device__ __forceinline__ bool live(const SysDev &S, int kstep) { return S.step + kstep < S.step_end; }
-__device__ __forceinline__ bool due_nl(const SysDev &S, int kstep) {
-  return live(S, kstep) && ((S.step + kstep) % S.n_nl) == 0;
+// Loads through the scalar cache: one trip for all of a system's fields, where
+// vector loads of values that steer the wave each wait in turn (three to eight
+// trips to the L2 before a kernel's first bead).  For what no other block
+// writes in the launch, and this one only after its reads.  Steps of one
+// system: 128 beads 5.90 -> 5.51 us, 4,999 7.64 -> 7.04, 10,000 8.2 -> 7.6; 512
+// replicas 69.6 -> 66.5 (the fields also leave the vector registers); the
+// rebuild's decision 6.7 -> 5.7; rows, cells and filter of 200,000 beads 150
+// -> 100 us a rebuild.
+typedef const __attribute__((address_space(4))) SysDev SysConst;
+__device__ __forceinline__ SysConst &sys_const(const DevPtrs &p, int s) { return *(SysConst *)(uintptr_t)(p.sys + s); }
+__device__ __forceinline__ int sload(const int32_t *q) {
+  return *(const __attribute__((address_space(4))) int *)(uintptr_t)q;
 }
-__device__ __forceinline__ bool due_pl(const SysDev &S, int kstep) {
-  return live(S, kstep) && ((S.step + kstep) % S.n_pl) == 0;
+__device__ __forceinline__ int2 sload(const int2 *q) {
+  typedef int v2 __attribute__((ext_vector_type(2)));
+  const v2 v = *(const __attribute__((address_space(4))) v2 *)(uintptr_t)q;
+  return make_int2(v.x, v.y);
+}
+__device__ __forceinline__ int4 sload(const int4 *q) {
+  typedef int v4 __attribute__((ext_vector_type(4)));
+  const v4 v = *(const __attribute__((address_space(4))) v4 *)(uintptr_t)q;
+  return make_int4(v.x, v.y, v.z, v.w);
+}
+
+// Which rebuilds are due at step + kstep, or asked for by the flags.  The
+// schedule's fields are read together (a short circuit between them would make
+// each a round trip of its own), and steps below 2^32 take a 32-bit remainder.
+struct Due {
+  bool nl, pl;
+};
+__device__ __forceinline__ bool divides(int n, int64_t step) {
+  return (uint64_t)step >> 32 ? step % n == 0 : (uint32_t)step % (uint32_t)n == 0;
+}
+template <typename Sys>
+__device__ __forceinline__ Due rebuild_due(const Sys &S, int kstep, int flags) {
+  const int64_t step = S.step + kstep, end = S.step_end;
+  const int n_nl = S.n_nl, n_pl = S.n_pl;
+  const bool mat = (flags & MATERIALIZE_NL) != 0, live = step < end;
+  const bool nl = ((flags & FORCE_NL) != 0) | (live & divides(n_nl, step));
+  const bool pl = ((flags & FORCE_PL) != 0) | (live & divides(n_pl, step));
+  return Due{nl && !mat, pl && !mat};
 }
 
 template <typename G>
@@ -210,27 +257,36 @@ __device__ __forceinline__ int cell_index(const G &S, float4 x) {
 // the cell grid (BUILD_SHELL).
 
 // Systems whose rebuild sorts beads into a cell grid.
-__device__ __forceinline__ bool grid_build(const SysDev &S) {
+template <typename Sys>
+__device__ __forceinline__ bool grid_build(const Sys &S) {
   return S.build != BUILD_NONE && S.build != BUILD_SHELL;
 }
 
-__device__ __forceinline__ const float4 *build_src(const DevPtrs &p, const SysDev &S, int kstep) {
+template <typename Sys>
+__device__ __forceinline__ const float4 *build_src(const DevPtrs &p, const Sys &S, int kstep) {
   return S.build == BUILD_DIRECT ? buf_in(p, S.parity + kstep) : p.pos_ref;
 }
 
+// What a rebuild's decision reads, loaded with the system's other constants: in
+// the deciding thread it would be one more round trip, behind the barrier.
+struct BuildLimits {
+  float skin, shell_ok;
+  int32_t nl_valid, n_direct, n_shell, n_nl;
+};
+
 // A rebuild's decision for one system, from the largest displacements since
 // the two snapshots (one thread).  Returns S.build.
-__device__ __forceinline__ int decide_build(SysDev &S, int flags, bool nl, bool pl, bool shell_chk, float d2max,
-                                            float d2sh) {
+__device__ __forceinline__ int decide_build(SysDev &S, const BuildLimits &lim, int flags, bool nl, bool pl,
+                                            bool shell_chk, float d2max, float d2sh) {
   const float dmax = sqrtf(d2max), dsh = sqrtf(d2sh);
   int build = BUILD_NONE;
   if (flags & MATERIALIZE_NL) {
-    build = S.nl_valid ? BUILD_NONE : BUILD_NL_ONLY;
+    build = lim.nl_valid ? BUILD_NONE : BUILD_NL_ONLY;
   } else {
     if (nl) S.nl_valid = 0;
     if (pl) {
-      if (S.skin > 0.0f && (nl || 2.0f * dmax < S.skin))
-        build = shell_chk && 2.0f * dsh < S.shell_ok ? BUILD_SHELL : BUILD_DIRECT;
+      if (lim.skin > 0.0f && (nl || 2.0f * dmax < lim.skin))
+        build = shell_chk && 2.0f * dsh < lim.shell_ok ? BUILD_SHELL : BUILD_DIRECT;
       else
         build = BUILD_NL;
     } else if (flags & FORCE_NL) {
@@ -240,8 +296,9 @@ __device__ __forceinline__ int decide_build(SysDev &S, int flags, bool nl, bool 
   S.build = build;
   if (build == BUILD_DIRECT) S.sl_valid = 1;
   if (build == BUILD_NL) S.sl_valid = 0;  // k_rows writes its rows into the shell-row slots
-  if (build == BUILD_DIRECT || build == BUILD_SHELL || build == BUILD_NL)
-    ++S.nbuild[build == BUILD_DIRECT ? 0 : (build == BUILD_SHELL ? 1 : 2)];
+  if (build == BUILD_DIRECT) S.nbuild[0] = lim.n_direct + 1;
+  if (build == BUILD_SHELL) S.nbuild[1] = lim.n_shell + 1;
+  if (build == BUILD_NL) S.nbuild[2] = lim.n_nl + 1;
   return build;
 }
 
@@ -333,19 +390,20 @@ __global__ __launch_bounds__(SORT_THREADS) void k_rebuild(DevPtrs p, int kstep, 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nsys = *p.nsys;
   for (int q = *p.nbig + blockIdx.x; q < nsys; q += gridDim.x) {
-    const int s = p.syslist[q];
+    const int s = __builtin_amdgcn_readfirstlane(p.syslist[q]);
     SysDev &S = p.sys[s];
     // system constants in registers (the stores below may alias S)
-    const int bo = S.bead_off, n = S.n;
-    const float4 *x = buf_in(p, S.parity + kstep);
+    SysConst &C = sys_const(p, s);
+    const int bo = C.bead_off, n = C.n;
+    const float4 *x = buf_in(p, C.parity + kstep);
     float4 xs[SB];
     int build;
     bool loaded = false;
     if (PH & PH_DECIDE) {
-      const bool mat = (flags & MATERIALIZE_NL) != 0;
-      const bool nl = !mat && ((flags & FORCE_NL) || due_nl(S, kstep));
-      const bool pl = !mat && ((flags & FORCE_PL) || due_pl(S, kstep));
-      const bool shell_chk = pl && S.sl_valid;
+      const BuildLimits lim{C.skin, C.shell_ok, C.nl_valid, C.nbuild[0], C.nbuild[1], C.nbuild[2]};
+      const bool rows = C.sl_valid != 0;
+      const Due due = rebuild_due(C, kstep, flags);
+      const bool nl = due.nl, pl = due.pl, shell_chk = pl & rows;
       float d2max = 0.0f, d2sh = 0.0f;
       loaded = nl || pl;
       if (loaded) {
@@ -358,40 +416,39 @@ __global__ __launch_bounds__(SORT_THREADS) void k_rebuild(DevPtrs p, int kstep, 
 #pragma unroll
           for (int u = 0; u < SB; ++u)
             if (u * SORT_THREADS < n) p.pos_ref[bo + min(tid + u * SORT_THREADS, n - 1)] = xs[u];
-        } else {
+        }
+        // (the fences keep each group of loads ahead of its uses)
+        auto farthest = [&](const float4 *from) -> float {
+          float4 r[SB];
+          float m = 0.0f;
+#pragma unroll
+          for (int u = 0; u < SB; ++u) r[u] = from[bo + min(tid + u * SORT_THREADS, n - 1)];
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int u = 0; u < SB; ++u) {
-            const float4 r = p.pos_ref[bo + min(tid + u * SORT_THREADS, n - 1)];
-            const float dx = xs[u].x - r.x, dy = xs[u].y - r.y, dz = xs[u].z - r.z;
-            d2max = fmaxf(d2max, dx * dx + dy * dy + dz * dz);
+            const float dx = xs[u].x - r[u].x, dy = xs[u].y - r[u].y, dz = xs[u].z - r[u].z;
+            m = fmaxf(m, dx * dx + dy * dy + dz * dz);
           }
-        }
-        if (shell_chk) {
-#pragma unroll
-          for (int u = 0; u < SB; ++u) {
-            const float4 r = p.pos_shell[bo + min(tid + u * SORT_THREADS, n - 1)];
-            const float ex = xs[u].x - r.x, ey = xs[u].y - r.y, ez = xs[u].z - r.z;
-            d2sh = fmaxf(d2sh, ex * ex + ey * ey + ez * ez);
-          }
-        }
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-          d2max = fmaxf(d2max, __shfl_xor(d2max, o));
-          d2sh = fmaxf(d2sh, __shfl_xor(d2sh, o));
-        }
+          return m;
+        };
+        if (!nl) d2max = farthest(p.pos_ref);
+        if (shell_chk) d2sh = farthest(p.pos_shell);
+        d2max = wave_max63(d2max);
+        d2sh = wave_max63(d2sh);
       }
-      if (lane == 0) {
+      if (lane == 63) {
         s_red[0][wave] = d2max;
         s_red[1][wave] = d2sh;
       }
       __syncthreads();
       if (tid == 0) {
         float m0 = 0.0f, m1 = 0.0f;
+#pragma unroll
         for (int w = 0; w < NW; ++w) {
           m0 = fmaxf(m0, s_red[0][w]);
           m1 = fmaxf(m1, s_red[1][w]);
         }
-        s_build = decide_build(S, flags, nl, pl, shell_chk, m0, m1);
+        s_build = decide_build(S, lim, flags, nl, pl, shell_chk, m0, m1);
         if (s_build == BUILD_NL || s_build == BUILD_NL_ONLY) atomicOr(p.nlbuild, 1);
       }
       __syncthreads();
@@ -554,9 +611,8 @@ __global__ __launch_bounds__(BIG_THREADS) void k_big_skin(DevPtrs p, int kstep, 
   const int nbig = *p.nbig;
   for (int q = blockIdx.y; q < nbig; q += gridDim.y) {
     SysDev &S = p.sys[p.syslist[q]];
-    const bool mat = (flags & MATERIALIZE_NL) != 0;
-    const bool nl = !mat && ((flags & FORCE_NL) || due_nl(S, kstep));
-    const bool pl = !mat && ((flags & FORCE_PL) || due_pl(S, kstep));
+    const Due due = rebuild_due(S, kstep, flags);
+    const bool nl = due.nl, pl = due.pl;
     if (!nl && !pl) continue;
     const int bo = S.bead_off, n = S.n;
     const float4 *x = buf_in(p, S.parity + kstep);
@@ -620,9 +676,8 @@ __global__ __launch_bounds__(1024) void k_big_plan(DevPtrs p, int kstep, int fla
   for (int q = blockIdx.x; q < nbig; q += gridDim.x) {
     SysDev &S = p.sys[p.syslist[q]];
     if (tid == 0) {
-      const bool mat = (flags & MATERIALIZE_NL) != 0;
-      const bool nl = !mat && ((flags & FORCE_NL) || due_nl(S, kstep));
-      const bool pl = !mat && ((flags & FORCE_PL) || due_pl(S, kstep));
+      const Due due = rebuild_due(S, kstep, flags);
+      const bool nl = due.nl, pl = due.pl;
       float mn[3], mx[3];
       for (int d = 0; d < 3; ++d) {
         mn[d] = ord_f(S.acc[d]);
@@ -635,7 +690,8 @@ __global__ __launch_bounds__(1024) void k_big_plan(DevPtrs p, int kstep, int fla
           S.ref_box[d] = mn[d];
           S.ref_box[3 + d] = mx[d];
         }
-      const int build = decide_build(S, flags, nl, pl, pl && S.sl_valid, d2max, d2sh);
+      const BuildLimits lim{S.skin, S.shell_ok, S.nl_valid, S.nbuild[0], S.nbuild[1], S.nbuild[2]};
+      const int build = decide_build(S, lim, flags, nl, pl, pl && S.sl_valid, d2max, d2sh);
       int nc = 0;
       if (build != BUILD_NONE && build != BUILD_SHELL) {
         if (build != BUILD_DIRECT)  // sorted at the snapshot
@@ -660,7 +716,7 @@ __global__ __launch_bounds__(1024) void k_big_plan(DevPtrs p, int kstep, int fla
 __global__ __launch_bounds__(256) void k_cell_count(DevPtrs p, int kstep) {
   const int nbig = *p.nbig;
   for (int q = blockIdx.y; q < nbig; q += gridDim.y) {
-    const SysDev &S = p.sys[p.syslist[q]];
+    SysConst &S = sys_const(p, sload(p.syslist + q));
     if (!grid_build(S)) continue;
     const float4 *src = build_src(p, S, kstep);
     const bool direct = S.build == BUILD_DIRECT;
@@ -741,7 +797,7 @@ __global__ __launch_bounds__(1024) void k_cell_scan(DevPtrs p) {
 __global__ __launch_bounds__(256) void k_cell_scatter(DevPtrs p) {
   const int nbig = *p.nbig;
   for (int q = blockIdx.y; q < nbig; q += gridDim.y) {
-    const SysDev &S = p.sys[p.syslist[q]];
+    SysConst &S = sys_const(p, sload(p.syslist + q));
     if (!grid_build(S)) continue;
     const int bo = S.bead_off, n = S.n, cb = S.cell_base;
     for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < n; b += gridDim.x * blockDim.x) {
@@ -759,7 +815,7 @@ __global__ __launch_bounds__(256) void k_cell_scatter(DevPtrs p) {
 __global__ __launch_bounds__(256) void k_cell_rank(DevPtrs p, int kstep) {
   const int nbig = *p.nbig;
   for (int q = blockIdx.y; q < nbig; q += gridDim.y) {
-    const SysDev &S = p.sys[p.syslist[q]];
+    SysConst &S = sys_const(p, sload(p.syslist + q));
     if (!grid_build(S)) continue;
     const float4 *src = build_src(p, S, kstep);
     const int bo = S.bead_off, n = S.n, cb = S.cell_base;
@@ -815,7 +871,7 @@ __device__ __forceinline__ void natbits_mark(uint32_t *bits, const int32_t *natj
 // appended to out[0..cap) with ballot/mbcnt
 // compaction; returns the count (which may exceed cap).
 template <typename Extra, typename Emit>
-__device__ __forceinline__ int scan_cells(const DevPtrs &p, const SysDev &S, int i, float4 xi,
+__device__ __forceinline__ int scan_cells(const DevPtrs &p, SysConst &S, int i, float4 xi,
                                           float rcA, float rcB, int ns, int nn, uint32_t *bits, Extra extra,
                                           Emit emit) {
   const int lane = threadIdx.x & 63;
@@ -986,9 +1042,9 @@ __device__ __forceinline__ void pl_cells(const DevPtrs &p, int kstep, char *s_ra
   const int total = *p.ncellwork;
   for (int g = blockIdx.x; g < total; g += gridDim.x) {
     const int2 item = p.cellitems[g];
-    const int s = p.syslist[item.x];
+    const int s = sload(p.syslist + item.x);
     const int c = item.y;
-    const SysDev &S = p.sys[s];
+    SysConst &S = sys_const(p, s);
     const int bo = S.bead_off, cb = S.cell_base, n = S.n;
     const int pl_cap = S.pl_cap;
     const int64_t pl_base = S.pl_base;
@@ -1184,10 +1240,10 @@ __device__ __forceinline__ void nl_build(const DevPtrs &p, int kstep, char *s_ra
   constexpr int UNITS = TILE / NLB_BEADS;
   const int nunit = *p.nwork * UNITS;
   for (int w = blockIdx.x * 4 + wave; w < nunit; w += gridDim.x * 4) {
-    const int t = p.work[w / UNITS];
+    const int t = sload(p.work + w / UNITS);
     if (t < 0) continue;
-    const int s = p.tile_sys[t];
-    const SysDev &S = p.sys[s];
+    const int s = sload(p.tile_sys + t);
+    SysConst &S = sys_const(p, s);
     if (S.build != BUILD_NL && S.build != BUILD_NL_ONLY) continue;
     const bool plb = S.build == BUILD_NL;
     const float4 *ref = p.pos_ref;
@@ -1342,7 +1398,7 @@ __device__ __forceinline__ uint32_t mad16(uint32_t w, uint32_t base) {
 
 // Force of the chain terms on bead b0 + lane of a tile, one bead per lane.
 template <bool LDS>
-__device__ __forceinline__ float3 chain_force(const DevPtrs &p, const SysDev &S, int s, int b0,
+__device__ __forceinline__ float3 chain_force(const DevPtrs &p, SysConst &S, int s, int b0,
                                               const float4 *__restrict__ pin, const float4 *s_pos, int lds0, float t_br,
                                               float br_before) {
   const int lane = threadIdx.x & 63;
@@ -1407,7 +1463,7 @@ __device__ __forceinline__ float3 chain_force(const DevPtrs &p, const SysDev &S,
 // The move of bead b0 + lane (or the force output) from its force mf without
 // noise and its three normals n0, n1, n2 of this step.
 template <bool LDS>
-__device__ __forceinline__ void integrate(const DevPtrs &p, const SysDev &S, int s, int i, int mode,
+__device__ __forceinline__ void integrate(const DevPtrs &p, SysConst &S, int s, int i, int mode,
                                           const float4 *__restrict__ pin, float4 *__restrict__ pout,
                                           const float4 *s_pos, int lds0, float mfx, float mfy, float mfz, float n0,
                                           float n1, float n2) {
@@ -1457,7 +1513,7 @@ __device__ __forceinline__ void integrate(const DevPtrs &p, const SysDev &S, int
 // same type, so the force-field constants are wave-uniform (scalar registers).
 // GB partners are asked for together.
 template <int LPB, int MODE, bool LDS, bool IDX16, bool ONE, int GB>
-__device__ __forceinline__ void wave_tile(const DevPtrs &p, const SysDev &S, int s, int t, int kstep,
+__device__ __forceinline__ void wave_tile(const DevPtrs &p, SysConst &S, int s, int t, int kstep,
                                           const float4 *__restrict__ pin, float4 *__restrict__ pout,
                                           const float4 *s_pos, int lds0, int r0, int r1) {
   constexpr int GPW = 64 / LPB;
@@ -1733,7 +1789,7 @@ __device__ __forceinline__ void step_items(const DevPtrs &p, int kstep, float4 *
   int w0, w1;
   item_range<KLDS, false>(p, tier, w0, w1);
   for (int w = w0 + blockIdx.x; w < w1; w += gridDim.x) {
-    const int4 it = p.items[w];
+    const int4 it = sload(p.items + w);
     if (it.x < 0) continue;
     const bool staged = KLDS && (!MIXED || it.z >= 0);
     if (staged) {
@@ -1748,8 +1804,8 @@ __device__ __forceinline__ void step_items(const DevPtrs &p, int kstep, float4 *
     const int r0 = (wave % ns) * (LPB / ns), r1 = r0 + LPB / ns;
     if (tw >= item_tiles(it.y)) continue;
     const int t = it.x + tw;
-    const int s = __builtin_amdgcn_readfirstlane(p.tile_sys[t]);
-    const SysDev &S = p.sys[s];
+    const int s = sload(p.tile_sys + t);
+    SysConst &S = sys_const(p, s);
     const int par = S.parity + kstep;
     const float4 *__restrict__ pin = buf_in(p, par);
     float4 *__restrict__ pout = buf_out(p, par);
@@ -1818,7 +1874,7 @@ __device__ __forceinline__ int tile_order(const DevPtrs &p, int t, int build, bo
 // end tested only in chunks that reach it, and one word of keep bits per chunk
 // took it from 229 to 209 us.
 template <bool LDS, bool IDX16, bool STAGE, bool ONE>
-__device__ __forceinline__ void filter_tile(const DevPtrs &p, const SysDev &S, int s, int t,
+__device__ __forceinline__ void filter_tile(const DevPtrs &p, SysConst &S, int s, int t,
                                             const float4 *__restrict__ pin, const float4 *s_pos, int lds0,
                                             void *s_stage) {
   using ent_t = typename std::conditional<IDX16, uint16_t, uint32_t>::type;
@@ -2099,7 +2155,7 @@ __global__ __launch_bounds__(STEP_THREADS) void k_shell_filter(DevPtrs p, int ks
   int w0, w1;
   item_range<KLDS, true>(p, tier, w0, w1);
   for (int w = w0 + blockIdx.x; w < w1; w += gridDim.x) {
-    const int4 it = p.fitems[w];
+    const int4 it = sload(p.fitems + w);
     if (it.x < 0) continue;
     // one wave per tile (the tile order it computes first must come from one
     // wave); a tile is filtered when its system's build is one of `builds`
@@ -2118,8 +2174,8 @@ __global__ __launch_bounds__(STEP_THREADS) void k_shell_filter(DevPtrs p, int ks
     }
     if (((tiles_mine >> wave) & 1) == 0) continue;
     const int t = it.x + wave;
-    const int s = __builtin_amdgcn_readfirstlane(p.tile_sys[t]);
-    const SysDev &S = p.sys[s];
+    const int s = sload(p.tile_sys + t);
+    SysConst &S = sys_const(p, s);
     const float4 *pin = buf_in(p, S.parity + kstep);
     const int lds0 = KLDS ? it.z : 0;
     // each wave owns stage_bytes / STEP_WAVES bytes whatever the entry width
@@ -2162,7 +2218,7 @@ constexpr int FILTER_ROW_WAVES = 8, FILTER_NAT_WAVES = 4;
 constexpr int FILTER_TILE_THREADS = 64 * (FILTER_ROW_WAVES + FILTER_NAT_WAVES);
 
 template <bool ONE>
-__device__ __forceinline__ void filter_rows(const DevPtrs &p, const SysDev &S, int b0, int nb, int wave,
+__device__ __forceinline__ void filter_rows(const DevPtrs &p, SysConst &S, int b0, int nb, int wave,
                                             const float4 *__restrict__ pin, int *s_len, const int *s_nlen,
                                             const int2 *s_nat) {
   constexpr int R = TILE / FILTER_ROW_WAVES, NP = 2;  // rows of the wave, passes held in registers
@@ -2282,7 +2338,7 @@ __device__ __forceinline__ void filter_rows(const DevPtrs &p, const SysDev &S, i
 // decisions and counts, then the entries at the lists' places.  Keep bits hold
 // 32 batches of four (128 natives of a bead); past them the decision is made
 // again for the writes, and batches past the first NB are loaded again.
-__device__ __forceinline__ void filter_nats(const DevPtrs &p, const SysDev &S, int b0, int nb, int wave,
+__device__ __forceinline__ void filter_nats(const DevPtrs &p, SysConst &S, int b0, int nb, int wave,
                                             const float4 *__restrict__ pin, int *s_nlen, int2 *s_nat) {
   constexpr int NB = 4;
   const int lane = threadIdx.x & 63, g = lane >> 2, l = lane & 3;
@@ -2370,12 +2426,16 @@ __global__ __launch_bounds__(FILTER_TILE_THREADS) void k_filter_tile(DevPtrs p, 
     *p.ncellwork = 0;
     *p.nlbuild = 0;
   }
-  const int ntiles = *p.ntiles;
+  // (the table has room for every block of the grid)
+  const int ntiles = sload(p.ntiles);
+  int2 it = sload(p.tiles + blockIdx.x);
   for (int w = blockIdx.x; w < ntiles; w += gridDim.x) {
-    if (w != (int)blockIdx.x) __syncthreads();  // the previous tile's totals have been read
-    const int2 it = p.tiles[w];
+    if (w != (int)blockIdx.x) {
+      __syncthreads();  // the previous tile's totals have been read
+      it = sload(p.tiles + w);
+    }
     if (it.x < 0) continue;
-    const SysDev &S = p.sys[it.y];
+    SysConst &S = sys_const(p, it.y);
     if (((builds >> S.build) & 1) == 0) continue;
     const int b0 = it.x * TILE, nb = min(TILE, S.bead_off + S.n - b0);
     const float4 *__restrict__ pin = buf_in(p, S.parity + kstep);
@@ -2452,7 +2512,7 @@ __device__ __forceinline__ RoundAt round_at(int r, int b0, int bend, int ordm, u
 
 // Gathered native and non-native force on the lane group's bead.
 template <int LPB, bool ONE>
-__device__ __forceinline__ float3 tile_round(const DevPtrs &p, const SysDev &S, const float4 *__restrict__ pin, int self,
+__device__ __forceinline__ float3 tile_round(const DevPtrs &p, SysConst &S, const float4 *__restrict__ pin, int self,
                                              const RoundAt &a) {
   const int l = (int)(threadIdx.x & 63) % LPB;
   // buffer resources in scalar registers: the system's pair-list segment
@@ -2576,14 +2636,18 @@ __global__ __launch_bounds__(64 * (tile_waves(LPB) + 1)) void k_step_tile(DevPtr
   __shared__ float s_f[3][TILE];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: system data in scalar registers
-  const int ntiles = *p.ntiles;
+  // (the table has room for every block of the grid)
+  const int ntiles = sload(p.ntiles);
+  int2 it = sload(p.tiles + blockIdx.x);
   for (int w = blockIdx.x; w < ntiles; w += gridDim.x) {
-    if (w != (int)blockIdx.x) __syncthreads();  // the previous tile's forces have been read
-    const int2 it = p.tiles[w];
+    if (w != (int)blockIdx.x) {
+      __syncthreads();  // the previous tile's forces have been read
+      it = sload(p.tiles + w);
+    }
     if (it.x < 0) continue;
     const int t = it.x, s = it.y;
     const int b0 = t * TILE;
-    const SysDev &S = p.sys[s];
+    SysConst &S = sys_const(p, s);
     if (wave < W) {
       const int ordm = p.tile_ord[b0 + lane];
       const uint2 hd = p.plhead[b0 + lane];
@@ -2648,10 +2712,10 @@ __global__ __launch_bounds__(ENERGY_THREADS) void k_energy(DevPtrs p, int t0, in
   const int g = lane / LPB, l = lane % LPB;
   const int nwork = nt > 0 ? nt : *p.nwork;
   for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
-    const int t = nt > 0 ? t0 + w : p.work[w];
+    const int t = nt > 0 ? t0 + w : sload(p.work + w);
     if (t < 0) continue;
-    const int s = p.tile_sys[t];
-    const SysDev &S = p.sys[s];
+    const int s = sload(p.tile_sys + t);
+    SysConst &S = sys_const(p, s);
     const int bead_off = S.bead_off, n = S.n;
     const int b0 = t * TILE;
     const int bend = min(b0 + TILE, bead_off + n);
@@ -2795,8 +2859,8 @@ __global__ __launch_bounds__(256) void k_sys_reduce(DevPtrs p, int slot, double 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nsys = slot >= 0 ? 1 : *p.nsys;
   for (int q = blockIdx.x; q < nsys; q += gridDim.x) {
-    const int s = slot >= 0 ? slot : p.syslist[q];
-    const SysDev &S = p.sys[s];
+    const int s = slot >= 0 ? slot : sload(p.syslist + q);
+    SysConst &S = sys_const(p, s);
     const int nt = (S.n + TILE - 1) / TILE;
     const double *e = p.epart + (int64_t)(S.bead_off - p.epart_base) / TILE * TPART_N;
     double acc[TPART_N];
