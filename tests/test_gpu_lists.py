@@ -1,9 +1,10 @@
 """Half lists as the device counts, places and writes them, on device 0: one
 bead, a broken group of sixteen beads, the blocks of 1,024 beads that the
-places are summed over, and a list that leaves in more than one window (4 Mi
-pairs) from 32-bit rows.  Up to 2,100 beads against the FP64 oracle's lists;
-the large one against a k-d tree, whose count at the radius -+ 1e-4 A has to
-enclose it.  In all of them the pairs come by bead, i < j, and a shorter buffer
+places are summed over, cells of fewer and more members than the sort compares
+at a time (eight), and a list that leaves in more than one window (4 Mi pairs)
+from 32-bit rows.  Up to 2,100 beads against the FP64 oracle's lists;
+the large one against a k-d tree: every pair nearer than its longest is in it,
+or excluded.  In all of them the pairs come by bead, i < j, and a shorter buffer
 gets the list's first entries and nothing behind them.
 """
 import ctypes as C
@@ -32,7 +33,7 @@ def short_buffer(e, i, which, got, cap):
     assert np.array_equal(buf[:cap], got[:cap]) and np.all(buf[cap:] == -7)
 
 
-@pytest.mark.parametrize("n", [1, 2, 17, 1024, 1025, 2100])
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 17, 24, 1024, 1025, 2100])
 def test_lists_against_the_oracle(n):
     s = S.make_chain_system(810 + n % 89, n)
     (nla, nlr), (pla, plr) = Oracle(s).lists(s.xyz, grid=False)
