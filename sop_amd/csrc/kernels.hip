@@ -1375,22 +1375,21 @@ __device__ __forceinline__ float4 partner(const float4 *__restrict__ pin, const 
 }
 
 // The same by 32-bit byte offsets, for the pair loops: one instruction per
-// partner for its address.  In LDS the offset is the LDS address itself (at0
-// is arena bead 0's, modulo 2^32); global coordinates go through a buffer
-// resource.
+// partner for its address.  at0 is arena bead 0's, modulo 2^32.  In LDS the
+// offset is the LDS address itself; global coordinates go through a buffer
+// resource at the system's first bead (a system's rows are below 4 GiB, so its
+// coordinates are too, whatever the arena holds).
 typedef float vf4 __attribute__((ext_vector_type(4)));
 typedef float vf3 __attribute__((ext_vector_type(3)));
 template <bool LDS>
 struct PosAt {
   uint32_t at0;
   __amdgpu_buffer_rsrc_t r;
-  __device__ __forceinline__ PosAt(const float4 *__restrict__ pin, const float4 *s_pos, int lds0) {
-    if constexpr (LDS) {
-      at0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) float4 *)s_pos - 16u * (uint32_t)lds0;
-    } else {
-      at0 = 0;
-      r = buf_rsrc(pin, 0xFFFFFFFFu);
-    }
+  // first: the first staged bead (LDS), or the system's
+  __device__ __forceinline__ PosAt(const float4 *__restrict__ pin, const float4 *s_pos, int first) {
+    at0 = 0u - 16u * (uint32_t)first;
+    if constexpr (LDS) at0 += (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) float4 *)s_pos;
+    else r = buf_rsrc(pin + first, 0xFFFFFFFFu);
   }
   template <bool XYZ>
   __device__ __forceinline__ float4 get(uint32_t off) const {
@@ -1590,7 +1589,7 @@ __device__ __forceinline__ void wave_tile(const DevPtrs &p, SysConst &S, int s, 
   const __amdgpu_buffer_rsrc_t rrow =
       buf_rsrc(p.plrep_j + S.pl_base, (uint32_t)S.n * (uint32_t)S.pl_cap * ESZ);
   const __amdgpu_buffer_rsrc_t rnat = buf_rsrc(p.platt, 0xFFFFFFFFu);
-  const PosAt<LDS> pos(pin, s_pos, lds0);
+  const PosAt<LDS> pos(pin, s_pos, LDS ? lds0 : bead_off);
   const uint32_t row0 = pos.at0 + 16u * (uint32_t)bead_off;  // of row index 0
   float mfx = 0.0f, mfy = 0.0f, mfz = 0.0f;  // force on bead b0 + lane
   bool exact = false;                        // this round takes the guard at every pair
@@ -1922,7 +1921,7 @@ __device__ __forceinline__ void filter_tile(const DevPtrs &p, SysConst &S, int s
   const double plf = S.pl_factor;
   const float pla = S.pl_abs;
   ent_t *const seg = reinterpret_cast<ent_t *>(p.plrep_j + pl_base);
-  const PosAt<LDS> pos(pin, s_pos, lds0);
+  const PosAt<LDS> pos(pin, s_pos, LDS ? lds0 : bo);
   const uint32_t row0 = pos.at0 + 16u * (uint32_t)bo;  // of row index 0
   // this tile's region of the segment, and the rows packed so far; the same
   // for the native pair list, whose region is the tile's native CSR range
