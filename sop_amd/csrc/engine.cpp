@@ -1718,22 +1718,24 @@ sop_status sop_get_list(sop_engine *e, int32_t sys, int32_t which, int32_t *ij, 
     if (st) return st;
   }
   const int32_t nb = e->sys[sys].n;
-  if ((st = engine_io(e, e->io, 64))) return st;
-  HIPCK(launch_list_places(e->p, sys, nb, which, 0, static_cast<int64_t *>(e->io.ptr), e->stream));
-  HIPCK(hipStreamSynchronize(e->stream));
-  const int64_t total = *static_cast<const int64_t *>(e->io.ptr);
-  *n = total;
-  const int64_t want = ij ? std::min(total, cap) : 0;
-  constexpr int64_t WINDOW = (int64_t)4 << 20;  // pairs through the host buffer at a time
-  if (want > 0 && (st = engine_io(e, e->io, 8 * (size_t)(std::min(want, WINDOW) + 1)))) return st;
-  for (int64_t lo = 0; lo < want; lo += WINDOW) {
-    const int64_t m = std::min(WINDOW, want - lo);
-    if (lo)  // (the total again, behind the window)
-      HIPCK(launch_list_places(e->p, sys, nb, which, lo, static_cast<int64_t *>(e->io.ptr) + WINDOW, e->stream));
-    HIPCK(launch_list_write(e->p, sys, nb, which, static_cast<int2 *>(e->io.ptr), (int)m, e->stream));
+  // pairs go through the host buffer a window at a time, the total behind it;
+  // the first window is written before the total is known, with one wait for
+  // both (two updates and the four lists of 1,500 beads, counted and then
+  // fetched: 270 us with a wait for each, 246 with one)
+  constexpr int64_t WINDOW = (int64_t)4 << 20;
+  const int64_t room = ij ? std::max<int64_t>(cap, 0) : 0, m0 = std::min(room, WINDOW);
+  if ((st = engine_io(e, e->io, 8 * (size_t)(m0 + 1)))) return st;
+  int2 *const pairs = static_cast<int2 *>(e->io.ptr);
+  int64_t *const total = static_cast<int64_t *>(e->io.ptr) + m0;
+  for (int64_t lo = 0;; lo += m0) {
+    HIPCK(launch_list_places(e->p, sys, nb, which, lo, total, e->stream));
+    if (m0 > 0) HIPCK(launch_list_write(e->p, sys, nb, which, pairs, (int)std::min(m0, room - lo), e->stream));
     HIPCK(hipStreamSynchronize(e->stream));
-    std::memcpy(ij + 2 * lo, e->io.ptr, 8 * (size_t)m);
+    const int64_t want = std::min(*total, room);
+    if (want > lo) std::memcpy(ij + 2 * lo, pairs, 8 * (size_t)std::min(m0, want - lo));
+    if (want <= lo + m0) break;
   }
+  *n = *total;
   return SOP_OK;
 }
 
