@@ -1910,10 +1910,11 @@ sop_status sop_run_plain(sop_engine *e, const int32_t *sys, int32_t nsys, int64_
     HIPCK(launch_begin(e->p, nsteps, e->stream));
     st = engine_run_hostloop(e, nsteps);
     if (st) return st;
+    if (nsteps == 0) HIPCK(launch_report(e->p, e->stream));  // no k_advance to report the state as it is now
     mirror_advance(e, &sys[q], 1, nsteps);
   }
   HIPCK(hipStreamSynchronize(e->stream));
-  for (int q = 0; q < nsys; ++q) {  // as k_advance reported them
+  for (int q = 0; q < nsys; ++q) {  // as k_advance or k_report left them
     st = engine_error_status(e, sys[q], e->p.rep[sys[q]].x);
     if (st) return st;
   }
