@@ -919,9 +919,8 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   // staged beads}.  Systems that fit the LDS budget are staged whole:
   // arena-adjacent small systems share an item (one staged range), a larger
   // system gets one item per `per` tiles, each staging the whole system.
-  // Larger systems gather from global memory and keep their items on one XCD
-  // (runs of one XCD's share on several XCDs when they have more items than
-  // that).  The shell filter takes one wave per tile, STEP_WAVES tiles per item.
+  // Larger systems gather from global memory, their items in equal runs over the
+  // XCDs.  The shell filter takes one wave per tile, STEP_WAVES tiles per item.
   // The step kernel's items hold `per` tiles and run each tile on
   // min(lanes_per_bead, STEP_WAVES / tiles) waves (power of two), each wave
   // taking that share of the tile's rounds: an item's duration shrinks with
@@ -999,13 +998,23 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     int32_t n_lds = 0, n_big = 0, n_far = 0;
     size_t lds = 0, lds_big = 0;
   };
-  // tiles per item of the global-gather systems: one item per compute unit, of
-  // 4 to 16 tiles (a wave's share of a tile repeats the tile's chain terms and
-  // noise, and a second item on some of the units lasts as long as on all).
-  // Step times for chains of 500 beads by items of 4 / 8 / 16 tiles (us):
-  // 200,000 beads 53.6 / 42.8 / 36.2, by this rule (13) 34.2; 100,000 beads
-  // 26.9 / 21.8 / 34.0, by this rule (7) 21.2
-  const int32_t per_far = (int32_t)std::clamp<int64_t>((far_tiles + e->num_cu - 1) / e->num_cu, 4, STEP_WAVES);
+  // tiles per item of the global-gather systems: the fewest, 4 to 16, with at
+  // most one item per compute unit (a wave's share of a tile repeats the tile's
+  // chain terms and noise, and a second item on some of the units lasts as long
+  // as on all).  Counted system by system: 200 systems of 16 tiles are 200
+  // items of 16 tiles, and 400 of the 13 that their tiles over the units come
+  // to (run 52.9 and 74.2 us per step).  Run per step for chains of 500 beads
+  // by items of 4 / 8 / 16 tiles (us): 200,000 beads 56.5 / 49.4 / 46.0, by this
+  // rule (13) 42.8; 100,000 beads 33.2 / 29.8 / 41.8, by this rule (7) 27.7.
+  int32_t per_far = 4;
+  for (; per_far < STEP_WAVES; ++per_far) {
+    int64_t items = 0;
+    for (int32_t q = 0; q < nslots; ++q) {
+      const int64_t len = e->sys[slots[q]].bead_len;
+      if (len > lds_cap && len > big_cap) items += (len / TILE + per_far - 1) / per_far;
+    }
+    if (items <= e->num_cu) break;
+  }
   // in a mixed launch the fewest of 4, 8 or 16 tiles with which all items are
   // resident at once, two per unit (the batch's item size instead: 60 systems
   // of 1,500 beads and 3 of 18,000 60.8 us per step against 49.4, 120 and 8
@@ -1076,10 +1085,9 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     }
     flush();
     // XCD bins by load (item k runs on XCD k mod 8): the LDS items, longest
-    // first (an item lasts about one tile's rounds / its waves per tile), then
-    // whole non-LDS systems (largest first) so each keeps its gathers in one L2
+    // first (an item lasts about one tile's rounds / its waves per tile)
     std::vector<std::vector<int4>> ibins(NX), bbins(NX), fbins(NX);
-    std::vector<double> iload(NX, 0), bload(NX, 0), fload(NX, 0);
+    std::vector<double> iload(NX, 0), bload(NX, 0);
     auto by_dur = [&](const int4 &u, const int4 &v) {
       const double du = 1.0 / item_split(u.y), dv = 1.0 / item_split(v.y);
       return du != dv ? du > dv : item_tiles(u.y) > item_tiles(v.y);
@@ -1138,24 +1146,19 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     std::sort(far_items.begin(), far_items.end(), [](const std::vector<int4> &u, const std::vector<int4> &v) {
       return u.size() != v.size() ? u.size() > v.size() : u[0].x < v[0].x;
     });
-    // a system with more items than an XCD's share of them all (at most its
-    // share of the launch's two blocks per compute unit) goes out in contiguous
-    // runs of that share, each run to the least-loaded XCD: so large a system
-    // outgrows one L2 anyway.  (Runs of the launch's share alone: 391 items
-    // filled six XCDs and left one nearly idle and one idle; the shell filter's
-    // 196 filled three and took 124 us instead of 67.)
+    // the global-gather items, system after system, in equal contiguous runs,
+    // one per XCD: a system's items stay on one XCD or on neighbouring runs, and
+    // no XCD holds a second round of items while another has units free.  Step
+    // times with each system whole on the least-loaded XCD, and now (us): 6
+    // systems of 30,000 beads 57.5, 44.5; 14 of 16,000 57.6, 49.8; 3 of 60,000
+    // 63.2, 48.1 (with runs of at most an eighth of the items, each to the
+    // least-loaded XCD, which left two runs on some: 67.8, 73.1 and 73.2)
     size_t n_far = 0;
     for (const auto &v : far_items) n_far += v.size();
-    const size_t share = std::max<size_t>(1, std::min<size_t>(2 * e->num_cu / NX, (n_far + NX - 1) / NX));
-    for (const auto &v : far_items) {
-      for (size_t k0 = 0; k0 < v.size(); k0 += share) {
-        const int x = (int)(std::min_element(fload.begin(), fload.end()) - fload.begin());
-        for (size_t k = k0; k < std::min(v.size(), k0 + share); ++k) {
-          fbins[x].push_back(v[k]);
-          fload[x] += (double)item_tiles(v[k].y);
-        }
-      }
-    }
+    const size_t share = (n_far + NX - 1) / NX;
+    size_t k_far = 0;
+    for (const auto &v : far_items)
+      for (const int4 &it : v) fbins[k_far++ / share].push_back(it);
     size_t imx = 0, bmx = 0, fmx = 0;
     for (auto &bn : ibins) imx = std::max(imx, bn.size());
     for (auto &bn : bbins) bmx = std::max(bmx, bn.size());
