@@ -526,33 +526,30 @@ sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, in
     st = off < 0 ? SOP_ERR_BUSY : SOP_OK;
     return off;
   };
-  h.bead_off = alloc(e->a_beads, h.bead_len, TILE, 0);
-  if (st) return st;
-  h.nat_off = alloc(e->a_nat, h.nat_len, 1, 1);
-  if (st) { e->a_beads.release(h.bead_off, h.bead_len); return st; }
-  if ((h.nat_off + h.nat_len) * 8 > (int64_t)0xFFFFFFFF) {  // 32-bit byte offsets of the native pair list
-    e->a_beads.release(h.bead_off, h.bead_len); e->a_nat.release(h.nat_off, h.nat_len);
-    return set_error(e, SOP_ERR_CAPACITY, "native pool beyond 4 GiB");
-  }
-  h.nl_off = 0;
-  h.pl_off = alloc(e->a_pl, h.pl_len, 16, 3);
-  if (st) { e->a_beads.release(h.bead_off, h.bead_len); e->a_nat.release(h.nat_off, h.nat_len); return st; }
-  h.cell_off = alloc(e->a_cells, h.cell_len, 1, 4);
-  if (st) {
-    e->a_beads.release(h.bead_off, h.bead_len); e->a_nat.release(h.nat_off, h.nat_len);
-    e->a_pl.release(h.pl_off, h.pl_len);
+  // ranges taken so far, given back by every return before the system exists
+  struct Held {
+    std::vector<std::pair<RangeAlloc *, std::pair<int64_t, int64_t>>> ranges;
+    ~Held() {
+      for (const auto &r : ranges) r.first->release(r.second.first, r.second.second);
+    }
+  } held;
+  auto take = [&](RangeAlloc &a, int64_t len, int64_t align, int which, int64_t &off) {
+    off = alloc(a, len, align, which);
+    if (!st) held.ranges.push_back({&a, {off, len}});
     return st;
-  }
+  };
+  if (take(e->a_beads, h.bead_len, TILE, 0, h.bead_off)) return st;
+  if (take(e->a_nat, h.nat_len, 1, 1, h.nat_off)) return st;
+  if ((h.nat_off + h.nat_len) * 8 > (int64_t)0xFFFFFFFF)  // 32-bit byte offsets of the native pair list
+    return set_error(e, SOP_ERR_CAPACITY, "native pool beyond 4 GiB");
+  h.nl_off = 0;
+  if (take(e->a_pl, h.pl_len, 16, 3, h.pl_off)) return st;
+  if (take(e->a_cells, h.cell_len, 1, 4, h.cell_off)) return st;
   // slot
   int32_t slot = -1;
   for (size_t s = 0; s < e->sys.size(); ++s)
     if (!e->sys[s].used) { slot = (int32_t)s; break; }
-  if (slot < 0 && up) {
-    e->a_beads.release(h.bead_off, h.bead_len); e->a_nat.release(h.nat_off, h.nat_len);
-    e->a_pl.release(h.pl_off, h.pl_len);
-    e->a_cells.release(h.cell_off, h.cell_len);
-    return SOP_ERR_BUSY;
-  }
+  if (slot < 0 && up) return SOP_ERR_BUSY;
   if (slot < 0) {
     if (e->fixed_pools && (int64_t)e->sys.size() >= e->cap.slots && e->cap.slots > 0) {
       slot = -1;
@@ -692,6 +689,7 @@ sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, in
   up_a.has_vel = d->vel ? 1 : 0;
   HIPCK(launch_add_system(e->p, up_a, up ? up : e->stream));
   if (up) upl->used += (stage_need + 255) / 256 * 256;
+  held.ranges.clear();  // the system's own from here on
   e->sys[slot] = std::move(h);
   *slot_out = slot;
   return SOP_OK;
