@@ -22,7 +22,7 @@ using namespace sopk;
 
 struct sop_engine::Job {
   int64_t id = 0;
-  std::vector<float> xyz, bond_r0, nat_r0;
+  std::vector<float> xyz, bond_r0, nat_r0, vel;
   std::vector<int32_t> chain, type, nat_i, nat_j;
   sop_system_desc desc{};
   int64_t nsteps = 0;
@@ -387,6 +387,7 @@ sop_status sop_serve_submit(sop_engine *e, const sop_system_desc *d, int64_t nst
   if (d->chain) j->chain.assign(d->chain, d->chain + n);
   if (d->type) j->type.assign(d->type, d->type + n);
   if (d->bond_r0) j->bond_r0.assign(d->bond_r0, d->bond_r0 + n);
+  if (d->vel) j->vel.assign(d->vel, d->vel + 3 * (size_t)n);
   if (m > 0) {
     j->nat_i.assign(d->nat_i, d->nat_i + m);
     j->nat_j.assign(d->nat_j, d->nat_j + m);
@@ -400,6 +401,7 @@ sop_status sop_serve_submit(sop_engine *e, const sop_system_desc *d, int64_t nst
   j->desc.nat_i = m > 0 ? j->nat_i.data() : nullptr;
   j->desc.nat_j = m > 0 ? j->nat_j.data() : nullptr;
   j->desc.nat_r0 = m > 0 ? j->nat_r0.data() : nullptr;
+  j->desc.vel = d->vel ? j->vel.data() : nullptr;
   j->nsteps = nsteps;
   j->bytes = job_bytes_estimate(e, d);
   j->t_submit = sop_clock_seconds();
