@@ -187,7 +187,7 @@ static void bind_arrays(sop_engine *e) {
       {(void **)&p.platt_cnt, 4},  {(void **)&p.nlrep_cnt, 4},   {(void **)&p.plrep_cnt, 4},
       {(void **)&p.cell_of, 4},    {(void **)&p.cell_tmp, 4},    {(void **)&p.cell_sorted, 4},
       {(void **)&p.cell_pos, 4},   {(void **)&p.nat_sorted, 8},
-      {(void **)&p.fout, 16},      {(void **)&p.epart, 8 * EPART_N}, {(void **)&p.vel, 16},
+      {(void **)&p.fout, 16},      {(void **)&p.vel, 16},
       {(void **)&p.tile_ord, 1},   {(void **)&p.slrep_cnt, 4},   {(void **)&p.pos_shell, 16},
       {(void **)&p.plrep_off, 4},  {(void **)&p.platt_off, 4},  {(void **)&p.plhead, 8}};
   e->nat_arrays = {{(void **)&p.nat_j, 4},    {(void **)&p.nat_r0, 4},  {(void **)&p.nlatt_j, 4},
@@ -243,6 +243,8 @@ static sop_status ensure_capacity(sop_engine *e, int64_t beads, int64_t nat, int
       if (s) return s;
     }
     sop_status s = grow_array(e, (void **)&e->p.tile_sys, 4 * (size_t)(c.beads / TILE), 4 * (size_t)(nb / TILE));
+    if (s) return s;
+    s = grow_array(e, (void **)&e->p.epart, 0, 8 * TPART_N * (size_t)(nb / TILE));  // scratch of a call
     if (s) return s;
     e->a_beads.grow(nb);
     c.beads = nb;
@@ -391,19 +393,24 @@ sop_status engine_read_sys(sop_engine *e, int32_t slot, SysDev *out) {
   return SOP_OK;
 }
 
+// Pool bytes of `beads` beads (whole tiles) and `cells` cells: the per-bead and
+// per-cell arrays, and a tile's system slot and energy partials.
+static int64_t pool_bytes(const sop_engine *e, int64_t beads, int64_t cells) {
+  int64_t per_bead = 0, per_cell = 0;
+  for (const auto &a : e->bead_arrays) per_bead += (int64_t)a.second;
+  for (const auto &a : e->cell_arrays) per_cell += (int64_t)a.second;
+  return beads * per_bead + beads / TILE * (4 + 8 * TPART_N) + cells * per_cell;
+}
+
 int64_t job_bytes_estimate(const sop_engine *e, const sop_system_desc *d) {
   const int64_t n = d->n_beads;
   const int64_t pl_cap = pl_cap_start(e, d->n_beads);
   const int64_t beads = (n + TILE - 1) / TILE * TILE;
   const int64_t cell_cap = std::min<int64_t>(e->opts.cell_cap_max, std::max<int64_t>(64, 2 * n)) + 1;
-  int64_t per_bead = 4;  // tile table share
-  for (const auto &a : e->bead_arrays) per_bead += (int64_t)a.second;
   // pair-list and shell-row segments (16-bit entries up to 65,536 beads); the
   // neighbor list is materialized only on request, in a scratch segment
   const int64_t esz = n <= 65536 ? 2 : 4;
-  int64_t per_cell = 0;
-  for (const auto &a : e->cell_arrays) per_cell += (int64_t)a.second;
-  return beads * per_bead + 24 * 2 * (int64_t)d->n_native + 2 * esz * n * pl_cap + per_cell * cell_cap;
+  return pool_bytes(e, beads, cell_cap) + 24 * 2 * (int64_t)d->n_native + 2 * esz * n * pl_cap;
 }
 
 sop_status upload_drain(sop_engine *e, Upload *upl) {
@@ -704,11 +711,7 @@ static sop_status read_sys_all(sop_engine *e, std::vector<SysDev> &sd) {
 // Resident bytes of one system (what job_bytes_estimate predicts for it).
 int64_t engine_system_bytes(const sop_engine *e, int32_t slot) {
   const SysHost &h = e->sys[slot];
-  int64_t per_bead = 4;  // tile table share
-  for (const auto &a : e->bead_arrays) per_bead += (int64_t)a.second;
-  int64_t per_cell = 0;
-  for (const auto &a : e->cell_arrays) per_cell += (int64_t)a.second;
-  return h.bead_len * per_bead + 24 * 2 * (int64_t)h.n_nat + 2 * 4 * h.pl_len + per_cell * h.cell_len;
+  return pool_bytes(e, h.bead_len, h.cell_len) + 24 * 2 * (int64_t)h.n_nat + 2 * 4 * h.pl_len;
 }
 
 // Move one system's shell rows and pair-list tiles to a segment of row
@@ -1623,7 +1626,7 @@ void sop_engine_destroy(sop_engine *e) {
   for (auto &a : e->cell_arrays) if (*a.first) note(hipFree(*a.first), "hipFree(cell pool)");
   void *others[] = {e->p.nlrep_j, e->p.plrep_j, e->p.slrep_j,  e->p.tile_sys, e->p.sys,  e->p.sysout,
                     e->p.syslist, e->p.work,    e->p.nwork,    e->p.items,
-                    e->p.tiles};
+                    e->p.tiles,   e->p.epart};
   for (void *q : others) if (q) note(hipFree(q), "hipFree");
   for (void *q : {e->io.ptr, e->stage.ptr, (void *)e->p.rep}) if (q) note(hipHostFree(q), "hipHostFree");
   if (e->p.fitems) note(hipFree(e->p.fitems), "hipFree");

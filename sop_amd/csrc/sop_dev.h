@@ -248,8 +248,7 @@ __host__ __device__ inline int item_split(int y) { return y >> 8; }
 constexpr int SORT_N_MAX = 5120;
 constexpr int SORT_C_MAX = 2 * SORT_N_MAX;
 
-constexpr int EPART_N = 6;   // bond, angle, native, rep, virial, contacts
-constexpr int TPART_N = 10;  // per tile: the EPART_N sums, then sum x, y, z, |r|^2 of its beads
+constexpr int TPART_N = 10;  // per tile: bond, angle, native, rep, virial, contacts, then sum x, y, z, |r|^2 of its beads
 constexpr int SYSOUT_N = 16; // e[0..5], contacts, rgsq, sum x,y,z, n
 
 // Scratch of the allocation-free energy entry point: one system of up to
