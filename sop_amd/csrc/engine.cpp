@@ -210,7 +210,8 @@ namespace sopk {
 sop_status engine_io(sop_engine *e, HostBuf &b, size_t bytes) {
   if (b.bytes >= bytes) return SOP_OK;
   HIPCK(hipStreamSynchronize(e->stream));
-  const size_t nb = std::max<size_t>(bytes + bytes / 2, (size_t)64 << 10);
+  const size_t half = std::min(bytes / 2, (size_t)16 << 20);  // room for somewhat larger calls
+  const size_t nb = std::max<size_t>(bytes + half, (size_t)64 << 10);
   void *q = nullptr;
   HIPCK(hipHostMalloc(&q, nb, hipHostMallocDefault));
   if (b.ptr) (void)hipHostFree(b.ptr);
@@ -1271,6 +1272,12 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   size_t words = 0;
   for (const auto &q : parts) words += q.second.second;
   HIPCK(hipStreamSynchronize(e->stream));  // the launch that read the last tables has passed
+  // room for a large system's upload, which the tables need none of, is given back
+  constexpr size_t STAGE_KEEP = (size_t)96 << 20;
+  if (e->stage.bytes > STAGE_KEEP && 4 * words <= STAGE_KEEP) {
+    (void)hipHostFree(e->stage.ptr);
+    e->stage = HostBuf();
+  }
   sop_status st = engine_io(e, e->stage, 4 * words);
   if (st) return st;
   TableParts tp;
@@ -1724,22 +1731,28 @@ sop_status sop_get_list(sop_engine *e, int32_t sys, int32_t which, int32_t *ij, 
   const int32_t nb = e->sys[sys].n;
   // pairs go through the host buffer a window at a time, the total behind it;
   // the first window is written before the total is known, with one wait for
-  // both (two updates and the four lists of 1,500 beads, counted and then
-  // fetched: 270 us with a wait for each, 246 with one)
-  constexpr int64_t WINDOW = (int64_t)4 << 20;
-  const int64_t room = ij ? std::max<int64_t>(cap, 0) : 0, m0 = std::min(room, WINDOW);
-  if ((st = engine_io(e, e->io, 8 * (size_t)(m0 + 1)))) return st;
-  int2 *const pairs = static_cast<int2 *>(e->io.ptr);
-  int64_t *const total = static_cast<int64_t *>(e->io.ptr) + m0;
-  for (int64_t lo = 0;; lo += m0) {
-    HIPCK(launch_list_places(e->p, sys, nb, which, lo, total, e->stream));
-    if (m0 > 0) HIPCK(launch_list_write(e->p, sys, nb, which, pairs, (int)std::min(m0, room - lo), e->stream));
+  // both, and is what the buffer holds (at least FIRST pairs): a caller's array
+  // may be far longer than the list, and pinned memory for all of it costs 0.3
+  // ms a MiB.  Later windows, for which the buffer grows, hold up to WINDOW
+  constexpr int64_t WINDOW = (int64_t)4 << 20, FIRST = (int64_t)64 << 10;
+  const int64_t room = ij ? std::max<int64_t>(cap, 0) : 0;
+  int64_t m = std::min(room, std::clamp<int64_t>((int64_t)(e->io.bytes / 8) - 1, FIRST, WINDOW));
+  int64_t total = 0;
+  for (int64_t lo = 0;;) {
+    if ((st = engine_io(e, e->io, 8 * (size_t)(m + 1)))) return st;
+    int2 *const pairs = static_cast<int2 *>(e->io.ptr);
+    int64_t *const count = static_cast<int64_t *>(e->io.ptr) + m;
+    HIPCK(launch_list_places(e->p, sys, nb, which, lo, count, e->stream));
+    if (m > 0) HIPCK(launch_list_write(e->p, sys, nb, which, pairs, (int)m, e->stream));
     HIPCK(hipStreamSynchronize(e->stream));
-    const int64_t want = std::min(*total, room);
-    if (want > lo) std::memcpy(ij + 2 * lo, pairs, 8 * (size_t)std::min(m0, want - lo));
-    if (want <= lo + m0) break;
+    total = *count;
+    const int64_t want = std::min(total, room);
+    if (want > lo) std::memcpy(ij + 2 * lo, pairs, 8 * (size_t)std::min(m, want - lo));
+    lo += m;
+    if (lo >= want) break;
+    m = std::min(want - lo, WINDOW);
   }
-  *n = *total;
+  *n = total;
   return SOP_OK;
 }
 
