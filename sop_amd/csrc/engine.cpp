@@ -921,7 +921,7 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   // staged beads}.  Systems that fit the LDS budget are staged whole:
   // arena-adjacent small systems share an item (one staged range), a larger
   // system gets one item per `per` tiles, each staging the whole system.
-  // Larger systems gather from global memory, their items in equal runs over the
+  // Larger systems gather from global memory, their items in runs over all
   // XCDs.  The shell filter takes one wave per tile, STEP_WAVES tiles per item.
   // The step kernel's items hold `per` tiles and run each tile on
   // min(lanes_per_bead, STEP_WAVES / tiles) waves (power of two), each wave
@@ -1148,19 +1148,26 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
     std::sort(far_items.begin(), far_items.end(), [](const std::vector<int4> &u, const std::vector<int4> &v) {
       return u.size() != v.size() ? u.size() > v.size() : u[0].x < v[0].x;
     });
-    // the global-gather items, system after system, in equal contiguous runs,
-    // one per XCD: a system's items stay on one XCD or on neighbouring runs, and
-    // no XCD holds a second round of items while another has units free.  Step
-    // times with each system whole on the least-loaded XCD, and now (us): 6
-    // systems of 30,000 beads 57.5, 44.5; 14 of 16,000 57.6, 49.8; 3 of 60,000
-    // 63.2, 48.1 (with runs of at most an eighth of the items, each to the
-    // least-loaded XCD, which left two runs on some: 67.8, 73.1 and 73.2)
+    // the global-gather items: each system's in contiguous runs of at most an
+    // eighth of all items, to the XCD with the fewest, and no more to any than it
+    // takes in as many rounds as all need, so that none holds a second round of
+    // items while another has units free.  Step times
+    // with each system whole on the least-loaded XCD, and now (us): 6 systems of
+    // 30,000 beads 57.5, 44.5; 14 of 16,000 57.6, 49.8; 3 of 60,000 63.2, 48.1
+    // (runs of at most an eighth, each whole to the least-loaded XCD, left two
+    // on some: 67.8, 73.1 and 73.2)
     size_t n_far = 0;
     for (const auto &v : far_items) n_far += v.size();
-    const size_t share = (n_far + NX - 1) / NX;
-    size_t k_far = 0;
+    const size_t units = (size_t)std::max(1, e->num_cu / NX), share = (n_far + NX - 1) / NX;
+    const size_t most = share <= units ? share : (share + units - 1) / units * units;
     for (const auto &v : far_items)
-      for (const int4 &it : v) fbins[k_far++ / share].push_back(it);
+      for (size_t k = 0; k < v.size();) {
+        auto &bn = *std::min_element(fbins.begin(), fbins.end(),
+                                     [](const auto &u, const auto &w) { return u.size() < w.size(); });
+        const size_t run = std::min({v.size() - k, share, most - bn.size()});
+        bn.insert(bn.end(), v.begin() + k, v.begin() + k + run);
+        k += run;
+      }
     size_t imx = 0, bmx = 0, fmx = 0;
     for (auto &bn : ibins) imx = std::max(imx, bn.size());
     for (auto &bn : bbins) bmx = std::max(bmx, bn.size());

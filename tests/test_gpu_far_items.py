@@ -31,3 +31,18 @@ def test_gathered_systems_together_equal_alone(sizes, options):
             assert np.array_equal(a.coords(ia[k]), b.coords(ib)), sizes[k]
             assert np.array_equal(a.force_eval(ia[k]), b.force_eval(ib)), sizes[k]
             b.remove(ib)
+
+
+def test_a_large_system_beside_many():
+    # more items than units: the large system's runs fill some XCDs, the others
+    # go whole to the rest
+    sizes = [66000] + [8000 + 100 * k for k in range(12)] + [11000, 25000, 30000]
+    systems = [S.make_chain_system(380 + k, n) for k, n in enumerate(sizes)]
+    with S.Engine(0, lds_beads_max=-1) as a, S.Engine(0) as b:
+        ia = [a.add(s) for s in systems]
+        a.run(ia, 20)
+        for k in (0, 1, 12, 14, 15):
+            ib = b.add(systems[k])
+            b.run([ib], 20)
+            assert np.array_equal(a.coords(ia[k]), b.coords(ib)), sizes[k]
+            b.remove(ib)
