@@ -875,7 +875,6 @@ __device__ __forceinline__ bool native_pair(const int32_t *nj, int nn, int j) {
 // (local index mod 65536); a set bit is confirmed by the exact search unless
 // the system is small enough for the key to be the index itself.
 constexpr int NATBITS_WORDS = 2048;
-constexpr int NLB_BEADS = 1;  // beads of a wave's unit in neighbor-list builds
 
 __device__ __forceinline__ void natbits_mark(uint32_t *bits, const int32_t *natj, int nn, int bead_off, bool set) {
   const int lane = threadIdx.x & 63;
@@ -1257,13 +1256,12 @@ __device__ __forceinline__ void nl_build(const DevPtrs &p, int kstep, char *s_ra
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int k = lane; k < NATBITS_WORDS; k += 64) s_bits[wave][k] = 0u;
   __builtin_amdgcn_wave_barrier();
-  // units of NLB_BEADS beads: a wave scans a bead's 27 cells one load batch
-  // after another, so the beads go out over as many waves as the launch has
-  // (a wave took sixteen: 860 us for the neighbor list of 5,000 beads)
-  constexpr int UNITS = TILE / NLB_BEADS;
-  const int nunit = *p.nwork * UNITS;
-  for (int w = blockIdx.x * 4 + wave; w < nunit; w += gridDim.x * 4) {
-    const int t = sload(p.work + w / UNITS);
+  // a wave scans a bead's 27 cells one load batch after another, so the beads
+  // go out over as many waves as the launch has (a wave took sixteen: 860 us for
+  // the neighbor list of 5,000 beads)
+  const int nbead = *p.nwork * TILE;
+  for (int w = blockIdx.x * 4 + wave; w < nbead; w += gridDim.x * 4) {
+    const int t = sload(p.work + w / TILE);
     if (t < 0) continue;
     const int s = sload(p.tile_sys + t);
     SysConst &S = sys_const(p, s);
@@ -1273,80 +1271,78 @@ __device__ __forceinline__ void nl_build(const DevPtrs &p, int kstep, char *s_ra
     const float4 *pin = buf_in(p, S.parity + kstep);
     const float boxl = S.boxl;
     const int bend = min(t * TILE + TILE, S.bead_off + S.n);
-    for (int q = 0; q < NLB_BEADS; ++q) {
-      const int i = t * TILE + (w % UNITS) * NLB_BEADS + q;
-      if (i >= bend) break;
-      const float4 xi = ref[i];
-      const float4 xn = pin[i];
-      const int ti = __float_as_int(xi.w) & 3;
-      const int ns = p.nat_start[i], nn = p.nat_cnt[i];
-      int cnt = 0;
-      for (int k0 = 0; k0 < nn; k0 += 64) {
-        const int k = k0 + lane;
-        bool pred = false;
-        int j = 0;
-        float r0 = 0.0f;
-        if (k < nn) {
-          j = p.nat_j[ns + k];
-          r0 = p.nat_r0[ns + k];
-          const float rc = cutoff_of(S.nl_factor, S.nl_abs, r0);
-          pred = dist2_exact(xi, ref[j], boxl) < rc * rc;
-          if (plb && pred) {
-            const float rp = cutoff_of(S.pl_factor, S.pl_abs, r0);
-            pred = dist2_exact(xn, pin[j], boxl) < rp * rp;
-          }
+    const int i = t * TILE + w % TILE;
+    if (i >= bend) continue;
+    const float4 xi = ref[i];
+    const float4 xn = pin[i];
+    const int ti = __float_as_int(xi.w) & 3;
+    const int ns = p.nat_start[i], nn = p.nat_cnt[i];
+    int cnt = 0;
+    for (int k0 = 0; k0 < nn; k0 += 64) {
+      const int k = k0 + lane;
+      bool pred = false;
+      int j = 0;
+      float r0 = 0.0f;
+      if (k < nn) {
+        j = p.nat_j[ns + k];
+        r0 = p.nat_r0[ns + k];
+        const float rc = cutoff_of(S.nl_factor, S.nl_abs, r0);
+        pred = dist2_exact(xi, ref[j], boxl) < rc * rc;
+        if (plb && pred) {
+          const float rp = cutoff_of(S.pl_factor, S.pl_abs, r0);
+          pred = dist2_exact(xn, pin[j], boxl) < rp * rp;
         }
-        const uint64_t m = __ballot(pred);
-        if (pred) {
-          const int o = ns + cnt + lanes_below(m);
-          if (plb) {
-            p.platt[o] = make_int2(j, __float_as_int(r0));
-          } else {
-            p.nlatt_j[o] = j;
-            p.nlatt_r0[o] = r0;
-          }
-        }
-        cnt += __popcll(m);
       }
-      const float rcA = S.rc2_nl_rep[(ti - 1) * 2], rcB = S.rc2_nl_rep[(ti - 1) * 2 + 1];
-      if (plb) {
-        if (lane == 0) {
-          p.platt_cnt[i] = cnt;
-          p.platt_off[i] = ns;  // in the bead's own native slots
+      const uint64_t m = __ballot(pred);
+      if (pred) {
+        const int o = ns + cnt + lanes_below(m);
+        if (plb) {
+          p.platt[o] = make_int2(j, __float_as_int(r0));
+        } else {
+          p.nlatt_j[o] = j;
+          p.nlatt_r0[o] = r0;
         }
-        const float pA = S.rc2_pl_rep[(ti - 1) * 2], pB = S.rc2_pl_rep[(ti - 1) * 2 + 1];
-        const int64_t row = (int64_t)(i - S.bead_off) * S.pl_cap;  // the bead's shell-row slot
-        uint16_t *r16 = (uint16_t *)(p.slrep_j + S.pl_base) + row;
-        int32_t *r32 = p.slrep_j + S.pl_base + row;
-        const int cap = S.pl_cap, bo = S.bead_off;
-        const bool i16 = S.idx16 != 0;
-        const int cr = scan_cells(
-            p, S, i, xi, rcA, rcB, ns, nn, s_bits[wave],
-            [&](int j, int wj) { return dist2_exact(xn, pin[j], boxl) < ((wj & 3) == 2 ? pB : pA); },
-            [&](int o, int j) {
-              if (o < cap) {
-                if (i16) r16[o] = (uint16_t)(j - bo);
-                else r32[o] = j;
-              }
-            });
-        if (lane == 0) {
-          p.slrep_cnt[i] = min(cr, cap);
-          if (cr > cap) atomicOr(&p.sys[s].err, ERR_PL_OVF);
-          atomicMax(&p.sys[s].row_max, cr);
-        }
-      } else {
-        if (lane == 0) p.nlatt_cnt[i] = cnt;
-        int32_t *out = p.nlrep_j + S.nl_base + (int64_t)(i - S.bead_off) * S.nl_cap;
-        const int cap = S.nl_cap;
-        const int cr = scan_cells(p, S, i, xi, rcA, rcB, ns, nn, s_bits[wave], [](int, int) { return true; },
-                                  [&](int o, int j) {
-                                    if (o < cap) out[o] = j;
-                                  });
-        if (lane == 0) {
-          p.nlrep_cnt[i] = min(cr, cap);
-          if (cr > cap) atomicOr(&p.sys[s].err, ERR_NL_OVF);
-          p.sys[s].nl_valid = 1;
-        }
+      }
+      cnt += __popcll(m);
+    }
+    const float rcA = S.rc2_nl_rep[(ti - 1) * 2], rcB = S.rc2_nl_rep[(ti - 1) * 2 + 1];
+    if (plb) {
+      if (lane == 0) {
+        p.platt_cnt[i] = cnt;
+        p.platt_off[i] = ns;  // in the bead's own native slots
+      }
+      const float pA = S.rc2_pl_rep[(ti - 1) * 2], pB = S.rc2_pl_rep[(ti - 1) * 2 + 1];
+      const int64_t row = (int64_t)(i - S.bead_off) * S.pl_cap;  // the bead's shell-row slot
+      uint16_t *r16 = (uint16_t *)(p.slrep_j + S.pl_base) + row;
+      int32_t *r32 = p.slrep_j + S.pl_base + row;
+      const int cap = S.pl_cap, bo = S.bead_off;
+      const bool i16 = S.idx16 != 0;
+      const int cr = scan_cells(
+          p, S, i, xi, rcA, rcB, ns, nn, s_bits[wave],
+          [&](int j, int wj) { return dist2_exact(xn, pin[j], boxl) < ((wj & 3) == 2 ? pB : pA); },
+          [&](int o, int j) {
+            if (o < cap) {
+              if (i16) r16[o] = (uint16_t)(j - bo);
+              else r32[o] = j;
+            }
+          });
+      if (lane == 0) {
+        p.slrep_cnt[i] = min(cr, cap);
+        if (cr > cap) atomicOr(&p.sys[s].err, ERR_PL_OVF);
+        atomicMax(&p.sys[s].row_max, cr);
+      }
+    } else {
+      if (lane == 0) p.nlatt_cnt[i] = cnt;
+      int32_t *out = p.nlrep_j + S.nl_base + (int64_t)(i - S.bead_off) * S.nl_cap;
+      const int cap = S.nl_cap;
+      const int cr = scan_cells(p, S, i, xi, rcA, rcB, ns, nn, s_bits[wave], [](int, int) { return true; },
+                                [&](int o, int j) {
+                                  if (o < cap) out[o] = j;
+                                });
+      if (lane == 0) {
+        p.nlrep_cnt[i] = min(cr, cap);
+        if (cr > cap) atomicOr(&p.sys[s].err, ERR_NL_OVF);
+        p.sys[s].nl_valid = 1;
       }
     }
   }
