@@ -89,8 +89,8 @@ int grid_sys(const sop_engine *e) {
   return std::max(1, std::min(e->cur_nsys, 2048));
 }
 
-// k_rebuild: a block per system of up to SORT_N_MAX beads (two are resident
-// per compute unit)
+// k_rebuild: a block per system of up to SORT_N_MAX beads (one that sorts is
+// resident per compute unit, two that only decide)
 static int grid_rebuild(const sop_engine *e) {
   if (e->fixed_grids) return 2 * e->num_cu;
   return std::min(e->cur_nsys - e->cur_nbig, 2048);
@@ -139,9 +139,10 @@ int grid_items(const sop_engine *e) {
                     e->cur_nitems + (e->cur_mixed ? e->cur_nitems_far : 0));
 }
 
-// A block per tile; while serving a fixed grid whenever the batch has such
-// tiles (three blocks are resident per compute unit).
 int grid_items_far(const sop_engine *e) { return items_grid(2 * e->num_cu, e->fixed_grids, e->cur_nitems_far); }
+// A block per tile; while serving a fixed grid whenever the batch has such
+// tiles (two five-wave blocks of k_step_tile are resident per compute unit, one
+// of nine waves, one of k_filter_tile; a block takes the rest in turn).
 int grid_step_tiles(const sop_engine *e) {
   if (e->cur_ntiles == 0) return 0;
   return e->fixed_grids ? 4 * e->num_cu : e->cur_ntiles;
@@ -964,11 +965,13 @@ sop_status engine_set_batch(sop_engine *e, const int32_t *slots, int32_t nslots)
   // TILE_STEP_PER_CU tiles per compute unit; else the systems too large for
   // two LDS blocks per unit while theirs are that few, and the ones too large
   // for any LDS tier up to TILE_STEP_FAR_PER_CU.  Step times by tile against
-  // the other kernel (us): 2 x 8,000 beads 8.2 / 13.8 whole-CU, 6 x 8,000
-  // 17.9 / 14.4; 32 x 4,000 and 4 x 8,000 together 34.8 / 40.8; 12 x 4,000
-  // 14.0 / 12.9 LDS; against global-gather items, step and run per step:
-  // 20,000 beads 12.7 and 18.6 / 17.8 and 29.2, 45,000 19.2 and 29.1 / 18.8 and
-  // 31.8, 65,000 27.0 and 39.8 / 20.0 and 34.5.
+  // the other kernel (us), on either side of the lines: 2 x 8,000 beads 7.7 /
+  // 13.7 whole-CU, 4 x 8,000 12.6 / 14.1, 6 x 8,000 17.0 / 14.3; 8 x 4,000 11.2 /
+  // 12.7 LDS, 12 x 4,000 16.4 / 13.0; 32 x 4,000 and 4 x 8,000 together 33.5 /
+  // 40.3.  Against global-gather items, step, and run per step with its rebuilds:
+  // 20,000 beads 11.7, 16.8 / 17.2, 24.8; 45,000 17.1, 26.1 / 18.3, 27.8; 60,000
+  // 21.8, 32.8 / 18.7, 28.4; chains of 500 together, 40,000 13.2, 18.7 / 13.3,
+  // 19.2; 60,000 17.1, 24.2 / 13.5, 19.4.
   const int64_t tile_cap = (int64_t)TILE_STEP_PER_CU * e->num_cu;
   int64_t mid_tiles = 0, far_tiles = 0;
   for (int32_t q = 0; q < nslots; ++q) {

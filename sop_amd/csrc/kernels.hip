@@ -357,22 +357,6 @@ __device__ __forceinline__ int plan_grid(SysDev &S, const float *mn, const float
   return nc;
 }
 
-// Rebuild of the systems whose cell sort fits one block's LDS (n <=
-// SORT_N_MAX; at most 2 n cells, so every such system), one 1024-thread block
-// per system.
-//   PH_DECIDE  neighbor-list snapshot, displacements, which build it is
-//   PH_GRID    for grid builds: bounding box, cell grid, the whole counting
-//              sort in LDS -- cell of each bead, histogram, exclusive scan,
-//              member lists, and the rank of each bead among its cell's
-//              members by index, so the in-cell order is the index order --
-//              the cell-ordered arrays, and the occupied cells appended to the
-//              batch's home-cell list (in any order: each writes its own rows)
-// What bounds it is latency: dependent round trips and block barriers of one
-// block.  Both phases in one launch (a system's beads are loaded once) when
-// the batch is small: the chain of eleven kernels it replaced, most of them
-// with nothing to do at most rebuilds, took 64 us per rebuild of one 128-bead
-// system (a rebuild and its step 107 us; now 48).  A batch that fills the device launches the phases apart, the
-// second on the side stream beside the shell builds' filter.
 // The entries s[st .. en) below b, eight at a time (s 16-byte aligned): the
 // ranks read each cell once per member, bound by the block's one compute unit.
 // Rebuild of 5,000 beads into 32 A cells of some 230 members: 75 us one entry
@@ -398,6 +382,25 @@ __device__ __forceinline__ int count_below(const uint16_t *s, int st, int en, in
   return r + acc.x + acc.y;
 }
 
+// Rebuild of the systems whose cell sort fits one block's LDS (n <=
+// SORT_N_MAX; at most 2 n cells, so every such system), one 1024-thread block
+// per system.
+//   PH_DECIDE  neighbor-list snapshot, displacements, which build it is
+//   PH_GRID    for grid builds: bounding box, cell grid, the whole counting
+//              sort in LDS -- cell of each bead, histogram, exclusive scan,
+//              member lists, and the rank of each bead among its cell's
+//              members by index, so the in-cell order is the index order --
+//              the cell-ordered arrays, and the occupied cells appended to the
+//              batch's home-cell list (in any order: each writes its own rows)
+// What bounds it is latency: dependent round trips and block barriers of one
+// block.  Both phases in one launch (a system's beads are loaded once) when
+// the batch is small.  Run per step of one 128-bead system with lists at every
+// step, by the chain of eleven kernels it replaced (most with nothing to do at
+// most rebuilds) and by it: shell builds 46 and 18 us, grid builds 81 and 36.  A
+// batch that fills the device launches the phases apart, the second on the side
+// stream beside the shell builds' filter.  The sort's loads in flight take 128
+// registers, one block per compute unit (and eight of them spill where both
+// phases are one launch); the decision alone takes 63, two blocks.
 constexpr int SORT_THREADS = 1024;
 constexpr int PH_DECIDE = 1, PH_GRID = 2;
 
@@ -2231,7 +2234,9 @@ __global__ __launch_bounds__(STEP_THREADS) void k_shell_filter(DevPtrs p, int ks
 // beads each; one exchange of the waves' totals gives every list its place,
 // and the kept entries are written from registers.  Lane 16 q + 4 e + l takes
 // entry 16 q + 4 l + e of its pass: a row's kept entries come out in the order
-// of the item kernel.  The native lists are packed in bead order.
+// of the item kernel.  The native lists are packed in bead order.  What a lane
+// holds takes 125 registers: one block per compute unit, so two or three tiles a
+// unit go through in as many rounds.
 constexpr int FILTER_ROW_WAVES = 8, FILTER_NAT_WAVES = 4;
 constexpr int FILTER_TILE_THREADS = 64 * (FILTER_ROW_WAVES + FILTER_NAT_WAVES);
 
@@ -2991,9 +2996,9 @@ __global__ __launch_bounds__(256) void k_read(DevPtrs p, int slot, int what, flo
 // Half lists for the host (pairs i < j, by bead and row order): 16 lanes per
 // bead count the entries above the bead, one block turns the counts into
 // places, and the pairs of a window of the list are written to pinned memory.
-// Bound by the calls' round trips.  The four lists of 1,500 beads, each asked
-// for its length and then fetched: 246 us, against 910 us with the row
-// segments copied to the host and walked there.
+// Bound by the calls' round trips.  The two pair lists of 1,500 beads, each
+// asked for its length and then fetched: 105 us, against 720 with the row
+// segments copied to the host and walked there (all four lists 470 and 4,100).
 struct ListRow {
   int64_t at;   // first entry
   int cnt;

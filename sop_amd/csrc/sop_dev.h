@@ -180,9 +180,11 @@ constexpr int STEP_WAVES = 16;
 constexpr int STEP_THREADS = 64 * STEP_WAVES;
 
 // Batches of up to this many tiles per compute unit step with a block per
-// tile (k_step_tile), whatever their systems' sizes.
+// tile (k_step_tile), whatever their systems' sizes: as many as are resident
+// with 4 lanes per bead (134 registers, two five-wave blocks).
 constexpr int TILE_STEP_PER_CU = 2;
-// The tiles of systems that gather from global memory do so up to this many.
+// The tiles of systems that gather from global memory do so up to this many,
+// in two rounds then: the line lies where the item kernel catches up.
 constexpr int TILE_STEP_FAR_PER_CU = 3;
 
 // Grids of the step's launches: items staged in LDS at two blocks per compute
