@@ -5,7 +5,8 @@
  * device, its memory pools and streams; systems (replicas) live on the device
  * until removed.  An engine is driven by one host thread and is not
  * thread-safe, except that the serve loop runs an internal thread behind
- * sop_serve_submit / sop_serve_poll.
+ * sop_serve_submit / sop_serve_poll: beside it the driving thread may make any
+ * call, on the systems it added before, that is not refused while serving.
  *
  * Reference interface replaced (samchogroup/SOP):
  *   force/energy entry points  energy.h:13-24 (set_potential, clear_forces,

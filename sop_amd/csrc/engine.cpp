@@ -431,6 +431,7 @@ sop_status upload_drain(sop_engine *e, Upload *upl) {
 // Validate and upload one system, without its first lists (engine_init_lists).
 sop_status engine_add_system_nolists(sop_engine *e, const sop_system_desc *d, int64_t step_end, int32_t *slot_out,
                                      Upload *upl) {
+  const EngineLock lk(e->mu);
   hipStream_t up = upl ? upl->stream : nullptr;
   if (!d || d->n_beads < 1 || !d->xyz) return set_error(e, SOP_ERR_INVALID, "system: need n_beads >= 1 and xyz");
   const int32_t n = d->n_beads;
@@ -1668,8 +1669,12 @@ const char *sop_last_error(const sop_engine *e) { return e ? e->err.c_str() : "n
 
 sop_status sop_synchronize(sop_engine *e) {
   if (!e) return SOP_ERR_INVALID;
+  const EngineLock lk(e->mu);
   return hip_check(e, hipStreamSynchronize(e->stream), "hipStreamSynchronize");
 }
+
+// The lock of a call, which may be given no engine.
+static EngineLock call_lock(sop_engine *e) { return e ? EngineLock(e->mu) : EngineLock(); }
 
 static bool valid_sys(sop_engine *e, int32_t s) {
   return e && s >= 0 && s < (int32_t)e->sys.size() && e->sys[s].used;
@@ -1683,11 +1688,13 @@ sop_status sop_system_add(sop_engine *e, const sop_system_desc *d, int32_t *sys)
 
 sop_status sop_system_remove(sop_engine *e, int32_t sys) {
   if (!e) return SOP_ERR_INVALID;
+  const EngineLock lk(e->mu);
   HIPCK(hipStreamSynchronize(e->stream));
   return engine_remove_system(e, sys);
 }
 
 sop_status sop_system_info(sop_engine *e, int32_t sys, int32_t *n_beads, int64_t *step) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys)) return set_error(e, SOP_ERR_INVALID, "no such system");
   if (n_beads) *n_beads = e->sys[sys].n;
   if (step) *step = e->sys[sys].step;
@@ -1708,6 +1715,7 @@ static sop_status nl_scratch_for(sop_engine *e, int32_t sys) {
 }
 
 sop_status sop_update_neighbor_list(sop_engine *e, int32_t sys) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys)) return set_error(e, SOP_ERR_INVALID, "no such system");
   sop_status st = nl_scratch_for(e, sys);
   if (st) return st;
@@ -1718,6 +1726,7 @@ sop_status sop_update_neighbor_list(sop_engine *e, int32_t sys) {
 }
 
 sop_status sop_update_pair_list(sop_engine *e, int32_t sys) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys)) return set_error(e, SOP_ERR_INVALID, "no such system");
   sop_status st = engine_set_batch(e, &sys, 1);
   if (st) return st;
@@ -1736,6 +1745,7 @@ static sop_status materialize_nl(sop_engine *e, int32_t sys) {
 }
 
 sop_status sop_get_list(sop_engine *e, int32_t sys, int32_t which, int32_t *ij, int64_t cap, int64_t *n) {
+  const EngineLock lk = call_lock(e);
   static_assert(LIST_NL_ATT == SOP_LIST_NL_NATIVE && LIST_NL_REP == SOP_LIST_NL_REP &&
                     LIST_PL_ATT == SOP_LIST_PL_NATIVE && LIST_PL_REP == SOP_LIST_PL_REP, "list ids");
   if (!valid_sys(e, sys) || !n) return set_error(e, SOP_ERR_INVALID, "bad arguments");
@@ -1774,6 +1784,7 @@ sop_status sop_get_list(sop_engine *e, int32_t sys, int32_t which, int32_t *ij, 
 }
 
 sop_status sop_system_rows(sop_engine *e, int32_t sys, int32_t *capacity, int32_t *longest) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys)) return set_error(e, SOP_ERR_INVALID, "no such system");
   HIPCK(hipStreamSynchronize(e->stream));
   SysDev S;
@@ -1797,6 +1808,7 @@ sop_status sop_system_reserve_rows(sop_engine *e, int32_t sys, int32_t capacity)
 }
 
 sop_status sop_list_stats_get(sop_engine *e, int32_t sys, sop_list_stats *stt) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys) || !stt) return set_error(e, SOP_ERR_INVALID, "bad arguments");
   HIPCK(hipStreamSynchronize(e->stream));
   sop_status st = materialize_nl(e, sys);
@@ -1828,6 +1840,7 @@ sop_status sop_list_stats_get(sop_engine *e, int32_t sys, sop_list_stats *stt) {
 }
 
 sop_status sop_force_eval(sop_engine *e, int32_t sys, int32_t with_noise) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys)) return set_error(e, SOP_ERR_INVALID, "no such system");
   sop_status st = engine_set_batch(e, &sys, 1);
   if (st) return st;
@@ -1851,6 +1864,7 @@ static sop_status read_beads(sop_engine *e, int32_t sys, int what, const float *
 }
 
 sop_status sop_get_forces(sop_engine *e, int32_t sys, float *f3n) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys) || !f3n) return set_error(e, SOP_ERR_INVALID, "bad arguments");
   const float *f = nullptr;
   const sop_status st = read_beads(e, sys, READ_FORCES, &f, nullptr);
@@ -1872,6 +1886,7 @@ static sop_status eval_energy(sop_engine *e, int32_t sys, double *out) {
 }
 
 sop_status sop_energy_eval(sop_engine *e, int32_t sys, double *energies) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys) || !energies) return set_error(e, SOP_ERR_INVALID, "bad arguments");
   double o[SYSOUT_N];
   sop_status st = eval_energy(e, sys, o);
@@ -1881,6 +1896,7 @@ sop_status sop_energy_eval(sop_engine *e, int32_t sys, double *energies) {
 }
 
 sop_status sop_energy_eval_noalloc(sop_engine *e, int32_t sys, double *energies) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys) || !energies) return set_error(e, SOP_ERR_INVALID, "bad arguments");
   if (!e->scratch) return set_error(e, SOP_ERR_HIP, "sop_energy_eval_noalloc: no scratch address on this device");
   const SysHost &h = e->sys[sys];
@@ -1907,6 +1923,7 @@ sop_status sop_energy_eval_noalloc(sop_engine *e, int32_t sys, double *energies)
 }
 
 sop_status sop_observables(sop_engine *e, int32_t sys, double *Q, int32_t *contacts, double *rgsq) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys)) return set_error(e, SOP_ERR_INVALID, "no such system");
   double o[SYSOUT_N];
   sop_status st = eval_energy(e, sys, o);
@@ -1956,6 +1973,7 @@ sop_status sop_run_plain(sop_engine *e, const int32_t *sys, int32_t nsys, int64_
 }
 
 sop_status sop_get_coords(sop_engine *e, int32_t sys, float *xyz, int64_t *step) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys)) return set_error(e, SOP_ERR_INVALID, "no such system");
   const float *x = nullptr;
   const sop_status st = read_beads(e, sys, READ_COORDS, &x, step);
@@ -1965,6 +1983,7 @@ sop_status sop_get_coords(sop_engine *e, int32_t sys, float *xyz, int64_t *step)
 }
 
 sop_status sop_get_wrapped_coords(sop_engine *e, int32_t sys, float *xyz) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys) || !xyz) return set_error(e, SOP_ERR_INVALID, "bad arguments");
   const float *x = nullptr;
   const sop_status st = read_beads(e, sys, READ_COORDS, &x, nullptr);
@@ -2006,6 +2025,7 @@ static bool incr_flag(const float4 &s) {
 }
 
 sop_status sop_get_velocities(sop_engine *e, int32_t sys, float *v3n) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys) || !v3n) return set_error(e, SOP_ERR_INVALID, "bad arguments");
   const SysHost &h = e->sys[sys];
   if (h.params.dynamics != SOP_DYN_UNDERDAMPED) {
@@ -2037,6 +2057,7 @@ sop_status sop_get_velocities(sop_engine *e, int32_t sys, float *v3n) {
 }
 
 sop_status sop_get_increments(sop_engine *e, int32_t sys, float *d3n) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys) || !d3n) return set_error(e, SOP_ERR_INVALID, "bad arguments");
   const SysHost &h = e->sys[sys];
   std::vector<float4> v;
@@ -2071,6 +2092,7 @@ sop_status sop_get_increments(sop_engine *e, int32_t sys, float *d3n) {
 }
 
 sop_status sop_set_rng(sop_engine *e, int32_t sys, uint64_t seed, int64_t step) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys)) return set_error(e, SOP_ERR_INVALID, "no such system");
   if (step < 0) return set_error(e, SOP_ERR_INVALID, "step must be >= 0");
   SysDev S;
@@ -2088,6 +2110,7 @@ sop_status sop_set_rng(sop_engine *e, int32_t sys, uint64_t seed, int64_t step) 
 }
 
 sop_status sop_set_coords(sop_engine *e, int32_t sys, const float *xyz) {
+  const EngineLock lk = call_lock(e);
   if (!valid_sys(e, sys) || !xyz) return set_error(e, SOP_ERR_INVALID, "bad arguments");
   const size_t bytes = 12 * (size_t)e->sys[sys].n;
   sop_status st = engine_io(e, e->io, bytes);

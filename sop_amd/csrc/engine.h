@@ -90,6 +90,12 @@ struct sop_engine {
   bool fixed_pools = false;
   bool grow_rows = true;  // row capacities grow after runs (off while the autotuner times trials)
 
+  // Beside the serve loop the driving thread may make every call that is not
+  // refused while serving: each holds this lock, and the loop holds it wherever
+  // it uses the engine (tables and launch of a block, uploads, retirement), but
+  // not while it waits for a block
+  std::recursive_mutex mu;
+
   sopk::Pools cap;
   sopk::RangeAlloc a_beads, a_nat, a_pl, a_cells;
   int32_t nl_owner = -1;  // system whose neighbor list the scratch holds
@@ -146,6 +152,7 @@ struct sop_engine {
 
 namespace sopk {
 // engine internals shared with serve.cpp
+using EngineLock = std::unique_lock<std::recursive_mutex>;
 sop_status set_error(sop_engine *e, sop_status st, const std::string &msg);
 sop_status hip_check(sop_engine *e, hipError_t h, const char *what);
 sop_status engine_add_system(sop_engine *e, const sop_system_desc *d, int32_t *slot);

@@ -67,6 +67,7 @@ sop_status retire_and_start(sop_engine *e, sop_engine::Serve *sv, const std::vec
   // wait for the block: its last kernel reported every running job's state
   sop_status st = hip_check(e, hipStreamSynchronize(e->stream), "retire");
   if (st) return st;
+  const EngineLock lk_e(e->mu);
   std::vector<sop_engine::Job *> keep, fin;
   std::vector<int32_t> slots;
   for (sop_engine::Job *j : sv->running) {
@@ -231,6 +232,7 @@ void admit(sop_engine *e, sop_engine::Serve *sv, Upload *up, std::vector<sop_eng
 sop_status start_jobs(sop_engine *e, sop_engine::Serve *sv, const std::vector<sop_engine::Job *> &added,
                       const std::vector<int32_t> &added_slots) {
   if (added.empty()) return SOP_OK;
+  const EngineLock lk_e(e->mu);
   std::vector<sop_status> ok(added.size(), SOP_OK);
   const sop_status st = engine_init_lists(e, added_slots.data(), (int32_t)added.size(), ok.data());
   if (st != SOP_OK) return st;
@@ -272,6 +274,7 @@ void serve_loop(sop_engine *e) {
     double t2 = t0, t3 = t0;
     int64_t block_bead_steps = 0;
     if (run) {
+      const EngineLock lk_e(e->mu);
       std::vector<int32_t> slots;
       for (sop_engine::Job *j : sv->running) {
         slots.push_back(j->slot);
